@@ -420,6 +420,9 @@ __device__ __forceinline__ void force_final_ops(double acc[3], double &dte, cons
     if (h_i >= 0.99 * max_hsml) dte = 0;
 }
 
+// this workgroup's copy of a stage's counters
+__device__ __forceinline__ Counters *ctr_slot(Counters *c) { return c + (blockIdx.x & (kCtrSpread - 1)); }
+
 // wavefront-wide sum, then one atomic per wavefront
 __device__ __forceinline__ void wave_add_u64(unsigned long long *dst, unsigned long long v)
 {

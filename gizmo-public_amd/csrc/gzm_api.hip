@@ -328,15 +328,31 @@ gzm_status download_sorted(gzm_ctx *c, const double *src, double *host, int widt
 
 gzm_status reset_counters(gzm_ctx *c, int slot)
 {
-    launch_clear_counters(c->stream, c->d_ctr + slot);
+    launch_clear_counters(c->stream, c->d_ctr + slot * kCtrSpread);
     GZM_HIP(hipGetLastError());
     return GZM_OK;
 }
 
+// the sum of a stage's kCtrSpread counter copies
+void fold_counters(const Counters *part, Counters *h)
+{
+    *h = Counters{};
+    for (int k = 0; k < kCtrSpread; k++) {
+        h->interactions += part[k].interactions;
+        h->retries += part[k].retries;
+        h->exact_calls += part[k].exact_calls;
+        h->status = std::max(h->status, part[k].status);
+        h->redo_n += part[k].redo_n;
+        h->overflow_slices += part[k].overflow_slices;
+    }
+}
+
 gzm_status read_counters(gzm_ctx *c, int slot, Counters *h)
 {
-    GZM_HIP(hipMemcpyAsync(h, c->d_ctr + slot, sizeof(Counters), hipMemcpyDeviceToHost, c->stream));
+    Counters part[kCtrSpread];
+    GZM_HIP(hipMemcpyAsync(part, c->d_ctr + slot * kCtrSpread, sizeof(part), hipMemcpyDeviceToHost, c->stream));
     GZM_HIP(hipStreamSynchronize(c->stream));
+    fold_counters(part, h);
     return GZM_OK;
 }
 
@@ -543,7 +559,7 @@ gzm_status gzm_ctx_create(gzm_ctx **out, const gzm_params *params)
     c->G.G7 = (0.5 * (g - 1.0));
     c->G.G8 = (1.0 / g);
     c->G.G9 = (g - 1.0);
-    if (dev_alloc(&c->d_ctr, kCtrSlots) || dev_alloc(&c->d_count, 1) || dev_alloc(&c->d_count_heavy, 1) ||
+    if (dev_alloc(&c->d_ctr, kCtrSlots * kCtrSpread) || dev_alloc(&c->d_count, 1) || dev_alloc(&c->d_count_heavy, 1) ||
         dev_alloc(&c->d_hmax, 1)) {
         gzm_ctx_destroy(c);
         return GZM_ERR_NOMEM;
@@ -945,7 +961,7 @@ struct Plan {
 gzm_status density_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
 {
     gzm_status s;
-    Counters *ctr = c->d_ctr + kCtrDensity;
+    Counters *ctr = c->d_ctr + kCtrDensity * kCtrSpread;
     c->hmax_valid = false;
     if (!gp) {
         s = reset_counters(c, kCtrDensity);
@@ -1084,7 +1100,7 @@ gzm_status density_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
         sums_fp32 = false;
         a.edge_list = nullptr;
         a.n_edge = nullptr;
-        a.ctr = c->d_ctr + kCtrMisc;
+        a.ctr = c->d_ctr + kCtrMisc * kCtrSpread;
         if (gp) {
             const int ne = gp->edge_live.empty() ? 0 : gp->edge_live[0];
             if (ne > 0) {
@@ -1207,7 +1223,7 @@ gzm_status gradients_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
     a.pres = c->d_pres;
     a.recf = c->d_grecf;
     a.f32 = f32_geom(c);
-    a.ctr = c->d_ctr + kCtrGradients;
+    a.ctr = c->d_ctr + kCtrGradients * kCtrSpread;
     // every particle active: the gradient kernel also writes the force records
     // (the force stage then skips its pack kernel)
     const bool fuse_records = c->all_active && c->n_active == c->n;
@@ -1340,7 +1356,7 @@ gzm_status force_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
     a.redo_count = c->d_redo_count;
     a.n = c->n;
     a.f32 = f32_geom(c);
-    a.ctr = c->d_ctr + kCtrForce;
+    a.ctr = c->d_ctr + kCtrForce * kCtrSpread;
     const bool use_list = c->list_valid && c->list_version == c->active_version;
     if (use_list) {
         a.list.idx = c->d_list;
@@ -1654,7 +1670,7 @@ gzm_status gzm_run_passes(gzm_ctx *c, int32_t n_passes, gzm_pass_stats *stats)
     hipGraph_t graph = nullptr;
     GZM_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     c->capturing = true;
-    for (int k = 0; k < kCtrSlots; k++) launch_clear_counters(c->stream, c->d_ctr + k);
+    for (int k = 0; k < kCtrSlots; k++) launch_clear_counters(c->stream, c->d_ctr + k * kCtrSpread);
     for (int p = 0; p < n_passes && s == GZM_OK; p++) {
         s = restore_state(c);
         s = s ? s : density_impl(c, &gp, nullptr);
@@ -1697,8 +1713,9 @@ gzm_status gzm_run_passes(gzm_ctx *c, int32_t n_passes, gzm_pass_stats *stats)
         set_error("graph launch failed: %s", hipGetErrorString(el != hipSuccess ? el : es));
         return GZM_ERR_HIP;
     }
-    Counters h[kCtrSlots];
-    GZM_HIP(hipMemcpy(h, c->d_ctr, sizeof(h), hipMemcpyDeviceToHost));
+    Counters h[kCtrSlots], part[kCtrSlots * kCtrSpread];
+    GZM_HIP(hipMemcpy(part, c->d_ctr, sizeof(part), hipMemcpyDeviceToHost));
+    for (int k = 0; k < kCtrSlots; k++) fold_counters(part + k * kCtrSpread, h + k);
     int status = 0;
     for (int k = 0; k < kCtrSlots; k++) status = std::max(status, h[k].status);
     if (status == 6) status = GZM_ERR_BRACKET;
@@ -1796,7 +1813,7 @@ gzm_status gzm_neighbor_counts(gzm_ctx *c, int32_t mode, const int32_t *active, 
     s = compute_hmax(c);
     if (s) return s;
     launch_neighbor_counts(c->stream, c->d_boxes, c->d_box_of, c->tree, mode, na, c->d_live, c->d_posm, c->d_hsml,
-                           counts ? c->d_flags : nullptr, c->d_ctr + kCtrMisc);
+                           counts ? c->d_flags : nullptr, c->d_ctr + kCtrMisc * kCtrSpread);
     GZM_HIP(hipGetLastError());
     if (counts) GZM_HIP(hipMemcpyAsync(counts, c->d_flags, sizeof(int) * na, hipMemcpyDeviceToHost, c->stream));
     Counters h;

@@ -125,14 +125,7 @@ __global__ void flag_unconverged_kernel(const int *n_live_dev, Counters *ctr)
 
 __global__ void clear_counters_kernel(Counters *ctr)
 {
-    if (threadIdx.x == 0) {
-        ctr->interactions = 0;
-        ctr->retries = 0;
-        ctr->exact_calls = 0;
-        ctr->redo_n = 0;
-        ctr->status = 0;
-        ctr->overflow_slices = 0;
-    }
+    ctr[threadIdx.x] = Counters{};  // kCtrSpread threads
 }
 
 __global__ void map_active_kernel(int n_active, const int *active_caller, const int *inv, int *active_sorted)
@@ -257,7 +250,7 @@ __device__ __forceinline__ int density_store(const DensitySweepArgs &a, int t, i
 #pragma unroll
     for (int k = 0; k < 6; k++) a.nvt[6 * (size_t)i + k] = R.nvt[k];
     a.redo[t] = (res == 1) ? 1 : 0;
-    if (res < 0) atomicMax(&a.ctr->status, (int)6);
+    if (res < 0) atomicMax(&ctr_slot(a.ctr)->status, (int)6);
     return res;
 }
 
@@ -363,7 +356,7 @@ __global__ __launch_bounds__(MAXB, 4) void density_sweep_kernel(DensitySweepArgs
             a.pvel[3 * (size_t)i + 2] = pv[2];
         }
     });
-    wave_add_u64(&a.ctr->interactions, cnt);
+    wave_add_u64(&ctr_slot(a.ctr)->interactions, cnt);
 }
 
 // The particles that passed the candidate budget: one wavefront each, its
@@ -410,7 +403,7 @@ __global__ __launch_bounds__(kBlock) void density_heavy_kernel(DensitySweepArgs 
         S.t11 = wave_sum(S.t11); S.t12 = wave_sum(S.t12); S.t22 = wave_sum(S.t22);
         S.f0 = wave_sum(S.f0); S.f1 = wave_sum(S.f1); S.f2 = wave_sum(S.f2);
         if (MFV) { pv[0] = wave_sum(pv[0]); pv[1] = wave_sum(pv[1]); pv[2] = wave_sum(pv[2]); }
-        wave_add_u64(&a.ctr->interactions, c);
+        wave_add_u64(&ctr_slot(a.ctr)->interactions, c);
         if (lane == 0) {
             const int res = density_store(a, t, i, h, S);
             if (res == 0 && any_edge && a.edge_list) a.edge_list[atomicAdd(a.n_edge, 1)] = i;
@@ -718,10 +711,10 @@ __global__ __launch_bounds__(BS) void gradients_kernel(GradientArgs a)
         const bool over = __any(listed > a.list.cap);
         if ((threadIdx.x & 63) == 0 && t < a.n_active) {
             a.list.overflow[t >> 6] = over ? 1 : 0;
-            if (over) atomicAdd(&a.ctr->overflow_slices, 1);
+            if (over) atomicAdd(&ctr_slot(a.ctr)->overflow_slices, 1);
         }
     }
-    wave_add_u64(&a.ctr->interactions, cnt);
+    wave_add_u64(&ctr_slot(a.ctr)->interactions, cnt);
 }
 
 // ---------------------------------------------------------------------------
@@ -847,7 +840,7 @@ __global__ __launch_bounds__((USE_LIST && THREE_PHASE) ? kMaxBlock : kBlock) voi
                 a.defer.mask[t] = dmask;
                 a.defer.count[t] = n_deferred;
                 a.defer.raw[t] = 1;
-                if (status) atomicMax(&a.ctr->status, status);
+                if (status) atomicMax(&ctr_slot(a.ctr)->status, status);
                 return;
             }
             if (vmax < out_vsig) vmax = out_vsig;
@@ -864,11 +857,11 @@ __global__ __launch_bounds__((USE_LIST && THREE_PHASE) ? kMaxBlock : kBlock) voi
         a.acc[3 * (size_t)i + 2] = acc[2];
         a.dtu[i] = dte;
         a.vsig[i] = vmax;
-        if (status) atomicMax(&a.ctr->status, status);
+        if (status) atomicMax(&ctr_slot(a.ctr)->status, status);
     });
-    wave_add_u64(&a.ctr->interactions, cnt);
-    wave_add_u64(&a.ctr->retries, nretry);
-    wave_add_u64(&a.ctr->exact_calls, nexact);
+    wave_add_u64(&ctr_slot(a.ctr)->interactions, cnt);
+    wave_add_u64(&ctr_slot(a.ctr)->retries, nretry);
+    wave_add_u64(&ctr_slot(a.ctr)->exact_calls, nexact);
 }
 
 // Deferred pairs q in [q_begin, min(total, q_end)): one pair per lane, with
@@ -905,10 +898,10 @@ __global__ __launch_bounds__(kBlock) void force_deferred_kernel(ForceArgs a)
         if (a.is_active && !a.is_active[j]) {
             if (vsig > kWakeup * a.vsig_old[j]) a.wakeup[j] = 1;
         }
-        if (e) atomicMax(&a.ctr->status, e);
+        if (e) atomicMax(&ctr_slot(a.ctr)->status, e);
     });
-    wave_add_u64(&a.ctr->retries, nretry);
-    wave_add_u64(&a.ctr->exact_calls, nexact);
+    wave_add_u64(&ctr_slot(a.ctr)->retries, nretry);
+    wave_add_u64(&ctr_slot(a.ctr)->exact_calls, nexact);
 }
 
 // Add the deferred pairs of this round to the raw sums (in list order) and,
@@ -981,7 +974,7 @@ __global__ __launch_bounds__(kBlock) void neighbor_count_kernel(const BoxDesc *b
         });
         if (counts) counts[t] = (int)cnt;
     });
-    wave_add_u64(&ctr->interactions, cnt);
+    wave_add_u64(&ctr_slot(ctr)->interactions, cnt);
 }
 
 inline unsigned nblocks(long long n) { return (unsigned)((n + kBlock - 1) / kBlock); }
@@ -1033,7 +1026,7 @@ void launch_flag_unconverged(hipStream_t s, const int *n_live_dev, Counters *ctr
 }
 void launch_clear_counters(hipStream_t s, Counters *ctr)
 {
-    hipLaunchKernelGGL(clear_counters_kernel, dim3(1), dim3(64), 0, s, ctr);
+    hipLaunchKernelGGL(clear_counters_kernel, dim3(1), dim3(kCtrSpread), 0, s, ctr);
 }
 void launch_map_active(hipStream_t s, int n_active, const int *active_caller, const int *inv, int *active_sorted)
 {

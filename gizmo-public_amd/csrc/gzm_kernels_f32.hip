@@ -271,9 +271,9 @@ __global__ __launch_bounds__(MAXB) void density_sweep_f32_kernel(DensitySweepArg
 #pragma unroll
         for (int k = 0; k < 6; k++) a.nvt[6 * (size_t)i + k] = R.nvt[k];
         a.redo[t] = (res == 1) ? 1 : 0;
-        if (res < 0) atomicMax(&a.ctr->status, (int)6);
+        if (res < 0) atomicMax(&ctr_slot(a.ctr)->status, (int)6);
     });
-    wave_add_u64(&a.ctr->interactions, cnt);
+    wave_add_u64(&ctr_slot(a.ctr)->interactions, cnt);
 }
 
 // ---------------------------------------------------------------------------
@@ -500,10 +500,10 @@ __global__ __launch_bounds__(BS, 4) void gradients_f32_kernel(GradientArgs a)
         const bool over = __any(listed > a.list.cap);
         if ((threadIdx.x & 63) == 0 && t < a.n_active) {
             a.list.overflow[t >> 6] = over ? 1 : 0;
-            if (over) atomicAdd(&a.ctr->overflow_slices, 1);
+            if (over) atomicAdd(&ctr_slot(a.ctr)->overflow_slices, 1);
         }
     }
-    wave_add_u64(&a.ctr->interactions, cnt);
+    wave_add_u64(&ctr_slot(a.ctr)->interactions, cnt);
 }
 
 // ---------------------------------------------------------------------------
@@ -767,7 +767,7 @@ __global__ __launch_bounds__((USE_LIST && THREE_PHASE) ? kMaxBlock : kBlock) voi
                 a.defer.mask[t] = dmask;
                 a.defer.count[t] = n_deferred;
                 a.defer.raw[t] = 1;
-                if (status) atomicMax(&a.ctr->status, status);
+                if (status) atomicMax(&ctr_slot(a.ctr)->status, status);
                 return;
             }
             if (vmax < out_vsig) vmax = out_vsig;
@@ -786,11 +786,11 @@ __global__ __launch_bounds__((USE_LIST && THREE_PHASE) ? kMaxBlock : kBlock) voi
         a.acc[3 * (size_t)i + 2] = acc[2];
         a.dtu[i] = dte;
         a.vsig[i] = vmax;
-        if (status) atomicMax(&a.ctr->status, status);
+        if (status) atomicMax(&ctr_slot(a.ctr)->status, status);
     });
-    wave_add_u64(&a.ctr->interactions, cnt);
-    wave_add_u64(&a.ctr->retries, nretry);
-    wave_add_u64(&a.ctr->exact_calls, nexact);
+    wave_add_u64(&ctr_slot(a.ctr)->interactions, cnt);
+    wave_add_u64(&ctr_slot(a.ctr)->retries, nretry);
+    wave_add_u64(&ctr_slot(a.ctr)->exact_calls, nexact);
 }
 
 // Deferred pairs of the FP32 list kernel, one per lane: exact-solver pairs
@@ -835,10 +835,10 @@ __global__ __launch_bounds__(kBlock, 4) void force_deferred_f32_kernel(ForceArgs
             nretry += (mask & 8) ? 1 : 0;
             nexact += (mask & 4) ? 1 : 0;
         }
-        if (e) atomicMax(&a.ctr->status, e);
+        if (e) atomicMax(&ctr_slot(a.ctr)->status, e);
     });
-    wave_add_u64(&a.ctr->retries, nretry);
-    wave_add_u64(&a.ctr->exact_calls, nexact);
+    wave_add_u64(&ctr_slot(a.ctr)->retries, nretry);
+    wave_add_u64(&ctr_slot(a.ctr)->exact_calls, nexact);
 }
 
 // The gradients of each particle listed by mark_redo, again, in FP64 from the
@@ -952,7 +952,7 @@ template <bool REDO>
 __global__ __launch_bounds__(kBlock) void force_wave_fp64_kernel(ForceArgs a, const int *list, const int *count)
 {
     const int n_redo = *count;
-    if (REDO && blockIdx.x == 0 && threadIdx.x == 0 && n_redo > 0) atomicAdd(&a.ctr->redo_n, n_redo);
+    if (REDO && blockIdx.x == 0 && threadIdx.x == 0 && n_redo > 0) atomicAdd(&ctr_slot(a.ctr)->redo_n, n_redo);
     const int lane = threadIdx.x & 63;
     const int n_waves = gridDim.x * (kBlock / 64);
     unsigned long long cnt = 0, nretry = 0, nexact = 0;
@@ -1025,13 +1025,13 @@ __global__ __launch_bounds__(kBlock) void force_wave_fp64_kernel(ForceArgs a, co
             a.dtu[i] = dte;
             a.vsig[i] = vmax;
             if (REDO) a.redo_flag[i] = 0;
-            if (status) atomicMax(&a.ctr->status, status);
+            if (status) atomicMax(&ctr_slot(a.ctr)->status, status);
         }
     }
     if (!REDO) {
-        wave_add_u64(&a.ctr->interactions, cnt);
-        wave_add_u64(&a.ctr->retries, nretry);
-        wave_add_u64(&a.ctr->exact_calls, nexact);
+        wave_add_u64(&ctr_slot(a.ctr)->interactions, cnt);
+        wave_add_u64(&ctr_slot(a.ctr)->retries, nretry);
+        wave_add_u64(&ctr_slot(a.ctr)->exact_calls, nexact);
     }
 }
 

@@ -183,7 +183,7 @@ __global__ __launch_bounds__(THREE_PHASE ? kMaxBlock : kBlock) void force_mfv_ke
                     a.defer.mask[t] = dmask;
                     a.defer.count[t] = n_deferred;
                     a.defer.raw[t] = 1;
-                    if (status) atomicMax(&a.ctr->status, status);
+                    if (status) atomicMax(&ctr_slot(a.ctr)->status, status);
                     return;
                 }
                 if (vmax < out_vsig) vmax = out_vsig;
@@ -194,12 +194,12 @@ __global__ __launch_bounds__(THREE_PHASE ? kMaxBlock : kBlock) void force_mfv_ke
             }
             atomicAdd(&m.d_mass[i], dm);
             mfv_store(a, m, i, acc, dte, vmax, dtm, gw, true);
-            if (status) atomicMax(&a.ctr->status, status);
+            if (status) atomicMax(&ctr_slot(a.ctr)->status, status);
         });
     }
-    wave_add_u64(&a.ctr->interactions, cnt);
-    wave_add_u64(&a.ctr->retries, nretry);
-    wave_add_u64(&a.ctr->exact_calls, nexact);
+    wave_add_u64(&ctr_slot(a.ctr)->interactions, cnt);
+    wave_add_u64(&ctr_slot(a.ctr)->retries, nretry);
+    wave_add_u64(&ctr_slot(a.ctr)->exact_calls, nexact);
 }
 
 // Deferred MFV pairs q in [q_begin, min(total, q_end)), one per lane, with
@@ -236,10 +236,10 @@ __global__ __launch_bounds__(kBlock) void force_mfv_deferred_kernel(ForceArgs a,
         if (a.is_active && !a.is_active[j]) {
             if (vsig > kWakeup * a.vsig_old[j]) a.wakeup[j] = 1;
         }
-        if (e) atomicMax(&a.ctr->status, e);
+        if (e) atomicMax(&ctr_slot(a.ctr)->status, e);
     });
-    wave_add_u64(&a.ctr->retries, nretry);
-    wave_add_u64(&a.ctr->exact_calls, nexact);
+    wave_add_u64(&ctr_slot(a.ctr)->retries, nretry);
+    wave_add_u64(&ctr_slot(a.ctr)->exact_calls, nexact);
 }
 
 // Add the round's deferred pairs to the raw sums in list order and, for the
