@@ -32,7 +32,7 @@ HIP_FLAGS = [
     "-Wall", f"-I{INC}",
 ]
 
-HIP_SOURCES = ["csrc/gzm_api.hip", "csrc/gzm_kernels.hip", "csrc/gzm_kernels_f32.hip", "csrc/gzm_tree.hip",
+HIP_SOURCES = ["csrc/gzm_api.hip", "csrc/gzm_kernels.hip", "csrc/gzm_density.hip", "csrc/gzm_kernels_f32.hip", "csrc/gzm_tree.hip",
                "csrc/gzm_elements.hip", "csrc/gzm_mfv.hip"]
 # per-file flags after HIP_FLAGS.  The FP32-bulk kernels stay at
 # -ffp-contract=off too: fused multiply-adds gained nothing measurable there,

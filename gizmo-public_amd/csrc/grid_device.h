@@ -128,6 +128,58 @@ __device__ __forceinline__ void for_each_cell(const Grid &g, const double xs[3],
     }
 }
 
+// for_each_cell's cells in the same order, consecutive cells of a z column
+// joined where their slot ranges adjoin (the Morton order stores cells 2k and
+// 2k + 1 of a column side by side): f(full, cx, cy, cz, begin, end) with the
+// unwrapped coordinates of the first cell of the run; runs do not cross the
+// periodic boundary.  An f returning false ends the walk.
+template <typename F>
+__device__ __forceinline__ void for_each_run(const Grid &g, const double xs[3], double R, F &&f)
+{
+    int lo[3], hi[3];
+    bool full[3];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        full[a] = !(R * g.inv_s[a] < 0.5 * g.nc[a] - 2.0);
+        lo[a] = full[a] ? 0 : (int)floor((xs[a] - R) * g.inv_s[a] - 1e-6);
+        hi[a] = full[a] ? g.nc[a] - 1 : (int)floor((xs[a] + R) * g.inv_s[a] + 1e-6);
+    }
+    const double R2 = R * R * (1.0 + 1e-9);
+    for (int cx = lo[0]; cx <= hi[0]; ++cx) {
+        const int wx = (cx < 0) ? cx + g.nc[0] : ((cx >= g.nc[0]) ? cx - g.nc[0] : cx);
+        const double gx = full[0] ? 0.0 : axis_gap(xs[0], cx * g.s[0], g.s[0]);
+        const double gx2 = gx * gx;
+        if (gx2 > R2) continue;
+        for (int cy = lo[1]; cy <= hi[1]; ++cy) {
+            const int wy = (cy < 0) ? cy + g.nc[1] : ((cy >= g.nc[1]) ? cy - g.nc[1] : cy);
+            const double gy = full[1] ? 0.0 : axis_gap(xs[1], cy * g.s[1], g.s[1]);
+            const double gxy2 = gx2 + gy * gy;
+            if (gxy2 > R2) continue;
+            const int2 *column = g.range + (wx * g.nc[1] + wy) * g.nc[2];
+            int beg = 0, end = 0, first = 0;
+            // one step past the last cell hands over the last run
+            for (int cz = lo[2]; cz <= hi[2] + 1; ++cz) {
+                int2 r = make_int2(0, 0);
+                if (cz <= hi[2]) {
+                    const double gz = full[2] ? 0.0 : axis_gap(xs[2], cz * g.s[2], g.s[2]);
+                    if (gxy2 + gz * gz > R2) continue;
+                    const int wz = (cz < 0) ? cz + g.nc[2] : ((cz >= g.nc[2]) ? cz - g.nc[2] : cz);
+                    r = column[wz];
+                    if (r.x == r.y) continue;
+                    if (r.x == end && end > beg && wz > 0) {
+                        end = r.y;
+                        continue;
+                    }
+                }
+                if (end > beg && !f(full, cx, cy, first, beg, end)) return;
+                beg = r.x;
+                end = r.y;
+                first = cz;
+            }
+        }
+    }
+}
+
 // Visit every sorted slot k whose cell may hold a particle within distance R
 // of (x, y, z), periodic.
 template <typename F>
@@ -147,6 +199,17 @@ __device__ __forceinline__ void wrap_dp(const BoxInfo &box, double dp[3])
     dp[1] = wrap_axis(dp[1], box.L[1], box.half[1]);
     dp[0] = wrap_axis(dp[0], box.L[0], box.half[0]);
     dp[2] = wrap_axis(dp[2], box.L[2], box.half[2]);
+}
+
+// The same image for displacements whose nearest image is shorter than 0.45 of
+// each side (BoxInfo::narrow2), in three instructions an axis instead of about
+// ten: the multiple of L subtracted is 0 or +-L exactly, so dp rounds as in
+// wrap_dp.  (A displacement near half a side may take the other image; it is
+// longer than the caller's radius either way.)
+__device__ __forceinline__ void wrap_near(const BoxInfo &box, double dp[3])
+{
+#pragma unroll
+    for (int k = 0; k < 3; k++) dp[k] = fma(-rint(dp[k] * box.inv[k]), box.L[k], dp[k]);
 }
 
 // periodic distance from x to the interval [lo, hi] (both inside [0, L))
@@ -306,6 +369,59 @@ __device__ __forceinline__ void wave_candidates(const TreeArgs &T, const BoxDesc
             for (int k = beg + lane; k < end; k += 64) f(k);
         }, h_pair);
     }
+}
+
+// Every candidate of one particle within R of x, spread over W lanes that walk
+// the tree or the grid in step (`sub` = 0 .. W - 1): f(k) for each lane's share.
+// With budget > 0 the walk ends, returning false, once it has passed that many
+// candidates (charged a cell or bucket at a time, so alike on every lane).
+template <int W, typename F>
+__device__ __forceinline__ bool group_candidates(const TreeArgs &T, const BoxDesc &G, const double x[3], double R,
+                                                 int sub, int budget, F &&f)
+{
+    int visited = 0;
+    if (T.nodes) {
+        int node = G.root;
+        for (int steps = 2 * G.count; node != kTreeEnd && steps > 0; steps--) {
+            int beg, end;
+            if (node < 0) {
+                beg = end = -node - 1;
+                node = T.leaf_esc[beg];
+            } else {
+                const TreeNode nd = T.nodes[node];
+                const double gx = periodic_gap(x[0], nd.lo.x, nd.hi.x, G.box.L[0]);
+                const double gy = periodic_gap(x[1], nd.lo.y, nd.hi.y, G.box.L[1]);
+                const double gz = periodic_gap(x[2], nd.lo.z, nd.hi.z, G.box.L[2]);
+                const int esc = __float_as_int(nd.hi.w);
+                if (!(gx * gx + gy * gy + gz * gz <= R * R * (1.0 + 1e-9))) {
+                    node = esc;
+                    continue;
+                }
+                beg = nd.link.y;
+                end = nd.link.z;
+                if (end - beg >= W) {
+                    node = nd.link.x;
+                    continue;
+                }
+                node = esc;
+            }
+            visited += end - beg + 1;
+            if (budget && visited > budget) return false;
+            if (beg + sub <= end) f(beg + sub);
+        }
+        return true;
+    }
+    bool full[3], ok = true;
+    for_each_cell(G.grid, x, R, full, [&](int, int, int, int beg, int end) -> bool {
+        visited += end - beg;
+        if (budget && visited > budget) {
+            ok = false;
+            return false;
+        }
+        for (int k = beg + sub; k < end; k += W) f(k);
+        return true;
+    });
+    return ok;
 }
 
 // The pair-search candidates of one particle (R = max(h_i, box hsml max),

@@ -90,7 +90,8 @@ struct gzm_ctx {
     uint8_t *d_wakeup = nullptr, *d_is_active = nullptr;
     int *d_active_caller = nullptr, *d_active = nullptr, *d_live = nullptr, *d_live2 = nullptr, *d_flags = nullptr;
     int *d_count = nullptr, *d_count_heavy = nullptr;
-    int *d_heavy_list = nullptr;  // density sweeps: live positions past the candidate budget
+    int *d_heavy_list = nullptr;  // density: particles (precision 2: live positions) past the candidate budget
+    int *d_iter = nullptr;        // density: sweeps done by the particles of the lists
     // precision 2: particles whose iteration is redone in FP64 (kEdgeBand),
     // their count, and every particle's hsml at the start of the stage
     int *d_edge_list = nullptr, *d_n_edge = nullptr;
@@ -135,7 +136,6 @@ struct gzm_ctx {
     int list_overflow_slices = 0;
     uint64_t active_version = 0, list_version = 0;
     std::vector<int> last_sweep_live;  // particles of each density sweep of the last eager call
-    std::vector<int> last_edge_live;   // precision 2: particles of each FP64 redo sweep of the last eager call
     // neighbour-search tree (search = 1)
     int2 *d_t_child = nullptr, *d_t_range = nullptr;
     int *d_t_large = nullptr, *d_t_large_count = nullptr, *d_t_split = nullptr,
@@ -143,8 +143,9 @@ struct gzm_ctx {
     double4 *d_t_lo = nullptr, *d_t_hi = nullptr;
     float *d_t_wmax = nullptr;
     TreeNode *d_t_nodes = nullptr;
-    int *d_dcache_idx = nullptr, *d_dcache_n = nullptr;  // density candidate cache (tree search)
+    int *d_dcache_idx = nullptr, *d_dcache_n = nullptr;  // density candidate rows (NULL: no memory for them)
     double *d_dcache_r2 = nullptr;
+    float4 *d_posf = nullptr;  // FP32 positions (grid rows)
     int *d_brow = nullptr, *d_bcount = nullptr;          // symmetric pair rows of the gradient stage
     int *d_bwave = nullptr, *d_bwave_n = nullptr;        //   and the particles that walk for them
     bool dcache_all = false;  // every particle's candidate row built since the last upload
@@ -263,7 +264,7 @@ void free_particles(gzm_ctx *c)
     dev_free(c->d_wakeup); dev_free(c->d_is_active);
     dev_free(c->d_active_caller); dev_free(c->d_active); dev_free(c->d_live); dev_free(c->d_live2);
     dev_free(c->d_flags); dev_free(c->d_grec); dev_free(c->d_frec);
-    dev_free(c->d_heavy_list);
+    dev_free(c->d_heavy_list); dev_free(c->d_iter);
     dev_free(c->d_edge_list); dev_free(c->d_n_edge); dev_free(c->d_hsml_entry);
     dev_free(c->d_pvel); dev_free(c->d_ti); dev_free(c->d_dtmass); dev_free(c->d_dmass); dev_free(c->d_dmass0);
     dev_free(c->d_gravwork);
@@ -279,7 +280,7 @@ void free_particles(gzm_ctx *c)
     dev_free(c->d_t_split); dev_free(c->d_t_esc); dev_free(c->d_t_leaf_esc); dev_free(c->d_t_flag);
     dev_free(c->d_t_lo); dev_free(c->d_t_hi); dev_free(c->d_t_wmax); dev_free(c->d_t_nodes);
     dev_free(c->d_dcache_idx); dev_free(c->d_dcache_n); dev_free(c->d_dcache_r2);
-    dev_free(c->d_brow); dev_free(c->d_bcount); dev_free(c->d_bwave); dev_free(c->d_bwave_n);
+    dev_free(c->d_posf); dev_free(c->d_brow); dev_free(c->d_bcount); dev_free(c->d_bwave); dev_free(c->d_bwave_n);
     c->dcache_all = false;
     c->tree = TreeArgs{};
     c->defer_result_cap = 0;
@@ -344,6 +345,8 @@ void fold_counters(const Counters *part, Counters *h)
         h->status = std::max(h->status, part[k].status);
         h->redo_n += part[k].redo_n;
         h->overflow_slices += part[k].overflow_slices;
+        h->sweeps = std::max(h->sweeps, part[k].sweeps);
+        h->updates += part[k].updates;
     }
 }
 
@@ -559,7 +562,7 @@ gzm_status gzm_ctx_create(gzm_ctx **out, const gzm_params *params)
     c->G.G7 = (0.5 * (g - 1.0));
     c->G.G8 = (1.0 / g);
     c->G.G9 = (g - 1.0);
-    if (dev_alloc(&c->d_ctr, kCtrSlots * kCtrSpread) || dev_alloc(&c->d_count, 1) || dev_alloc(&c->d_count_heavy, 1) ||
+    if (dev_alloc(&c->d_ctr, kCtrSlots * kCtrSpread) || dev_alloc(&c->d_count, 3) || dev_alloc(&c->d_count_heavy, 1) ||
         dev_alloc(&c->d_hmax, 1)) {
         gzm_ctx_destroy(c);
         return GZM_ERR_NOMEM;
@@ -629,8 +632,11 @@ gzm_status setup_boxes(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const do
             B.s_f[ax] = (float)B.grid.s[ax];
             B.box.L[ax] = L[ax];
             B.box.half[ax] = 0.5 * L[ax];
+            B.box.inv[ax] = 1.0 / L[ax];
             nb *= nc;
         }
+        const double side = 0.45 * std::min(L[0], std::min(L[1], L[2]));
+        B.box.narrow2 = side * side;
         B.cell_base = (int)ncell;
         ncell += nb;
         if (ncell > ((int64_t)1 << 30)) { set_error("grids of %lld cells too large", (long long)ncell); return GZM_ERR_ARG; }
@@ -723,6 +729,7 @@ gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const 
         s = s ? s : dev_alloc(&c->d_live2, n);
         s = s ? s : dev_alloc(&c->d_flags, n);
         s = s ? s : dev_alloc(&c->d_heavy_list, n);
+        s = s ? s : dev_alloc(&c->d_iter, n);
         if (c->p.precision == 0) {
             s = s ? s : dev_alloc(&c->d_grec, n);
             s = s ? s : dev_alloc(&c->d_frec, n);
@@ -761,15 +768,21 @@ gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const 
             s = s ? s : dev_alloc(&c->d_t_lo, n);
             s = s ? s : dev_alloc(&c->d_t_hi, n);
             s = s ? s : dev_alloc(&c->d_t_nodes, n);
-            s = s ? s : dev_alloc(&c->d_dcache_idx, (size_t)n * kDensityCacheCap);
-            s = s ? s : dev_alloc(&c->d_dcache_n, n);
-            s = s ? s : dev_alloc(&c->d_dcache_r2, n);
             s = s ? s : dev_alloc(&c->d_brow, (size_t)n * kPairRowCap);
             s = s ? s : dev_alloc(&c->d_bcount, n);
             s = s ? s : dev_alloc(&c->d_bwave, n);
             s = s ? s : dev_alloc(&c->d_bwave_n, 1);
         }
         if (s) { free_particles(c); return s; }
+        if (c->p.precision != 2) {
+            // the candidate rows are an optimisation (up to 412 B per particle): a set
+            // that fills the memory without them runs without them
+            if (dev_alloc(&c->d_dcache_idx, (size_t)n * kDensityCacheCap) || dev_alloc(&c->d_dcache_n, n) ||
+                dev_alloc(&c->d_dcache_r2, n) || (c->p.search == 0 && dev_alloc(&c->d_posf, n))) {
+                (void)hipGetLastError();
+                dev_free(c->d_dcache_idx); dev_free(c->d_dcache_n); dev_free(c->d_dcache_r2); dev_free(c->d_posf);
+            }
+        }
     }
     if (c->d_redo_flag) launch_fill_int(c->stream, c->d_redo_flag, n, 0);
     gzm_status s = setup_boxes(c, v, n_boxes, box_sizes, offsets);
@@ -809,7 +822,7 @@ gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const 
         GZM_HIP(rocprim::radix_sort_pairs(c->d_temp, bytes, c->d_keys, c->d_keys_sorted, c->d_iota, c->d_perm, n, 0,
                                           key_bits, c->stream));
         launch_gather_sorted(c->stream, n, c->d_perm, st_pos, st_vel, st_mass, st_u, d_box_caller, c->d_posm,
-                             c->d_velu, c->d_inv, c->d_box_of);
+                             c->d_velu, c->d_posf, c->d_inv, c->d_box_of);
         if (!tree) launch_cell_ranges(c->stream, n, c->d_posm, c->d_boxes, c->d_box_of, c->d_range, c->ncell);
         if (c->p.precision != 0)
             launch_pack_geom_f32(c->stream, n, c->d_posm, c->d_velu, c->d_boxes, c->d_box_of, c->d_offm, c->d_velf,
@@ -861,10 +874,10 @@ gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const 
         GZM_HIP(hipGetLastError());
         c->tree.nodes = c->d_t_nodes;
         c->tree.leaf_esc = c->d_t_leaf_esc;
-        // new positions: no candidate row is valid
-        launch_fill_int(c->stream, c->d_dcache_n, n, kDensityCacheCap + 1);
-        c->dcache_all = false;
     }
+    // new positions: no candidate row is valid
+    if (c->d_dcache_n) launch_fill_int(c->stream, c->d_dcache_n, n, kDensityCacheCap + 1);
+    c->dcache_all = false;
 
     // optional state of particles that may stay inactive
     struct Opt { const double *h; double *d; int w; } opts[] = {
@@ -947,47 +960,98 @@ gzm_status restore_state(gzm_ctx *c)
     return GZM_OK;
 }
 
-// What a captured pass cannot learn on the host: the number of density
-// sweeps and whether the pair list overflowed, both taken from a probe pass
-// on the same initial state.
+// What a captured pass cannot learn on the host, taken from a probe pass on
+// the same initial state: whether the pair list overflowed, how many pairs
+// were deferred, and for precision 2 its density sweeps.
 struct Plan {
     int sweeps;
     bool overflow;
     int64_t deferred;             // exact-solver pairs deferred out of the force loop
-    std::vector<int> sweep_live;  // particles of each density sweep
-    std::vector<int> edge_live;   // precision 2: particles of each FP64 redo sweep
+    std::vector<int> sweep_live;  // precision 2: particles of each density sweep
 };
 
-gzm_status density_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
+// the arguments that every density kernel of precisions 0 and 1 reads
+DensityStageArgs density_stage_args(gzm_ctx *c)
+{
+    DensityStageArgs a;
+    memset(&a, 0, sizeof(a));
+    a.boxes = c->d_boxes;
+    a.box_of = c->d_box_of;
+    a.tree = c->tree;
+    a.hp.des_num_ngb = c->p.des_num_ngb;
+    a.hp.max_num_ngb_dev = c->p.max_num_ngb_dev;
+    a.hp.min_hsml = c->p.min_hsml;
+    a.hp.max_hsml = c->p.max_hsml;
+    a.hp.first_step = c->p.first_step;
+    a.maxiter = c->p.maxiter;
+    a.gm1 = c->G.G9;
+    a.active = c->d_active;
+    a.n_active = c->n_active;
+    a.posm = c->d_posm;
+    a.velu = c->d_velu;
+    a.posf = c->d_posf;
+    a.hsml = c->d_hsml; a.left = c->d_left; a.right = c->d_right; a.cn = c->d_cn;
+    a.num_ngb = c->d_num_ngb; a.dhsml = c->d_dhsml; a.divvel = c->d_divvel; a.rho = c->d_rho; a.pres = c->d_pres;
+    a.fce = c->d_fce; a.nvt = c->d_nvt;
+    a.pvel = (c->p.method == 1) ? c->d_pvel : nullptr;
+    a.row_idx = c->d_dcache_idx; a.row_n = c->d_dcache_n; a.row_r2 = c->d_dcache_r2;
+    a.iter = c->d_iter;
+    a.tail_list = c->d_live;
+    a.n_tail = c->d_count + 1;
+    a.far_list = c->d_heavy_list;
+    a.n_far = c->d_count + 2;
+    a.budget = c->p.density_budget == 0 ? kDensityBudget : (c->p.density_budget < 0 ? 0 : c->p.density_budget);
+    a.lanes = c->n_active <= kFewParticles ? 8 : 1;
+    a.ctr = c->d_ctr + kCtrDensity * kCtrSpread;
+    return a;
+}
+
+gzm_status density_fp64(gzm_ctx *c, bool captured)
+{
+    const DensityStageArgs a = density_stage_args(c);
+    {
+        Timed tm(c, kOther);
+        launch_density_begin(c->stream, captured ? nullptr : a.ctr, c->d_count + 1);
+    }
+    if (a.n_active > 0) {
+        {
+            Timed tm(c, kDensity);
+            if (a.row_idx) launch_density_rows(c->stream, a);
+            launch_density_stage(c->stream, a);
+        }
+        Timed tm(c, kDensityWave);
+        launch_density_tail(c->stream, a);
+    }
+    GZM_HIP(hipGetLastError());
+    if (a.row_idx && a.n_active == c->n) c->dcache_all = true;
+    return GZM_OK;
+}
+
+// Precision 2: sweeps with FP32 sums, one launch each, then the FP64 redo.
+gzm_status density_fp32(gzm_ctx *c, const Plan *gp, int *status, int *sweeps_out, int64_t *updates_out, int *n_edge_out)
 {
     gzm_status s;
     Counters *ctr = c->d_ctr + kCtrDensity * kCtrSpread;
-    c->hmax_valid = false;
     if (!gp) {
         s = reset_counters(c, kCtrDensity);
         if (s) return s;
-    }
-    const int na = c->n_active;
-    int n_live = 0;
-    // candidate cache of the FP64 tree sweeps (not with FP32 sums: their FP64
-    // redo sweeps restart the iteration of a few particles)
-    const bool dcache = c->tree.nodes && c->d_dcache_idx && c->p.precision != 2;
-    if (na > 0) {
-        {
-            Timed tm(c, kOther);
-            launch_density_init(c->stream, na, c->d_active, c->d_posm, dcache ? c->d_dcache_n : nullptr, c->d_hsml,
-                                c->d_left, c->d_right, c->p.max_hsml, c->d_flags);
-        }
-        s = compact(c, c->d_active, c->d_flags, na, c->d_live, gp ? nullptr : &n_live);
+        s = reset_counters(c, kCtrMisc);
         if (s) return s;
     }
-    const bool fp32_sums = c->p.precision == 2;
-    if (fp32_sums && na > 0) {
-        // the stage's entry hsml, from which an FP64 redo restarts, and an empty redo list
-        GZM_HIP(hipMemcpyAsync(c->d_hsml_entry, c->d_hsml, sizeof(double) * (size_t)c->n, hipMemcpyDeviceToDevice,
-                               c->stream));
-        launch_fill_int(c->stream, c->d_n_edge, 1, 0);
+    const int na = c->n_active;
+    if (na == 0) return GZM_OK;
+    int n_live = 0;
+    {
+        Timed tm(c, kOther);
+        launch_density_init(c->stream, na, c->d_active, c->d_posm, c->d_hsml, c->d_left, c->d_right, c->p.max_hsml,
+                            c->d_flags);
     }
+    s = compact(c, c->d_active, c->d_flags, na, c->d_live, gp ? nullptr : &n_live);
+    if (s) return s;
+    // the stage's entry hsml, from which an FP64 redo restarts, and an empty redo list
+    GZM_HIP(hipMemcpyAsync(c->d_hsml_entry, c->d_hsml, sizeof(double) * (size_t)c->n, hipMemcpyDeviceToDevice,
+                           c->stream));
+    launch_fill_int(c->stream, c->d_n_edge, 1, 0);
     DensitySweepArgs a;
     memset(&a, 0, sizeof(a));
     a.boxes = c->d_boxes;
@@ -1003,181 +1067,130 @@ gzm_status density_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
     a.hsml = c->d_hsml; a.left = c->d_left; a.right = c->d_right; a.cn = c->d_cn;
     a.num_ngb = c->d_num_ngb; a.dhsml = c->d_dhsml; a.divvel = c->d_divvel; a.rho = c->d_rho;
     a.fce = c->d_fce; a.nvt = c->d_nvt;
-    a.pvel = (c->p.method == 1) ? c->d_pvel : nullptr;
-    if (dcache) {
-        a.dcache_idx = c->d_dcache_idx;
-        a.dcache_n = c->d_dcache_n;
-        a.dcache_r2 = c->d_dcache_r2;
-    }
     a.redo = c->d_flags;
     a.budget = c->p.density_budget == 0 ? kDensityBudget : (c->p.density_budget < 0 ? 0 : c->p.density_budget);
     a.heavy_list = c->d_heavy_list;
     a.n_heavy = c->d_count_heavy;
+    a.edge_list = c->d_edge_list;
+    a.n_edge = c->d_n_edge;
     a.f32 = f32_geom(c);
     a.ctr = ctr;
     a.block = c->block[0];
-    if (fp32_sums) {
-        a.edge_list = c->d_edge_list;
-        a.n_edge = c->d_n_edge;
-    }
-    bool sums_fp32 = fp32_sums;  // false for the FP64 redo sweeps
-    // one sweep over up to `cap` live entries: the budgeted launch (entries
-    // past the budget are listed on the device), then one wavefront per listed
-    // entry
-    // (a sweep over at most wave_sweep_max entries gives every entry a wavefront)
-    auto sweep = [&](int cap, int expected) -> gzm_status {
+    // One sweep over up to `cap` live entries: the budgeted launch (entries past the budget are listed on the device),
+    // then one wavefront per listed entry; a sweep over at most wave_sweep_max entries gives every entry a wavefront.
+    // The list also takes the particles whose hsml step FP32 sums cannot decide, so it is worked off without a budget too.
+    auto sweep = [&](int cap, int expected) {
         if (expected <= c->wave_sweep_max) {
             Timed tm(c, kDensityWave);
             DensitySweepArgs w = a;
             w.wave_all = 1;
             launch_density_heavy(c->stream, w, expected);
-            return GZM_OK;
+            return;
         }
-        if (a.budget) launch_fill_int(c->stream, c->d_count_heavy, 1, 0);
+        launch_fill_int(c->stream, c->d_count_heavy, 1, 0);
         {
             Timed tm(c, kDensity);
-            if (sums_fp32) launch_density_sweep_f32(c->stream, a);
-            else launch_density_sweep(c->stream, a);
+            launch_density_sweep_f32(c->stream, a);
         }
-        if (a.budget) {
-            Timed tm(c, kDensityWave);
-            launch_density_heavy(c->stream, a, cap);
-        }
-        return GZM_OK;
+        Timed tm(c, kDensityWave);
+        launch_density_heavy(c->stream, a, cap);
     };
-    int iter = 0, sweeps = 0;
-    if (!gp) {
-        c->last_sweep_live.clear();
-        c->last_edge_live.clear();
-    }
-    int64_t updates = 0;
-    int status = GZM_OK;
-    int n_edge = 0;
     if (gp) {
         // captured: every sweep is sized for all active particles and reads the
         // live count from the device; the probe pass fixed the number of sweeps
-        if (na > 0) {
-            for (int sw = 0; sw < gp->sweeps; sw++) {
-                a.hp.iter = sw;
-                a.live = c->d_live;
-                a.n_live = na;
-                a.n_live_dev = c->d_count;
-                s = sweep(na, sw < (int)gp->sweep_live.size() ? gp->sweep_live[sw] : na);
-                if (s) return s;
-                s = compact(c, c->d_live, c->d_flags, na, c->d_live2, nullptr);
-                if (s) return s;
-                std::swap(c->d_live, c->d_live2);
-            }
-            launch_flag_unconverged(c->stream, c->d_count, ctr);
+        for (int sw = 0; sw < gp->sweeps; sw++) {
+            a.hp.iter = sw;
+            a.live = c->d_live;
+            a.n_live = na;
+            a.n_live_dev = c->d_count;
+            sweep(na, sw < (int)gp->sweep_live.size() ? gp->sweep_live[sw] : na);
+            s = compact(c, c->d_live, c->d_flags, na, c->d_live2, nullptr);
+            if (s) return s;
+            std::swap(c->d_live, c->d_live2);
         }
+        launch_flag_unconverged(c->stream, c->d_count, ctr);
     } else {
+        c->last_sweep_live.clear();
+        int iter = 0;
         while (n_live > 0) {
-            updates += n_live;
+            *updates_out += n_live;
             a.hp.iter = iter;
             a.live = c->d_live;
             a.n_live = n_live;
             c->last_sweep_live.push_back(n_live);
-            s = sweep(n_live, n_live);
-            if (s) return s;
+            sweep(n_live, n_live);
             GZM_HIP(hipGetLastError());
-            sweeps++;
+            ++*sweeps_out;
             int n_next = 0;
             s = compact(c, c->d_live, c->d_flags, n_live, c->d_live2, &n_next);
             if (s) return s;
             std::swap(c->d_live, c->d_live2);
             n_live = n_next;
-            if (n_live > 0) {
-                iter++;
-                if (iter > c->p.maxiter) { status = GZM_ERR_HSML_NOT_CONVERGED; break; }
-            }
+            if (n_live > 0 && ++iter > c->p.maxiter) { *status = GZM_ERR_HSML_NOT_CONVERGED; break; }
         }
     }
-    // Precision 2: the particles that converged next to a kernel edge
-    // (kEdgeBand) repeat their whole iteration with FP64 sums, from the entry
-    // hsml, so that their hsml and neighbour sets are the FP64 pass's.  Their
-    // sweeps count into the misc counter slot, not the density interactions.
-    if (fp32_sums && na > 0 && status == GZM_OK) {
-        sums_fp32 = false;
-        a.edge_list = nullptr;
-        a.n_edge = nullptr;
-        a.ctr = c->d_ctr + kCtrMisc * kCtrSpread;
-        if (gp) {
-            const int ne = gp->edge_live.empty() ? 0 : gp->edge_live[0];
-            if (ne > 0) {
-                launch_edge_reset(c->stream, ne, c->d_n_edge, c->d_edge_list, c->d_hsml_entry, c->d_hsml, c->d_left,
-                                  c->d_right);
-                GZM_HIP(hipMemcpyAsync(c->d_live, c->d_edge_list, sizeof(int) * (size_t)ne, hipMemcpyDeviceToDevice,
-                                       c->stream));
-                GZM_HIP(hipMemcpyAsync(c->d_count, c->d_n_edge, sizeof(int), hipMemcpyDeviceToDevice, c->stream));
-                for (int sw = 0; sw < (int)gp->edge_live.size(); sw++) {
-                    a.hp.iter = sw;
-                    a.live = c->d_live;
-                    a.n_live = ne;
-                    a.n_live_dev = c->d_count;
-                    s = sweep(ne, gp->edge_live[sw]);
-                    if (s) return s;
-                    s = compact(c, c->d_live, c->d_flags, ne, c->d_live2, nullptr);
-                    if (s) return s;
-                    std::swap(c->d_live, c->d_live2);
-                }
-                launch_flag_unconverged(c->stream, c->d_count, ctr);
-            }
-        } else {
-            GZM_HIP(hipMemcpyAsync(&n_edge, c->d_n_edge, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-            GZM_HIP(hipStreamSynchronize(c->stream));
-            if (n_edge > 0) {
-                s = reset_counters(c, kCtrMisc);
-                if (s) return s;
-                {
-                    Timed tm(c, kOther);
-                    launch_edge_reset(c->stream, n_edge, c->d_n_edge, c->d_edge_list, c->d_hsml_entry, c->d_hsml,
-                                      c->d_left, c->d_right);
-                }
-                GZM_HIP(hipMemcpyAsync(c->d_live, c->d_edge_list, sizeof(int) * (size_t)n_edge,
-                                       hipMemcpyDeviceToDevice, c->stream));
-                n_live = n_edge;
-                int it = 0;
-                while (n_live > 0) {
-                    a.hp.iter = it;
-                    a.live = c->d_live;
-                    a.n_live = n_live;
-                    a.n_live_dev = nullptr;
-                    c->last_edge_live.push_back(n_live);
-                    s = sweep(n_live, n_live);
-                    if (s) return s;
-                    GZM_HIP(hipGetLastError());
-                    int n_next = 0;
-                    s = compact(c, c->d_live, c->d_flags, n_live, c->d_live2, &n_next);
-                    if (s) return s;
-                    std::swap(c->d_live, c->d_live2);
-                    n_live = n_next;
-                    if (n_live > 0 && ++it > c->p.maxiter) { status = GZM_ERR_HSML_NOT_CONVERGED; break; }
-                }
-                Counters hm;
-                s = read_counters(c, kCtrMisc, &hm);
-                if (s) return s;
-                if (hm.status == 6 && status == GZM_OK) status = GZM_ERR_BRACKET;
-            }
-        }
-        a.ctr = ctr;
-    }
-    if (na > 0) {
+    {
         Timed tm(c, kOther);
-        launch_density_finalize(c->stream, na, c->d_active, c->d_posm, c->d_velu, c->d_hsml, c->d_num_ngb,
-                                c->d_rho, c->d_pres, c->G.G9, (c->p.method == 1) ? c->d_pvel : nullptr);
+        launch_density_finalize(c->stream, na, c->d_active, c->d_posm, c->d_velu, c->d_hsml, c->d_num_ngb, c->d_rho,
+                                c->d_pres, c->G.G9);
     }
+    // The particles that converged next to a kernel edge (kEdgeBand) repeat
+    // their whole iteration with FP64 sums, from the entry hsml, so that their
+    // hsml and neighbour sets are the FP64 pass's.  Their sweeps count into the
+    // misc counter slot, not the density interactions.
+    if (*status == GZM_OK) {
+        DensityStageArgs r = density_stage_args(c);
+        r.row_idx = nullptr;
+        r.row_n = nullptr;
+        r.tail_list = c->d_edge_list;
+        r.n_tail = c->d_n_edge;
+        r.ctr = c->d_ctr + kCtrMisc * kCtrSpread;
+        {
+            Timed tm(c, kOther);
+            launch_density_begin(c->stream, nullptr, c->d_count + 1);
+            launch_edge_reset(c->stream, na, c->d_n_edge, c->d_edge_list, c->d_hsml_entry, c->d_hsml, c->d_left,
+                              c->d_right, c->d_iter);
+        }
+        {
+            Timed tm(c, kDensityWave);
+            launch_density_tail(c->stream, r);
+        }
+        GZM_HIP(hipGetLastError());
+        if (!gp) {
+            GZM_HIP(hipMemcpyAsync(n_edge_out, c->d_n_edge, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+            Counters hm;
+            s = read_counters(c, kCtrMisc, &hm);
+            if (s) return s;
+            if (hm.status == 6) *status = GZM_ERR_BRACKET;
+            else if (hm.status) *status = hm.status;
+        }
+    }
+    return GZM_OK;
+}
+
+gzm_status density_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
+{
+    c->hmax_valid = false;
+    int status = GZM_OK, sweeps = 0, n_edge = 0;
+    int64_t updates = 0;
+    const bool fp32_sums = c->p.precision == 2;
+    gzm_status s = fp32_sums ? density_fp32(c, gp, &status, &sweeps, &updates, &n_edge) : density_fp64(c, gp != nullptr);
+    if (s) return s;
     GZM_HIP(hipGetLastError());
     c->have_density = true;
     c->have_gradients = false;
     c->list_valid = false;
     c->frec_fresh = false;
-    if (dcache && na == c->n) c->dcache_all = true;  // every particle went through the first sweep
     if (gp) return GZM_OK;
     Counters h;
     s = read_counters(c, kCtrDensity, &h);
     if (s) return s;
     collect_timings(c);
-    if (h.status == 6 && status == GZM_OK) status = GZM_ERR_BRACKET;
+    if (!fp32_sums) {
+        sweeps = h.sweeps;
+        updates = (int64_t)h.updates;
+    }
+    if (h.status && status == GZM_OK) status = h.status == 6 ? (int)GZM_ERR_BRACKET : h.status;
     if (stats) {
         stats->density_sweeps = sweeps;
         stats->density_interactions = (int64_t)h.interactions;
@@ -1654,8 +1667,7 @@ gzm_status gzm_run_passes(gzm_ctx *c, int32_t n_passes, gzm_pass_stats *stats)
     s = s ? s : gradients_impl(c, nullptr, &probe);
     s = s ? s : force_impl(c, nullptr, &probe);
     if (s) return s;
-    const Plan gp = {probe.density_sweeps, c->list_overflow_slices > 0, c->last_deferred, c->last_sweep_live,
-                     c->last_edge_live};
+    const Plan gp = {probe.density_sweeps, c->list_overflow_slices > 0, c->last_deferred, c->last_sweep_live};
     {
         // the captured compactions run over the whole active list
         size_t bytes = 0;

@@ -1,0 +1,504 @@
+// gzm_density.hip -- the density stage of the FP64 hsml iteration (precisions
+// 0 and 1; also the FP64 redo of precision 2) for gfx950.
+//
+// A particle's iteration reads only its own sums, so no sweep has to be a
+// launch of its own and nothing is compacted or counted on the host between
+// sweeps.  Four kernels per stage:
+//
+//   density_rows_kernel   candidates of every active particle within
+//                         kDensityCacheFactor * hsml, in walk order (a pure
+//                         distance filter over the grid or tree)
+//   density_stage_kernel  the first two sweeps over the rows, a launch each
+//                         (nearly every particle needs exactly two)
+//   density_tail_kernel   particles not converged by then, or without a usable
+//                         row: 16 lanes each, iterating to convergence
+//   density_far_kernel    particles whose walk passes the candidate budget: a
+//                         wavefront each, iterating to convergence
+//
+// The lists between them live on the device.
+//
+// 128^3 blast (2.1 M particles, 33 pairs and 1.97 sweeps each): rows 0.86, sweeps
+// 0.66 + 0.66, tail and far 0.03 ms; the launch per sweep with its walk that this
+// replaces took 2 x 1.41 ms and a host round trip per sweep.  32^3 lattice: rows
+// 0.038, sweeps 2 x 0.024 ms (2 x 0.11 ms).  Bound by the latency of the
+// candidate loads (45 % VALU busy, 500 cycles per load at 5 waves per SIMD).
+#include "grid_device.h"
+#include "gzm_internal.h"
+
+namespace gzm {
+
+namespace {
+
+constexpr int kTailLanes = 16;
+constexpr int kNoRow = kDensityCacheCap + 1;
+
+// sums of one candidate already known to lie within h (density.c:252-347).
+// MFV: also m_j W_ij v_j into pv (density.c:291-293 for r = 0, 331-334 as
+// v_i - (v_i - v_j) otherwise), the sum behind ParticleVel.
+template <bool MFV>
+__device__ __forceinline__ void density_add(const double dp[3], double r2, double m_j, const double4 &vi,
+                                            const double4 *__restrict__ velu, int j, double hinv, double hinv3,
+                                            double hinv4, DensitySums &S, double *pv)
+{
+    const double r = sqrt(r2);
+    const double u = r * hinv;
+    double wk, dwk;
+    kernel_wdw(u, hinv3, hinv4, wk, dwk);
+    S.ngb += wk;
+    S.rho += m_j * wk;
+    S.dhsml += -(3 * hinv * wk + u * dwk);
+    if (r > 0) {
+        S.t00 += wk * dp[0] * dp[0];
+        S.t01 += wk * dp[0] * dp[1];
+        S.t02 += wk * dp[0] * dp[2];
+        S.t11 += wk * dp[1] * dp[1];
+        S.t12 += wk * dp[1] * dp[2];
+        S.t22 += wk * dp[2] * dp[2];
+        S.f0 += wk * dp[0];
+        S.f1 += wk * dp[1];
+        S.f2 += wk * dp[2];
+        const double4 vj = velu[j];
+        const double dv0 = vi.x - vj.x, dv1 = vi.y - vj.y, dv2 = vi.z - vj.z;
+        if (MFV) {
+            const double mj_wk = m_j * wk;
+            pv[0] += mj_wk * (vi.x - dv0);
+            pv[1] += mj_wk * (vi.y - dv1);
+            pv[2] += mj_wk * (vi.z - dv2);
+        }
+        S.divvel -= dwk * (dp[0] * dv0 + dp[1] * dv1 + dp[2] * dv2) / r;
+    } else if (MFV) {
+        const double4 vj = velu[j];
+        const double mj_wk = m_j * wk;
+        pv[0] += mj_wk * vj.x;
+        pv[1] += mj_wk * vj.y;
+        pv[2] += mj_wk * vj.z;
+    }
+}
+
+// sum over the G lanes of one particle (every lane gets the result)
+template <int G>
+__device__ __forceinline__ double group_sum(double v)
+{
+#pragma unroll
+    for (int off = G / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    return v;
+}
+
+template <int G, bool MFV>
+__device__ __forceinline__ void group_sums(DensitySums &S, double *pv)
+{
+    S.ngb = group_sum<G>(S.ngb); S.rho = group_sum<G>(S.rho); S.dhsml = group_sum<G>(S.dhsml);
+    S.divvel = group_sum<G>(S.divvel);
+    S.t00 = group_sum<G>(S.t00); S.t01 = group_sum<G>(S.t01); S.t02 = group_sum<G>(S.t02);
+    S.t11 = group_sum<G>(S.t11); S.t12 = group_sum<G>(S.t12); S.t22 = group_sum<G>(S.t22);
+    S.f0 = group_sum<G>(S.f0); S.f1 = group_sum<G>(S.f1); S.f2 = group_sum<G>(S.f2);
+    if (MFV) {
+        pv[0] = group_sum<G>(pv[0]);
+        pv[1] = group_sum<G>(pv[1]);
+        pv[2] = group_sum<G>(pv[2]);
+    }
+}
+
+// where one particle stands in its iteration
+struct Iterate {
+    double h, left, right, cn;
+    int iter;
+};
+
+// One hsml step from the sums of sweep s.iter; true: sweep again.  On the
+// last sweep (converged, a bracket failure, or the sweep limit) `write` stores
+// the outputs with the final operations of density.c:880-1031.
+__device__ __forceinline__ bool density_step(const DensityStageArgs &a, int i, bool write, const DensitySums &S,
+                                             const double *pv, Iterate &s)
+{
+    DensityResult R;
+    HsmlParams hp = a.hp;
+    hp.iter = s.iter;
+    const int res = hsml_update(hp, S, s.h, s.left, s.right, s.cn, R);
+    s.cn = R.cn_stored;
+    s.iter++;
+    const bool again = (res == 1) && (s.iter <= a.maxiter);
+    if (again || !write) return again;
+    if (res != 0) atomicMax(&ctr_slot(a.ctr)->status, res < 0 ? 6 : 1155);
+    a.hsml[i] = s.h;
+    a.cn[i] = s.cn;
+    a.dhsml[i] = R.dhsml;
+    a.divvel[i] = R.divvel;
+    a.fce[i] = R.fce;
+#pragma unroll
+    for (int k = 0; k < 6; k++) a.nvt[6 * (size_t)i + k] = R.nvt[k];
+    const double4 vi = a.velu[i];
+    if (a.pvel) {
+        // MFV mesh motion 5 (density.c:886-894): 0.7 VelPred + 0.3 the kernel-weighted mean velocity
+        const double eps_pvel = 0.3, d_sum = R.rho_sum;
+        const double vv[3] = {vi.x, vi.y, vi.z};
+        for (int k = 0; k < 3; k++)
+            a.pvel[3 * (size_t)i + k] = (d_sum > 0) ? (1. - eps_pvel) * vv[k] + eps_pvel * pv[k] / d_sum : pv[k];
+    }
+    const double h = s.h, nn = R.num_ngb, m = a.posm[i].w;
+    double d;
+    // density.c:967-978 (MFM: own mass times the kernel number density)
+    if ((h > 0) && (nn > 0)) d = m * nn / (kNormCoeff * cube(h));
+    else if (h <= 0) d = 0;
+    else d = m / (kNormCoeff * cube(h));
+    a.rho[i] = d;
+    a.pres[i] = a.gm1 * vi.w * d;                       // eos.c:58-61
+    a.num_ngb[i] = (nn > 0) ? cbrt(nn) : 0;  // density.c:1020
+    return again;
+}
+
+// leave particle i to the next sweep, or to the kernel that works through `list`
+__device__ __forceinline__ void hand_on(const DensityStageArgs &a, int i, const Iterate &s, int *list, int *count)
+{
+    a.hsml[i] = s.h;
+    a.left[i] = s.left;
+    a.right[i] = s.right;
+    a.cn[i] = s.cn;
+    a.iter[i] = s.iter;
+    if (list) list[atomicAdd(count, 1)] = i;
+}
+
+__device__ __forceinline__ Iterate take_up(const DensityStageArgs &a, int i)
+{
+    return {a.hsml[i], a.left[i], a.right[i], a.cn[i], a.iter[i]};
+}
+
+__device__ __forceinline__ void count_sweeps(const DensityStageArgs &a, unsigned long long pairs,
+                                             unsigned long long sweeps, int max_iter)
+{
+    wave_add_u64(&ctr_slot(a.ctr)->interactions, pairs);
+    wave_add_u64(&ctr_slot(a.ctr)->updates, sweeps);
+    for (int off = 32; off > 0; off >>= 1) {
+        const int o = __shfl_xor(max_iter, off, 64);
+        max_iter = o > max_iter ? o : max_iter;
+    }
+    if ((threadIdx.x & 63) == 0 && max_iter > 0) atomicMax(&ctr_slot(a.ctr)->sweeps, max_iter);
+}
+
+// Candidate rows.  The walk tests every particle of the cells (nodes) that the
+// radius touches, some 250 for 32 neighbours; testing only distances here and
+// summing over the ~55 row entries afterwards keeps the lanes of the sums
+// together (in one loop nearly every candidate step of a wavefront runs the
+// pair body for the few lanes that have a neighbour there).  G = 1: one lane
+// per particle, entries staged in LDS and stored as whole 64-byte chunks.
+// G > 1 (few particles): G lanes share a cell, entries packed by ballot, same
+// order.
+template <bool TREE, int G>
+__global__ __launch_bounds__(kBlock) void density_rows_kernel(DensityStageArgs a)
+{
+    __shared__ int stage[G == 1 ? kListChunk * kBlock : 1];
+    const int gt = xcd_block() * kBlock + (int)threadIdx.x;
+    const int t = gt / G, sub = gt % G;
+    const bool valid = t < a.n_active;
+    for_box(a.boxes, a.box_of, valid ? a.active[t] : 0, valid, [&](const BoxDesc &B) {
+        const int i = a.active[t];
+        const double4 pi = a.posm[i];
+        if (!(pi.w > 0)) {  // density_isactive: gas with mass > 0 (density.c:85)
+            if (sub == 0) a.row_n[i] = kNoRow;
+            return;
+        }
+        double h = a.hsml[i];
+        if ((h < 0) || !isfinite(h) || (h > 0.99 * a.hp.max_hsml)) {  // density.c:484
+            h = 0.99 * a.hp.max_hsml;
+            if (sub == 0) a.hsml[i] = h;
+        }
+        const double Rc = (TREE ? kDensityCacheFactor : kDensityCacheFactorGrid) * h, Rc2 = Rc * Rc;
+        const double xs[3] = {pi.x, pi.y, pi.z};
+        constexpr int cap = kDensityCacheCap;
+        int *row = a.row_idx + (size_t)i * cap;
+        // a row past its cap is of no use, so its walk ends there; the budget
+        // bounds the walk where cells hold many more particles than neighbours
+        const int limit = a.budget ? 2 * a.budget : 0x7fffffff;
+        int m = 0, visited = 0;
+        auto append = [&](int j, bool in) {
+            if constexpr (G == 1) {
+                if (!in) return;
+                if (m < cap) {
+                    const int c = m & (kListChunk - 1);
+                    stage[c * kBlock + threadIdx.x] = j;
+                    if (c == kListChunk - 1) flush_list_chunk(stage, row + (m - c), kBlock);
+                }
+                m++;
+            } else {
+                const int first = (int)(threadIdx.x & 63) & ~(G - 1);
+                const unsigned bits = (unsigned)(__ballot(in) >> first) & ((1u << G) - 1);
+                const int k = m + __popc(bits & ((1u << sub) - 1));
+                if (in && k < cap) row[k] = j;
+                m += __popc(bits);
+            }
+        };
+        if constexpr (TREE) {
+            auto visit = [&](int j) -> bool {
+                if (++visited > limit) return false;
+                const double4 pj = a.posm[j];
+                double dp[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
+                wrap_dp(B.box, dp);
+                const double r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
+                append(j, r2 < Rc2 && pj.w > 0);
+                return m <= cap;
+            };
+            static_assert(G == 1, "the tree rows take one lane per particle");
+            tree_walk_grouped(a.tree, B, xs, Rc, visit);
+        } else {
+            // FP32 distances with a margin for their rounding (2^-24 of a side per
+            // coordinate): the row may hold a few more than the exact radius
+            // asks for, never fewer, and a candidate is one 16-byte load.
+            const float Lmax = (float)fmax(B.box.L[0], fmax(B.box.L[1], B.box.L[2]));
+            const float Rf = (float)Rc * (1 + 1e-6f) + 5e-7f * Lmax, Rf2 = Rf * Rf * (1 + 1e-6f);
+            const float4 fi = a.posf[i];
+            for_each_run(B.grid, xs, Rc, [&](const bool full[3], int cx, int cy, int cz, int beg, int end) -> bool {
+                visited += end - beg;
+                if (visited > limit) return false;
+                // the image of this cell that the walk reached is the nearest
+                // one wherever the axis is not walked whole
+                const bool whole = full[0] || full[1] || full[2];
+                const float Lx = (float)B.box.L[0], Ly = (float)B.box.L[1], Lz = (float)B.box.L[2];
+                const float ox = fi.x - (cx < 0 ? -Lx : (cx >= B.grid.nc[0] ? Lx : 0.0f));
+                const float oy = fi.y - (cy < 0 ? -Ly : (cy >= B.grid.nc[1] ? Ly : 0.0f));
+                const float oz = fi.z - (cz < 0 ? -Lz : (cz >= B.grid.nc[2] ? Lz : 0.0f));
+                auto test = [&](const float4 &pj) {
+                    float dx = ox - pj.x, dy = oy - pj.y, dz = oz - pj.z;
+                    if (whole) {
+                        dx -= Lx * rintf(dx / Lx);
+                        dy -= Ly * rintf(dy / Ly);
+                        dz -= Lz * rintf(dz / Lz);
+                    }
+                    return dx * dx + dy * dy + dz * dz < Rf2 && pj.w > 0;
+                };
+                // two candidates in flight: the walk waits on these loads
+                constexpr int U = 2;
+                for (int k = beg + sub; k - sub < end; k += U * G) {
+                    float4 p[U];
+#pragma unroll
+                    for (int c = 0; c < U; c++) p[c] = a.posf[min(k + c * G, end - 1)];
+#pragma unroll
+                    for (int c = 0; c < U; c++)
+                        if (G > 1 || c == 0 || k + c < end) append(k + c * G, k + c * G < end && test(p[c]));
+                }
+                return m <= cap;
+            });
+        }
+        if (visited > limit) m = kNoRow;
+        if (G == 1 && m < cap && (m & (kListChunk - 1)))
+            flush_list_chunk(stage, row + (m & ~(kListChunk - 1)), kBlock);
+        if (sub == 0) {
+            a.row_n[i] = m <= cap ? m : kNoRow;
+            a.row_r2[i] = Rc2;
+        }
+    });
+}
+
+// Sweep IT (0 or 1) over the rows, one launch each: nearly every particle of a
+// run needs two.  The few that need more leave after the second, so that they
+// do not hold a wavefront of finished ones.  IT is a compile-time constant
+// because it decides most of the step's branches; both sweeps in one kernel
+// spilled 119 registers (2.88 ms for the two at 2.1 M particles).  Three waves
+// per SIMD: four spill 28 to 42 registers (0.73 and 0.78 against 0.66 ms).
+template <bool MFV, int G, int IT>
+__global__ __launch_bounds__(kBlock, 3) void density_stage_kernel(DensityStageArgs a)
+{
+    const int gt = xcd_block() * kBlock + (int)threadIdx.x;
+    const int t = gt / G, sub = gt % G;
+    const bool valid = t < a.n_active;
+    unsigned long long cnt = 0, sweeps = 0;
+    int max_iter = 0;
+    for_box(a.boxes, a.box_of, valid ? a.active[t] : 0, valid, [&](const BoxDesc &B) {
+        const int i = a.active[t];
+        const double4 pi = a.posm[i];
+        if (!(pi.w > 0)) return;
+        if (IT == 1 && a.iter[i] != 1) return;  // done, or in the tail list
+        const double4 vi = a.velu[i];
+        Iterate s = {a.hsml[i], IT ? a.left[i] : 0.0, IT ? a.right[i] : 0.0, a.cn[i], IT};
+        const int n = a.row_n[i];
+        const int *row = a.row_idx + (size_t)i * kDensityCacheCap;
+        bool again = true;
+        const double h2 = s.h * s.h;
+        if (n <= kDensityCacheCap && h2 <= a.row_r2[i]) {
+            double hinv, hinv3, hinv4;
+            kernel_hinv(s.h, hinv, hinv3, hinv4);
+            DensitySums S = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+            double pv[3] = {0, 0, 0};
+            auto pair = [&](auto near, int j, const double4 &pj) {
+                double dp[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
+                if constexpr (near.value) wrap_near(B.box, dp);
+                else wrap_dp(B.box, dp);
+                const double r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
+                if (!(r2 < h2)) return;
+                cnt++;
+                density_add<MFV>(dp, r2, pj.w, vi, a.velu, j, hinv, hinv3, hinv4, S, pv);
+            };
+            auto scan = [&](auto near) {
+                if constexpr (G == 1) {
+                    // four candidates' positions in flight at a time
+                    const int4 *row4 = reinterpret_cast<const int4 *>(row);
+                    for (int k = 0; k < n; k += 4) {
+                        const int4 q = row4[k >> 2];
+                        const int j1 = k + 1 < n ? q.y : q.x, j2 = k + 2 < n ? q.z : q.x, j3 = k + 3 < n ? q.w : q.x;
+                        const double4 p0 = a.posm[q.x], p1 = a.posm[j1], p2 = a.posm[j2], p3 = a.posm[j3];
+                        pair(near, q.x, p0);
+                        if (k + 1 < n) pair(near, j1, p1);
+                        if (k + 2 < n) pair(near, j2, p2);
+                        if (k + 3 < n) pair(near, j3, p3);
+                    }
+                } else {
+                    for (int k = sub; k < n; k += G) pair(near, row[k], a.posm[row[k]]);
+                }
+            };
+            if (__all(a.row_r2[i] < B.box.narrow2)) scan(std::true_type{});
+            else scan(std::false_type{});
+            if constexpr (G > 1) group_sums<G, MFV>(S, pv);
+            if (sub == 0) sweeps++;
+            again = density_step(a, i, sub == 0, S, pv, s);
+        }
+        if (sub == 0) {
+            max_iter = s.iter;
+            if (!again) a.iter[i] = 0;
+            else if (IT == 0 && s.iter == 1) hand_on(a, i, s, nullptr, nullptr);
+            else hand_on(a, i, s, a.tail_list, a.n_tail);
+        }
+    });
+    count_sweeps(a, cnt, sweeps, max_iter);
+}
+
+// The listed particles, W lanes each, iterating to convergence: over the
+// particle's row while hsml stays inside it, else over a walk shared by the
+// lanes.  BUDGET: a walk past the candidate budget leaves the particle to
+// density_far_kernel.  A fixed grid strides over the device-side count.
+template <bool MFV, int W, bool BUDGET>
+__device__ __forceinline__ void density_iterate(const DensityStageArgs &a, const int *list, const int *count)
+{
+    const int sub = (int)threadIdx.x % W;
+    const int n_groups = (int)(gridDim.x * (kBlock / W));
+    const int n = *count;
+    unsigned long long cnt = 0, sweeps = 0;
+    int max_iter = 0;
+    for (int u = (int)(blockIdx.x * kBlock + threadIdx.x) / W; u < n; u += n_groups) {
+        const int i = list[u];
+        const BoxDesc &B = a.boxes[a.box_of[i]];
+        const double4 pi = a.posm[i];
+        const double4 vi = a.velu[i];
+        Iterate s = take_up(a, i);
+        const int n_row = a.row_n ? a.row_n[i] : kNoRow;
+        const double Rc2 = n_row <= kDensityCacheCap ? a.row_r2[i] : -1.0;
+        const double xs[3] = {pi.x, pi.y, pi.z};
+        bool again = true, far = false;
+        while (again) {
+            const double h2 = s.h * s.h;
+            double hinv, hinv3, hinv4;
+            kernel_hinv(s.h, hinv, hinv3, hinv4);
+            DensitySums S = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+            double pv[3] = {0, 0, 0};
+            unsigned long long c = 0;
+            auto pair = [&](int j) {
+                const double4 pj = a.posm[j];
+                double dp[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
+                wrap_dp(B.box, dp);
+                const double r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
+                if (!(r2 < h2 && pj.w > 0)) return;
+                c++;
+                density_add<MFV>(dp, r2, pj.w, vi, a.velu, j, hinv, hinv3, hinv4, S, pv);
+            };
+            if (h2 <= Rc2) {
+                const int *row = a.row_idx + (size_t)i * kDensityCacheCap;
+                for (int k = sub; k < n_row; k += W) pair(row[k]);
+            } else {
+                const int budget = BUDGET ? a.budget : 0;
+                if (!group_candidates<W>(a.tree, B, xs, s.h, sub, budget, pair)) {
+                    far = true;
+                    break;
+                }
+            }
+            group_sums<W, MFV>(S, pv);
+            cnt += c;
+            if (sub == 0) sweeps++;
+            again = density_step(a, i, sub == 0, S, pv, s);
+        }
+        if (sub == 0) {
+            if (far) hand_on(a, i, s, a.far_list, a.n_far);
+            max_iter = s.iter > max_iter ? s.iter : max_iter;
+        }
+    }
+    count_sweeps(a, cnt, sweeps, max_iter);
+}
+
+template <bool MFV>
+__global__ __launch_bounds__(kBlock) void density_tail_kernel(DensityStageArgs a)
+{
+    density_iterate<MFV, kTailLanes, true>(a, a.tail_list, a.n_tail);
+}
+
+template <bool MFV>
+__global__ __launch_bounds__(kBlock) void density_far_kernel(DensityStageArgs a)
+{
+    density_iterate<MFV, 64, false>(a, a.far_list, a.n_far);
+}
+
+// no rows: every active particle starts in the tail list
+__global__ void density_list_all_kernel(DensityStageArgs a)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= a.n_active) return;
+    const int i = a.active[t];
+    if (!(a.posm[i].w > 0)) return;
+    double h = a.hsml[i];
+    if ((h < 0) || !isfinite(h) || (h > 0.99 * a.hp.max_hsml)) h = 0.99 * a.hp.max_hsml;  // density.c:484
+    const Iterate s = {h, 0, 0, a.cn[i], 0};
+    hand_on(a, i, s, a.tail_list, a.n_tail);
+}
+
+inline unsigned nblocks(long long n) { return (unsigned)((n + kBlock - 1) / kBlock); }
+
+}  // namespace
+
+void launch_density_rows(hipStream_t s, const DensityStageArgs &a)
+{
+    if (a.n_active <= 0) return;
+    const dim3 block(kBlock);
+    if (a.tree.nodes)
+        hipLaunchKernelGGL((density_rows_kernel<true, 1>), dim3(nblocks(a.n_active)), block, 0, s, a);
+    else if (a.lanes == 8)
+        hipLaunchKernelGGL((density_rows_kernel<false, 8>), dim3(nblocks(8LL * a.n_active)), block, 0, s, a);
+    else
+        hipLaunchKernelGGL((density_rows_kernel<false, 1>), dim3(nblocks(a.n_active)), block, 0, s, a);
+}
+
+template <int G>
+static void launch_stage_lanes(hipStream_t s, const DensityStageArgs &a)
+{
+    const dim3 grid(nblocks((long long)G * a.n_active)), block(kBlock);
+    if (a.pvel) {
+        hipLaunchKernelGGL((density_stage_kernel<true, G, 0>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((density_stage_kernel<true, G, 1>), grid, block, 0, s, a);
+    } else {
+        hipLaunchKernelGGL((density_stage_kernel<false, G, 0>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((density_stage_kernel<false, G, 1>), grid, block, 0, s, a);
+    }
+}
+
+void launch_density_stage(hipStream_t s, const DensityStageArgs &a)
+{
+    if (a.n_active <= 0) return;
+    const dim3 block(kBlock);
+    if (!a.row_idx) {
+        hipLaunchKernelGGL(density_list_all_kernel, dim3(nblocks(a.n_active)), block, 0, s, a);
+    } else if (a.lanes == 8) {
+        launch_stage_lanes<8>(s, a);
+    } else {
+        launch_stage_lanes<1>(s, a);
+    }
+}
+
+void launch_density_tail(hipStream_t s, const DensityStageArgs &a)
+{
+    if (a.n_active <= 0) return;
+    // the count is on the device: enough workgroups to fill the chip, at most one group per particle
+    const dim3 grid(std::min(2048u, nblocks((long long)kTailLanes * a.n_active))), block(kBlock);
+    if (a.pvel) hipLaunchKernelGGL(density_tail_kernel<true>, grid, block, 0, s, a);
+    else hipLaunchKernelGGL(density_tail_kernel<false>, grid, block, 0, s, a);
+    if (!a.budget) return;
+    const dim3 far(std::min(2048u, nblocks(64LL * a.n_active)));
+    if (a.pvel) hipLaunchKernelGGL(density_far_kernel<true>, far, block, 0, s, a);
+    else hipLaunchKernelGGL(density_far_kernel<false>, far, block, 0, s, a);
+}
+
+}  // namespace gzm

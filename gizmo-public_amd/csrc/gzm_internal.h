@@ -155,20 +155,30 @@ struct alignas(128) Counters {
     int status;
     int redo_n;  // FP32 force: particles redone in FP64 (summed over stages)
     int overflow_slices;
+    int sweeps;  // density: sweeps of the particle that took most
+    unsigned long long updates;  // density: sum over particles of their sweeps
 };
 
 // candidates a density-sweep lane walks before it defers its particle to the
 // second, load-balanced launch (gzm_params.density_budget = 0)
 constexpr int kDensityBudget = 512;
 
-// Density candidate cache of the FP64 tree sweeps: the first sweep of a stage
-// walks the tree with radius kDensityCacheFactor * hsml and keeps, per
-// particle, the candidates within that radius in walk order (at most
-// kDensityCacheCap; more marks the particle uncached).  A later sweep whose
-// hsml still lies inside the radius scans that row instead of the tree: the
-// candidates within hsml come out of it in the order the walk would give.
-constexpr double kDensityCacheFactor = 1.2;
+// Candidate rows of the FP64 density sums: the particles (of mass > 0) within
+// kDensityCacheFactor times the stage's entry hsml, in walk order, at most
+// kDensityCacheCap (more: no usable row).  A sweep whose hsml lies inside the
+// radius scans the row: its neighbours come out in the order the walk gives.
+// In the grid a smaller radius: 43 instead of 55 entries a row for 32
+// neighbours (sweeps of 2.1 M particles 0.73 against 0.96 ms each), still
+// beyond the few percent by which hsml changes within a stage.
+constexpr double kDensityCacheFactor = 1.2;      // tree
+constexpr double kDensityCacheFactorGrid = 1.1;  // grid
 constexpr int kDensityCacheCap = 96;  // a multiple of 4: rows are read as int4
+
+// At most this many active particles: 8 lanes per particle in the density stage
+// instead of one, which would leave most SIMDs without a wavefront (rows + two
+// sweeps of 32^3 particles 0.086 against 0.147 ms, of 16^3 0.051 against 0.140);
+// with 61^3 one lane each is faster (0.41 against 0.68 ms).
+constexpr int kFewParticles = 65536;
 
 // Symmetric pair rows of the FP64 gradient stage (tree search, every particle
 // active).  The gradient pair set of i is {j : r_ij < h_i or r_ij < h_j}; with
@@ -204,6 +214,33 @@ constexpr int kWaveSweepMax = 4096;
 // (measured 2.3e-7 on 31.5 M particles), and FP32 r^2 carries up to 2e-6 h^2.
 constexpr double kEdgeBand = 1e-5;
 
+// The density stage of precisions 0 and 1 (gzm_density.hip)
+struct DensityStageArgs {
+    const BoxDesc *boxes;
+    const int *box_of;
+    TreeArgs tree;
+    HsmlParams hp;         // hp.iter is each particle's own
+    int maxiter;
+    double gm1;
+    const int *active;
+    int n_active;
+    const double4 *posm, *velu;
+    const float4 *posf;    // positions in FP32, w = 1 for mass > 0, else 0 (grid rows)
+    double *hsml, *left, *right, *cn;
+    double *num_ngb, *dhsml, *divvel, *rho, *pres, *fce, *nvt;  // nvt: 6 per particle
+    double *pvel;          // MFV: ParticleVel (NULL: MFM)
+    // candidate rows: kDensityCacheCap slots per particle, their number (above
+    // the cap: no row) and squared radius; NULL: no memory for rows
+    int *row_idx, *row_n;
+    double *row_r2;
+    int *iter;             // sweeps done by a particle handed on to a list
+    int *tail_list, *n_tail;
+    int *far_list, *n_far;
+    int budget;            // candidates of one walk in the tail kernel; 0: no limit
+    int lanes;             // lanes per particle of the row and stage kernels: 1 or 8
+    Counters *ctr;
+};
+
 struct DensitySweepArgs {
     const BoxDesc *boxes;  // per box
     const int *box_of;     // box of each sorted slot
@@ -216,9 +253,6 @@ struct DensitySweepArgs {
     const double4 *velu;   // vx, vy, vz, u
     double *hsml, *left, *right, *cn;
     double *num_ngb, *dhsml, *divvel, *rho, *fce, *nvt;  // nvt: 6 per particle
-    // MFV (FP64 sweeps only): the sweep's sum of m_j W_ij v_j per particle, 3
-    // per particle; the finalize turns the last one into ParticleVel.  NULL: MFM
-    double *pvel;
     int *redo;             // per live entry: 1 = sweep again
     // Load balance: a particle whose walk passes `budget` candidates (0: no
     // limit) stops and appends its live position to heavy_list (count
@@ -229,18 +263,10 @@ struct DensitySweepArgs {
     int *heavy_list;
     int *n_heavy;
     int wave_all;          // wavefront-per-particle launch over all live entries (a small sweep)
-    // Density candidate cache (tree search, FP64 sums; NULL otherwise): row
-    // dcache_idx[i * kDensityCacheCap ...] of dcache_n[i] candidates within
-    // sqrt(dcache_r2[i]) of particle i, in walk order; dcache_n[i] above the
-    // cap: no valid row (set for every active particle by the stage's init).
-    int *dcache_idx;
-    int *dcache_n;
-    double *dcache_r2;
     // FP32 density sums (precision 2): a particle that converges with a
     // candidate whose r^2 lies within kEdgeBand of h^2 is appended to
     // edge_list (count n_edge); the stage then redoes its whole iteration in
     // FP64, so that its hsml and neighbour sets are those of the FP64 pass.
-    // NULL in the FP64 kernels' own sweeps.
     int *edge_list;
     int *n_edge;
     F32Geom f32;           // FP32-bulk kernels only
@@ -366,7 +392,7 @@ void launch_cell_keys(hipStream_t s, int n, const double *pos, const BoxDesc *bo
                       uint64_t *keys, int *iota);
 void launch_gather_sorted(hipStream_t s, int n, const int *perm, const double *pos, const double *vel,
                           const double *mass, const double *u, const int *box_caller, double4 *posm,
-                          double4 *velu, int *inv, int *box_of);
+                          double4 *velu, float4 *posf, int *inv, int *box_of);
 void launch_gather_scalar(hipStream_t s, int n, const int *perm, const double *src, double *dst, int width);
 void launch_scatter_scalar(hipStream_t s, int n, const int *perm, const double *src, double *dst, int width);
 void launch_cell_ranges(hipStream_t s, int n, const double4 *posm, const BoxDesc *boxes, const int *box_of,
@@ -379,18 +405,22 @@ void launch_box_hmax(hipStream_t s, int n_boxes, BoxDesc *boxes, const double *h
 void launch_flag_unconverged(hipStream_t s, const int *n_live_dev, Counters *ctr);
 void launch_clear_counters(hipStream_t s, Counters *ctr);
 void launch_map_active(hipStream_t s, int n_active, const int *active_caller, const int *inv, int *active_sorted);
-void launch_density_init(hipStream_t s, int n_active, const int *active, const double4 *posm, int *dcache_n, double *hsml,
+// density stage of precisions 0 and 1, in this order; counts[0] and [1] (tail
+// and far list) are cleared by the first, the counter block when ctr is given
+void launch_density_begin(hipStream_t s, Counters *ctr, int *counts);
+void launch_density_rows(hipStream_t s, const DensityStageArgs &a);
+void launch_density_stage(hipStream_t s, const DensityStageArgs &a);
+void launch_density_tail(hipStream_t s, const DensityStageArgs &a);
+// precision 2: FP32 sweeps, one launch each
+void launch_density_init(hipStream_t s, int n_active, const int *active, const double4 *posm, double *hsml,
                          double *left, double *right, double max_hsml, int *live_flag);
-void launch_density_sweep(hipStream_t s, const DensitySweepArgs &a);
-// precision 2: the listed particles (count on the device) restart their hsml
-// iteration from the stage's entry hsml, with empty brackets
+// the listed particles (count on the device) restart their hsml iteration
+// from the stage's entry hsml, with empty brackets
 void launch_edge_reset(hipStream_t s, int cap, const int *n_edge, const int *edge_list, const double *hsml_entry,
-                       double *hsml, double *left, double *right);
-// pvel (MFV, else NULL): the last sweep's sums of m_j W_ij v_j become
-// ParticleVel before the density sum they are divided by is replaced
+                       double *hsml, double *left, double *right, int *iter);
 void launch_density_finalize(hipStream_t s, int n_active, const int *active, const double4 *posm,
                              const double4 *velu, const double *hsml, double *num_ngb, double *rho,
-                             double *pres, double gamma_minus_1, double *pvel);
+                             double *pres, double gamma_minus_1);
 void launch_pack_grad(hipStream_t s, int n, const double4 *posm, const double4 *velu, const double *hsml,
                       const double *rho, const double *pres, GradRec *rec);
 void launch_sym_rows(hipStream_t s, const SymRowArgs &a);
@@ -423,7 +453,7 @@ void launch_force_long_lists(hipStream_t s, const ForceArgs &a, int *list, int *
 void launch_force_deferred_f32(hipStream_t s, const ForceArgs &a, int n_pairs);
 
 // density sweep of the entries in a.heavy_list (*a.n_heavy of them), one
-// wavefront each, FP64 sums (also for the FP32-bulk sweeps)
+// wavefront each, FP64 sums (the FP32 sweeps of precision 2)
 void launch_density_heavy(hipStream_t s, const DensitySweepArgs &a, int max_entries);
 
 void launch_neighbor_counts(hipStream_t s, const BoxDesc *boxes, const int *box_of, const TreeArgs &tree, int mode,

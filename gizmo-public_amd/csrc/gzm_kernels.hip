@@ -46,13 +46,15 @@ __global__ void cell_keys_kernel(int n, const double *pos, const BoxDesc *boxes,
 
 __global__ void gather_sorted_kernel(int n, const int *perm, const double *pos, const double *vel,
                                      const double *mass, const double *u, const int *box_caller, double4 *posm,
-                                     double4 *velu, int *inv, int *box_of)
+                                     double4 *velu, float4 *posf, int *inv, int *box_of)
 {
     int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
     int i = perm[k];
     posm[k] = make_double4(pos[3 * i + 0], pos[3 * i + 1], pos[3 * i + 2], mass[i]);
     velu[k] = make_double4(vel[3 * i + 0], vel[3 * i + 1], vel[3 * i + 2], u[i]);
+    if (posf)
+        posf[k] = make_float4((float)pos[3 * i + 0], (float)pos[3 * i + 1], (float)pos[3 * i + 2], mass[i] > 0 ? 1.0f : 0.0f);
     inv[i] = k;
     box_of[k] = box_caller ? box_caller[i] : 0;
 }
@@ -128,6 +130,15 @@ __global__ void clear_counters_kernel(Counters *ctr)
     ctr[threadIdx.x] = Counters{};  // kCtrSpread threads
 }
 
+__global__ void density_begin_kernel(Counters *ctr, int *counts)
+{
+    if (threadIdx.x == 0) {
+        counts[0] = 0;
+        counts[1] = 0;
+    }
+    if (ctr) ctr[threadIdx.x] = Counters{};  // kCtrSpread threads
+}
+
 __global__ void map_active_kernel(int n_active, const int *active_caller, const int *inv, int *active_sorted)
 {
     int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -160,15 +171,15 @@ __global__ void set_flags_kernel(int n_active, const int *active, uint8_t *flags
 }
 
 // ---------------------------------------------------------------------------
-// density (density.c:252-347 pair sums + 505-850 iteration, fused)
+// density (density.c:252-347 pair sums + 505-850 iteration, fused): the parts
+// that the FP32 sweeps of precision 2 use; precisions 0 and 1 have gzm_density.hip
 // ---------------------------------------------------------------------------
-__global__ void density_init_kernel(int n_active, const int *active, const double4 *posm, int *dcache_n,
-                                    double *hsml, double *left, double *right, double max_hsml, int *live_flag)
+__global__ void density_init_kernel(int n_active, const int *active, const double4 *posm, double *hsml, double *left,
+                                    double *right, double max_hsml, int *live_flag)
 {
     int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n_active) return;
     int i = active[t];
-    if (dcache_n) dcache_n[i] = kDensityCacheCap + 1;  // no candidate row until this stage's first sweep
     int live = posm[i].w > 0;  // density_isactive: gas with mass > 0 (density.c:85)
     live_flag[t] = live;
     if (!live) return;
@@ -179,21 +190,16 @@ __global__ void density_init_kernel(int n_active, const int *active, const doubl
 }
 
 // one density pair (density.c:252-347): j's terms into S when r_ij < h_i.
-// EDGE: also set `edge` when r_ij^2 lies within kEdgeBand of h_i^2.  MFV:
-// also m_j W_ij v_j into pv (density.c:291-293 for r = 0, 331-334 as
-// v_i - (v_i - v_j) otherwise), the sum behind ParticleVel.
-template <bool EDGE = false, bool MFV = false>
+// Also sets `edge` when r_ij^2 lies within kEdgeBand of h_i^2.
 __device__ __forceinline__ bool density_pair(const BoxDesc &G, const double4 &pi, const double4 &vi,
                                              const DensitySweepArgs &a, int j, double h2, double hinv,
-                                             double hinv3, double hinv4, DensitySums &S, bool *edge = nullptr,
-                                             double *pv = nullptr, double *r2_out = nullptr)
+                                             double hinv3, double hinv4, DensitySums &S, bool &edge)
 {
     const double4 pj = a.posm[j];
     double dp[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
     wrap_dp(G.box, dp);
     const double r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
-    if (r2_out) *r2_out = r2;
-    if (EDGE && pj.w > 0 && fabs(r2 - h2) <= kEdgeBand * h2) *edge = true;
+    if (pj.w > 0 && fabs(r2 - h2) <= kEdgeBand * h2) edge = true;
     if (!(r2 < h2 && pj.w > 0)) return false;
     const double r = sqrt(r2);
     const double u = r * hinv;
@@ -214,19 +220,7 @@ __device__ __forceinline__ bool density_pair(const BoxDesc &G, const double4 &pi
         S.f2 += wk * dp[2];
         const double4 vj = a.velu[j];
         const double dv0 = vi.x - vj.x, dv1 = vi.y - vj.y, dv2 = vi.z - vj.z;
-        if (MFV) {
-            const double mj_wk = pj.w * wk;
-            pv[0] += mj_wk * (vi.x - dv0);
-            pv[1] += mj_wk * (vi.y - dv1);
-            pv[2] += mj_wk * (vi.z - dv2);
-        }
         S.divvel -= dwk * (dp[0] * dv0 + dp[1] * dv1 + dp[2] * dv2) / r;
-    } else if (MFV) {
-        const double4 vj = a.velu[j];
-        const double mj_wk = pj.w * wk;
-        pv[0] += mj_wk * vj.x;
-        pv[1] += mj_wk * vj.y;
-        pv[2] += mj_wk * vj.z;
     }
     return true;
 }
@@ -254,117 +248,11 @@ __device__ __forceinline__ int density_store(const DensitySweepArgs &a, int t, i
     return res;
 }
 
-// 4 waves per SIMD: fits 128 VGPRs without spills, and the extra wave hides
-// the candidate loads (sweeps 10 % faster than at the compiler's 146 VGPRs)
-template <bool TREE, int MAXB, bool MFV = false>
-__global__ __launch_bounds__(MAXB, 4) void density_sweep_kernel(DensitySweepArgs a)
-{
-    const int t = xcd_block() * (int)blockDim.x + threadIdx.x;
-    const int n_live = a.n_live_dev ? *a.n_live_dev : a.n_live;
-    const bool valid = t < n_live;
-    if (!valid && a.n_live_dev && t < a.n_live) a.redo[t] = 0;  // captured pass: clear up to the capacity
-    unsigned long long cnt = 0;
-    for_box(a.boxes, a.box_of, valid ? a.live[t] : 0, valid, [&](const BoxDesc &G) {
-        const int i = a.live[t];
-        const double4 pi = a.posm[i];
-        const double4 vi = a.velu[i];
-        const double h = a.hsml[i];
-        double hinv, hinv3, hinv4;
-        kernel_hinv(h, hinv, hinv3, hinv4);
-        const double h2 = h * h;
-        DensitySums S = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-        double pv[3] = {0, 0, 0};
-        const double xs[3] = {pi.x, pi.y, pi.z};
-        const int budget = a.budget;
-        int visited = 0;
-        bool heavy = false;
-        unsigned long long lane_cnt = 0;
-        auto pair = [&](int j) {
-            if (density_pair<false, MFV>(G, pi, vi, a, j, h2, hinv, hinv3, hinv4, S, nullptr, pv)) lane_cnt++;
-        };
-        if (TREE) {
-            const int cap = kDensityCacheCap;
-            int *row = a.dcache_idx ? a.dcache_idx + (size_t)i * cap : nullptr;
-            const int n_row = (row && a.hp.iter > 0) ? a.dcache_n[i] : cap + 1;
-            if (n_row <= cap && h2 <= a.dcache_r2[i]) {
-                // every candidate within h is in the row, in walk order
-                const int4 *row4 = reinterpret_cast<const int4 *>(row);
-                for (int k = 0; k < n_row; k += 4) {
-                    const int4 q = row4[k >> 2];
-                    pair(q.x);
-                    if (k + 1 < n_row) pair(q.y);
-                    if (k + 2 < n_row) pair(q.z);
-                    if (k + 3 < n_row) pair(q.w);
-                }
-            } else if (row && a.hp.iter == 0) {
-                // first sweep: walk the cache radius, keep its candidates (the
-                // candidate budget doubles with the wider radius)
-                const double Rc = kDensityCacheFactor * h, Rc2 = Rc * Rc;
-                int m = 0;
-                tree_walk_grouped(a.tree, G, xs, Rc, [&](int j) -> bool {
-                    if (budget && ++visited > 2 * budget) {
-                        heavy = true;
-                        return false;
-                    }
-                    double r2;
-                    if (density_pair<false, MFV>(G, pi, vi, a, j, h2, hinv, hinv3, hinv4, S, nullptr, pv, &r2))
-                        lane_cnt++;
-                    if (r2 < Rc2) {
-                        if (m < cap) row[m] = j;
-                        m++;
-                    }
-                    return true;
-                });
-                a.dcache_n[i] = heavy ? cap + 1 : m;
-                a.dcache_r2[i] = Rc2;
-            } else if (row && budget) {
-                // a later sweep without a usable row: one wavefront for this
-                // particle's walk, so that it does not hold a wavefront of row scans
-                heavy = true;
-            } else {
-                tree_walk_grouped(a.tree, G, xs, h, [&](int j) -> bool {
-                    if (budget && ++visited > budget) {
-                        heavy = true;
-                        return false;
-                    }
-                    pair(j);
-                    return true;
-                });
-            }
-        } else {
-            // the budget is charged a cell at a time, outside the candidate loop
-            bool full[3];
-            for_each_cell(G.grid, xs, h, full, [&](int, int, int, int beg, int end) -> bool {
-                visited += end - beg;
-                if (budget && visited > budget) {
-                    heavy = true;
-                    return false;
-                }
-                for (int j = beg; j < end; ++j) pair(j);
-                return true;
-            });
-        }
-        if (heavy) {  // left to density_heavy_kernel
-            a.heavy_list[atomicAdd(a.n_heavy, 1)] = t;
-            return;
-        }
-        cnt += lane_cnt;
-        density_store(a, t, i, h, S);
-        if (MFV) {
-            a.pvel[3 * (size_t)i + 0] = pv[0];
-            a.pvel[3 * (size_t)i + 1] = pv[1];
-            a.pvel[3 * (size_t)i + 2] = pv[2];
-        }
-    });
-    wave_add_u64(&ctr_slot(a.ctr)->interactions, cnt);
-}
-
 // The particles that passed the candidate budget: one wavefront each, its
 // lanes sharing the walk (wave_candidates); the sums are reduced across the
 // wavefront (another summation order than a single lane's, FP64 throughout).
 // A fixed grid strides over the list, so the launch is sized independently of
 // the (device-side) count.
-template <bool MFV = false>
 __global__ __launch_bounds__(kBlock) void density_heavy_kernel(DensitySweepArgs a)
 {
     const int lane = threadIdx.x & 63;
@@ -385,16 +273,11 @@ __global__ __launch_bounds__(kBlock) void density_heavy_kernel(DensitySweepArgs 
         kernel_hinv(h, hinv, hinv3, hinv4);
         const double h2 = h * h;
         DensitySums S = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-        double pv[3] = {0, 0, 0};
         const double xs[3] = {pi.x, pi.y, pi.z};
         unsigned long long c = 0;
         bool edge = false;
         wave_candidates(a.tree, G, xs, h, lane, [&](int j) {
-            if (a.edge_list) {
-                if (density_pair<true>(G, pi, vi, a, j, h2, hinv, hinv3, hinv4, S, &edge)) c++;
-            } else {
-                if (density_pair<false, MFV>(G, pi, vi, a, j, h2, hinv, hinv3, hinv4, S, nullptr, pv)) c++;
-            }
+            if (density_pair(G, pi, vi, a, j, h2, hinv, hinv3, hinv4, S, edge)) c++;
         });
         const bool any_edge = __any(edge);
         S.ngb = wave_sum(S.ngb); S.rho = wave_sum(S.rho); S.dhsml = wave_sum(S.dhsml);
@@ -402,22 +285,16 @@ __global__ __launch_bounds__(kBlock) void density_heavy_kernel(DensitySweepArgs 
         S.t00 = wave_sum(S.t00); S.t01 = wave_sum(S.t01); S.t02 = wave_sum(S.t02);
         S.t11 = wave_sum(S.t11); S.t12 = wave_sum(S.t12); S.t22 = wave_sum(S.t22);
         S.f0 = wave_sum(S.f0); S.f1 = wave_sum(S.f1); S.f2 = wave_sum(S.f2);
-        if (MFV) { pv[0] = wave_sum(pv[0]); pv[1] = wave_sum(pv[1]); pv[2] = wave_sum(pv[2]); }
         wave_add_u64(&ctr_slot(a.ctr)->interactions, c);
         if (lane == 0) {
             const int res = density_store(a, t, i, h, S);
-            if (res == 0 && any_edge && a.edge_list) a.edge_list[atomicAdd(a.n_edge, 1)] = i;
-            if (MFV) {
-                a.pvel[3 * (size_t)i + 0] = pv[0];
-                a.pvel[3 * (size_t)i + 1] = pv[1];
-                a.pvel[3 * (size_t)i + 2] = pv[2];
-            }
+            if (res == 0 && any_edge) a.edge_list[atomicAdd(a.n_edge, 1)] = i;
         }
     }
 }
 
 __global__ void edge_reset_kernel(int cap, const int *n_edge, const int *edge_list, const double *hsml_entry,
-                                  double *hsml, double *left, double *right)
+                                  double *hsml, double *left, double *right, int *iter)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= cap || t >= *n_edge) return;
@@ -425,34 +302,25 @@ __global__ void edge_reset_kernel(int cap, const int *n_edge, const int *edge_li
     hsml[i] = hsml_entry[i];
     left[i] = 0;
     right[i] = 0;
+    iter[i] = 0;
 }
 
 __global__ void density_finalize_kernel(int n_active, const int *active, const double4 *posm, const double4 *velu,
-                                        const double *hsml, double *num_ngb, double *rho, double *pres, double gm1,
-                                        double *pvel)
+                                        const double *hsml, double *num_ngb, double *rho, double *pres, double gm1)
 {
     int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n_active) return;
     int i = active[t];
     double m = posm[i].w;
     if (!(m > 0)) return;
-    if (pvel && rho[i] > 0) {
-        // MFV mesh motion 5 (density.c:886-894): 0.7 VelPred + 0.3 the kernel-weighted
-        // mean velocity, over the density sum the last sweep left in rho
-        const double4 v = velu[i];
-        const double eps_pvel = 0.3, d_sum = rho[i];
-        const double vv[3] = {v.x, v.y, v.z};
-        for (int k = 0; k < 3; k++)
-            pvel[3 * (size_t)i + k] = (1. - eps_pvel) * vv[k] + eps_pvel * pvel[3 * (size_t)i + k] / d_sum;
-    }
     double h = hsml[i], nn = num_ngb[i], d;
     // density.c:967-978 (MFM: own mass times the kernel number density)
-    if ((h > 0) && (nn > 0)) d = m * nn / (kNormCoeff * pow(h, 3.0));
+    if ((h > 0) && (nn > 0)) d = m * nn / (kNormCoeff * cube(h));
     else if (h <= 0) d = 0;
-    else d = m / (kNormCoeff * pow(h, 3.0));
+    else d = m / (kNormCoeff * cube(h));
     rho[i] = d;
     pres[i] = gm1 * velu[i].w * d;  // eos.c:58-61
-    num_ngb[i] = (nn > 0) ? pow(nn, 1. / 3.) : 0;  // density.c:1020
+    num_ngb[i] = (nn > 0) ? cbrt(nn) : 0;  // density.c:1020
 }
 
 // ---------------------------------------------------------------------------
@@ -993,11 +861,11 @@ void launch_cell_keys(hipStream_t s, int n, const double *pos, const BoxDesc *bo
 }
 void launch_gather_sorted(hipStream_t s, int n, const int *perm, const double *pos, const double *vel,
                           const double *mass, const double *u, const int *box_caller, double4 *posm,
-                          double4 *velu, int *inv, int *box_of)
+                          double4 *velu, float4 *posf, int *inv, int *box_of)
 {
     if (n > 0)
         hipLaunchKernelGGL(gather_sorted_kernel, dim3(nblocks(n)), dim3(kBlock), 0, s, n, perm, pos, vel, mass, u, box_caller,
-                           posm, velu, inv, box_of);
+                           posm, velu, posf, inv, box_of);
 }
 void launch_gather_scalar(hipStream_t s, int n, const int *perm, const double *src, double *dst, int width)
 {
@@ -1033,42 +901,29 @@ void launch_map_active(hipStream_t s, int n_active, const int *active_caller, co
     if ((n_active) > 0) hipLaunchKernelGGL(map_active_kernel, dim3(nblocks(n_active)), dim3(kBlock), 0, s, n_active, active_caller, inv,
                        active_sorted);
 }
-void launch_density_init(hipStream_t s, int n_active, const int *active, const double4 *posm, int *dcache_n, double *hsml,
-                         double *left, double *right, double max_hsml, int *live_flag)
+void launch_density_begin(hipStream_t s, Counters *ctr, int *counts)
+{
+    hipLaunchKernelGGL(density_begin_kernel, dim3(1), dim3(kCtrSpread), 0, s, ctr, counts);
+}
+void launch_density_init(hipStream_t s, int n_active, const int *active, const double4 *posm, double *hsml, double *left,
+                         double *right, double max_hsml, int *live_flag)
 {
     if ((n_active) > 0) hipLaunchKernelGGL(density_init_kernel, dim3(nblocks(n_active)), dim3(kBlock), 0, s, n_active, active, posm,
-                       dcache_n, hsml, left, right, max_hsml, live_flag);
-}
-void launch_density_sweep(hipStream_t s, const DensitySweepArgs &a)
-{
-    if (a.n_live <= 0) return;
-    // workgroups of 512 take their own instantiation: the bound shapes the register allocation
-    const int b = a.block;
-    const dim3 grid(nblocks(a.n_live, b)), block(b);
-    if (a.pvel) {  // MFV: one instantiation per search, 256-thread workgroups
-        if (a.tree.nodes) hipLaunchKernelGGL((density_sweep_kernel<true, kBlock, true>), dim3(nblocks(a.n_live)), dim3(kBlock), 0, s, a);
-        else hipLaunchKernelGGL((density_sweep_kernel<false, kBlock, true>), dim3(nblocks(a.n_live)), dim3(kBlock), 0, s, a);
-    } else if (b > kBlock) {
-        if (a.tree.nodes) hipLaunchKernelGGL((density_sweep_kernel<true, kMaxBlock>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((density_sweep_kernel<false, kMaxBlock>), grid, block, 0, s, a);
-    } else {
-        if (a.tree.nodes) hipLaunchKernelGGL((density_sweep_kernel<true, kBlock>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((density_sweep_kernel<false, kBlock>), grid, block, 0, s, a);
-    }
+                       hsml, left, right, max_hsml, live_flag);
 }
 void launch_edge_reset(hipStream_t s, int cap, const int *n_edge, const int *edge_list, const double *hsml_entry,
-                       double *hsml, double *left, double *right)
+                       double *hsml, double *left, double *right, int *iter)
 {
     if (cap > 0)
         hipLaunchKernelGGL(edge_reset_kernel, dim3(nblocks(cap)), dim3(kBlock), 0, s, cap, n_edge, edge_list,
-                           hsml_entry, hsml, left, right);
+                           hsml_entry, hsml, left, right, iter);
 }
 void launch_density_finalize(hipStream_t s, int n_active, const int *active, const double4 *posm,
                              const double4 *velu, const double *hsml, double *num_ngb, double *rho, double *pres,
-                             double gm1, double *pvel)
+                             double gm1)
 {
     if ((n_active) > 0) hipLaunchKernelGGL(density_finalize_kernel, dim3(nblocks(n_active)), dim3(kBlock), 0, s, n_active, active, posm,
-                       velu, hsml, num_ngb, rho, pres, gm1, pvel);
+                       velu, hsml, num_ngb, rho, pres, gm1);
 }
 void launch_pack_grad(hipStream_t s, int n, const double4 *posm, const double4 *velu, const double *hsml,
                       const double *rho, const double *pres, GradRec *rec)
@@ -1168,8 +1023,7 @@ void launch_density_heavy(hipStream_t s, const DensitySweepArgs &a, int max_entr
     // up to 2048 workgroups of 4 wavefronts stride over the entries
     const long long blocks = ((long long)max_entries + 3) / 4;
     const dim3 grid((unsigned)(blocks < 2048 ? blocks : 2048));
-    if (a.pvel) hipLaunchKernelGGL(density_heavy_kernel<true>, grid, dim3(kBlock), 0, s, a);
-    else hipLaunchKernelGGL(density_heavy_kernel<false>, grid, dim3(kBlock), 0, s, a);
+    hipLaunchKernelGGL(density_heavy_kernel, grid, dim3(kBlock), 0, s, a);
 }
 
 namespace {

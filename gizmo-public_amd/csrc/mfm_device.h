@@ -58,7 +58,19 @@ struct GammaConsts {
 struct BoxInfo {
     double L[3];
     double half[3];
+    double inv[3];  // 1 / L
+    double narrow2; // (0.45 of the shortest side)^2: displacements below it have one image near the origin
 };
+
+// h^3 to the last bit but for rare ties: the rounding errors of both products
+// are carried along (pow(h, 3.0), which the reference calls, costs a few
+// hundred instructions on the GPU).  Where the product overflows, it stands.
+__device__ __forceinline__ double cube(double h)
+{
+    const double p = h * h, q = p * h;
+    const double e = fma(h, h, -p), f = fma(p, h, -q);
+    return isfinite(q) ? q + fma(e, h, f) : q;
+}
 
 // ---------------------------------------------------------------------------
 // cubic-spline kernel (kernel.h:182-197, 225-242, 373-374)
@@ -196,7 +208,7 @@ __device__ inline void hsml_prepare(const HsmlParams &P, const DensitySums &S, d
     if (NumNgb > 0) {
         Dhsml *= h / (3 * NumNgb);
         DivVel /= NumNgb;
-        NumNgb *= kNormCoeff * pow(h, 3.0);
+        NumNgb *= kNormCoeff * cube(h);
     } else {
         NumNgb = Dhsml = DivVel = 0;
     }
@@ -206,9 +218,9 @@ __device__ inline void hsml_prepare(const HsmlParams &P, const DensitySums &S, d
     // NV_T inversion with diagonal preconditioning, face-closure error
     double ConditionNumber;
     {
-        double V_i = kNormCoeff * pow(h, 3.0) / NumNgb;
+        double V_i = kNormCoeff * cube(h) / NumNgb;
         double dx_i = sqrt(V_i * (S.t00 + S.t11 + S.t22));
-        double norm = pow(h, -1.0);
+        double norm = 1.0 / h;
         double a = S.t00 / norm, b = S.t01 / norm, c = S.t02 / norm;
         double d = S.t11 / norm, e = S.t12 / norm, f = S.t22 / norm;
         const double cn_thresh = 10. * kCondDanger;
@@ -235,7 +247,7 @@ __device__ inline void hsml_prepare(const HsmlParams &P, const DensitySums &S, d
             for (int k2 = 0; k2 < 3; k2++) o += 2. * V_i * row[k1][k2] * fin[k2];
             leak += fabs(o) / 3;
         }
-        R.fce = leak / (2. * 3 * pow(dx_i, 2.0));
+        R.fce = leak / (2. * 3 * (dx_i * dx_i));
     }
 
     // neighbour-number target (density.c:565-595)
@@ -321,7 +333,7 @@ __device__ inline int hsml_step(const HsmlParams &P, const HsmlStep &X, double &
                 } else {
                     if (h > Right) h = Right;
                     if (h < Left) h = Left;
-                    h = pow(h * Left * Right, 1.0 / 3.0);
+                    h = cbrt(h * Left * Right);
                 }
             } else {
                 if (Right == 0 && Left == 0) { cn_out = cn_stored; return -1; }

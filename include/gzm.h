@@ -81,17 +81,17 @@ typedef struct gzm_params {
     int32_t search;         /* neighbour search: 0 = cell grid (default); 1 = tree over
                                Morton-sorted particles with per-node hsml maxima, for
                                strongly clustered sets */
-    int32_t density_budget; /* candidates a density-sweep thread tests before its particle
-                               is deferred to a second launch over such particles only
+    int32_t density_budget; /* candidates a density walk tests before its particle
+                               is deferred to a launch that gives it a wavefront
                                (load balance where a few hsml jump far in one iteration):
                                0 = default (512), < 0 = no limit; results do not depend
                                on it */
     int32_t block_size[3];  /* threads per workgroup of the per-particle loop kernels of
-                               [0] the density sweeps, [1] the gradient loop, [2] the force
+                               [0] the density sweeps of precision 2, [1] the gradient loop, [2] the force
                                loop: 64, 128, 256 or 512 (the force loop's grid-scanning
                                fallbacks stay at 256); 0 = 256.  Results do not depend on
                                it */
-    int32_t wave_sweep_max; /* a density sweep over at most this many particles gives each
+    int32_t wave_sweep_max; /* precision 2: a density sweep over at most this many particles gives each
                                one a wavefront whose lanes share its walk: 0 = default
                                (4096), < 0 = never.  Sums then run in another order (lane
                                partial sums), within the parity bar */
@@ -173,7 +173,7 @@ typedef struct gzm_pass_stats {
 /* Per-kernel device time (HIP events on the context stream), accumulated
  * since the last gzm_timing_reset. */
 typedef struct gzm_timing {
-    double density_ms;   int64_t density_launches;  /* density sweeps, one thread per particle */
+    double density_ms;   int64_t density_launches;  /* density candidate rows and sweeps over them (precision 2: sweeps) */
     double gradients_ms; int64_t gradients_launches;
     double force_ms;     int64_t force_launches;
     double other_ms;     int64_t other_launches;   /* grid build, packing, finalize */
@@ -181,9 +181,8 @@ typedef struct gzm_timing {
     int64_t graph_passes;                          /* passes inside those graphs */
     double force_deferred_ms; int64_t force_deferred_launches;  /* exact-solver pairs deferred
                                                    out of the force loop, their scan and finish */
-    double density_wave_ms; int64_t density_wave_launches;  /* density sweeps run one wavefront
-                                                   per particle: the particles past the candidate
-                                                   budget, and sweeps of few particles */
+    double density_wave_ms; int64_t density_wave_launches;  /* the particles left over by them: late
+                                                   sweeps, walks past the candidate budget */
 } gzm_timing;
 
 typedef struct gzm_ctx gzm_ctx;
