@@ -477,6 +477,63 @@ __device__ __forceinline__ void wave_pair_candidates(const TreeArgs &T, const Bo
     }
 }
 
+// sum over the G lanes of one particle (every lane gets the result)
+template <int G>
+__device__ __forceinline__ double group_sum(double v)
+{
+#pragma unroll
+    for (int off = G / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    return v;
+}
+
+template <int G>
+__device__ __forceinline__ double group_max(double v)
+{
+#pragma unroll
+    for (int off = G / 2; off > 0; off >>= 1) {
+        const double o = __shfl_xor(v, off, 64);
+        v = (o > v) ? o : v;
+    }
+    return v;
+}
+
+template <int G>
+__device__ __forceinline__ double group_min(double v)
+{
+#pragma unroll
+    for (int off = G / 2; off > 0; off >>= 1) {
+        const double o = __shfl_xor(v, off, 64);
+        v = (o < v) ? o : v;
+    }
+    return v;
+}
+
+// Whether the candidate row of radius^2 r2 around x holds the whole pair set
+// {j : r < h_i or r < h_j}: no particle beyond the radius has an hsml that
+// reaches x.  The box's largest hsml answers for most sets; else the cells in
+// its reach do, each by its own largest.
+__device__ __forceinline__ bool row_holds_pairs(const BoxDesc &B, const double x[3], double h_i, double r2)
+{
+    if (!(h_i * h_i <= r2)) return false;
+    if (B.hmax * B.hmax <= r2) return true;
+    const Grid &g = B.grid;
+    bool full[3], holds = true;
+    for_each_cell(g, x, B.hmax, full, [&](int cx, int cy, int cz, int beg, int end) -> bool {
+        if (beg == end) return true;
+        const int wx = (cx < 0) ? cx + g.nc[0] : ((cx >= g.nc[0]) ? cx - g.nc[0] : cx);
+        const int wy = (cy < 0) ? cy + g.nc[1] : ((cy >= g.nc[1]) ? cy - g.nc[1] : cy);
+        const int wz = (cz < 0) ? cz + g.nc[2] : ((cz >= g.nc[2]) ? cz - g.nc[2] : cz);
+        const double hm = g.hmax[(wx * g.nc[1] + wy) * g.nc[2] + wz], hm2 = hm * hm * (1.0 + 1e-9);
+        if (hm2 <= r2) return true;
+        const double gx = full[0] ? 0.0 : axis_gap(x[0], cx * g.s[0], g.s[0]);
+        const double gy = full[1] ? 0.0 : axis_gap(x[1], cy * g.s[1], g.s[1]);
+        const double gz = full[2] ? 0.0 : axis_gap(x[2], cz * g.s[2], g.s[2]);
+        holds = gx * gx + gy * gy + gz * gz > hm2;
+        return holds;
+    });
+    return holds;
+}
+
 __device__ __forceinline__ double wave_sum(double v)
 {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
@@ -559,15 +616,97 @@ __device__ __forceinline__ void minmax_check(T x, T &mn, T &mx)
     mx = gt ? x : mx;
 }
 
-// One lane's staged list chunk (column threadIdx.x of `stage`, rows `stride`
-// ints apart: the workgroup size) -> 64 bytes of its row.
-__device__ __forceinline__ void flush_list_chunk(const int *stage, int *dst, int stride)
+// LDS of one wavefront for index rows: kListChunk entries per lane, entry c of
+// lane l at [c * 64 + l], so that same-c accesses hit distinct banks.
+constexpr int kWaveChunk = kListChunk * 64;
+
+__device__ __forceinline__ int *wave_chunk(int *lds) { return lds + (threadIdx.x >> 6) * kWaveChunk; }
+
+// One lane's staged chunk -> 64 bytes of its row.
+__device__ __forceinline__ void flush_list_chunk(const int *chunk, int *dst)
 {
+    const int *c = chunk + (threadIdx.x & 63);
     int4 *d = reinterpret_cast<int4 *>(dst);
 #pragma unroll
     for (int q = 0; q < kListChunk / 4; q++)
-        d[q] = make_int4(stage[(4 * q + 0) * stride + threadIdx.x], stage[(4 * q + 1) * stride + threadIdx.x],
-                         stage[(4 * q + 2) * stride + threadIdx.x], stage[(4 * q + 3) * stride + threadIdx.x]);
+        d[q] = make_int4(c[(4 * q + 0) * 64], c[(4 * q + 1) * 64], c[(4 * q + 2) * 64], c[(4 * q + 3) * 64]);
+}
+
+// 64 bytes of a lane's row -> its chunk.  Read entry by entry as the loop goes,
+// the row's line is out of the 32 KB L1 again before the next entry (64 rows of
+// a wavefront are 64 lines).
+__device__ __forceinline__ void load_list_chunk(int *chunk, const int *src)
+{
+    int *c = chunk + (threadIdx.x & 63);
+    const int4 *q4 = reinterpret_cast<const int4 *>(src);
+#pragma unroll
+    for (int q = 0; q < kListChunk / 4; q++) {
+        const int4 v = q4[q];
+        c[(4 * q + 0) * 64] = v.x;
+        c[(4 * q + 1) * 64] = v.y;
+        c[(4 * q + 2) * 64] = v.z;
+        c[(4 * q + 3) * 64] = v.w;
+    }
+}
+
+// f(entry) for the n entries of a lane's row, in order, through its chunk
+// (a row's memory is whole chunks).
+template <typename F>
+__device__ __forceinline__ void for_row(int *chunk, const int *row, int n, F &&f)
+{
+    const int *c = chunk + (threadIdx.x & 63);
+    for (int k = 0; k < n; k += kListChunk) {
+        load_list_chunk(chunk, row + k);
+        const int m = min(kListChunk, n - k);
+        for (int e = 0; e < m; e++) f(c[e * 64]);
+    }
+}
+
+// f(entry a, entry b, whether b counts) two at a time, for loads in flight
+template <typename F>
+__device__ __forceinline__ void for_row_pairs(int *chunk, const int *row, int n, F &&f)
+{
+    const int *c = chunk + (threadIdx.x & 63);
+    for (int k = 0; k < n; k += kListChunk) {
+        load_list_chunk(chunk, row + k);
+        const int m = min(kListChunk, n - k);
+        for (int e = 0; e < m; e += 2) {
+            const bool second = e + 1 < m;
+            const int j = c[e * 64];
+            f(j, second ? c[(e + 1) * 64] : j, second);
+        }
+    }
+}
+
+// Store N 8-byte words of each lane's record i (stride in words, from base)
+// through the wavefront's LDS (1024 ints): eight lanes write 64 adjacent bytes of
+// one record.  A lane's own stores of a record go out as one request per lane
+// and 8 or 16 bytes (2,364 requests per wavefront of the gradient kernel).
+// Called by all 64 lanes; `valid` lanes store.
+template <int N>
+__device__ __forceinline__ void wave_store_records(int *lds, double *base, size_t stride, int i, bool valid,
+                                                   const double (&w)[N])
+{
+    double *buf = reinterpret_cast<double *>(lds);
+    const int lane = threadIdx.x & 63, word = lane & 7;
+#pragma unroll
+    for (int p = 0; p < N; p += 8) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int c = 0; c < 8; c++)
+            if (p + c < N) buf[lane * 8 + (c ^ word)] = w[p + c];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int it = 0; it < 8; it++) {
+            const int l = it * 8 + (lane >> 3);  // whose record
+            const int il = __shfl(i, l, 64);
+            const bool ok = __shfl((int)valid, l, 64) != 0;
+            const double v = buf[l * 8 + (word ^ (l & 7))];
+            if (ok && p + word < N) base[(size_t)il * stride + p + word] = v;
+        }
+    }
 }
 
 }  // namespace gzm

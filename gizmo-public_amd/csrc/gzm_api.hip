@@ -101,11 +101,13 @@ struct gzm_ctx {
     double *d_pvel = nullptr, *d_ti = nullptr, *d_dtmass = nullptr, *d_dmass = nullptr, *d_dmass0 = nullptr,
            *d_gravwork = nullptr;
     double *d_hmax = nullptr;
+    double4 *d_gxh = nullptr;
     GradRec *d_grec = nullptr;
     ForceRec *d_frec = nullptr;
     // FP32-bulk records (precision 1 and 2)
     float4 *d_offm = nullptr, *d_velf = nullptr;
     uint32_t *d_cellc = nullptr;
+    float4 *d_gxhf = nullptr;
     GradRecF *d_grecf = nullptr;
     ForceRecF *d_frecf = nullptr;
     int *d_redo_flag = nullptr, *d_redo_list = nullptr, *d_redo_count = nullptr;  // FP32 force: FP64 redo
@@ -126,7 +128,6 @@ struct gzm_ctx {
     int64_t last_deferred = 0;     // deferred pairs of the last force call
     // pair list written by the gradient kernel, read by the force kernel
     int *d_list = nullptr, *d_list_count = nullptr;
-    uint8_t *d_list_over = nullptr;
     size_t list_entries = 0;
     int list_cap = 64;
     int block[3] = {kBlock, kBlock, kBlock};  // workgroup size of the density, gradient and force loops
@@ -263,15 +264,15 @@ void free_particles(gzm_ctx *c)
     dev_free(c->d_nvt); dev_free(c->d_fce); dev_free(c->d_grad); dev_free(c->d_acc); dev_free(c->d_dtu);
     dev_free(c->d_wakeup); dev_free(c->d_is_active);
     dev_free(c->d_active_caller); dev_free(c->d_active); dev_free(c->d_live); dev_free(c->d_live2);
-    dev_free(c->d_flags); dev_free(c->d_grec); dev_free(c->d_frec);
+    dev_free(c->d_flags); dev_free(c->d_gxh); dev_free(c->d_grec); dev_free(c->d_frec);
     dev_free(c->d_heavy_list); dev_free(c->d_iter);
     dev_free(c->d_edge_list); dev_free(c->d_n_edge); dev_free(c->d_hsml_entry);
     dev_free(c->d_pvel); dev_free(c->d_ti); dev_free(c->d_dtmass); dev_free(c->d_dmass); dev_free(c->d_dmass0);
     dev_free(c->d_gravwork);
-    dev_free(c->d_offm); dev_free(c->d_velf); dev_free(c->d_cellc); dev_free(c->d_grecf); dev_free(c->d_frecf);
+    dev_free(c->d_offm); dev_free(c->d_velf); dev_free(c->d_cellc); dev_free(c->d_gxhf); dev_free(c->d_grecf); dev_free(c->d_frecf);
     dev_free(c->d_redo_flag); dev_free(c->d_redo_list); dev_free(c->d_redo_count);
     dev_free(c->d_long_list); dev_free(c->d_long_count);
-    dev_free(c->d_list); dev_free(c->d_list_count); dev_free(c->d_list_over);
+    dev_free(c->d_list); dev_free(c->d_list_count);
     dev_free(c->d_box_of);
     dev_free(c->d_defer_mask); dev_free(c->d_defer_count); dev_free(c->d_defer_off); dev_free(c->d_defer_total);
     dev_free(c->d_defer_raw); dev_free(c->d_defer_result); dev_free(c->d_defer_pair);
@@ -433,11 +434,10 @@ gzm_status ensure_list(gzm_ctx *c)
     size_t slices = ((size_t)c->n_active + 63) / 64;
     size_t entries = slices * (size_t)c->list_cap * 64;
     if (entries <= c->list_entries && c->d_list_count) return GZM_OK;
-    dev_free(c->d_list); dev_free(c->d_list_count); dev_free(c->d_list_over);
+    dev_free(c->d_list); dev_free(c->d_list_count);
     c->list_entries = 0;
     gzm_status s = dev_alloc(&c->d_list, entries);
     s = s ? s : dev_alloc(&c->d_list_count, (size_t)c->n + 64);
-    s = s ? s : dev_alloc(&c->d_list_over, slices + 1);
     if (s) return s;
     c->list_entries = entries;
     return GZM_OK;
@@ -731,12 +731,14 @@ gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const 
         s = s ? s : dev_alloc(&c->d_heavy_list, n);
         s = s ? s : dev_alloc(&c->d_iter, n);
         if (c->p.precision == 0) {
+            s = s ? s : dev_alloc(&c->d_gxh, n);
             s = s ? s : dev_alloc(&c->d_grec, n);
             s = s ? s : dev_alloc(&c->d_frec, n);
         } else {
             s = s ? s : dev_alloc(&c->d_offm, n);
             s = s ? s : dev_alloc(&c->d_velf, n);
             s = s ? s : dev_alloc(&c->d_cellc, n);
+            s = s ? s : dev_alloc(&c->d_gxhf, n);
             s = s ? s : dev_alloc(&c->d_grecf, n);
             s = s ? s : dev_alloc(&c->d_frecf, n);
             s = s ? s : dev_alloc(&c->d_redo_flag, n);
@@ -1214,9 +1216,11 @@ gzm_status gradients_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
     {
         Timed tm(c, kOther);
         if (c->p.precision != 0)
-            launch_pack_grad_f32(c->stream, c->n, c->d_offm, c->d_velf, c->d_hsml, c->d_rho, c->d_pres, c->d_grecf);
+            launch_pack_grad_f32(c->stream, c->n, c->d_offm, c->d_velf, c->d_hsml, c->d_rho, c->d_pres, c->d_gxhf,
+                                 c->d_grecf);
         else
-            launch_pack_grad(c->stream, c->n, c->d_posm, c->d_velu, c->d_hsml, c->d_rho, c->d_pres, c->d_grec);
+            launch_pack_grad(c->stream, c->n, c->d_posm, c->d_velu, c->d_hsml, c->d_rho, c->d_pres, c->d_gxh,
+                             c->d_grec);
     }
     GradientArgs a;
     memset(&a, 0, sizeof(a));
@@ -1226,6 +1230,7 @@ gzm_status gradients_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
     a.tree = c->tree;
     a.active = c->d_active;
     a.n_active = c->n_active;
+    a.xh = c->d_gxh;
     a.rec = c->d_grec;
     a.nvt = c->d_nvt;
     a.cn = c->d_cn;
@@ -1234,6 +1239,7 @@ gzm_status gradients_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
     a.hsml = c->d_hsml;
     a.rho = c->d_rho;
     a.pres = c->d_pres;
+    a.xhf = c->d_gxhf;
     a.recf = c->d_grecf;
     a.f32 = f32_geom(c);
     a.ctr = c->d_ctr + kCtrGradients * kCtrSpread;
@@ -1256,7 +1262,6 @@ gzm_status gradients_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
         if (s) return s;
         a.list.idx = c->d_list;
         a.list.count = c->d_list_count;
-        a.list.overflow = c->d_list_over;
         a.list.cap = c->list_cap;
     }
     // symmetric pair rows instead of the pair walk (tree search, FP64 density
@@ -1286,7 +1291,12 @@ gzm_status gradients_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
         a.dcache_r2 = c->d_dcache_r2;
         a.brow = c->d_brow;
         a.bcount = c->d_bcount;
+    } else if (!c->tree.nodes && c->d_dcache_idx) {
+        a.dcache_idx = c->d_dcache_idx;
+        a.dcache_n = c->d_dcache_n;
+        a.dcache_r2 = c->d_dcache_r2;
     }
+    a.lanes = (!c->tree.nodes && c->n_active <= kFewParticles) ? 8 : 1;
     if (c->n_active > 0) {
         Timed tm(c, kGradients);
         if (c->p.precision != 0) launch_gradients_f32(c->stream, a);
@@ -1374,7 +1384,6 @@ gzm_status force_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
     if (use_list) {
         a.list.idx = c->d_list;
         a.list.count = c->d_list_count;
-        a.list.overflow = c->d_list_over;
         a.list.cap = c->list_cap;
     }
     const bool mfv = c->p.method == 1;
@@ -1388,6 +1397,7 @@ gzm_status force_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
         m.d_mass = c->d_dmass;
         m.grav_work = c->d_gravwork;
     }
+    a.lanes = c->n_active <= kFewParticles ? 8 : 1;
     // exact-solver pairs leave the list loop for a kernel of their own (lists of <= 64)
     const bool three_phase = use_list && c->list_cap <= 64 && c->n_active > 0;
     if (three_phase) {

@@ -75,15 +75,6 @@ __device__ __forceinline__ void density_add(const double dp[3], double r2, doubl
     }
 }
 
-// sum over the G lanes of one particle (every lane gets the result)
-template <int G>
-__device__ __forceinline__ double group_sum(double v)
-{
-#pragma unroll
-    for (int off = G / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
 template <int G, bool MFV>
 __device__ __forceinline__ void group_sums(DensitySums &S, double *pv)
 {
@@ -125,8 +116,9 @@ __device__ __forceinline__ bool density_step(const DensityStageArgs &a, int i, b
     a.dhsml[i] = R.dhsml;
     a.divvel[i] = R.divvel;
     a.fce[i] = R.fce;
+    double2 *t2 = reinterpret_cast<double2 *>(a.nvt + 6 * (size_t)i);
 #pragma unroll
-    for (int k = 0; k < 6; k++) a.nvt[6 * (size_t)i + k] = R.nvt[k];
+    for (int k = 0; k < 3; k++) t2[k] = make_double2(R.nvt[2 * k], R.nvt[2 * k + 1]);
     const double4 vi = a.velu[i];
     if (a.pvel) {
         // MFV mesh motion 5 (density.c:886-894): 0.7 VelPred + 0.3 the kernel-weighted mean velocity
@@ -186,7 +178,8 @@ __device__ __forceinline__ void count_sweeps(const DensityStageArgs &a, unsigned
 template <bool TREE, int G>
 __global__ __launch_bounds__(kBlock) void density_rows_kernel(DensityStageArgs a)
 {
-    __shared__ int stage[G == 1 ? kListChunk * kBlock : 1];
+    __shared__ __align__(16) int lds[G == 1 ? kListChunk * kBlock : 1];
+    int *stage = wave_chunk(lds);
     const int gt = xcd_block() * kBlock + (int)threadIdx.x;
     const int t = gt / G, sub = gt % G;
     const bool valid = t < a.n_active;
@@ -215,8 +208,8 @@ __global__ __launch_bounds__(kBlock) void density_rows_kernel(DensityStageArgs a
                 if (!in) return;
                 if (m < cap) {
                     const int c = m & (kListChunk - 1);
-                    stage[c * kBlock + threadIdx.x] = j;
-                    if (c == kListChunk - 1) flush_list_chunk(stage, row + (m - c), kBlock);
+                    stage[c * 64 + (threadIdx.x & 63)] = j;
+                    if (c == kListChunk - 1) flush_list_chunk(stage, row + (m - c));
                 }
                 m++;
             } else {
@@ -280,7 +273,7 @@ __global__ __launch_bounds__(kBlock) void density_rows_kernel(DensityStageArgs a
         }
         if (visited > limit) m = kNoRow;
         if (G == 1 && m < cap && (m & (kListChunk - 1)))
-            flush_list_chunk(stage, row + (m & ~(kListChunk - 1)), kBlock);
+            flush_list_chunk(stage, row + (m & ~(kListChunk - 1)));
         if (sub == 0) {
             a.row_n[i] = m <= cap ? m : kNoRow;
             a.row_r2[i] = Rc2;
@@ -300,6 +293,8 @@ __global__ __launch_bounds__(kBlock, 3) void density_stage_kernel(DensityStageAr
     const int gt = xcd_block() * kBlock + (int)threadIdx.x;
     const int t = gt / G, sub = gt % G;
     const bool valid = t < a.n_active;
+    __shared__ __align__(16) int lds[G == 1 ? kListChunk * kBlock : 1];
+    int *chunk = wave_chunk(lds);
     unsigned long long cnt = 0, sweeps = 0;
     int max_iter = 0;
     for_box(a.boxes, a.box_of, valid ? a.active[t] : 0, valid, [&](const BoxDesc &B) {
@@ -329,17 +324,11 @@ __global__ __launch_bounds__(kBlock, 3) void density_stage_kernel(DensityStageAr
             };
             auto scan = [&](auto near) {
                 if constexpr (G == 1) {
-                    // four candidates' positions in flight at a time
-                    const int4 *row4 = reinterpret_cast<const int4 *>(row);
-                    for (int k = 0; k < n; k += 4) {
-                        const int4 q = row4[k >> 2];
-                        const int j1 = k + 1 < n ? q.y : q.x, j2 = k + 2 < n ? q.z : q.x, j3 = k + 3 < n ? q.w : q.x;
-                        const double4 p0 = a.posm[q.x], p1 = a.posm[j1], p2 = a.posm[j2], p3 = a.posm[j3];
-                        pair(near, q.x, p0);
-                        if (k + 1 < n) pair(near, j1, p1);
-                        if (k + 2 < n) pair(near, j2, p2);
-                        if (k + 3 < n) pair(near, j3, p3);
-                    }
+                    for_row_pairs(chunk, row, n, [&](int j0, int j1, bool second) {
+                        const double4 p0 = a.posm[j0], p1 = a.posm[j1];
+                        pair(near, j0, p0);
+                        if (second) pair(near, j1, p1);
+                    });
                 } else {
                     for (int k = sub; k < n; k += G) pair(near, row[k], a.posm[row[k]]);
                 }

@@ -94,9 +94,10 @@ __device__ __forceinline__ void unpack_side(const ForceRec &r, PairSide<double> 
     S.gv[6] = r.g3.x; S.gv[7] = r.g3.y; S.gv[8] = r.g3.z;
 }
 
-// Per-particle record read by the gradient loop for the neighbour j.
-struct alignas(32) GradRec {
-    double4 xh;    // x, y, z, hsml
+// Read by the gradient loop for the neighbour j: position and hsml of every
+// candidate (double4, four to a cache line), the rest of each neighbour in one
+// half line.
+struct alignas(64) GradRec {
     double4 vr;    // vx, vy, vz, rho
     double2 pm;    // P, m
 };
@@ -114,13 +115,13 @@ struct F32Geom {
     const uint32_t *cellc;     // cx | cy << 10 | cz << 20 (cell within the particle's box)
 };
 
-// Per-particle record of the FP32 gradient loop (48 bytes).  rho and P are
+// Per-particle record of the FP32 gradient loop (32 bytes, beside a float4 of
+// offset x, y, z and hsml, which every candidate is tested with).  rho and P are
 // split into a high FP32 word and the FP32 rounding of the remainder, so that
 // a pair difference (hi_j - hi_i) + (lo_j - lo_i) is the FP64 difference to
 // FP32 rounding of the difference itself, not of the values: neighbour
 // densities and pressures agree to many digits in smooth flow.
-struct alignas(16) GradRecF {
-    float4 xh;     // off x, y, z, hsml
+struct alignas(32) GradRecF {
     float4 vr;     // vx, vy, vz, rho (high word)
     float4 pm;     // P (high word), m, rho and P low words
 };
@@ -277,14 +278,12 @@ struct DensitySweepArgs {
 // Pair list: row t (entry t of the active list) holds the force-loop pair
 // set of that particle in scan order, idx[t * cap + k]; cap is a multiple of
 // 16 so each row is a whole number of 64-byte chunks.  A particle with more
-// than `cap` pairs (count > cap) is left to the scanning fallback; the 64
-// consecutive entries of the active list that one wavefront handles form a
-// slice, flagged when it holds such a particle (the fallback kernel runs
-// only when some slice is flagged).
+// than `cap` pairs (count > cap) is left to the scanning fallback, which runs
+// only when some wavefront of the gradient kernel counted such a particle
+// (Counters::overflow_slices).
 struct PairList {
     int *idx;              // (n_slices * 64 * cap)
     int *count;            // per active entry
-    uint8_t *overflow;     // per slice
     int cap;
 };
 
@@ -294,6 +293,7 @@ struct GradientArgs {
     TreeArgs tree;
     const int *active;
     int n_active;
+    const double4 *xh;     // x, y, z, hsml
     const GradRec *rec;
     const double *nvt;     // 6 per particle
     const double *cn;
@@ -303,6 +303,7 @@ struct GradientArgs {
     const double *hsml;    // FP64 hsml (FP32 kernels: exact re-tests)
     const double *rho;     // FP64 density and pressure of i (FP32 kernels: limiter)
     const double *pres;
+    const float4 *xhf;     // FP32 kernels: offset x, y, z, hsml
     const GradRecF *recf;  // FP32 kernels
     F32Geom f32;
     Counters *ctr;
@@ -313,7 +314,9 @@ struct GradientArgs {
     const double *dhsml, *fce;
     double gamma;
     int block;             // threads per workgroup of the gradient kernel (64 .. kMaxBlock)
-    // symmetric pair rows (tree search; NULL: every particle walks the tree)
+    int lanes;             // lanes per particle of the FP64 grid kernel: 1 or 8
+    // candidate rows of the density stage (NULL: every particle walks), for the
+    // tree with the symmetric pair rows beside them
     const int *dcache_idx;
     const int *dcache_n;
     const double *dcache_r2;
@@ -374,6 +377,7 @@ struct ForceArgs {
     F32Geom f32;
     Counters *ctr;
     int block;             // threads per workgroup of the force loop kernel (64 .. kMaxBlock)
+    int lanes;             // lanes per particle of the three-phase list kernels: 1 or 8
 };
 
 // MFV force loop: ParticleVel (3 per particle), the integer timestep of each
@@ -422,7 +426,7 @@ void launch_density_finalize(hipStream_t s, int n_active, const int *active, con
                              const double4 *velu, const double *hsml, double *num_ngb, double *rho,
                              double *pres, double gamma_minus_1);
 void launch_pack_grad(hipStream_t s, int n, const double4 *posm, const double4 *velu, const double *hsml,
-                      const double *rho, const double *pres, GradRec *rec);
+                      const double *rho, const double *pres, double4 *xh, GradRec *rec);
 void launch_sym_rows(hipStream_t s, const SymRowArgs &a);
 void launch_gradients(hipStream_t s, const GradientArgs &a);
 void launch_pack_force(hipStream_t s, int n, const double4 *posm, const double4 *velu, const double *hsml,
@@ -440,7 +444,7 @@ void launch_pack_geom_f32(hipStream_t s, int n, const double4 *posm, const doubl
                           const int *box_of, float4 *offm, float4 *velf, uint32_t *cellc);
 void launch_density_sweep_f32(hipStream_t s, const DensitySweepArgs &a);
 void launch_pack_grad_f32(hipStream_t s, int n, const float4 *offm, const float4 *velf, const double *hsml,
-                          const double *rho, const double *pres, GradRecF *rec);
+                          const double *rho, const double *pres, float4 *xh, GradRecF *rec);
 void launch_gradients_f32(hipStream_t s, const GradientArgs &a);
 void launch_pack_force_f32(hipStream_t s, int n, const float4 *offm, const float4 *velf, const uint32_t *cellc,
                            const double4 *posm, const double *hsml, const double *rho, const double *pres,

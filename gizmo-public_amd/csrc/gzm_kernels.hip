@@ -327,13 +327,13 @@ __global__ void density_finalize_kernel(int n_active, const int *active, const d
 // gradients (gradients.c:1477-2089 pair loop, 1052-1253 finalize)
 // ---------------------------------------------------------------------------
 __global__ void pack_grad_kernel(int n, const double4 *posm, const double4 *velu, const double *hsml,
-                                 const double *rho, const double *pres, GradRec *rec)
+                                 const double *rho, const double *pres, double4 *xh, GradRec *rec)
 {
     int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
     double4 p = posm[k], v = velu[k];
     GradRec r;
-    r.xh = make_double4(p.x, p.y, p.z, hsml[k]);
+    xh[k] = make_double4(p.x, p.y, p.z, hsml[k]);
     r.vr = make_double4(v.x, v.y, v.z, rho[k]);
     r.pm = make_double2(pres[k], p.w);
     rec[k] = r;
@@ -441,54 +441,86 @@ __global__ __launch_bounds__(kBlock) void sym_rows_sort_kernel(int n, int *brow,
     }
 }
 
-template <int BS, bool ROWS = false>
-__global__ __launch_bounds__(BS) void gradients_kernel(GradientArgs a)
+// where a gradient kernel takes its candidates from: a walk (grid or tree), the
+// tree's candidate and pair rows, the grid's candidate rows (the last two fall
+// back to the walk for a particle whose rows do not hold its pair set)
+enum GradSource { kFromWalk, kFromTreeRows, kFromGridRows };
+
+// Bound by the L2 reads of the neighbours (5,500 lines per wavefront before the
+// split of GradRec and the chunked row reads): of 2.1 M particles 2.36 ms from
+// the walk, 1.72 from the rows entry by entry, 1.27 with rows read 64 bytes at
+// a time, positions apart from the rest of the record, and whole-record stores.
+//
+// G lanes per particle (more than one for few particles, which would leave most
+// SIMDs without a wavefront): each takes every G-th candidate, the sums are
+// reduced at the end and every lane finishes the particle (32^3 particles: 0.036
+// against 0.145 ms from the walk with one lane).
+template <int BS, GradSource SRC, int G = 1>
+__global__ __launch_bounds__(BS, 3) void gradients_kernel(GradientArgs a)
 {
-    // Pair-list entries are staged in LDS, column-major (entry c of thread x
-    // at stage[c * BS + x], so same-c stores of a wave hit distinct banks),
-    // and leave as whole 64-byte chunks: single 4-byte stores spread over the
-    // loop would reach HBM as partial-line write-backs.  BS = blockDim.x.
-    __shared__ int stage[kListChunk * BS];
-    constexpr int bs = BS;
-    const int t = xcd_block() * bs + threadIdx.x;
+    // Pair-list entries are staged in LDS and leave as whole 64-byte chunks:
+    // single 4-byte stores spread over the loop would reach HBM as partial-line
+    // write-backs.  BS = blockDim.x.  With G > 1 the entries of a step are packed
+    // by ballot and adjoin anyway.
+    __shared__ __align__(16) int lds[G == 1 ? kListChunk * BS : 1];
+    __shared__ __align__(16) int lds_row[G == 1 && SRC == kFromGridRows ? kListChunk * BS : 1];
+    int *stage = wave_chunk(lds), *chunk = wave_chunk(lds_row);
+    const int t = (xcd_block() * BS + (int)threadIdx.x) / G, sub = (int)threadIdx.x % G;
     const bool valid = t < a.n_active;
     unsigned long long cnt = 0;
-    int listed = 0;
-    for_box(a.boxes, a.box_of, valid ? a.active[t] : 0, valid, [&](const BoxDesc &G) {
+    int listed = 0, out_i = 0;
+    double g_out[15];  // the particle's gradients and force record, stored by the whole wavefront
+    ForceRec f_out;
+    for_box(a.boxes, a.box_of, valid ? a.active[t] : 0, valid, [&](const BoxDesc &B) {
         const int i = a.active[t];
+        out_i = i;
         const GradRec ri = a.rec[i];
+        const double4 xi = a.xh[i];
         double gr0 = 0, gr1 = 0, gr2 = 0, gp0 = 0, gp1 = 0, gp2 = 0;
         double gv00 = 0, gv01 = 0, gv02 = 0, gv10 = 0, gv11 = 0, gv12 = 0, gv20 = 0, gv21 = 0, gv22 = 0;
         double maxd = 0, mn_r = 0, mx_r = 0, mn_p = 0, mx_p = 0;
         double mn_v0 = 0, mx_v0 = 0, mn_v1 = 0, mx_v1 = 0, mn_v2 = 0, mx_v2 = 0;
-        const double h_i = ri.xh.w, rho_i = ri.vr.w, p_i = ri.pm.x, m_i = ri.pm.y;
+        const double h_i = xi.w, rho_i = ri.vr.w, p_i = ri.pm.x, m_i = ri.pm.y;
         int *list_row = a.list.idx ? a.list.idx + (size_t)t * a.list.cap : nullptr;
         if ((m_i > 0) && (rho_i > 0) && (h_i > 0)) {  // GasGrad_isactive (gradients.c:66-75)
             double hinv, hinv3, hinv4;
             kernel_hinv(h_i, hinv, hinv3, hinv4);
             const double h2_i = h_i * h_i;
-            const double xs[3] = {ri.xh.x, ri.xh.y, ri.xh.z};
-            auto visit = [&](int j) {
-                const double4 xj = a.rec[j].xh;
-                double dp[3] = {xs[0] - xj.x, xs[1] - xj.y, xs[2] - xj.z};
-                wrap_dp(G.box, dp);
-                const double r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
-                const double h_j = xj.w;
-                if (r2 <= 0) return;
-                if ((r2 >= h2_i) && (r2 >= h_j * h_j)) return;
-                const double4 vr = a.rec[j].vr;
-                const double2 pm = a.rec[j].pm;
-                if (!((pm.y > 0) && (vr.w > 0))) return;
-                // the list holds the force loop's pair set (m_j > 0, rho_j > 0,
-                // hydro_evaluate.h:149-150); gradients also need h_j > 0
-                if (list_row) {
+            const double xs[3] = {xi.x, xi.y, xi.z};
+            // the force loop's pair set (hydro_evaluate.h:149-150)
+            auto is_pair = [&](auto near, const double4 &xj, const GradRec &rj, double dp[3], double &r2) {
+                dp[0] = xs[0] - xj.x;
+                dp[1] = xs[1] - xj.y;
+                dp[2] = xs[2] - xj.z;
+                if constexpr (near.value) wrap_near(B.box, dp);
+                else wrap_dp(B.box, dp);
+                r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
+                if (r2 <= 0) return false;
+                if ((r2 >= h2_i) && (r2 >= xj.w * xj.w)) return false;
+                return (rj.pm.y > 0) && (rj.vr.w > 0);
+            };
+            // list entry (m_j > 0, rho_j > 0; gradients also need h_j > 0)
+            auto enlist = [&](int j, bool in) {
+                if (!list_row) return;
+                if constexpr (G == 1) {
+                    if (!in) return;
                     if (listed < a.list.cap) {
                         const int c = listed & (kListChunk - 1);
-                        stage[c * bs + threadIdx.x] = j;
-                        if (c == kListChunk - 1) flush_list_chunk(stage, list_row + (listed - c), bs);
+                        stage[c * 64 + (threadIdx.x & 63)] = j;
+                        if (c == kListChunk - 1) flush_list_chunk(stage, list_row + (listed - c));
                     }
                     listed++;
+                } else {
+                    const unsigned bits = (unsigned)(__ballot(in) >> ((threadIdx.x & 63) & ~(G - 1))) & ((1u << G) - 1);
+                    const int k = listed + __popc(bits & ((1u << sub) - 1));
+                    if (in && k < a.list.cap) list_row[k] = j;
+                    listed += __popc(bits);
                 }
+            };
+            auto add = [&](const double4 &xj, const GradRec &rj, const double dp[3], double r2) {
+                const double h_j = xj.w;
+                const double4 vr = rj.vr;
+                const double2 pm = rj.pm;
                 if (!(h_j > 0)) return;
                 cnt++;
                 const double r = sqrt(r2);
@@ -511,9 +543,50 @@ __global__ __launch_bounds__(BS) void gradients_kernel(GradientArgs a)
                     gv20 += w0 * dv2; gv21 += w1 * dv2; gv22 += w2 * dv2;
                 }
             };
-            const int n_a = ROWS ? a.dcache_n[i] : 0;
-            const int n_b = ROWS ? a.bcount[i] : 0;
-            if (ROWS && n_a <= kDensityCacheCap && h2_i <= a.dcache_r2[i] && n_b <= kPairRowCap) {
+            auto visit = [&](int j) {
+                const double4 xj = a.xh[j];
+                double dp[3], r2;
+                if (!is_pair(std::false_type{}, xj, a.rec[j], dp, r2)) return;
+                enlist(j, true);
+                add(xj, a.rec[j], dp, r2);
+            };
+            // G > 1: candidate k + sub of a run of `end` for each lane, all lanes in step
+            auto visit_step = [&](auto near, int j, bool valid_j) {
+                double dp[3], r2;
+                double4 xj;
+                bool in = valid_j;
+                if (in) {
+                    xj = a.xh[j];
+                    in = is_pair(near, xj, a.rec[j], dp, r2);
+                }
+                enlist(j, in);
+                if (in) add(xj, a.rec[j], dp, r2);
+            };
+            const int n_a = SRC != kFromWalk ? a.dcache_n[i] : kDensityCacheCap + 1;
+            const int n_b = SRC == kFromTreeRows ? a.bcount[i] : 0;
+            if (SRC == kFromGridRows && n_a <= kDensityCacheCap && row_holds_pairs(B, xs, h_i, a.dcache_r2[i])) {
+                const int *row = a.dcache_idx + (size_t)i * kDensityCacheCap;
+                auto scan = [&](auto near) {
+                    if constexpr (G > 1) {
+                        for (int k = 0; k < n_a; k += G) visit_step(near, row[min(k + sub, n_a - 1)], k + sub < n_a);
+                    } else {
+                        for_row_pairs(chunk, row, n_a, [&](int j0, int j1, bool second) {
+                            const double4 x0 = a.xh[j0], x1 = a.xh[j1];
+                            double dp[3], r2;
+                            if (is_pair(near, x0, a.rec[j0], dp, r2)) {
+                                enlist(j0, true);
+                                add(x0, a.rec[j0], dp, r2);
+                            }
+                            if (second && is_pair(near, x1, a.rec[j1], dp, r2)) {
+                                enlist(j1, true);
+                                add(x1, a.rec[j1], dp, r2);
+                            }
+                        });
+                    }
+                };
+                if (__all(a.dcache_r2[i] * 1.01 < B.box.narrow2)) scan(std::true_type{});
+                else scan(std::false_type{});
+            } else if (SRC == kFromTreeRows && n_a <= kDensityCacheCap && h2_i <= a.dcache_r2[i] && n_b <= kPairRowCap) {
                 // ascending merge of i's candidate row and its pair row
                 const int *ra = a.dcache_idx + (size_t)i * kDensityCacheCap;
                 const int *rb = a.brow + (size_t)i * kPairRowCap;
@@ -530,14 +603,33 @@ __global__ __launch_bounds__(BS) void gradients_kernel(GradientArgs a)
                         jb = (kb < n_b) ? rb[kb] : kNoSlot;
                     }
                 }
+            } else if constexpr (G > 1) {  // grid
+                const double R = (B.hmax > h_i) ? B.hmax : h_i;
+                bool full[3];
+                for_each_cell(B.grid, xs, R, full, [&](int, int, int, int beg, int end) {
+                    for (int k = beg; k < end; k += G) visit_step(std::false_type{}, k + sub, k + sub < end);
+                }, h_i);
             } else {
-                for_each_neighbour_candidate(a.tree, G, xs, h_i, true, visit);
+                for_each_neighbour_candidate(a.tree, B, xs, h_i, true, visit);
             }
             // the partly filled last chunk (entries past `listed` are never read)
-            if (list_row && listed < a.list.cap && (listed & (kListChunk - 1)))
-                flush_list_chunk(stage, list_row + (listed & ~(kListChunk - 1)), bs);
+            if (G == 1 && list_row && listed < a.list.cap && (listed & (kListChunk - 1)))
+                flush_list_chunk(stage, list_row + (listed & ~(kListChunk - 1)));
         } else if ((m_i > 0) && (rho_i > 0)) {
             listed = a.list.cap + 1;  // the force loop still runs for i: send it to the scan
+        }
+        if constexpr (G > 1) {
+            gr0 = group_sum<G>(gr0); gr1 = group_sum<G>(gr1); gr2 = group_sum<G>(gr2);
+            gp0 = group_sum<G>(gp0); gp1 = group_sum<G>(gp1); gp2 = group_sum<G>(gp2);
+            gv00 = group_sum<G>(gv00); gv01 = group_sum<G>(gv01); gv02 = group_sum<G>(gv02);
+            gv10 = group_sum<G>(gv10); gv11 = group_sum<G>(gv11); gv12 = group_sum<G>(gv12);
+            gv20 = group_sum<G>(gv20); gv21 = group_sum<G>(gv21); gv22 = group_sum<G>(gv22);
+            maxd = group_max<G>(maxd);
+            mn_r = group_min<G>(mn_r); mx_r = group_max<G>(mx_r);
+            mn_p = group_min<G>(mn_p); mx_p = group_max<G>(mx_p);
+            mn_v0 = group_min<G>(mn_v0); mx_v0 = group_max<G>(mx_v0);
+            mn_v1 = group_min<G>(mn_v1); mx_v1 = group_max<G>(mx_v1);
+            mn_v2 = group_min<G>(mn_v2); mx_v2 = group_max<G>(mx_v2);
         }
         double nvt[6];
 #pragma unroll
@@ -559,28 +651,30 @@ __global__ __launch_bounds__(BS) void gradients_kernel(GradientArgs a)
         slope_limit(gv0, mx_v0, mn_v0, a_lim, h_i, 0.1, 0, 0, 0);
         slope_limit(gv1, mx_v1, mn_v1, a_lim, h_i, 0.1, 0, 0, 0);
         slope_limit(gv2, mx_v2, mn_v2, a_lim, h_i, 0.1, 0, 0, 0);
-        double *o = a.grad + 15 * (size_t)i;
-        o[0] = gr[0]; o[1] = gr[1]; o[2] = gr[2];
-        o[3] = gp[0]; o[4] = gp[1]; o[5] = gp[2];
-        o[6] = gv0[0]; o[7] = gv0[1]; o[8] = gv0[2];
-        o[9] = gv1[0]; o[10] = gv1[1]; o[11] = gv1[2];
-        o[12] = gv2[0]; o[13] = gv2[1]; o[14] = gv2[2];
-        if (a.frec_out) {  // every particle active: its force record, as pack_force_kernel writes it
-            const double g[15] = {gr[0], gr[1], gr[2], gp[0], gp[1], gp[2], gv0[0], gv0[1], gv0[2],
-                                  gv1[0], gv1[1], gv1[2], gv2[0], gv2[1], gv2[2]};
-            a.frec_out[i] = make_force_rec(make_double4(ri.xh.x, ri.xh.y, ri.xh.z, m_i),
-                                           make_double4(ri.vr.x, ri.vr.y, ri.vr.z, 0.0), rho_i, p_i, h_i,
-                                           a.dhsml[i], cn, a.fce[i], nvt, g, a.gamma);
-        }
-        if (a.list.idx) a.list.count[t] = listed;
+        const double g[15] = {gr[0], gr[1], gr[2], gp[0], gp[1], gp[2], gv0[0], gv0[1], gv0[2],
+                              gv1[0], gv1[1], gv1[2], gv2[0], gv2[1], gv2[2]};
+#pragma unroll
+        for (int k = 0; k < 15; k++) g_out[k] = g[k];
+        if (a.frec_out)  // every particle active: its force record, as pack_force_kernel writes it
+            f_out = make_force_rec(make_double4(xi.x, xi.y, xi.z, m_i), make_double4(ri.vr.x, ri.vr.y, ri.vr.z, 0.0),
+                                   rho_i, p_i, h_i, a.dhsml[i], cn, a.fce[i], nvt, g, a.gamma);
+        if (a.list.idx && sub == 0) a.list.count[t] = listed;
     });
-    if (a.list.idx) {
-        // a slice overflows when any of its lanes listed more than cap neighbours
-        const bool over = __any(listed > a.list.cap);
-        if ((threadIdx.x & 63) == 0 && t < a.n_active) {
-            a.list.overflow[t >> 6] = over ? 1 : 0;
-            if (over) atomicAdd(&ctr_slot(a.ctr)->overflow_slices, 1);
+    if constexpr (G == 1) {
+        wave_store_records(stage, a.grad, 15, out_i, valid, g_out);
+        if (a.frec_out) {
+            double w[sizeof(ForceRec) / 8];
+            __builtin_memcpy(w, &f_out, sizeof(ForceRec));
+            wave_store_records(stage, reinterpret_cast<double *>(a.frec_out), sizeof(ForceRec) / 8, out_i, valid, w);
         }
+    } else if (valid && sub == 0) {
+        for (int k = 0; k < 15; k++) a.grad[15 * (size_t)out_i + k] = g_out[k];
+        if (a.frec_out) a.frec_out[out_i] = f_out;
+    }
+    if (a.list.idx) {
+        // wavefronts with a particle of more than cap neighbours
+        const bool over = __any(listed > a.list.cap);
+        if ((threadIdx.x & 63) == 0 && over) atomicAdd(&ctr_slot(a.ctr)->overflow_slices, 1);
     }
     wave_add_u64(&ctr_slot(a.ctr)->interactions, cnt);
 }
@@ -926,9 +1020,9 @@ void launch_density_finalize(hipStream_t s, int n_active, const int *active, con
                        velu, hsml, num_ngb, rho, pres, gm1);
 }
 void launch_pack_grad(hipStream_t s, int n, const double4 *posm, const double4 *velu, const double *hsml,
-                      const double *rho, const double *pres, GradRec *rec)
+                      const double *rho, const double *pres, double4 *xh, GradRec *rec)
 {
-    if ((n) > 0) hipLaunchKernelGGL(pack_grad_kernel, dim3(nblocks(n)), dim3(kBlock), 0, s, n, posm, velu, hsml, rho, pres, rec);
+    if ((n) > 0) hipLaunchKernelGGL(pack_grad_kernel, dim3(nblocks(n)), dim3(kBlock), 0, s, n, posm, velu, hsml, rho, pres, xh, rec);
 }
 void launch_sym_rows(hipStream_t s, const SymRowArgs &a)
 {
@@ -939,21 +1033,29 @@ void launch_sym_rows(hipStream_t s, const SymRowArgs &a)
     hipLaunchKernelGGL(sym_rows_wave_kernel, dim3(2048), dim3(kBlock), 0, s, a);
     hipLaunchKernelGGL(sym_rows_sort_kernel, dim3(nblocks(a.n)), dim3(kBlock), 0, s, a.n, a.brow, a.bcount);
 }
+template <GradSource SRC>
+static void launch_gradients_from(hipStream_t s, const GradientArgs &a, dim3 grid, dim3 block)
+{
+    if (a.block == 64) hipLaunchKernelGGL((gradients_kernel<64, SRC>), grid, block, 0, s, a);
+    else if (a.block == 128) hipLaunchKernelGGL((gradients_kernel<128, SRC>), grid, block, 0, s, a);
+    else if (a.block == 512) hipLaunchKernelGGL((gradients_kernel<512, SRC>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((gradients_kernel<kBlock, SRC>), grid, block, 0, s, a);
+}
 void launch_gradients(hipStream_t s, const GradientArgs &a)
 {
     if (a.n_active <= 0) return;
     const dim3 grid(nblocks(a.n_active, a.block)), block(a.block);
-    if (a.brow) {
-        if (a.block == 64) hipLaunchKernelGGL((gradients_kernel<64, true>), grid, block, 0, s, a);
-        else if (a.block == 128) hipLaunchKernelGGL((gradients_kernel<128, true>), grid, block, 0, s, a);
-        else if (a.block == 512) hipLaunchKernelGGL((gradients_kernel<512, true>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((gradients_kernel<kBlock, true>), grid, block, 0, s, a);
-        return;
+    if (a.lanes == 8 && !a.tree.nodes) {
+        const dim3 few(nblocks(8LL * a.n_active));
+        if (a.dcache_idx) hipLaunchKernelGGL((gradients_kernel<kBlock, kFromGridRows, 8>), few, dim3(kBlock), 0, s, a);
+        else hipLaunchKernelGGL((gradients_kernel<kBlock, kFromWalk, 8>), few, dim3(kBlock), 0, s, a);
+    } else if (a.brow) {
+        launch_gradients_from<kFromTreeRows>(s, a, grid, block);
+    } else if (a.dcache_idx && !a.tree.nodes) {
+        launch_gradients_from<kFromGridRows>(s, a, grid, block);
+    } else {
+        launch_gradients_from<kFromWalk>(s, a, grid, block);
     }
-    if (a.block == 64) hipLaunchKernelGGL(gradients_kernel<64>, grid, block, 0, s, a);
-    else if (a.block == 128) hipLaunchKernelGGL(gradients_kernel<128>, grid, block, 0, s, a);
-    else if (a.block == 512) hipLaunchKernelGGL(gradients_kernel<512>, grid, block, 0, s, a);
-    else hipLaunchKernelGGL(gradients_kernel<kBlock>, grid, block, 0, s, a);
 }
 void launch_pack_force(hipStream_t s, int n, const double4 *posm, const double4 *velu, const double *hsml,
                        const double *rho, const double *pres, const double *dhsml, const double *cn,

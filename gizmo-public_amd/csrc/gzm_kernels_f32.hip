@@ -283,7 +283,7 @@ __global__ __launch_bounds__(MAXB) void density_sweep_f32_kernel(DensitySweepArg
 __device__ __forceinline__ float low_word(double x, float hi) { return (float)(x - (double)hi); }
 
 __global__ void pack_grad_f32_kernel(int n, const float4 *offm, const float4 *velf, const double *hsml,
-                                     const double *rho, const double *pres, GradRecF *rec)
+                                     const double *rho, const double *pres, float4 *xh, GradRecF *rec)
 {
     int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
@@ -291,7 +291,7 @@ __global__ void pack_grad_f32_kernel(int n, const float4 *offm, const float4 *ve
     const double d = rho[k], P = pres[k];
     const float df = (float)d, Pf = (float)P;
     GradRecF r;
-    r.xh = make_float4(o.x, o.y, o.z, (float)hsml[k]);
+    xh[k] = make_float4(o.x, o.y, o.z, (float)hsml[k]);
     r.vr = make_float4(v.x, v.y, v.z, df);
     r.pm = make_float4(Pf, o.w, low_word(d, df), low_word(P, Pf));
     rec[k] = r;
@@ -318,20 +318,61 @@ __device__ __forceinline__ ForceRecF make_force_rec_f(const float4 &o, const flo
     return r;
 }
 
+// the record as 8-byte words, in memory order (element by element: a copy
+// through memory would go through scratch)
+__device__ __forceinline__ void record_words(const ForceRecF &r, double (&w)[sizeof(ForceRecF) / 8])
+{
+    const float4 f[9] = {r.xh, r.vc, r.th, r.t0, r.t1, r.g0, r.g1, r.g2, r.g3};
+    auto word = [](float lo, float hi) { return __hiloint2double(__float_as_int(hi), __float_as_int(lo)); };
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        w[2 * k] = word(f[k].x, f[k].y);
+        w[2 * k + 1] = word(f[k].z, f[k].w);
+    }
+    w[18] = r.cn;
+    w[19] = r.e;
+}
+
 constexpr int kNoSlotF = 0x7fffffff;  // above every sorted slot: the end of a merged row
+
+// whether for_each_cell walks axis ax whole for search radius R
+__device__ __forceinline__ bool walks_whole(const Grid &g, double R, int ax)
+{
+    return !(R * g.inv_s[ax] < 0.5 * g.nc[ax] - 2.0);
+}
+
+// Particle i's density candidate row instead of the grid walk of radius R: it
+// holds the pair set, and its walk visited the cells in the same order (an axis
+// walked whole starts at cell 0, else at the first cell in reach).
+__device__ __forceinline__ bool grid_row_usable(const GradientArgs &a, const BoxDesc &G, int i, const double xs[3],
+                                                double h_i, double R)
+{
+    if (!a.dcache_idx || a.dcache_n[i] > kDensityCacheCap) return false;
+    const double r2 = a.dcache_r2[i], Rc = sqrt(r2);
+    bool same = true;
+#pragma unroll
+    for (int ax = 0; ax < 3; ax++) same = same && (walks_whole(G.grid, Rc, ax) == walks_whole(G.grid, R, ax));
+    return same && row_holds_pairs(G, xs, h_i, r2);
+}
 
 template <bool TREE, int BS>
 __global__ __launch_bounds__(BS, 4) void gradients_f32_kernel(GradientArgs a)
 {
-    __shared__ int stage[kListChunk * BS];  // as in gradients_kernel; BS = blockDim.x
-    constexpr int bs = BS;
-    const int t = xcd_block() * bs + threadIdx.x;
+    // as in gradients_kernel; BS = blockDim.x
+    __shared__ __align__(16) int lds[kListChunk * BS];
+    __shared__ __align__(16) int lds_row[TREE ? 1 : kListChunk * BS];
+    int *stage = wave_chunk(lds), *chunk = wave_chunk(lds_row);
+    const int t = xcd_block() * BS + threadIdx.x;
     const bool valid = t < a.n_active;
     unsigned long long cnt = 0;
-    int listed = 0;
+    int listed = 0, out_i = 0;
+    double g_out[15];
+    ForceRecF f_out;
     for_box(a.boxes, a.box_of, valid ? a.active[t] : 0, valid, [&](const BoxDesc &G) {
         const int i = a.active[t];
+        out_i = i;
         const double4 pi = a.posm[i];
+        const float4 xi = a.xhf[i];
         const GradRecF ri = a.recf[i];
         int ci[3];
         unpack_cell(a.f32.cellc[i], ci);
@@ -352,18 +393,18 @@ __global__ __launch_bounds__(BS, 4) void gradients_f32_kernel(GradientArgs a)
             const double xs[3] = {pi.x, pi.y, pi.z};
             const double R = (h_i > G.hmax) ? h_i : G.hmax;
             const float h_fine = smax_of(G) / kFineCells;  // pairs with a smaller hsml: FP64 geometry
-            const bool fine_i = ri.xh.w < h_fine;
+            const bool fine_i = xi.w < h_fine;
             auto visit = [&](int k, float sh0, float sh1, float sh2, bool exact_geom) {
                 if (k == i) return;  // r2 = 0 exactly
-                const float4 xj = a.recf[k].xh;
+                const float4 xj = a.xhf[k];
                 const float hj2 = xj.w * xj.w;
                 float dp[3];
                 float r2;
                 int in_i, in_j, pos;
                 if (!exact_geom && !(xj.w < h_fine)) {
-                    dp[0] = sh0 + (ri.xh.x - xj.x);
-                    dp[1] = sh1 + (ri.xh.y - xj.y);
-                    dp[2] = sh2 + (ri.xh.z - xj.z);
+                    dp[0] = sh0 + (xi.x - xj.x);
+                    dp[1] = sh1 + (xi.y - xj.y);
+                    dp[2] = sh2 + (xi.z - xj.z);
                     r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
                     if ((r2 >= bi.hi) && (r2 >= hj2 * (1 + kBandF))) return;  // clearly outside both
                     in_i = decide(r2, bi);
@@ -396,8 +437,8 @@ __global__ __launch_bounds__(BS, 4) void gradients_f32_kernel(GradientArgs a)
                 if (list_row) {
                     if (listed < a.list.cap) {
                         const int c = listed & (kListChunk - 1);
-                        stage[c * bs + threadIdx.x] = k;
-                        if (c == kListChunk - 1) flush_list_chunk(stage, list_row + (listed - c), bs);
+                        stage[c * 64 + (threadIdx.x & 63)] = k;
+                        if (c == kListChunk - 1) flush_list_chunk(stage, list_row + (listed - c));
                     }
                     listed++;
                 }
@@ -447,6 +488,20 @@ __global__ __launch_bounds__(BS, 4) void gradients_f32_kernel(GradientArgs a)
                 } else {
                     tree_walk(a.tree, G, xs, h_i, true, [&](int k) { visit(k, 0.0f, 0.0f, 0.0f, true); });
                 }
+            } else if (grid_row_usable(a, G, i, xs, h_i, R)) {
+                // the row in the order of the walk, so that the FP32 sums are the walk's
+                bool exact_geom = fine_i;
+#pragma unroll
+                for (int ax = 0; ax < 3; ax++) exact_geom = exact_geom || walks_whole(G.grid, R, ax);
+                const int n_row = a.dcache_n[i];
+                const int *row = a.dcache_idx + (size_t)i * kDensityCacheCap;
+                for_row(chunk, row, n_row, [&](int k) {
+                    int cj[3];
+                    unpack_cell(a.f32.cellc[k], cj);
+                    visit(k, cell_shift(wrap_cell(ci[0] - cj[0], G.grid.nc[0]), G.s_f[0]),
+                          cell_shift(wrap_cell(ci[1] - cj[1], G.grid.nc[1]), G.s_f[1]),
+                          cell_shift(wrap_cell(ci[2] - cj[2], G.grid.nc[2]), G.s_f[2]), exact_geom);
+                });
             } else {
                 bool full[3];
                 for_each_cell(G.grid, xs, R, full, [&](int cx, int cy, int cz, int beg, int end) {
@@ -458,7 +513,7 @@ __global__ __launch_bounds__(BS, 4) void gradients_f32_kernel(GradientArgs a)
                 }, h_i);
             }
             if (list_row && listed < a.list.cap && (listed & (kListChunk - 1)))
-                flush_list_chunk(stage, list_row + (listed & ~(kListChunk - 1)), bs);
+                flush_list_chunk(stage, list_row + (listed & ~(kListChunk - 1)));
         } else if ((m_i > 0) && (rho_i > 0)) {
             listed = a.list.cap + 1;  // the force loop still runs for i: send it to the scan
         }
@@ -482,26 +537,24 @@ __global__ __launch_bounds__(BS, 4) void gradients_f32_kernel(GradientArgs a)
         slope_limit(gv0, mx_v0, mn_v0, a_lim, h_i, 0.1, 0, 0, 0);
         slope_limit(gv1, mx_v1, mn_v1, a_lim, h_i, 0.1, 0, 0, 0);
         slope_limit(gv2, mx_v2, mn_v2, a_lim, h_i, 0.1, 0, 0, 0);
-        double *o = a.grad + 15 * (size_t)i;
-        o[0] = gr[0]; o[1] = gr[1]; o[2] = gr[2];
-        o[3] = gp[0]; o[4] = gp[1]; o[5] = gp[2];
-        o[6] = gv0[0]; o[7] = gv0[1]; o[8] = gv0[2];
-        o[9] = gv1[0]; o[10] = gv1[1]; o[11] = gv1[2];
-        o[12] = gv2[0]; o[13] = gv2[1]; o[14] = gv2[2];
-        if (a.frecf_out) {  // every particle active: its force record, as pack_force_f32_kernel writes it
-            const double g[15] = {gr[0], gr[1], gr[2], gp[0], gp[1], gp[2], gv0[0], gv0[1], gv0[2],
-                                  gv1[0], gv1[1], gv1[2], gv2[0], gv2[1], gv2[2]};
-            a.frecf_out[i] = make_force_rec_f(make_float4(ri.xh.x, ri.xh.y, ri.xh.z, 0.0f), ri.vr, a.f32.cellc[i], m_i,
-                                              rho_i, p_i, h_i, a.dhsml[i], cn, a.fce[i], nvt, g, a.gamma);
-        }
+        const double g[15] = {gr[0], gr[1], gr[2], gp[0], gp[1], gp[2], gv0[0], gv0[1], gv0[2],
+                              gv1[0], gv1[1], gv1[2], gv2[0], gv2[1], gv2[2]};
+#pragma unroll
+        for (int k = 0; k < 15; k++) g_out[k] = g[k];
+        if (a.frecf_out)  // every particle active: its force record, as pack_force_f32_kernel writes it
+            f_out = make_force_rec_f(make_float4(xi.x, xi.y, xi.z, 0.0f), ri.vr, a.f32.cellc[i], m_i, rho_i, p_i, h_i,
+                                     a.dhsml[i], cn, a.fce[i], nvt, g, a.gamma);
         if (a.list.idx) a.list.count[t] = listed;
     });
+    wave_store_records(stage, a.grad, 15, out_i, valid, g_out);
+    if (a.frecf_out) {
+        double w[sizeof(ForceRecF) / 8];
+        record_words(f_out, w);
+        wave_store_records(stage, reinterpret_cast<double *>(a.frecf_out), sizeof(ForceRecF) / 8, out_i, valid, w);
+    }
     if (a.list.idx) {
         const bool over = __any(listed > a.list.cap);
-        if ((threadIdx.x & 63) == 0 && t < a.n_active) {
-            a.list.overflow[t >> 6] = over ? 1 : 0;
-            if (over) atomicAdd(&ctr_slot(a.ctr)->overflow_slices, 1);
-        }
+        if ((threadIdx.x & 63) == 0 && over) atomicAdd(&ctr_slot(a.ctr)->overflow_slices, 1);
     }
     wave_add_u64(&ctr_slot(a.ctr)->interactions, cnt);
 }
@@ -1069,9 +1122,9 @@ void launch_density_sweep_f32(hipStream_t s, const DensitySweepArgs &a)
     }
 }
 void launch_pack_grad_f32(hipStream_t s, int n, const float4 *offm, const float4 *velf, const double *hsml,
-                          const double *rho, const double *pres, GradRecF *rec)
+                          const double *rho, const double *pres, float4 *xh, GradRecF *rec)
 {
-    if (n > 0) hipLaunchKernelGGL(pack_grad_f32_kernel, dim3(nblocks(n)), dim3(kBlock), 0, s, n, offm, velf, hsml, rho, pres, rec);
+    if (n > 0) hipLaunchKernelGGL(pack_grad_f32_kernel, dim3(nblocks(n)), dim3(kBlock), 0, s, n, offm, velf, hsml, rho, pres, xh, rec);
 }
 void launch_gradients_f32(hipStream_t s, const GradientArgs &a)
 {
