@@ -508,6 +508,108 @@ __device__ __forceinline__ double group_min(double v)
     return v;
 }
 
+template <int G>
+__device__ __forceinline__ int group_sum_int(int v)
+{
+#pragma unroll
+    for (int off = G / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    return v;
+}
+
+// bitwise or over the G lanes of one particle
+template <int G>
+__device__ __forceinline__ uint64_t group_or(uint64_t v)
+{
+#pragma unroll
+    for (int off = G / 2; off > 0; off >>= 1) v |= __shfl_xor((unsigned long long)v, off, 64);
+    return v;
+}
+
+// order this wavefront's LDS writes before its later reads
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The pair lists of 64 / kForceLanes particles, one wavefront (a workgroup of its
+// own), kForceLanes lanes per particle: step by step each lane takes one pair,
+// visit(own, other, x_j, j, k) with both records in LDS.
+//
+// A lane that reads its neighbour's record itself costs the address unit one
+// cycle per lane and 16 bytes (20 loads of 64 lanes: 1,280 cycles a step for the
+// FP64 record, more than the 1,000 of the arithmetic on a CU's four SIMDs).
+// Four lanes reading 64 adjacent bytes cost one, so the wavefront fetches the 64
+// records of a step together and passes them on through LDS; the loads of the
+// next step are in flight while this one computes.  Eight lanes per particle
+// instead of one keep the neighbours of all particles in flight on an XCD within
+// its 4 MB L2 (L2 misses 5,150 against 318 lines per 64 particles of a 2.1 M set)
+// and let them share i's record in LDS instead of each holding it in registers.
+template <typename REC>
+struct PairLoopLds {
+    REC other[64];
+    REC own[64 / kForceLanes];
+};
+
+template <typename REC, typename F>
+__device__ __forceinline__ void pair_list_loop(PairLoopLds<REC> &lds, const REC *__restrict__ rec,
+                                               const double4 *__restrict__ posm, const int *row, int n, int i,
+                                               F &&visit)
+{
+    constexpr int kChunks = (int)(sizeof(REC) / 16), kSegments = kChunks / 4, kRest = kChunks % 4;
+    static_assert(sizeof(REC) % 16 == 0, "records of whole 16-byte chunks");
+    using Chunk = double __attribute__((ext_vector_type(2)));
+    const int lane = threadIdx.x & 63, sub = lane % kForceLanes, g = lane / kForceLanes;
+    int steps = (n + kForceLanes - 1) / kForceLanes;
+    for (int off = 32; off >= kForceLanes; off >>= 1) steps = max(steps, __shfl_xor(steps, off, 64));
+    // i's record
+    {
+        const double *src = reinterpret_cast<const double *>(rec + i);
+        double *dst = reinterpret_cast<double *>(lds.own + g);
+        for (int w = sub; w < (int)(sizeof(REC) / 8); w += kForceLanes) dst[w] = src[w];
+    }
+    Chunk seg[4][kSegments], rest[kRest > 0 ? kRest : 1];
+    double4 xj;
+    auto fetch = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const Chunk *src = reinterpret_cast<const Chunk *>(rec + __shfl(j, 16 * q + (lane >> 2), 64));
+#pragma unroll
+            for (int m = 0; m < kSegments; m++) seg[q][m] = src[4 * m + (lane & 3)];
+        }
+        const Chunk *src = reinterpret_cast<const Chunk *>(rec + j);
+#pragma unroll
+        for (int m = 0; m < kRest; m++) rest[m] = src[4 * kSegments + m];
+        xj = posm[j];
+    };
+    // lanes past their list fetch i itself
+    int j = sub < n ? row[sub] : i;
+    int j_next = sub + kForceLanes < n ? row[sub + kForceLanes] : i;
+    if (steps > 0) fetch(j);
+    for (int it = 0; it < steps; it++) {
+        wave_lds_fence();
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            Chunk *dst = reinterpret_cast<Chunk *>(lds.other + 16 * q + (lane >> 2));
+#pragma unroll
+            for (int m = 0; m < kSegments; m++) dst[4 * m + (lane & 3)] = seg[q][m];
+        }
+        Chunk *dst = reinterpret_cast<Chunk *>(lds.other + lane);
+#pragma unroll
+        for (int m = 0; m < kRest; m++) dst[4 * kSegments + m] = rest[m];
+        wave_lds_fence();
+        const int k = it * kForceLanes + sub, j_now = j;
+        const double4 x_now = xj;
+        if (it + 1 < steps) {
+            j = j_next;
+            fetch(j);
+            const int k2 = k + 2 * kForceLanes;
+            j_next = k2 < n ? row[k2] : i;
+        }
+        if (k < n) visit(lds.own[g], lds.other[lane], x_now, j_now, k);
+    }
+}
+
 // Whether the candidate row of radius^2 r2 around x holds the whole pair set
 // {j : r < h_i or r < h_j}: no particle beyond the radius has an hsml that
 // reaches x.  The box's largest hsml answers for most sets; else the cells in
@@ -691,13 +793,11 @@ __device__ __forceinline__ void wave_store_records(int *lds, double *base, size_
     const int lane = threadIdx.x & 63, word = lane & 7;
 #pragma unroll
     for (int p = 0; p < N; p += 8) {
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
 #pragma unroll
         for (int c = 0; c < 8; c++)
             if (p + c < N) buf[lane * 8 + (c ^ word)] = w[p + c];
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
 #pragma unroll
         for (int it = 0; it < 8; it++) {
             const int l = it * 8 + (lane >> 3);  // whose record

@@ -1397,7 +1397,6 @@ gzm_status force_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
         m.d_mass = c->d_dmass;
         m.grav_work = c->d_gravwork;
     }
-    a.lanes = c->n_active <= kFewParticles ? 8 : 1;
     // exact-solver pairs leave the list loop for a kernel of their own (lists of <= 64)
     const bool three_phase = use_list && c->list_cap <= 64 && c->n_active > 0;
     if (three_phase) {

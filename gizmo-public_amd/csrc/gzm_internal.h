@@ -63,36 +63,12 @@ struct TreeArgs {
     const int *leaf_esc = nullptr;    // sorted slot: next node after the leaf
 };
 
-// Per-particle record read by the force loop for the neighbour j (and for i).
-// 320 bytes: one aligned block so a gather touches 2.5 cache lines.
-struct alignas(64) ForceRec {
-    double4 xh;    // x, y, z, hsml
-    double4 vc;    // vx, vy, vz, sound speed sqrt(gamma P / rho)
-    double4 th;    // rho, P, V = m / rho, DhsmlNgbFactor
-    double4 mc;    // m, ConditionNumber, FaceClosureError, P / rho
-    double4 t0;    // NV_T: i00 i01 i02 i11
-    double4 t1;    // NV_T: i12 i22, 1 / hsml, 0
-    double4 g0;    // grad rho (3), grad P x
-    double4 g1;    // grad P y, z, grad v row 0 (x, y)
-    double4 g2;    // grad v row 0 z, row 1 (x, y, z)
-    double4 g3;    // grad v row 2 (x, y, z), 0
-};
-
-// ForceRec -> the pair-side quantities (moves only)
-__device__ __forceinline__ void unpack_side(const ForceRec &r, PairSide<double> &S)
-{
-    S.v[0] = r.vc.x; S.v[1] = r.vc.y; S.v[2] = r.vc.z; S.cs = r.vc.w;
-    S.h = r.xh.w; S.hinv = r.t1.z;
-    S.rho = r.th.x; S.P = r.th.y; S.V = r.th.z; S.dhsml = r.th.w;
-    S.cn = r.mc.y; S.fce = r.mc.z; S.e = r.mc.w;
-    S.nvt[0] = r.t0.x; S.nvt[1] = r.t0.y; S.nvt[2] = r.t0.z; S.nvt[3] = r.t0.w;
-    S.nvt[4] = r.t1.x; S.nvt[5] = r.t1.y;
-    S.gr[0] = r.g0.x; S.gr[1] = r.g0.y; S.gr[2] = r.g0.z;
-    S.gp[0] = r.g0.w; S.gp[1] = r.g1.x; S.gp[2] = r.g1.y;
-    S.gv[0] = r.g1.z; S.gv[1] = r.g1.w; S.gv[2] = r.g2.x;
-    S.gv[3] = r.g2.y; S.gv[4] = r.g2.z; S.gv[5] = r.g2.w;
-    S.gv[6] = r.g3.x; S.gv[7] = r.g3.y; S.gv[8] = r.g3.z;
-}
+// Per-particle record of the FP64 force loop (beside posm: x, y, z, m), the
+// pair side itself: 34 words, 272 bytes, an odd number of 16-byte chunks, so
+// that the copies of a wavefront's 64 neighbours in LDS meet no bank conflict
+// when each lane reads its own.
+using ForceRec = PairSide<double>;
+static_assert(sizeof(ForceRec) == 272, "34 words");
 
 // Read by the gradient loop for the neighbour j: position and hsml of every
 // candidate (double4, four to a cache line), the rest of each neighbour in one
@@ -342,6 +318,10 @@ struct DeferArgs {
     int q_begin, q_end;    // deferred pairs handled by this round
 };
 
+// Lanes per particle of the three-phase list kernels (each takes every
+// kForceLanes-th pair of the list).
+constexpr int kForceLanes = 8;
+
 struct ForceArgs {
     const BoxDesc *boxes;
     const int *box_of;
@@ -377,7 +357,6 @@ struct ForceArgs {
     F32Geom f32;
     Counters *ctr;
     int block;             // threads per workgroup of the force loop kernel (64 .. kMaxBlock)
-    int lanes;             // lanes per particle of the three-phase list kernels: 1 or 8
 };
 
 // MFV force loop: ParticleVel (3 per particle), the integer timestep of each

@@ -346,16 +346,15 @@ __device__ __forceinline__ ForceRec make_force_rec(const double4 &p, const doubl
                                                    double gamma)
 {
     ForceRec r;
-    r.xh = make_double4(p.x, p.y, p.z, h);
-    r.vc = make_double4(v.x, v.y, v.z, sqrt(gamma * P / d));  // eos.c:245-254
-    r.th = make_double4(d, P, p.w / d, dh);
-    r.mc = make_double4(p.w, cn, fce, P / d);
-    r.t0 = make_double4(t[0], t[1], t[2], t[3]);
-    r.t1 = make_double4(t[4], t[5], 1.0 / h, 0.0);
-    r.g0 = make_double4(g[0], g[1], g[2], g[3]);
-    r.g1 = make_double4(g[4], g[5], g[6], g[7]);
-    r.g2 = make_double4(g[8], g[9], g[10], g[11]);
-    r.g3 = make_double4(g[12], g[13], g[14], 0.0);
+    r.v[0] = v.x; r.v[1] = v.y; r.v[2] = v.z;
+    r.h = h; r.hinv = 1.0 / h;
+    r.rho = d; r.P = P;
+    r.cs = sqrt(gamma * P / d);  // eos.c:245-254
+    r.V = p.w / d; r.dhsml = dh; r.fce = fce;
+    for (int k = 0; k < 6; k++) r.nvt[k] = t[k];
+    for (int k = 0; k < 3; k++) { r.gr[k] = g[k]; r.gp[k] = g[3 + k]; }
+    for (int k = 0; k < 9; k++) r.gv[k] = g[6 + k];
+    r.cn = cn; r.e = P / d;
     return r;
 }
 
@@ -663,8 +662,11 @@ __global__ __launch_bounds__(BS, 3) void gradients_kernel(GradientArgs a)
     if constexpr (G == 1) {
         wave_store_records(stage, a.grad, 15, out_i, valid, g_out);
         if (a.frec_out) {
-            double w[sizeof(ForceRec) / 8];
-            __builtin_memcpy(w, &f_out, sizeof(ForceRec));
+            const ForceRec &r = f_out;
+            const double w[sizeof(ForceRec) / 8] = {
+                r.v[0], r.v[1], r.v[2], r.h, r.hinv, r.rho, r.P, r.cs, r.V, r.dhsml, r.fce, r.nvt[0], r.nvt[1], r.nvt[2],
+                r.nvt[3], r.nvt[4], r.nvt[5], r.gr[0], r.gr[1], r.gr[2], r.gp[0], r.gp[1], r.gp[2], r.gv[0], r.gv[1],
+                r.gv[2], r.gv[3], r.gv[4], r.gv[5], r.gv[6], r.gv[7], r.gv[8], r.cn, r.e};
             wave_store_records(stage, reinterpret_cast<double *>(a.frec_out), sizeof(ForceRec) / 8, out_i, valid, w);
         }
     } else if (valid && sub == 0) {
@@ -695,124 +697,184 @@ __global__ void pack_force_kernel(int n, const double4 *posm, const double4 *vel
 }
 
 
-// One particle's force loop.  USE_LIST: walk the pair list written by the
-// gradient kernel (particles that overflowed it are skipped and left to
-// force_wave_fp64_kernel); otherwise scan the grid or tree (no list: every
-// particle).  Pairs that reach the exact Riemann
-// solver are summed after all other pairs of the particle: THREE_PHASE (list
-// kernel with defer buffers) leaves them to force_deferred_kernel and
-// force_finish_kernel, otherwise the loop walks the pairs a second time and
-// evaluates them in place -- the same order, so every variant gives the same
-// bits.
-template <bool USE_LIST, bool THREE_PHASE>
-__global__ __launch_bounds__((USE_LIST && THREE_PHASE) ? kMaxBlock : kBlock) void force_kernel(ForceArgs a)
+// The force loop over the pair lists (lists of <= 64): pairs that reach the
+// exact Riemann solver (or the KT flux of a failed estimate) are left to
+// force_deferred_kernel and added by force_finish_kernel, after all other pairs
+// of the particle; particles whose list overflowed are left to
+// force_wave_fp64_kernel.
+// Bounded by the latency of the pair's serial arithmetic at two wavefronts per
+// SIMD (vector units 64 % busy; a third would need the records of its 64 pairs
+// in 13 KB of LDS).  33 k particles: 61 us against 145 us with one lane per
+// particle; 2.1 M: 3.43 against 3.38 ms.
+__global__ __launch_bounds__(64, 2) void force_list_kernel(ForceArgs a)
 {
-    const int t = xcd_block() * (int)blockDim.x + threadIdx.x;
+    __shared__ PairLoopLds<ForceRec> lds;
+    const int lane = threadIdx.x, sub = lane % kForceLanes;
+    const int t = xcd_block() * (64 / kForceLanes) + lane / kForceLanes;
     bool valid = t < a.n_active;
-    if (USE_LIST) {
-        if (valid && a.list.count[t] > a.list.cap) {
-            valid = false;
-            if (THREE_PHASE) {  // evaluated by the wavefront loop for long pair sets
+    int n = 0, i = 0;
+    if (valid) {
+        n = a.list.count[t];
+        i = a.active[t];
+        if (n > a.list.cap) {  // evaluated by the wavefront loop for long pair sets
+            if (sub == 0) {
                 a.defer.count[t] = 0;
                 a.defer.raw[t] = 0;
             }
+            valid = false;
         }
     }
+    const double4 pi = a.posm[i];
+    const double rho_i = a.rec[i].rho, cs_i = a.rec[i].cs;
+    const bool live = valid && (pi.w > 0) && (rho_i > 0);
+    if (!live) n = 0;
+    const BoxInfo &box = a.boxes[a.box_of[i]].box;
+    const double L[3] = {box.L[0], box.L[1], box.L[2]};
+    double acc[3] = {0, 0, 0}, dte = 0, out_vsig = cs_i;
+    int status = 0, n_deferred = 0;
+    uint64_t dmask = 0;
+    unsigned long long cnt = 0;
+    ROut<double> ro = {0, 0, {0, 0, 0}, 0};
+    pair_list_loop(lds, a.rec, a.posm, a.list.idx + (size_t)t * a.list.cap, n, i,
+                   [&](const ForceRec &I, const ForceRec &J, const double4 &xj, int j, int k) {
+        double dp[3] = {pi.x - xj.x, pi.y - xj.y, pi.z - xj.z};
+#pragma unroll
+        for (int c = 0; c < 3; c++) dp[c] = wrap_axis(dp[c], L[c], 0.5 * L[c]);
+        const double r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
+        double Fv[3], Fp, vsig;
+        int mask;
+        const int e = force_pair<double, true, false, true>(I, J, dp, r2, a.G, ro, Fv, Fp, vsig, mask);
+        cnt++;
+        if (e == kDeferred) {
+            dmask |= 1ull << k;
+            n_deferred++;
+            return;
+        }
+        if (e > status) status = e;
+        acc[0] += Fv[0];
+        acc[1] += Fv[1];
+        acc[2] += Fv[2];
+        dte += Fp;
+        if (vsig > out_vsig) out_vsig = vsig;
+        if (a.is_active && !a.is_active[j]) {
+            if (vsig > kWakeup * a.vsig_old[j]) a.wakeup[j] = 1;  // WAKEUP (hydro_evaluate.h:485-495)
+        }
+    });
+    if (status) atomicMax(&ctr_slot(a.ctr)->status, status);
+    for (int c = 0; c < 3; c++) acc[c] = group_sum<kForceLanes>(acc[c]);
+    dte = group_sum<kForceLanes>(dte);
+    out_vsig = group_max<kForceLanes>(out_vsig);
+    dmask = group_or<kForceLanes>(dmask);
+    n_deferred = group_sum_int<kForceLanes>(n_deferred);
+    if (valid && sub == 0) {
+        if (live) {
+            // raw sums: finished by force_finish_kernel after the deferred pairs
+            a.defer.mask[t] = dmask;
+        } else {
+            if (pi.w > 0) dte /= pi.w;
+            out_vsig = kMinReal;
+        }
+        a.defer.count[t] = n_deferred;
+        a.defer.raw[t] = live ? 1 : 0;
+        a.acc[3 * (size_t)i + 0] = acc[0];
+        a.acc[3 * (size_t)i + 1] = acc[1];
+        a.acc[3 * (size_t)i + 2] = acc[2];
+        a.dtu[i] = dte;
+        a.vsig[i] = out_vsig;
+    }
+    wave_add_u64(&ctr_slot(a.ctr)->interactions, cnt);
+}
+
+// One lane's force loop where no list of at most 64 pairs holds the set.
+// USE_LIST: walk the pair list written by the gradient kernel (particles that
+// overflowed it are skipped and left to force_wave_fp64_kernel); otherwise scan
+// the grid or tree (no list: every particle).  Pairs that reach the exact
+// Riemann solver are summed after all other pairs of the particle, in a second
+// walk over the pairs.
+template <bool USE_LIST>
+__global__ __launch_bounds__(kBlock) void force_kernel(ForceArgs a)
+{
+    const int t = xcd_block() * (int)blockDim.x + threadIdx.x;
+    bool valid = t < a.n_active;
+    if (USE_LIST && valid && a.list.count[t] > a.list.cap) valid = false;
     unsigned long long cnt = 0, nretry = 0, nexact = 0;
     for_box(a.boxes, a.box_of, valid ? a.active[t] : 0, valid, [&](const BoxDesc &G) {
         const int i = a.active[t];
-        const ForceRec ri = a.rec[i];
+        const double4 pi = a.posm[i];
         double acc[3] = {0, 0, 0}, dte = 0, vmax = kMinReal;
-        const double m_i = ri.mc.x, rho_i = ri.th.x;
+        const double m_i = pi.w;
+        const ForceRec I = a.rec[i];
         int status = 0;
-        uint64_t dmask = 0;
-        if ((m_i > 0) && (rho_i > 0)) {
-            PairI<double> I;
-            unpack_side(ri, I);
-            const double x_i[3] = {ri.xh.x, ri.xh.y, ri.xh.z};
-            I.hinv3 = I.hinv * I.hinv * I.hinv;
-            I.hinv4 = I.hinv3 * I.hinv;
-            I.cnumcrit2 = kCondDanger * kCondDanger - I.cn * I.cn;
+        if ((m_i > 0) && (I.rho > 0)) {
+            const double x_i[3] = {pi.x, pi.y, pi.z};
             double out_vsig = I.cs;
             ROut<double> ro = {0, 0, {0, 0, 0}, 0};
             const double h2_i = I.h * I.h;
-            int n_deferred = 0;
-            auto add = [&](int j, const double Fv[3], double Fp, double vsig, int mask, int e) {
+            int n_deferred = 0, k_pair = 0;
+            // the sums of force_list_kernel's lanes, added up in its order
+            double part[kForceLanes][4] = {};
+            auto add = [&](double *sum, int j, const double Fv[3], double Fp, double vsig, int mask, int e) {
                 if (e > status) status = e;
                 nretry += (mask & 8) ? 1 : 0;
                 nexact += (mask & 4) ? 1 : 0;
-                acc[0] += Fv[0];
-                acc[1] += Fv[1];
-                acc[2] += Fv[2];
-                dte += Fp;
+                for (int c = 0; c < 3; c++) sum[c] += Fv[c];
+                sum[3] += Fp;
                 if (vsig > out_vsig) out_vsig = vsig;
                 if (a.is_active && !a.is_active[j]) {
                     if (vsig > kWakeup * a.vsig_old[j]) a.wakeup[j] = 1;  // WAKEUP (hydro_evaluate.h:485-495)
                 }
             };
             // pass 0: every pair but the deferred ones; pass 1: only those
-            auto visit = [&](int j, int k, bool check, int pass) {
-                const double4 xj = a.rec[j].xh;
+            auto visit = [&](int j, bool check, int pass) {
+                const double4 xj = a.posm[j];
                 double dp[3] = {x_i[0] - xj.x, x_i[1] - xj.y, x_i[2] - xj.z};
                 wrap_dp(G.box, dp);
                 const double r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
+                const ForceRec J = a.rec[j];
                 if (check) {
-                    const double h_j = xj.w;
-                    if ((r2 >= h2_i) && (r2 >= h_j * h_j)) return;
+                    if ((r2 >= h2_i) && (r2 >= J.h * J.h)) return;
                     if (r2 <= 0) return;
-                    if (!(a.rec[j].mc.x > 0) || !(a.rec[j].th.x > 0)) return;  // hydro_evaluate.h:149-150
+                    if (!(xj.w > 0) || !(J.rho > 0)) return;  // hydro_evaluate.h:149-150
                 }
-                PairSide<double> J;
-                unpack_side(a.rec[j], J);
                 double Fv[3], Fp, vsig;
                 int mask;
                 const int e = force_pair<double, true>(I, J, dp, r2, a.G, ro, Fv, Fp, vsig, mask);
                 if (pass == 0) {
                     cnt++;
+                    const int k = k_pair++;
                     if (e == kDeferred) {
-                        if (THREE_PHASE) dmask |= 1ull << k;
                         n_deferred++;
                         return;
                     }
-                    add(j, Fv, Fp, vsig, mask, e);
-                } else if (!THREE_PHASE && e == kDeferred) {
+                    add(part[k % kForceLanes], j, Fv, Fp, vsig, mask, e);
+                } else if (e == kDeferred) {
                     const int e2 = force_pair<double, false>(I, J, dp, r2, a.G, ro, Fv, Fp, vsig, mask);
-                    add(j, Fv, Fp, vsig, mask, e2);
+                    add(part[0], j, Fv, Fp, vsig, mask, e2);
                 }
             };
             for (int pass = 0; pass < 2; pass++) {
-                if (pass == 1 && (THREE_PHASE || n_deferred == 0)) break;
+                if (pass == 1) {
+                    for (int off = kForceLanes / 2; off > 0; off >>= 1)
+                        for (int l = 0; l < off; l++)
+                            for (int c = 0; c < 4; c++) part[l][c] += part[l + off][c];
+                    if (n_deferred == 0) break;
+                }
                 if (USE_LIST) {
                     // the list holds the pair set in the gradient kernel's scan order,
                     // which is this kernel's scan order as well (same predicate, same R)
                     const int n = a.list.count[t];
                     const int *row = a.list.idx + (size_t)t * a.list.cap;
-                    for (int k = 0; k < n; k++) visit(row[k], k, false, pass);
+                    for (int k = 0; k < n; k++) visit(row[k], false, pass);
                 } else {
-                    for_each_neighbour_candidate(a.tree, G, x_i, I.h, true, [&](int j) { visit(j, 0, true, pass); });
+                    for_each_neighbour_candidate(a.tree, G, x_i, I.h, true, [&](int j) { visit(j, true, pass); });
                 }
             }
-            if (THREE_PHASE) {
-                // raw sums: finished by force_finish_kernel after the deferred pairs
-                a.acc[3 * (size_t)i + 0] = acc[0];
-                a.acc[3 * (size_t)i + 1] = acc[1];
-                a.acc[3 * (size_t)i + 2] = acc[2];
-                a.dtu[i] = dte;
-                a.vsig[i] = out_vsig;
-                a.defer.mask[t] = dmask;
-                a.defer.count[t] = n_deferred;
-                a.defer.raw[t] = 1;
-                if (status) atomicMax(&ctr_slot(a.ctr)->status, status);
-                return;
-            }
+            for (int c = 0; c < 3; c++) acc[c] = part[0][c];
+            dte = part[0][3];
             if (vmax < out_vsig) vmax = out_vsig;
             force_final_ops(acc, dte, I.v, m_i, I.h, a.max_hsml);
         } else if (m_i > 0) {
             dte /= m_i;
-        }
-        if (THREE_PHASE) {
-            a.defer.count[t] = 0;
-            a.defer.raw[t] = 0;
         }
         a.acc[3 * (size_t)i + 0] = acc[0];
         a.acc[3 * (size_t)i + 1] = acc[1];
@@ -837,18 +899,11 @@ __global__ __launch_bounds__(kBlock) void force_deferred_kernel(ForceArgs a)
     unsigned long long nretry = 0, nexact = 0;
     for_box(a.boxes, a.box_of, ij.x, valid, [&](const BoxDesc &G) {
         const int i = ij.x, j = ij.y;
-        const ForceRec ri = a.rec[i];
-        PairI<double> I;
-        unpack_side(ri, I);
-        I.hinv3 = I.hinv * I.hinv * I.hinv;
-        I.hinv4 = I.hinv3 * I.hinv;
-        I.cnumcrit2 = kCondDanger * kCondDanger - I.cn * I.cn;
-        const double4 xj = a.rec[j].xh;
-        double dp[3] = {ri.xh.x - xj.x, ri.xh.y - xj.y, ri.xh.z - xj.z};
+        const ForceRec I = a.rec[i], J = a.rec[j];
+        const double4 pi = a.posm[i], xj = a.posm[j];
+        double dp[3] = {pi.x - xj.x, pi.y - xj.y, pi.z - xj.z};
         wrap_dp(G.box, dp);
         const double r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
-        PairSide<double> J;
-        unpack_side(a.rec[j], J);
         ROut<double> ro = {0, 0, {0, 0, 0}, 0};
         double Fv[3], Fp, vsig;
         int mask;
@@ -1067,15 +1122,12 @@ void launch_pack_force(hipStream_t s, int n, const double4 *posm, const double4 
 void launch_force(hipStream_t s, const ForceArgs &a)
 {
     if (a.n_active <= 0) return;
-    // only the three-phase list kernel takes workgroups above kBlock
-    const int b = (a.list.idx && a.defer.mask) ? a.block : min(a.block, kBlock);
+    const int b = min(a.block, kBlock);
     const dim3 grid(nblocks(a.n_active, b)), block(b);
-    if (a.list.idx) {
-        if (a.defer.mask) hipLaunchKernelGGL((force_kernel<true, true>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((force_kernel<true, false>), grid, block, 0, s, a);
-    } else {
-        hipLaunchKernelGGL((force_kernel<false, false>), grid, block, 0, s, a);
-    }
+    if (a.list.idx && a.defer.mask)
+        hipLaunchKernelGGL(force_list_kernel, dim3(nblocks((long long)kForceLanes * a.n_active, 64)), dim3(64), 0, s, a);
+    else if (a.list.idx) hipLaunchKernelGGL(force_kernel<true>, grid, block, 0, s, a);
+    else hipLaunchKernelGGL(force_kernel<false>, grid, block, 0, s, a);
 }
 namespace {
 

@@ -30,36 +30,31 @@ __global__ void mfv_preloop_kernel(int n_active, const int *active, MfvArgs m)
     for (int k = 0; k < 3; k++) m.grav_work[3 * (size_t)i + k] = 0;
 }
 
-// i's side of an MFV pair
-struct MfvSide {
-    PairI<double> I;
+// i's values of an MFV pair beside its record
+struct MfvOwn {
     double w[3];   // ParticleVel
     double ti, dt; // integer timestep (as a double) and physical timestep
     double m;
 };
 
-__device__ __forceinline__ void mfv_side(const ForceArgs &a, const MfvArgs &m, int i, const ForceRec &ri, MfvSide &S)
+__device__ __forceinline__ void mfv_own(const ForceArgs &a, const MfvArgs &m, int i, MfvOwn &S)
 {
-    unpack_side(ri, S.I);
-    S.I.hinv3 = S.I.hinv * S.I.hinv * S.I.hinv;
-    S.I.hinv4 = S.I.hinv3 * S.I.hinv;
-    S.I.cnumcrit2 = kCondDanger * kCondDanger - S.I.cn * S.I.cn;
     for (int k = 0; k < 3; k++) S.w[k] = m.pvel[3 * (size_t)i + k];
     S.ti = m.ti ? m.ti[i] : 1.0;
     S.dt = S.ti * m.timebase;  // hydro_evaluate.h:82
-    S.m = ri.mc.x;
+    S.m = a.posm[i].w;
 }
 
 // The mass exchange of one pair (hydro_evaluate.h:379-392) with the
 // reference's 10 % limiter; j_is_active_for_fluxes is always 0 there
 // (hydro_evaluate.h:158-168): a smaller step than j's gives j the whole
 // share, an equal step half of it.  Returns i's share; j's goes to j now.
-__device__ __forceinline__ double mfv_mass_exchange(const ForceArgs &a, const MfvArgs &m, const MfvSide &S, int j,
+__device__ __forceinline__ double mfv_mass_exchange(const ForceArgs &a, const MfvArgs &m, const MfvOwn &S, int j,
                                                     double Frho)
 {
     const double ti_j = m.ti ? m.ti[j] : 1.0;
     double dmh = Frho * S.dt, lim;
-    if (dmh > 0) lim = a.rec[j].mc.x; else lim = S.m;
+    if (dmh > 0) lim = a.posm[j].w; else lim = S.m;
     lim *= 0.1;
     if (fabs(dmh) > lim) dmh *= lim / fabs(dmh);
     double own = 0;
@@ -95,71 +90,133 @@ __device__ __forceinline__ void mfv_store(const ForceArgs &a, const MfvArgs &m, 
     for (int k = 0; k < 3; k++) m.grav_work[3 * (size_t)i + k] = gw[k];
 }
 
-// One active particle's MFV force loop (hydro_evaluate.h:146-498).
-// THREE_PHASE (pair lists of <= 64): walk the gradient kernel's pair list,
-// leave the pairs that reach the exact Riemann solver to
-// force_mfv_deferred_kernel (bit k of the particle's defer mask) and the
-// particles whose pair set overflowed the list to this kernel's scanning
-// form; write raw sums for force_mfv_finish_kernel.  Otherwise (the scanning
-// form) every pair in place, in one pass, with the final operations: over
-// every active particle (USE_LIST: the pair list where it holds the whole
-// set), or over rows[0, *n_rows) (active entries), striding.
-template <bool USE_LIST, bool THREE_PHASE>
-__global__ __launch_bounds__(THREE_PHASE ? kMaxBlock : kBlock) void force_mfv_kernel(ForceArgs a, MfvArgs m,
-                                                                                    const int *rows,
-                                                                                    const int *n_rows)
+// The MFV force loop (hydro_evaluate.h:146-498) over the pair lists (lists of
+// <= 64): pairs that reach the exact Riemann solver are left to
+// force_mfv_deferred_kernel (bit k of the particle's defer mask) and particles
+// whose pair set overflowed the list to force_mfv_kernel; raw sums go to
+// force_mfv_finish_kernel.  384 k particles: 1.37 ms against 1.79 ms with one lane
+// per particle, whose two records and nine sums spilled 82 registers.
+__global__ __launch_bounds__(64, 2) void force_mfv_list_kernel(ForceArgs a, MfvArgs m)
+{
+    __shared__ PairLoopLds<ForceRec> lds;
+    const int lane = threadIdx.x, sub = lane % kForceLanes;
+    const int t = xcd_block() * (64 / kForceLanes) + lane / kForceLanes;
+    bool valid = t < a.n_active;
+    int n = 0, i = 0;
+    if (valid) {
+        n = a.list.count[t];
+        i = a.active[t];
+        if (n > a.list.cap) {  // evaluated by the scanning form
+            if (sub == 0) {
+                a.defer.count[t] = 0;
+                a.defer.raw[t] = 0;
+            }
+            valid = false;
+        }
+    }
+    const double4 pi = a.posm[i];
+    const double rho_i = a.rec[i].rho, cs_i = a.rec[i].cs;
+    const bool live = valid && (pi.w > 0) && (rho_i > 0);
+    if (!live) n = 0;
+    MfvOwn own;
+    mfv_own(a, m, i, own);
+    const BoxInfo &box = a.boxes[a.box_of[i]].box;
+    const double L[3] = {box.L[0], box.L[1], box.L[2]};
+    double acc[3] = {0, 0, 0}, dte = 0, dtm = 0, dm = 0, gw[3] = {0, 0, 0}, out_vsig = cs_i;
+    int status = 0, n_deferred = 0;
+    uint64_t dmask = 0;
+    unsigned long long cnt = 0;
+    pair_list_loop(lds, a.rec, a.posm, a.list.idx + (size_t)t * a.list.cap, n, i,
+                   [&](const ForceRec &I, const ForceRec &J, const double4 &xj, int j, int k) {
+        double dp[3] = {pi.x - xj.x, pi.y - xj.y, pi.z - xj.z};
+#pragma unroll
+        for (int c = 0; c < 3; c++) dp[c] = wrap_axis(dp[c], L[c], 0.5 * L[c]);
+        const double r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
+        double Fv[3], Fp, Frho, vsig;
+        int mask;
+        const int e = force_pair_mfv<true, false, true>(I, J, own.w, dp, r2, a.G, Fv, Fp, Frho, vsig, mask);
+        cnt++;
+        if (e == kDeferred) {
+            dmask |= 1ull << k;
+            n_deferred++;
+            return;
+        }
+        if (e > status) status = e;
+        dm += mfv_mass_exchange(a, m, own, j, Frho);
+        dtm += Frho;
+        for (int c = 0; c < 3; c++) gw[c] += Frho * dp[c];
+        for (int c = 0; c < 3; c++) acc[c] += Fv[c];
+        dte += Fp;
+        if (vsig > out_vsig) out_vsig = vsig;
+        if (a.is_active && !a.is_active[j]) {
+            if (vsig > kWakeup * a.vsig_old[j]) a.wakeup[j] = 1;  // WAKEUP (hydro_evaluate.h:485-495)
+        }
+    });
+    if (status) atomicMax(&ctr_slot(a.ctr)->status, status);
+    for (int c = 0; c < 3; c++) acc[c] = group_sum<kForceLanes>(acc[c]);
+    for (int c = 0; c < 3; c++) gw[c] = group_sum<kForceLanes>(gw[c]);
+    dte = group_sum<kForceLanes>(dte);
+    dtm = group_sum<kForceLanes>(dtm);
+    dm = group_sum<kForceLanes>(dm);
+    out_vsig = group_max<kForceLanes>(out_vsig);
+    dmask = group_or<kForceLanes>(dmask);
+    n_deferred = group_sum_int<kForceLanes>(n_deferred);
+    if (valid && sub == 0) {
+        if (live) a.defer.mask[t] = dmask;
+        a.defer.count[t] = n_deferred;
+        a.defer.raw[t] = live ? 1 : 0;
+        atomicAdd(&m.d_mass[i], dm);
+        mfv_store(a, m, i, acc, dte, live ? out_vsig : kMinReal, dtm, gw, !live);
+    }
+    wave_add_u64(&ctr_slot(a.ctr)->interactions, cnt);
+}
+
+// The scanning form, one particle per lane: every pair in place, in one pass,
+// with the final operations, over every active particle (USE_LIST: the pair list
+// where it holds the whole set), or over rows[0, *n_rows) (active entries),
+// striding.
+template <bool USE_LIST>
+__global__ __launch_bounds__(kBlock) void force_mfv_kernel(ForceArgs a, MfvArgs m, const int *rows, const int *n_rows)
 {
     const int n = rows ? *n_rows : a.n_active;
     const int stride = (int)(gridDim.x * blockDim.x);
     unsigned long long cnt = 0, nretry = 0, nexact = 0;
     for (int base = xcd_block() * (int)blockDim.x; base < n; base += stride) {
         const int q = base + (int)threadIdx.x;
-        bool valid = q < n;
+        const bool valid = q < n;
         const int t = valid ? (rows ? rows[q] : q) : 0;
         const bool listed = USE_LIST && valid && a.list.count[t] <= a.list.cap;
-        if (THREE_PHASE && valid && !listed) {  // evaluated by the scanning form
-            valid = false;
-            a.defer.count[t] = 0;
-            a.defer.raw[t] = 0;
-        }
         for_box(a.boxes, a.box_of, valid ? a.active[t] : 0, valid, [&](const BoxDesc &G) {
             const int i = a.active[t];
-            const ForceRec ri = a.rec[i];
-            MfvSide S;
-            mfv_side(a, m, i, ri, S);
+            const double4 pi = a.posm[i];
+            const ForceRec I = a.rec[i];
+            MfvOwn own;
+            mfv_own(a, m, i, own);
             double acc[3] = {0, 0, 0}, dte = 0, dtm = 0, dm = 0, gw[3] = {0, 0, 0}, vmax = kMinReal;
-            int status = 0, n_deferred = 0;
-            uint64_t dmask = 0;
-            if ((S.m > 0) && (ri.th.x > 0)) {
-                double out_vsig = S.I.cs;
-                const double x_i[3] = {ri.xh.x, ri.xh.y, ri.xh.z};
-                const double h2_i = S.I.h * S.I.h;
-                auto visit = [&](int j, int k, bool check) {
-                    const double4 xj = a.rec[j].xh;
+            int status = 0;
+            if ((own.m > 0) && (I.rho > 0)) {
+                double out_vsig = I.cs;
+                const double x_i[3] = {pi.x, pi.y, pi.z};
+                const double h2_i = I.h * I.h;
+                auto visit = [&](int j, bool check) {
+                    const double4 xj = a.posm[j];
+                    const ForceRec J = a.rec[j];
                     double dp[3] = {x_i[0] - xj.x, x_i[1] - xj.y, x_i[2] - xj.z};
                     wrap_dp(G.box, dp);
                     const double r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
                     if (check) {
-                        const double h_j = xj.w;
-                        if ((r2 >= h2_i) && (r2 >= h_j * h_j)) return;
+                        if ((r2 >= h2_i) && (r2 >= J.h * J.h)) return;
                         if (r2 <= 0) return;
-                        if (!(a.rec[j].mc.x > 0) || !(a.rec[j].th.x > 0)) return;  // hydro_evaluate.h:149-150
+                        if (!(xj.w > 0) || !(J.rho > 0)) return;  // hydro_evaluate.h:149-150
                     }
-                    PairSide<double> J;
-                    unpack_side(a.rec[j], J);
                     double Fv[3], Fp, Frho, vsig;
                     int mask;
-                    const int e = force_pair_mfv<THREE_PHASE>(S.I, J, S.w, dp, r2, a.G, Fv, Fp, Frho, vsig, mask);
+                    const int e = force_pair_mfv<false>(I, J, own.w, dp, r2, a.G, Fv, Fp, Frho, vsig, mask);
                     cnt++;
-                    if (THREE_PHASE && e == kDeferred) {
-                        dmask |= 1ull << k;
-                        n_deferred++;
-                        return;
-                    }
                     if (e > status) status = e;
                     nretry += (mask & 8) ? 1 : 0;
                     nexact += (mask & 4) ? 1 : 0;
-                    dm += mfv_mass_exchange(a, m, S, j, Frho);
+                    dm += mfv_mass_exchange(a, m, own, j, Frho);
                     dtm += Frho;
                     for (int c = 0; c < 3; c++) gw[c] += Frho * dp[c];
                     for (int c = 0; c < 3; c++) acc[c] += Fv[c];
@@ -172,25 +229,11 @@ __global__ __launch_bounds__(THREE_PHASE ? kMaxBlock : kBlock) void force_mfv_ke
                 if (listed) {
                     const int nl = a.list.count[t];
                     const int *row = a.list.idx + (size_t)t * a.list.cap;
-                    for (int k = 0; k < nl; k++) visit(row[k], k, false);
+                    for (int k = 0; k < nl; k++) visit(row[k], false);
                 } else {
-                    for_each_neighbour_candidate(a.tree, G, x_i, S.I.h, true, [&](int j) { visit(j, 0, true); });
-                }
-                if (THREE_PHASE) {
-                    // raw sums; force_mfv_finish_kernel adds the deferred pairs and finishes
-                    atomicAdd(&m.d_mass[i], dm);
-                    mfv_store(a, m, i, acc, dte, out_vsig, dtm, gw, false);
-                    a.defer.mask[t] = dmask;
-                    a.defer.count[t] = n_deferred;
-                    a.defer.raw[t] = 1;
-                    if (status) atomicMax(&ctr_slot(a.ctr)->status, status);
-                    return;
+                    for_each_neighbour_candidate(a.tree, G, x_i, I.h, true, [&](int j) { visit(j, true); });
                 }
                 if (vmax < out_vsig) vmax = out_vsig;
-            }
-            if (THREE_PHASE) {
-                a.defer.count[t] = 0;
-                a.defer.raw[t] = 0;
             }
             atomicAdd(&m.d_mass[i], dm);
             mfv_store(a, m, i, acc, dte, vmax, dtm, gw, true);
@@ -215,21 +258,20 @@ __global__ __launch_bounds__(kBlock) void force_mfv_deferred_kernel(ForceArgs a,
     unsigned long long nretry = 0, nexact = 0;
     for_box(a.boxes, a.box_of, ij.x, valid, [&](const BoxDesc &G) {
         const int i = ij.x, j = ij.y;
-        const ForceRec ri = a.rec[i];
-        MfvSide S;
-        mfv_side(a, m, i, ri, S);
-        const double4 xj = a.rec[j].xh;
-        double dp[3] = {ri.xh.x - xj.x, ri.xh.y - xj.y, ri.xh.z - xj.z};
+        MfvOwn own;
+        mfv_own(a, m, i, own);
+        const ForceRec I = a.rec[i];
+        const double4 pi = a.posm[i], xj = a.posm[j];
+        double dp[3] = {pi.x - xj.x, pi.y - xj.y, pi.z - xj.z};
         wrap_dp(G.box, dp);
         const double r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
-        PairSide<double> J;
-        unpack_side(a.rec[j], J);
+        const ForceRec J = a.rec[j];
         double Fv[3], Fp, Frho, vsig;
         int mask;
-        const int e = force_pair_mfv<false, true>(S.I, J, S.w, dp, r2, a.G, Fv, Fp, Frho, vsig, mask);
+        const int e = force_pair_mfv<false, true>(I, J, own.w, dp, r2, a.G, Fv, Fp, Frho, vsig, mask);
         nretry += (mask & 8) ? 1 : 0;
         nexact += (mask & 4) ? 1 : 0;
-        atomicAdd(&m.d_mass[i], mfv_mass_exchange(a, m, S, j, Frho));
+        atomicAdd(&m.d_mass[i], mfv_mass_exchange(a, m, own, j, Frho));
         double *o = a.defer.result + 9 * (size_t)(q - a.defer.q_begin);
         o[0] = Fv[0]; o[1] = Fv[1]; o[2] = Fv[2]; o[3] = Fp; o[4] = Frho; o[5] = vsig;
         o[6] = Frho * dp[0]; o[7] = Frho * dp[1]; o[8] = Frho * dp[2];
@@ -344,14 +386,13 @@ void launch_force_mfv(hipStream_t s, const ForceArgs &a, const MfvArgs &m)
 {
     if (a.n_active <= 0) return;
     if (a.list.idx && a.defer.mask) {
-        const int b = a.block;
-        hipLaunchKernelGGL((force_mfv_kernel<true, true>), dim3((unsigned)((a.n_active + b - 1) / b)), dim3(b), 0, s, a,
-                           m, (const int *)nullptr, (const int *)nullptr);
+        const long long lanes = (long long)kForceLanes * a.n_active;
+        hipLaunchKernelGGL(force_mfv_list_kernel, dim3((unsigned)((lanes + 63) / 64)), dim3(64), 0, s, a, m);
     } else if (a.list.idx) {
-        hipLaunchKernelGGL((force_mfv_kernel<true, false>), dim3(nblocks_mfv(a.n_active)), dim3(kBlock), 0, s, a, m,
+        hipLaunchKernelGGL(force_mfv_kernel<true>, dim3(nblocks_mfv(a.n_active)), dim3(kBlock), 0, s, a, m,
                            (const int *)nullptr, (const int *)nullptr);
     } else {
-        hipLaunchKernelGGL((force_mfv_kernel<false, false>), dim3(nblocks_mfv(a.n_active)), dim3(kBlock), 0, s, a, m,
+        hipLaunchKernelGGL(force_mfv_kernel<false>, dim3(nblocks_mfv(a.n_active)), dim3(kBlock), 0, s, a, m,
                            (const int *)nullptr, (const int *)nullptr);
     }
 }
@@ -362,7 +403,7 @@ void launch_force_mfv_overflow(hipStream_t s, const ForceArgs &a, const MfvArgs 
     hipLaunchKernelGGL(collect_overflow_rows_kernel, dim3(nblocks_mfv(a.n_active)), dim3(kBlock), 0, s, a.n_active,
                        a.list.count, a.list.cap, rows, n_rows);
     // a fixed grid strides over the rows, whose count is on the device
-    hipLaunchKernelGGL((force_mfv_kernel<false, false>), dim3(1024), dim3(kBlock), 0, s, a, m, (const int *)rows,
+    hipLaunchKernelGGL(force_mfv_kernel<false>, dim3(1024), dim3(kBlock), 0, s, a, m, (const int *)rows,
                        (const int *)n_rows);
 }
 

@@ -50,6 +50,71 @@ template <> struct Real<float> {
     static __device__ __forceinline__ float root(float a) { return __builtin_amdgcn_sqrtf(a); }
 };
 
+// ---------------------------------------------------------------------------
+// FP64 arithmetic of the pair fluxes.  The force loops are bound by VALU issue
+// (about 1,000 instructions per pair step before), much of it IEEE division (11
+// instructions), square root (about 18), products and sums rounded apart, and
+// 64-bit selects.  Written out here: fused multiply-adds (never less exact than
+// a product and a sum), one reciprocal for quotients of one denominator, each
+// quotient corrected by its residual (the steps, and so the bits, of the
+// compiler's division without its scaling for extreme exponents), square root
+// (likewise) and reciprocal root from one v_rsq_f64.  The fusing is explicit,
+// not left to the compiler, so that a pair gives the same bits in every kernel;
+// the Riemann solver's own products and sums stay apart, it gives the
+// reference's bits on given states.
+// FP32 keeps separate products and sums: fma1(a, b, c) is a * b + c there.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ double fma1(double a, double b, double c) { return fma(a, b, c); }
+__device__ __forceinline__ float fma1(float a, float b, float c) { return a * b + c; }
+
+// whether x > 0 lies where the sequences below neither overflow nor underflow
+__device__ __forceinline__ bool plain_range(double x) { return x > 1e-280 && x < 1e280; }
+
+// 1 / x for normal x (two Newton steps on v_rcp_f64)
+__device__ __forceinline__ double rcp_newton(double x)
+{
+    double y = __builtin_amdgcn_rcp(x);
+    y = fma(y, fma(-x, y, 1.0), y);
+    return fma(y, fma(-x, y, 1.0), y);
+}
+
+// a / x given y = rcp_newton(x)
+__device__ __forceinline__ double quotient(double a, double x, double y)
+{
+    const double q = a * y;
+    return fma(fma(-x, q, a), y, q);
+}
+
+// sqrt(x) and 1 / sqrt(x) for x in plain_range
+__device__ __forceinline__ void root_newton(double x, double &r, double &rinv)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    double d = fma(-h, g, 0.5);
+    g = fma(g, d, g);
+    h = fma(h, d, h);
+    d = fma(-g, g, x);
+    g = fma(d, h, g);
+    d = fma(-g, g, x);
+    r = fma(d, h, g);
+    h = h + h;
+    rinv = fma(h, fma(-r, h, 1.0), h);
+}
+
+// the same for any x
+template <typename T>
+__device__ __forceinline__ void root_and_inverse(T x, T &r, T &rinv)
+{
+    if constexpr (sizeof(T) == sizeof(double)) {
+        if (plain_range(x)) {
+            root_newton(x, r, rinv);
+            return;
+        }
+    }
+    r = Real<T>::root(x);
+    rinv = Real<T>::rcp(r);
+}
+
 // reimann.h:1-10 for the run's adiabatic index
 struct GammaConsts {
     double G0, G1, G2, G3, G4, G5, G6, G7, G8, G9;
@@ -83,12 +148,18 @@ __device__ __forceinline__ void kernel_hinv(T h, T &hinv, T &hinv3, T &hinv4)
     hinv4 = hinv3 * hinv;
 }
 
-template <typename T>
+template <bool FUSED = false, typename T>
 __device__ __forceinline__ void kernel_wdw(T u, T hinv3, T hinv4, T &wk, T &dwk)
 {
     if (u >= 1) { wk = 0; dwk = 0; return; }
     T w, dw;
-    if (u < T(0.5)) {
+    if constexpr (FUSED) {
+        // both pieces and a select: the lanes of a wavefront take both anyway
+        const T t = T(1.0) - u, t2 = t * t;
+        const bool inner = u < T(0.5);
+        dw = inner ? u * fma1(T(18.0), u, T(-12.0)) : T(-6.0) * t2;
+        w = inner ? fma1(T(-6.0) * (t * u), u, T(1.0)) : T(2.0) * t2 * t;
+    } else if (u < T(0.5)) {
         dw = u * (T(18.0) * u - T(12.0));
         w = (T(1.0) + T(6.0) * (u - T(1.0)) * u * u);
     } else {
@@ -432,11 +503,64 @@ __device__ __forceinline__ bool near_threshold(T x, T threshold, T scale)
 // returns true when that crossing lies within kDecideMargin of (Qmax - Qmin),
 // where the rounded operands may take the other side than in FP64.
 // ---------------------------------------------------------------------------
+//
+// FP64, the same limiter without branches.  Values of one sign are reflected to
+// the positive side, where only the lower bound can need the sign-preserving
+// quotient; for values on both sides of zero lo <= 0 <= hi and none does.  The
+// remaining minima and maxima of the general form (of Qmed_max with Qmax_eff, of
+// Qmed_min with Qmin_eff) never bind.  They drop a NaN extrapolation, which
+// keep_nan puts back; `odd` collects xR + xL to find one.
+__device__ __forceinline__ void extrapolate(double Qi, const double gi[3], double Qj, const double gj[3],
+                                            const double di[3], const double dj[3], double &xR, double &xL)
+{
+    xR = fma(gi[2], di[2], fma(gi[1], di[1], fma(gi[0], di[0], Qi)));
+    xL = fma(gj[2], dj[2], fma(gj[1], dj[1], fma(gj[0], dj[0], Qj)));
+}
+
+__device__ __forceinline__ double flip(double x, uint32_t sign)
+{
+    return __hiloint2double((int)((uint32_t)__double2hiint(x) ^ sign), __double2loint(x));
+}
+
+__device__ __forceinline__ void reconstruct_fp64(double Qi, const double gi[3], double Qj, const double gj[3],
+                                                 const double di[3], const double dj[3], double &QL, double &QR,
+                                                 double &odd)
+{
+    double xR, xL;
+    extrapolate(Qi, gi, Qj, gj, di, dj, xR, xL);
+    odd += xR + xL;
+    const double sum = Qi + Qj;
+    const bool neg = sum < 0;
+    const uint32_t sign = neg ? 0x80000000u : 0u;
+    const double a_i = flip(Qi, sign), a_j = flip(Qj, sign);
+    const double lo = fmin(a_i, a_j), hi = fmax(a_i, a_j);
+    const double dQ = hi - lo, med = 0.5 * fabs(sum);
+    const double e = fma(-0.5, dQ, lo), den = fmax(fma(0.5, dQ, lo), 1e-290);
+    const double b = quotient(lo * lo, den, rcp_newton(den));
+    const double lo_eff = (lo > 0 && e < 0) ? b : e, hi_eff = fma(0.5, dQ, hi);
+    const bool up = a_i < a_j;  // the R value is the lower of the two
+    xR = flip(xR, sign);
+    xL = flip(xL, sign);
+    const double rlo = fmin(fmax(up ? xR : xL, lo_eff), fma(0.375, dQ, med));
+    const double rhi = fmax(fmin(up ? xL : xR, hi_eff), fma(-0.375, dQ, med));
+    QR = flip(up ? rlo : rhi, sign);
+    QL = flip(up ? rhi : rlo, sign);
+}
+
+__device__ __forceinline__ void keep_nan(double Qi, const double gi[3], double Qj, const double gj[3],
+                                         const double di[3], const double dj[3], double &QL, double &QR)
+{
+    if (Qi == Qj) return;
+    double xR, xL;
+    extrapolate(Qi, gi, Qj, gj, di, dj, xR, xL);
+    if (isnan(xR)) QR = xR;
+    if (isnan(xL)) QL = xL;
+}
+
 template <typename T>
 __device__ __forceinline__ bool reconstruct(T Qi, const T gi[3], T Qj, const T gj[3], const T di[3], const T dj[3],
-                                            T &QL, T &QR, int mode)
+                                            T &QL, T &QR)
 {
-    if (mode == 0) { QR = Qi; QL = Qj; return false; }
     if (Qi == Qj) { QL = QR = Qi; return false; }
     QR = Qi + gi[0] * di[0] + gi[1] * di[1] + gi[2] * di[2];
     QL = Qj + gj[0] * dj[0] + gj[1] * dj[1] + gj[2] * dj[2];
@@ -491,10 +615,43 @@ struct ROut {
 //
 // S_LR (may be null): the outer wave speeds of the estimate that stands (both
 // 0 on the vacuum test and where P_M is floored), which the MFV fluxes read.
+//
+// Specific enthalpies of the two states, wanted only by the Roe estimate and
+// the KT flux.
+template <typename T>
+__device__ __forceinline__ void enthalpies(const RState<T> &L, const RState<T> &R, const GammaConsts &G, T &hL, T &hR)
+{
+    using M = Real<T>;
+    const T uL = M::div(L.p, (T(G.G9) * L.rho));
+    const T uR = M::div(R.p, (T(G.G9) * R.rho));
+    hL = M::div(L.p, L.rho) + uL + T(0.5) * (L.v[0] * L.v[0] + L.v[1] * L.v[1] + L.v[2] * L.v[2]);
+    hR = M::div(R.p, R.rho) + uR + T(0.5) * (R.v[0] * R.v[0] + R.v[1] * R.v[1] + R.v[2] * R.v[2]);
+}
+
+// sound speeds sqrt(gamma p / rho) of the two states
+template <typename T>
+__device__ __forceinline__ void sound_speeds(const RState<T> &L, const RState<T> &R, const GammaConsts &G, T &cL, T &cR)
+{
+    using M = Real<T>;
+    if constexpr (sizeof(T) == sizeof(double)) {
+        const double g = G.G0;
+        if (plain_range(L.rho) && plain_range(R.rho) && plain_range(L.p) && plain_range(R.p)) {
+            const double eL = quotient(g * L.p, L.rho, rcp_newton(L.rho)), eR = quotient(g * R.p, R.rho, rcp_newton(R.rho));
+            if (plain_range(eL) && plain_range(eR)) {
+                double inv;
+                root_newton(eL, cL, inv);
+                root_newton(eR, cR, inv);
+                return;
+            }
+        }
+    }
+    cL = M::root(M::div(T(G.G0) * L.p, L.rho));
+    cR = M::root(M::div(T(G.G0) * R.p, R.rho));
+}
+
 template <typename T>
 __device__ inline bool wavespeeds_pstar(const RState<T> &L, const RState<T> &R, const GammaConsts &G, const T n[3],
-                                        T vL, T vR, T cL, T cR, T hL, T hR, T limiter, ROut<T> &o,
-                                        T *S_LR = nullptr)
+                                        T vL, T vR, T cL, T cR, T limiter, ROut<T> &o, T *S_LR = nullptr)
 {
     using M = Real<T>;
     const T cmax = tmax(cL, cR);
@@ -509,12 +666,23 @@ __device__ inline bool wavespeeds_pstar(const RState<T> &L, const RState<T> &R, 
     T S_R = tmax(vL, vR) + tmax(cL, cR);
     T rwL = L.rho * (S_L - vL);
     T rwR = R.rho * (S_R - vR);
-    o.S_M = M::div(((PT_R - PT_L) + rwL * vL - rwR * vR), (rwL - rwR));
-    o.P_M = M::div((PT_L * rwR - PT_R * rwL + rwL * rwR * (vR - vL)), (rwR - rwL));
+    if constexpr (sizeof(T) == sizeof(double)) {
+        // one reciprocal for both quotients, the rounding of the divisions below.
+        // A zero denominator (two cold states at one velocity) gives NaN here and
+        // NaN or infinity there: the Roe estimate follows either way.
+        const double d = rwL - rwR, y = rcp_newton(d);
+        o.S_M = quotient(((PT_R - PT_L) + rwL * vL - rwR * vR), d, y);
+        o.P_M = quotient((PT_L * rwR - PT_R * rwL + rwL * rwR * (vR - vL)), -d, -y);
+    } else {
+        o.S_M = M::div(((PT_R - PT_L) + rwL * vL - rwR * vR), (rwL - rwR));
+        o.P_M = M::div((PT_L * rwR - PT_R * rwL + rwL * rwR * (vR - vL)), (rwR - rwL));
+    }
     if (near_threshold(o.P_M, limiter, limiter)) return true;
     if (o.P_M <= M::tiny) { o.P_M = M::tiny; o.S_M = 0; S_L = S_R = 0; }
     if (S_LR) { S_LR[0] = S_L; S_LR[1] = S_R; }
     if ((o.P_M <= 0) || isnan(o.P_M) || (o.P_M > limiter)) {
+        T hL, hR;
+        enthalpies(L, R, G, hL, hR);
         T sL = M::root(L.rho), sR = M::root(R.rho);
         T sinv = M::rcp(sL + sR);
         T vx = (sL * L.v[0] + sR * R.v[0]) * sinv;
@@ -699,7 +867,7 @@ __device__ __noinline__ ExactOut riemann_exact(double rL, double pL, double rR, 
 // Riemann_solver() for MFM hydro (reimann.h:286-388).  Returns a stage mask:
 // bit0 HLLC, bit1 KT, bit2 exact; err gets 1234545 on the exact solver's
 // negative-density exit.  The exact solver always runs in FP64.  DEFER: stop
-// where the exact solver would be called and return kDeferBit instead.
+// where the KT flux or the exact solver would be called and return kDeferBit.
 // FP32: kNearBit when the wavespeed estimate stopped at a near-threshold test.
 constexpr int kDeferBit = 32;
 constexpr int kNearBit = 64;
@@ -708,21 +876,21 @@ template <typename T, bool DEFER = false, bool INLINE = false>
 __device__ __forceinline__ int riemann_solve(const RState<T> &L, const RState<T> &R, const T n[3], T limiter,
                                              const GammaConsts &G, ROut<T> &o, int &err)
 {
-    using M = Real<T>;
     if ((L.p < 0 && R.p < 0) || (L.rho < 0) || (R.rho < 0)) { o.P_M = 0; return 0; }
-    T cL = M::root(M::div(T(G.G0) * L.p, L.rho));
-    T cR = M::root(M::div(T(G.G0) * R.p, R.rho));
-    T uL = M::div(L.p, (T(G.G9) * L.rho));
-    T uR = M::div(R.p, (T(G.G9) * R.rho));
-    T hL = M::div(L.p, L.rho) + uL + T(0.5) * (L.v[0] * L.v[0] + L.v[1] * L.v[1] + L.v[2] * L.v[2]);
-    T hR = M::div(R.p, R.rho) + uR + T(0.5) * (R.v[0] * R.v[0] + R.v[1] * R.v[1] + R.v[2] * R.v[2]);
+    T cL, cR;
+    sound_speeds(L, R, G, cL, cR);
     T vL = L.v[0] * n[0] + L.v[1] * n[1] + L.v[2] * n[2];
     T vR = R.v[0] * n[0] + R.v[1] * n[1] + R.v[2] * n[2];
     int mask = 1;
-    if (wavespeeds_pstar(L, R, G, n, vL, vR, cL, cR, hL, hR, limiter, o)) return mask | kNearBit;
+    if (wavespeeds_pstar(L, R, G, n, vL, vR, cL, cR, limiter, o)) return mask | kNearBit;
     for (int k = 0; k < 3; k++) o.Fv[k] = o.P_M * n[k];
     o.Fp = o.P_M * o.S_M;
     if ((o.P_M < 0) || isnan(o.P_M)) {
+        // a call here would cost the list loop the registers of a call in every
+        // step, for a flux that only NaN estimates reach
+        if (DEFER) return mask | kDeferBit;
+        T hL, hR;
+        enthalpies(L, R, G, hL, hR);
         if (INLINE)
             o = riemann_kt_body<T>(L.rho, L.p, L.v[0], L.v[1], L.v[2], R.rho, R.p, R.v[0], R.v[1], R.v[2], n[0], n[1],
                                    n[2], vL, vR, cL, cR, hL, hR);
@@ -761,13 +929,6 @@ struct PairSide {
     double cn, e;
 };
 
-// i-side extras: kernel factors and the condition-number threshold
-template <typename T>
-struct PairI : PairSide<T> {
-    T hinv3, hinv4;
-    double cnumcrit2;  // CONDITION_NUMBER_DANGER^2 - CN_i^2 (hydro_evaluate.h:203-210)
-};
-
 // dp = x_i - x_j (nearest image), r2 = |dp|^2.  Returns the status code
 // (0, 1234 or 1234545); Fv, Fp, vsig are the pair's flux terms for i, mask
 // the stages used (bit0 HLLC, bit1 KT, bit2 exact, bit3 retry).  DEFER:
@@ -779,28 +940,94 @@ struct PairI : PairSide<T> {
 constexpr int kDeferred = -1;
 constexpr int kNearThreshold = -2;
 
-template <typename T, bool DEFER = false, bool INLINE = false>
-__device__ __forceinline__ int force_pair(const PairI<T> &I, const PairSide<T> &J, const T dp[3], T r2,
+//
+// IN_LDS: I and J lie in LDS.  Fences then keep the compiler from reading them
+// (34 FP64 values each) into registers ahead of their use: they are read again
+// in each part below.
+template <bool IN_LDS>
+__device__ __forceinline__ void part_fence()
+{
+    if constexpr (IN_LDS) asm volatile("" ::: "memory");
+}
+
+// The states of both sides at the face; true (FP32) where a limiter's branch is
+// too near to decide.  `recon` false: the particles' own values.
+template <bool IN_LDS, typename T>
+__device__ __forceinline__ bool face_states(const PairSide<T> &I, const PairSide<T> &J, const T di[3], const T dj[3],
+                                            bool recon, RState<T> &SL, RState<T> &SR)
+{
+    if (!recon) {
+        SR.rho = I.rho; SL.rho = J.rho;
+        SR.p = I.P; SL.p = J.P;
+#pragma unroll
+        for (int k = 0; k < 3; k++) { SR.v[k] = I.v[k]; SL.v[k] = J.v[k]; }
+        return false;
+    }
+    if constexpr (sizeof(T) == sizeof(double)) {
+        double odd = 0;
+        reconstruct_fp64(I.rho, I.gr, J.rho, J.gr, di, dj, SL.rho, SR.rho, odd);
+        part_fence<IN_LDS>();
+        reconstruct_fp64(I.P, I.gp, J.P, J.gp, di, dj, SL.p, SR.p, odd);
+        part_fence<IN_LDS>();
+        bool moving = false;  // equal velocities, as of gas at rest, are their own states
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            SR.v[k] = SL.v[k] = I.v[k];
+            moving |= I.v[k] != J.v[k];
+        }
+        if (moving) {
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                reconstruct_fp64(I.v[k], I.gv + 3 * k, J.v[k], J.gv + 3 * k, di, dj, SL.v[k], SR.v[k], odd);
+                part_fence<IN_LDS>();
+            }
+        }
+        if (isnan(odd)) {
+            keep_nan(I.rho, I.gr, J.rho, J.gr, di, dj, SL.rho, SR.rho);
+            keep_nan(I.P, I.gp, J.P, J.gp, di, dj, SL.p, SR.p);
+#pragma unroll
+            for (int k = 0; k < 3; k++) keep_nan(I.v[k], I.gv + 3 * k, J.v[k], J.gv + 3 * k, di, dj, SL.v[k], SR.v[k]);
+        }
+        return false;
+    } else {
+        bool near = reconstruct(I.rho, I.gr, J.rho, J.gr, di, dj, SL.rho, SR.rho);
+        near |= reconstruct(I.P, I.gp, J.P, J.gp, di, dj, SL.p, SR.p);
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            near |= reconstruct(I.v[k], I.gv + 3 * k, J.v[k], J.gv + 3 * k, di, dj, SL.v[k], SR.v[k]);
+        return near;
+    }
+}
+
+template <typename T, bool DEFER = false, bool INLINE = false, bool IN_LDS = false>
+__device__ __forceinline__ int force_pair(const PairSide<T> &I, const PairSide<T> &J, const T dp[3], T r2,
                                           const GammaConsts &G, ROut<T> &ro, T Fv[3], T &Fp, T &vsig, int &mask)
 {
     using M = Real<T>;
+    constexpr bool fp64 = sizeof(T) == sizeof(double);
     int status = 0;
-    const T r = M::root(r2);
-    const T rinv = M::rcp(r);
+    T r, rinv;
+    root_and_inverse(r2, r, rinv);
     const T dv[3] = {I.v[0] - J.v[0], I.v[1] - J.v[1], I.v[2] - J.v[2]};
     vsig = I.cs + J.cs;
-    const T vdotr2 = dp[0] * dv[0] + dp[1] * dv[1] + dp[2] * dv[2];
+    const T vdotr2 = fma1(dp[2], dv[2], fma1(dp[1], dv[1], dp[0] * dv[0]));
     if (vdotr2 < 0) vsig -= T(1.0) * vdotr2 * rinv;  // MFM: fac_mu = 1 (hydro_evaluate.h:235-245)
     T wk_i = 0, dwk_i = 0, wk_j = 0, dwk_j = 0;
-    if (r < I.h) kernel_wdw(r * I.hinv, I.hinv3, I.hinv4, wk_i, dwk_i);
+    if (r < I.h) {
+        const T hinv3_i = I.hinv * I.hinv * I.hinv;
+        kernel_wdw<fp64>(r * I.hinv, hinv3_i, hinv3_i * I.hinv, wk_i, dwk_i);
+    }
     if (r < J.h) {
         const T hinv3_j = J.hinv * J.hinv * J.hinv;
-        kernel_wdw(r * J.hinv, hinv3_j, hinv3_j * J.hinv, wk_j, dwk_j);
+        kernel_wdw<fp64>(r * J.hinv, hinv3_j, hinv3_j * J.hinv, wk_j, dwk_j);
     }
+    part_fence<IN_LDS>();
     Fv[0] = Fv[1] = Fv[2] = 0;
     Fp = 0;
     mask = 0;
     const double leak = 0.5 * ((double)I.fce + (double)J.fce);
+    // CONDITION_NUMBER_DANGER^2 - CN_i^2 (hydro_evaluate.h:203-210)
+    const double cnumcrit2 = kCondDanger * kCondDanger - I.cn * I.cn;
     // FP32 only: a listed pair (r^2 < h^2 decided in FP64) whose FP32 r / h
     // rounds to 1 on both sides has no kernel weight; in FP64 its weights are
     // tiny but positive and the face vanishes, so give it no face here instead
@@ -817,28 +1044,35 @@ __device__ __forceinline__ int force_pair(const PairI<T> &I, const PairSide<T> &
         return DEFER ? kDeferred : kNearThreshold;
     // effective face (compute_finitevol_faces.h:14-106)
     T wt_i = I.V, wt_j = J.V;
-    const T vratio = M::div(M::div(fabs(I.V - J.V), tmin(I.V, J.V)), T(3));
-    if (near_threshold(vratio, T(1.25), T(1.25))) return DEFER ? kDeferred : kNearThreshold;
-    if (vratio > T(1.25)) {
+    bool uneven;
+    if constexpr (fp64) {
+        uneven = fabs(I.V - J.V) > 3.75 * tmin(I.V, J.V);
+    } else {
+        const T vratio = M::div(M::div(fabs(I.V - J.V), tmin(I.V, J.V)), T(3));
+        if (near_threshold(vratio, T(1.25), T(1.25))) return DEFER ? kDeferred : kNearThreshold;
+        uneven = vratio > T(1.25);
+    }
+    if (uneven) {
         wt_i = wt_j = M::div(I.V * J.V * (wk_i + wk_j), (I.V * wk_i + J.V * wk_j));
     }
     T A[3];
     T Anorm = 0, fdp = 0;
     {
-        const T ti_d[3] = {I.nvt[0] * dp[0] + I.nvt[1] * dp[1] + I.nvt[2] * dp[2],
-                           I.nvt[1] * dp[0] + I.nvt[3] * dp[1] + I.nvt[4] * dp[2],
-                           I.nvt[2] * dp[0] + I.nvt[4] * dp[1] + I.nvt[5] * dp[2]};
-        const T tj_d[3] = {J.nvt[0] * dp[0] + J.nvt[1] * dp[1] + J.nvt[2] * dp[2],
-                           J.nvt[1] * dp[0] + J.nvt[3] * dp[1] + J.nvt[4] * dp[2],
-                           J.nvt[2] * dp[0] + J.nvt[4] * dp[1] + J.nvt[5] * dp[2]};
+        auto dot = [&](T a, T b, T c) { return fma1(c, dp[2], fma1(b, dp[1], a * dp[0])); };
+        const T ti_d[3] = {dot(I.nvt[0], I.nvt[1], I.nvt[2]), dot(I.nvt[1], I.nvt[3], I.nvt[4]),
+                           dot(I.nvt[2], I.nvt[4], I.nvt[5])};
+        const T tj_d[3] = {dot(J.nvt[0], J.nvt[1], J.nvt[2]), dot(J.nvt[1], J.nvt[3], J.nvt[4]),
+                           dot(J.nvt[2], J.nvt[4], J.nvt[5])};
+        const T wi = wk_i * wt_i, wj = wk_j * wt_j;
 #pragma unroll
         for (int k = 0; k < 3; k++) {
-            A[k] = wk_i * wt_i * ti_d[k] + wk_j * wt_j * tj_d[k];
-            Anorm += A[k] * A[k];
-            fdp += A[k] * dp[k];
+            // both terms rounded alike, so that the faces of (i, j) and (j, i) are exact opposites
+            A[k] = wi * ti_d[k] + wj * tj_d[k];
+            Anorm = fma1(A[k], A[k], Anorm);
+            fdp = fma1(A[k], dp[k], fdp);
         }
     }
-    const bool cn_switch = J.cn * J.cn > 1.0e12 + I.cnumcrit2;
+    const bool cn_switch = J.cn * J.cn > 1.0e12 + cnumcrit2;
     if (!cn_switch && near_threshold(fdp, T(0), (fabs(A[0]) + fabs(A[1]) + fabs(A[2])) * r))
         return DEFER ? kDeferred : kNearThreshold;
     if (cn_switch || (fdp < 0)) {
@@ -848,10 +1082,25 @@ __device__ __forceinline__ int force_pair(const PairI<T> &I, const PairSide<T> &
         A[2] = An * dp[2];
         Anorm = An * An * r2;
     }
-    Anorm = M::root(Anorm);
-    if (Anorm == 0) return 0;
-
-    const T n[3] = {M::div(A[0], Anorm), M::div(A[1], Anorm), M::div(A[2], Anorm)};
+    T n[3];
+    if constexpr (fp64) {
+        if (plain_range(Anorm)) {
+            const double A2 = Anorm;
+            double ainv;
+            root_newton(A2, Anorm, ainv);
+#pragma unroll
+            for (int k = 0; k < 3; k++) n[k] = quotient(A[k], Anorm, ainv);
+        } else {
+            Anorm = sqrt(Anorm);
+            if (Anorm == 0) return 0;
+            for (int k = 0; k < 3; k++) n[k] = A[k] / Anorm;
+        }
+    } else {
+        Anorm = M::root(Anorm);
+        if (Anorm == 0) return 0;
+        for (int k = 0; k < 3; k++) n[k] = M::div(A[k], Anorm);
+    }
+    part_fence<IN_LDS>();
     // faces at the midpoint: s_i = -r/2, s_j = +r/2 (hydro_core_meshless.h:70-90)
     const T s_i = T(0) - T(0.5) * r, s_j = T(0) - (T(-0.5) * r);
     T di[3], dj[3], vf[3];
@@ -864,27 +1113,30 @@ __device__ __forceinline__ int force_pair(const PairI<T> &I, const PairSide<T> &
     }
     T fvi = 0, fvj = 0;
 #pragma unroll
-    for (int k = 0; k < 3; k++) { fvi += I.v[k] * n[k]; fvj += J.v[k] * n[k]; }
+    for (int k = 0; k < 3; k++) {
+        fvi = fma1(I.v[k], n[k], fvi);
+        fvj = fma1(J.v[k], n[k], fvj);
+    }
     const T fadv = rinv * (-s_i * fvj + s_j * fvi);
     T v2a = 0;
     T vdotr2_phys = vdotr2;
-    vdotr2_phys *= M::rcp(r * T(1.0));
+    vdotr2_phys *= fp64 ? rinv : M::rcp(r * T(1.0));
     if (vdotr2_phys < 0) v2a = vdotr2_phys * vdotr2_phys;
     const T vdotf2 = fvi - fvj;
     if (vdotf2 < 0) v2a = tmax(v2a, vdotf2 * vdotf2);
     const int recon = (leak > 1) ? 0 : 1;
     RState<T> SL, SR;
-    bool near = reconstruct(I.rho, I.gr, J.rho, J.gr, di, dj, SL.rho, SR.rho, recon);
-    near |= reconstruct(I.P, I.gp, J.P, J.gp, di, dj, SL.p, SR.p, recon);
+    part_fence<IN_LDS>();
+    const bool near = face_states<IN_LDS>(I, J, di, dj, recon != 0, SL, SR);
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-        near |= reconstruct(I.v[k], I.gv + 3 * k, J.v[k], J.gv + 3 * k, di, dj, SL.v[k], SR.v[k], recon);
         SL.v[k] -= vf[k];
         SR.v[k] -= vf[k];
     }
     if (sizeof(T) == sizeof(float) && near) return DEFER ? kDeferred : kNearThreshold;
-    const T pti = I.P + I.rho * v2a;
-    const T ptj = J.P + J.rho * v2a;
+    part_fence<IN_LDS>();
+    const T pti = fma1(I.rho, v2a, I.P);
+    const T ptj = fma1(J.rho, v2a, J.P);
     T lim = T(1.1) * T(1.0) * tmax(pti, ptj);
     if (recon == 0) lim = tmax(lim, tmax(tmax(I.P, J.P), T(2.) * tmax(I.rho, J.rho) * v2a));
     // Riemann problem with the reference's two retries (hydro_core_meshless.h:209-265):
@@ -898,6 +1150,8 @@ __device__ __forceinline__ int force_pair(const PairI<T> &I, const PairSide<T> &
         if (DEFER && (mask & kDeferBit)) return kDeferred;
         const bool bad = (ro.P_M < 0) || isnan(ro.P_M);
         if (attempt == 0 && near_threshold(ro.P_M, T(1.4) * lim, lim)) return DEFER ? kDeferred : kNearThreshold;
+        // a pressure that asks for a retry is past the limiter: deferred above
+        if (DEFER) break;
         if (attempt == 0) {
             if (!(bad || (ro.P_M > T(1.4) * lim))) break;
             mask |= 8;
@@ -918,14 +1172,18 @@ __device__ __forceinline__ int force_pair(const PairI<T> &I, const PairSide<T> &
         }
     }
     if (err) status = err;
+    part_fence<IN_LDS>();
     if ((ro.P_M > 0) && !isnan(ro.P_M)) {
 #pragma unroll
-        for (int k = 0; k < 3; k++) ro.Fp += vf[k] * ro.Fv[k];
+        for (int k = 0; k < 3; k++) ro.Fp = fma1(vf[k], ro.Fv[k], ro.Fp);
         Fp = Anorm * ro.Fp;
 #pragma unroll
         for (int k = 0; k < 3; k++) Fv[k] = Anorm * ro.Fv[k];
         // MFM adiabatic face correction (hydro_core_meshless.h:335-374)
-        const T sm_c = M::div(fabs(ro.S_M), tmin(I.cs, J.cs));
+        // |S_M| / c_min against 0.5 and 1e-3: FP64 compares |S_M| with c_min times them
+        const T cmin = tmin(I.cs, J.cs);
+        const T sm_c = fp64 ? fabs(ro.S_M) : M::div(fabs(ro.S_M), cmin);
+        const T sm_unit = fp64 ? cmin : T(1);
         // FP32: the switch's decisions (|S_M|/c against 0.5 and 1e-3, and the
         // signs of the energy transfer to j or i) flip the pair's energy flux
         // by du_new - du_old; one within the FP32 margin of its threshold is
@@ -935,7 +1193,7 @@ __device__ __forceinline__ int force_pair(const PairI<T> &I, const PairSide<T> &
         // absolute error and the margins below hold that with room (0.03 +
         // threshold scales kDecideMargin to 3e-4 of 1e-3 and 1e-5 of 0.5).
         if (!(leak > 1) && near_threshold(sm_c, T(0.5), T(0.5 + 0.03))) return DEFER ? kDeferred : kNearThreshold;
-        if ((sm_c < T(0.5)) || (leak > 1)) {
+        if ((sm_c < T(0.5) * sm_unit) || (leak > 1)) {
             int use = 1;
             const T fpm = ro.P_M * Anorm;
             const T pdv_fac = ro.P_M * vdotr2_phys / T(1.0);
@@ -944,9 +1202,9 @@ __device__ __forceinline__ int force_pair(const PairI<T> &I, const PairSide<T> &
             const T du_old = fpm * (ro.S_M + fadv);
             const T du_new = T(0.5) * (pdv_i - pdv_j + fpm * (fvi + fvj));
             const double cnum2 = J.cn * J.cn;
-            if (cnum2 < I.cnumcrit2 && (I.e != J.e) && near_threshold(sm_c, T(1.e-3), T(1.e-3 + 0.03)))
+            if (cnum2 < cnumcrit2 && (I.e != J.e) && near_threshold(sm_c, T(1.e-3), T(1.e-3 + 0.03)))
                 return DEFER ? kDeferred : kNearThreshold;
-            if (sm_c > T(1.e-3) && cnum2 < I.cnumcrit2) {
+            if (sm_c > T(1.e-3) * sm_unit && cnum2 < cnumcrit2) {
                 if (I.e != J.e) {
                     const T fpv = (I.e > J.e) ? fpm * fvj : fpm * fvi;
                     // dtoj = -du_old + fpm fvj, dtoi = du_old - fpm fvi: compared with 0 and with
@@ -968,7 +1226,7 @@ __device__ __forceinline__ int force_pair(const PairI<T> &I, const PairSide<T> &
                     }
                 }
             }
-            if (cnum2 >= I.cnumcrit2) use = 1;
+            if (cnum2 >= cnumcrit2) use = 1;
             if (use) Fp += du_new - du_old;
         }
     } else {

@@ -273,20 +273,21 @@ __device__ inline int riemann_solve_mfv(const RState<double> &L, const RState<do
                                         double limiter, const GammaConsts &G, ROutV &o, int &err)
 {
     if ((L.p < 0 && R.p < 0) || (L.rho < 0) || (R.rho < 0)) { o.P_M = 0; return 0; }
-    const double cL = sqrt(G.G0 * L.p / L.rho), cR = sqrt(G.G0 * R.p / R.rho);
-    const double uL = L.p / (G.G9 * L.rho), uR = R.p / (G.G9 * R.rho);
-    const double hL = L.p / L.rho + uL + 0.5 * (L.v[0] * L.v[0] + L.v[1] * L.v[1] + L.v[2] * L.v[2]);
-    const double hR = R.p / R.rho + uR + 0.5 * (R.v[0] * R.v[0] + R.v[1] * R.v[1] + R.v[2] * R.v[2]);
+    double cL, cR;
+    sound_speeds(L, R, G, cL, cR);
+    double hL, hR;
+    enthalpies(L, R, G, hL, hR);
     const double vL = L.v[0] * n[0] + L.v[1] * n[1] + L.v[2] * n[2];
     const double vR = R.v[0] * n[0] + R.v[1] * n[1] + R.v[2] * n[2];
     int mask = 1;
     ROut<double> e = {o.P_M, o.S_M, {0, 0, 0}, 0};
     double S_LR[2] = {0, 0};
-    wavespeeds_pstar<double>(L, R, G, n, vL, vR, cL, cR, hL, hR, limiter, e, S_LR);
+    wavespeeds_pstar<double>(L, R, G, n, vL, vR, cL, cR, limiter, e, S_LR);
     o.P_M = e.P_M;
     o.S_M = e.S_M;
     if ((o.P_M >= 0) && !isnan(o.P_M)) hllc_fluxes_mfv(L, R, o, n, vL, vR, hL, hR, S_LR[0], S_LR[1]);
     if ((o.P_M < 0) || isnan(o.P_M)) {
+        if (DEFER) return mask | kDeferBit;
         if (INLINE) riemann_kt_mfv(L, R, o, n, vL, vR, cL, cR, hL, hR);
         else
             o = riemann_kt_mfv_ool(L.rho, L.p, L.v[0], L.v[1], L.v[2], R.rho, R.p, R.v[0], R.v[1], R.v[2], n[0], n[1],
@@ -323,55 +324,68 @@ __device__ inline int riemann_solve_mfv(const RState<double> &L, const RState<do
 // kDeferred, with no flux terms, for a pair that would call the exact solver
 // (every first-order retry follows an exact solution, so retries happen only
 // in the caller's later evaluation of such a pair with DEFER = false).
-template <bool DEFER = false, bool INLINE = false>
-__device__ inline int force_pair_mfv(const PairI<double> &I, const PairSide<double> &J, const double w_i[3],
+template <bool DEFER = false, bool INLINE = false, bool IN_LDS = false>
+__device__ inline int force_pair_mfv(const PairSide<double> &I, const PairSide<double> &J, const double w_i[3],
                                      const double dp[3], double r2, const GammaConsts &G, double Fv[3], double &Fp,
                                      double &Frho, double &vsig, int &mask)
 {
     int status = 0;
-    const double r = sqrt(r2);
-    const double rinv = 1 / r;
+    double r, rinv;
+    root_and_inverse(r2, r, rinv);
     const double dv[3] = {I.v[0] - J.v[0], I.v[1] - J.v[1], I.v[2] - J.v[2]};
     vsig = I.cs + J.cs;
-    const double vdotr2 = dp[0] * dv[0] + dp[1] * dv[1] + dp[2] * dv[2];
+    const double vdotr2 = fma(dp[2], dv[2], fma(dp[1], dv[1], dp[0] * dv[0]));
     if (vdotr2 < 0) vsig -= 3 * 1.0 * vdotr2 * rinv;
     double wk_i = 0, dwk_i = 0, wk_j = 0, dwk_j = 0;
-    if (r < I.h) kernel_wdw(r * I.hinv, I.hinv3, I.hinv4, wk_i, dwk_i);
+    if (r < I.h) {
+        const double hinv3_i = I.hinv * I.hinv * I.hinv;
+        kernel_wdw<true>(r * I.hinv, hinv3_i, hinv3_i * I.hinv, wk_i, dwk_i);
+    }
     if (r < J.h) {
         const double hinv3_j = J.hinv * J.hinv * J.hinv;
-        kernel_wdw(r * J.hinv, hinv3_j, hinv3_j * J.hinv, wk_j, dwk_j);
+        kernel_wdw<true>(r * J.hinv, hinv3_j, hinv3_j * J.hinv, wk_j, dwk_j);
     }
+    part_fence<IN_LDS>();
     Fv[0] = Fv[1] = Fv[2] = 0;
     Fp = 0;
     Frho = 0;
     mask = 0;
     const double leak = 0.5 * (I.fce + J.fce);
+    const double cnumcrit2 = kCondDanger * kCondDanger - I.cn * I.cn;
     double wt_i = I.V, wt_j = J.V;
-    if ((fabs(I.V - J.V) / dmin(I.V, J.V)) / 3 > 1.25) wt_i = wt_j = I.V * J.V * (wk_i + wk_j) / (I.V * wk_i + J.V * wk_j);
+    if (fabs(I.V - J.V) > 3.75 * dmin(I.V, J.V)) wt_i = wt_j = I.V * J.V * (wk_i + wk_j) / (I.V * wk_i + J.V * wk_j);
     double A[3], Anorm = 0, fdp = 0;
     {
-        const double ti_d[3] = {I.nvt[0] * dp[0] + I.nvt[1] * dp[1] + I.nvt[2] * dp[2],
-                                I.nvt[1] * dp[0] + I.nvt[3] * dp[1] + I.nvt[4] * dp[2],
-                                I.nvt[2] * dp[0] + I.nvt[4] * dp[1] + I.nvt[5] * dp[2]};
-        const double tj_d[3] = {J.nvt[0] * dp[0] + J.nvt[1] * dp[1] + J.nvt[2] * dp[2],
-                                J.nvt[1] * dp[0] + J.nvt[3] * dp[1] + J.nvt[4] * dp[2],
-                                J.nvt[2] * dp[0] + J.nvt[4] * dp[1] + J.nvt[5] * dp[2]};
+        auto dot = [&](double a, double b, double c) { return fma(c, dp[2], fma(b, dp[1], a * dp[0])); };
+        const double ti_d[3] = {dot(I.nvt[0], I.nvt[1], I.nvt[2]), dot(I.nvt[1], I.nvt[3], I.nvt[4]),
+                                dot(I.nvt[2], I.nvt[4], I.nvt[5])};
+        const double tj_d[3] = {dot(J.nvt[0], J.nvt[1], J.nvt[2]), dot(J.nvt[1], J.nvt[3], J.nvt[4]),
+                                dot(J.nvt[2], J.nvt[4], J.nvt[5])};
+        const double wi = wk_i * wt_i, wj = wk_j * wt_j;
         for (int k = 0; k < 3; k++) {
-            A[k] = wk_i * wt_i * ti_d[k] + wk_j * wt_j * tj_d[k];
-            Anorm += A[k] * A[k];
-            fdp += A[k] * dp[k];
+            A[k] = wi * ti_d[k] + wj * tj_d[k];
+            Anorm = fma(A[k], A[k], Anorm);
+            fdp = fma(A[k], dp[k], fdp);
         }
     }
-    if ((J.cn * J.cn > 1.0e12 + I.cnumcrit2) || (fdp < 0)) {
+    if ((J.cn * J.cn > 1.0e12 + cnumcrit2) || (fdp < 0)) {
         const double An = -(wt_i * I.V * dwk_i + wt_j * J.V * dwk_j) / r;
         A[0] = An * dp[0];
         A[1] = An * dp[1];
         A[2] = An * dp[2];
         Anorm = An * An * r2;
     }
-    Anorm = sqrt(Anorm);
-    if (Anorm == 0) return 0;
-    const double n[3] = {A[0] / Anorm, A[1] / Anorm, A[2] / Anorm};
+    double n[3];
+    if (plain_range(Anorm)) {
+        const double A2 = Anorm;
+        double ainv;
+        root_newton(A2, Anorm, ainv);
+        for (int k = 0; k < 3; k++) n[k] = quotient(A[k], Anorm, ainv);
+    } else {
+        Anorm = sqrt(Anorm);
+        if (Anorm == 0) return 0;
+        for (int k = 0; k < 3; k++) n[k] = A[k] / Anorm;
+    }
     const double s_i = 0 - 0.5 * r, s_j = 0 - (-0.5 * r);
     double di[3], dj[3], vf[3];
     for (int k = 0; k < 3; k++) {
@@ -381,22 +395,25 @@ __device__ inline int force_pair_mfv(const PairI<double> &I, const PairSide<doub
         vf[k] = rinv * (-s_i * J.v[k] + s_j * w_i[k]);
     }
     double fvi = 0, fvj = 0;
-    for (int k = 0; k < 3; k++) { fvi += I.v[k] * n[k]; fvj += J.v[k] * n[k]; }
+    for (int k = 0; k < 3; k++) {
+        fvi = fma(I.v[k], n[k], fvi);
+        fvj = fma(J.v[k], n[k], fvj);
+    }
     double v2a = 0;
     double vdotr2_phys = vdotr2;
-    vdotr2_phys *= 1 / (r * 1.0);
+    vdotr2_phys *= rinv;
     if (vdotr2_phys < 0) v2a = vdotr2_phys * vdotr2_phys;
     const double vdotf2 = fvi - fvj;
     if (vdotf2 < 0) v2a = dmax(v2a, vdotf2 * vdotf2);
     const int recon = (leak > 1) ? 0 : 1;
     RState<double> SL, SR;
-    reconstruct(I.rho, I.gr, J.rho, J.gr, di, dj, SL.rho, SR.rho, recon);
-    reconstruct(I.P, I.gp, J.P, J.gp, di, dj, SL.p, SR.p, recon);
+    part_fence<IN_LDS>();
+    face_states<IN_LDS>(I, J, di, dj, recon != 0, SL, SR);
     for (int k = 0; k < 3; k++) {
-        reconstruct(I.v[k], I.gv + 3 * k, J.v[k], J.gv + 3 * k, di, dj, SL.v[k], SR.v[k], recon);
         SL.v[k] -= vf[k];
         SR.v[k] -= vf[k];
     }
+    part_fence<IN_LDS>();
     double lim = 1.1 * 1.0 * dmax(I.P + I.rho * v2a, J.P + J.rho * v2a);
     lim *= 2.0;
     if (recon == 0) lim = dmax(lim, dmax(dmax(I.P, J.P), 2. * dmax(I.rho, J.rho) * v2a));
@@ -408,6 +425,7 @@ __device__ inline int force_pair_mfv(const PairI<double> &I, const PairSide<doub
         mask |= riemann_solve_mfv<DEFER, INLINE>(SL, SR, n, lim_a, G, ro, err);
         if (DEFER && (mask & kDeferBit)) return kDeferred;
         const bool bad = (ro.P_M < 0) || isnan(ro.P_M);
+        if (DEFER) break;
         if (attempt == 0) {
             if (!(bad || (ro.P_M > 1.4 * lim))) break;
             mask |= 8;
@@ -429,9 +447,9 @@ __device__ inline int force_pair_mfv(const PairI<double> &I, const PairSide<doub
     if (err) status = err;
     if ((ro.P_M > 0) && !isnan(ro.P_M)) {
         for (int k = 0; k < 3; k++) {
-            ro.Fp += vf[k] * ro.Fv[k];
-            ro.Fp += (0.5 * vf[k] * vf[k]) * ro.Frho;
-            ro.Fv[k] += vf[k] * ro.Frho;
+            ro.Fp = fma(vf[k], ro.Fv[k], ro.Fp);
+            ro.Fp = fma(0.5 * vf[k] * vf[k], ro.Frho, ro.Fp);
+            ro.Fv[k] = fma(vf[k], ro.Frho, ro.Fv[k]);
         }
         Frho = Anorm * ro.Frho;
         Fp = Anorm * ro.Fp;

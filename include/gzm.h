@@ -89,8 +89,8 @@ typedef struct gzm_params {
     int32_t block_size[3];  /* threads per workgroup of the per-particle loop kernels of
                                [0] the density sweeps of precision 2, [1] the gradient loop, [2] the force
                                loop: 64, 128, 256 or 512 (the force loop's grid-scanning
-                               fallbacks stay at 256); 0 = 256.  Results do not depend on
-                               it */
+                               fallbacks stay at 256, its FP64 list loop at 64); 0 = 256.
+                               Results do not depend on it */
     int32_t wave_sweep_max; /* precision 2: a density sweep over at most this many particles gives each
                                one a wavefront whose lanes share its walk: 0 = default
                                (4096), < 0 = never.  Sums then run in another order (lane
