@@ -326,6 +326,220 @@ __device__ __forceinline__ void for_each_neighbour_candidate(const TreeArgs &T, 
     }
 }
 
+// order this wavefront's LDS writes before its later reads
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// the votes of a group of W lanes, from bit 0
+template <int W>
+__device__ __forceinline__ uint64_t group_ballot(bool v)
+{
+    const uint64_t bits = __ballot(v);
+    if constexpr (W == 64) return bits;
+    else return (bits >> ((threadIdx.x & 63) & ~(W - 1))) & ((1ull << W) - 1);
+}
+
+// LDS of the tree walk of W lanes (group_tree_walk).  Past kWide entries fewer
+// are taken at a time, in the end one by one, which adds at most an entry per
+// level, and the 95 bits of a Morton key and slot bound the levels.  (Taking W
+// from the end of the list adds up to W per level; at 5 W a dense clump's walk ran
+// entry by entry.)
+constexpr int kNodeTaken = 0x40000000;  // stack flag: a bucket whose test is passed
+template <int W>
+struct GroupWalkLds {
+    static constexpr int kWide = W == 64 ? 16 * W : 8 * W;
+    int stack[kWide + W + 96];
+    int cand[W * (kTreeBucket + 1)];
+};
+using WaveWalkLds = GroupWalkLds<64>;
+
+// The tree walk of one particle by W lanes (a power of two): the same visits as
+// tree_walk (h_pair < 0: radius R only; else max(h_pair, node hmax)), handed out
+// W slots at a time, f(slot, valid) called by the W lanes together.
+//
+// Walked alone, a node costs its load's full latency, and so does each step of
+// the next: the few particles whose search sphere reaches into a dense clump
+// (some 2,000 of 250,000 in a set of Plummer spheres) held a stage for
+// milliseconds.  Here the lanes test the first W entries of a stack of pending
+// nodes at once; a node that is opened leaves its two children in its place.
+// ORDERED: slots leave in ascending order, so a bucket past an opened node waits
+// on the stack.
+// With budget > 0 the walk ends, returning false, once it has passed that many
+// slots.
+template <int W, bool ORDERED, typename F>
+__device__ __forceinline__ bool group_tree_walk(const TreeArgs &T, const BoxDesc &G, const double x[3], double R,
+                                                double h_pair, int lane, GroupWalkLds<W> &lds, F &&f, int budget = 0)
+{
+    int top = 0, fill = 0, passed = 0;
+    if (G.root != kTreeEnd) {
+        if (lane == 0) lds.stack[0] = G.root;
+        top = 1;
+    }
+    wave_lds_fence();
+    // a well-formed tree has 2 count - 1 nodes, and each turn takes at least one off
+    for (int turns = 2 * G.count; top > 0 && turns > 0; turns--) {
+        const int m = min(min(top, W), max(1, lds.kWide + W - top));
+        const int item = lane < m ? lds.stack[top - 1 - lane] : kTreeEnd;
+        int beg = 0, end = -1, left = 0, right = 0;
+        bool open = false, range = false;
+        if (lane < m) {
+            if (item < 0) {
+                beg = end = -item - 1;
+                range = true;
+            } else {
+                const TreeNode nd = T.nodes[item & ~kNodeTaken];
+                beg = nd.link.y;
+                end = nd.link.z;
+                left = nd.link.x;
+                right = nd.link.w;
+                bool in = true;
+                if (!(item & kNodeTaken)) {
+                    const double hm = nd.lo.w;
+                    const double Rn = (h_pair < 0) ? R : ((hm > h_pair) ? hm : h_pair);
+                    const double gx = periodic_gap(x[0], nd.lo.x, nd.hi.x, G.box.L[0]);
+                    const double gy = periodic_gap(x[1], nd.lo.y, nd.hi.y, G.box.L[1]);
+                    const double gz = periodic_gap(x[2], nd.lo.z, nd.hi.z, G.box.L[2]);
+                    in = gx * gx + gy * gy + gz * gz <= Rn * Rn * (1.0 + 1e-9);
+                }
+                range = in && end - beg < kTreeBucket;
+                open = in && !range;
+            }
+        }
+        const uint64_t opened = group_ballot<W>(open);
+        const int front = ORDERED && opened ? __ffsll((unsigned long long)opened) - 1 : W;
+        const bool out = range && lane < front;
+        const int n_slots = out ? end - beg + 1 : 0, n_push = open ? 2 : (range && !out ? 1 : 0);
+        int sum = n_slots << 16 | n_push;
+#pragma unroll
+        for (int off = 1; off < W; off <<= 1) {
+            const int o = __shfl_up(sum, off, W);
+            if (lane >= off) sum += o;
+        }
+        const int total = __shfl(sum, W - 1, W);
+        int c = fill + (sum >> 16) - n_slots;
+        for (int j = beg; out && j <= end; j++) lds.cand[c++] = j;
+        top += (total & 0xffff) - m;
+        const int p = top - 1 - ((sum & 0xffff) - n_push);
+        if (open) {
+            lds.stack[p] = left;
+            lds.stack[p - 1] = right;
+        } else if (n_push) {
+            lds.stack[p] = item < 0 ? item : item | kNodeTaken;
+        }
+        fill += total >> 16;
+        passed += total >> 16;
+        if (budget && passed > budget) return false;
+        wave_lds_fence();
+        if (fill >= W) {
+            int done = 0;
+            for (; fill - done >= W; done += W) f(lds.cand[done + lane], true);
+            fill -= done;
+            const int rest = lds.cand[done + lane];
+            wave_lds_fence();
+            if (lane < fill) lds.cand[lane] = rest;
+            wave_lds_fence();
+        }
+    }
+    f(lane < fill ? lds.cand[lane] : 0, lane < fill);
+    wave_lds_fence();
+    return true;
+}
+
+template <bool ORDERED, typename F>
+__device__ __forceinline__ bool wave_tree_walk(const TreeArgs &T, const BoxDesc &G, const double x[3], double R,
+                                               double h_pair, int lane, WaveWalkLds &lds, F &&f, int budget = 0)
+{
+    return group_tree_walk<64, ORDERED>(T, G, x, R, h_pair, lane, lds, f, budget);
+}
+
+// The same walk (radius R only, slots in no order) by a workgroup of WAVES
+// wavefronts, for the walks over thousands of slots: stack and slots in common, so
+// that the wavefronts stay alike busy.  A split of the stack among them, each
+// going on alone, left most waiting for the one with the densest subtree.
+template <int WAVES>
+struct BlockWalkLds {
+    static constexpr int kThreads = 64 * WAVES, kWide = 8 * kThreads;
+    int stack[kWide + kThreads + 96];
+    int cand[kThreads * (kTreeBucket + 1)];
+    int total[WAVES];
+};
+
+template <int WAVES, typename F>
+__device__ __forceinline__ void block_tree_walk(const TreeArgs &T, const BoxDesc &G, const double x[3], double R,
+                                                BlockWalkLds<WAVES> &lds, F &&f)
+{
+    constexpr int kThreads = 64 * WAVES;
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int top = G.root != kTreeEnd ? 1 : 0, fill = 0;
+    if (tid == 0) lds.stack[0] = G.root;
+    __syncthreads();
+    for (int turns = 2 * G.count; top > 0 && turns > 0; turns--) {
+        const int m = min(min(top, kThreads), max(1, lds.kWide + kThreads - top));
+        const int item = tid < m ? lds.stack[top - 1 - tid] : kTreeEnd;
+        int beg = 0, end = -1, left = 0, right = 0;
+        bool open = false, range = false;
+        if (tid < m) {
+            if (item < 0) {
+                beg = end = -item - 1;
+                range = true;
+            } else {
+                const TreeNode nd = T.nodes[item];
+                beg = nd.link.y;
+                end = nd.link.z;
+                left = nd.link.x;
+                right = nd.link.w;
+                const double gx = periodic_gap(x[0], nd.lo.x, nd.hi.x, G.box.L[0]);
+                const double gy = periodic_gap(x[1], nd.lo.y, nd.hi.y, G.box.L[1]);
+                const double gz = periodic_gap(x[2], nd.lo.z, nd.hi.z, G.box.L[2]);
+                const bool in = gx * gx + gy * gy + gz * gz <= R * R * (1.0 + 1e-9);
+                range = in && end - beg < kTreeBucket;
+                open = in && !range;
+            }
+        }
+        const int n_slots = range ? end - beg + 1 : 0, n_push = open ? 2 : 0;
+        int sum = n_slots << 16 | n_push;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int o = __shfl_up(sum, off, 64);
+            if (lane >= off) sum += o;
+        }
+        if (lane == 63) lds.total[wave] = sum;
+        __syncthreads();
+        int before = 0, total = 0;
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) {
+            const int v = lds.total[w];
+            if (w < wave) before += v;
+            total += v;
+        }
+        sum += before;
+        int c = fill + (sum >> 16) - n_slots;
+        for (int j = beg; range && j <= end; j++) lds.cand[c++] = j;
+        top += (total & 0xffff) - m;
+        const int p = top - 1 - ((sum & 0xffff) - n_push);
+        if (open) {
+            lds.stack[p] = left;
+            lds.stack[p - 1] = right;
+        }
+        fill += total >> 16;
+        __syncthreads();
+        if (fill >= kThreads) {
+            int done = 0;
+            for (; fill - done >= kThreads; done += kThreads) f(lds.cand[done + tid], true);
+            fill -= done;
+            const int rest = lds.cand[done + tid];
+            __syncthreads();
+            if (tid < fill) lds.cand[tid] = rest;
+            __syncthreads();
+        }
+    }
+    f(tid < fill ? lds.cand[tid] : 0, tid < fill);
+    __syncthreads();
+}
+
 // Every candidate of one particle (search radius R around x), spread over the
 // 64 lanes of a wavefront that walks the tree or the grid in step: each lane
 // receives its share, f(k).  For the few particles whose search covers far
@@ -334,35 +548,12 @@ __device__ __forceinline__ void for_each_neighbour_candidate(const TreeArgs &T, 
 // by the largest hsml they hold, as in the pair walks.
 template <typename F>
 __device__ __forceinline__ void wave_candidates(const TreeArgs &T, const BoxDesc &G, const double x[3], double R,
-                                                int lane, F &&f, double h_pair = -1.0)
+                                                int lane, WaveWalkLds &lds, F &&f, double h_pair = -1.0)
 {
     if (T.nodes) {
-        int node = G.root;
-        for (int steps = 2 * G.count; node != kTreeEnd && steps > 0; steps--) {
-            if (node < 0) {
-                const int j = -node - 1;
-                if (lane == 0) f(j);
-                node = T.leaf_esc[j];
-                continue;
-            }
-            const TreeNode nd = T.nodes[node];
-            const double hm = nd.lo.w;
-            const double Rn = (h_pair < 0) ? R : ((hm > h_pair) ? hm : h_pair);
-            const double gx = periodic_gap(x[0], nd.lo.x, nd.hi.x, G.box.L[0]);
-            const double gy = periodic_gap(x[1], nd.lo.y, nd.hi.y, G.box.L[1]);
-            const double gz = periodic_gap(x[2], nd.lo.z, nd.hi.z, G.box.L[2]);
-            const int esc = __float_as_int(nd.hi.w);
-            if (!(gx * gx + gy * gy + gz * gz <= Rn * Rn * (1.0 + 1e-9))) {
-                node = esc;
-                continue;
-            }
-            if (nd.link.z - nd.link.y < 64) {
-                if (nd.link.y + lane <= nd.link.z) f(nd.link.y + lane);
-                node = esc;
-            } else {
-                node = nd.link.x;
-            }
-        }
+        wave_tree_walk<false>(T, G, x, R, h_pair, lane, lds, [&](int j, bool valid) {
+            if (valid) f(j);
+        });
     } else {
         bool full[3];
         for_each_cell(G.grid, x, R, full, [&](int, int, int, int beg, int end) {
@@ -371,46 +562,15 @@ __device__ __forceinline__ void wave_candidates(const TreeArgs &T, const BoxDesc
     }
 }
 
-// Every candidate of one particle within R of x, spread over W lanes that walk
-// the tree or the grid in step (`sub` = 0 .. W - 1): f(k) for each lane's share.
-// With budget > 0 the walk ends, returning false, once it has passed that many
-// candidates (charged a cell or bucket at a time, so alike on every lane).
+// Every grid candidate of one particle within R of x, spread over W lanes that
+// walk the cells in step (`sub` = 0 .. W - 1): f(k) for each lane's share.  With
+// budget > 0 the walk ends, returning false, once it has passed that many
+// candidates (charged a cell at a time, so alike on every lane).
 template <int W, typename F>
-__device__ __forceinline__ bool group_candidates(const TreeArgs &T, const BoxDesc &G, const double x[3], double R,
-                                                 int sub, int budget, F &&f)
+__device__ __forceinline__ bool group_candidates(const BoxDesc &G, const double x[3], double R, int sub, int budget,
+                                                 F &&f)
 {
     int visited = 0;
-    if (T.nodes) {
-        int node = G.root;
-        for (int steps = 2 * G.count; node != kTreeEnd && steps > 0; steps--) {
-            int beg, end;
-            if (node < 0) {
-                beg = end = -node - 1;
-                node = T.leaf_esc[beg];
-            } else {
-                const TreeNode nd = T.nodes[node];
-                const double gx = periodic_gap(x[0], nd.lo.x, nd.hi.x, G.box.L[0]);
-                const double gy = periodic_gap(x[1], nd.lo.y, nd.hi.y, G.box.L[1]);
-                const double gz = periodic_gap(x[2], nd.lo.z, nd.hi.z, G.box.L[2]);
-                const int esc = __float_as_int(nd.hi.w);
-                if (!(gx * gx + gy * gy + gz * gz <= R * R * (1.0 + 1e-9))) {
-                    node = esc;
-                    continue;
-                }
-                beg = nd.link.y;
-                end = nd.link.z;
-                if (end - beg >= W) {
-                    node = nd.link.x;
-                    continue;
-                }
-                node = esc;
-            }
-            visited += end - beg + 1;
-            if (budget && visited > budget) return false;
-            if (beg + sub <= end) f(beg + sub);
-        }
-        return true;
-    }
     bool full[3], ok = true;
     for_each_cell(G.grid, x, R, full, [&](int, int, int, int beg, int end) -> bool {
         visited += end - beg;
@@ -432,10 +592,10 @@ __device__ __forceinline__ bool group_candidates(const TreeArgs &T, const BoxDes
 // the lanes share each bucket.
 template <typename F>
 __device__ __forceinline__ void wave_pair_candidates(const TreeArgs &T, const BoxDesc &G, const double x[3],
-                                                     double R, double h_pair, int lane, F &&f)
+                                                     double R, double h_pair, int lane, WaveWalkLds &lds, F &&f)
 {
     if (T.nodes) {
-        wave_candidates(T, G, x, R, lane, f, h_pair);
+        wave_candidates(T, G, x, R, lane, lds, f, h_pair);
         return;
     }
     const Grid &g = G.grid;
@@ -523,13 +683,6 @@ __device__ __forceinline__ uint64_t group_or(uint64_t v)
 #pragma unroll
     for (int off = G / 2; off > 0; off >>= 1) v |= __shfl_xor((unsigned long long)v, off, 64);
     return v;
-}
-
-// order this wavefront's LDS writes before its later reads
-__device__ __forceinline__ void wave_lds_fence()
-{
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
 }
 
 // The pair lists of 64 / kForceLanes particles, one wavefront (a workgroup of its

@@ -562,7 +562,7 @@ gzm_status gzm_ctx_create(gzm_ctx **out, const gzm_params *params)
     c->G.G7 = (0.5 * (g - 1.0));
     c->G.G8 = (1.0 / g);
     c->G.G9 = (g - 1.0);
-    if (dev_alloc(&c->d_ctr, kCtrSlots * kCtrSpread) || dev_alloc(&c->d_count, 3) || dev_alloc(&c->d_count_heavy, 1) ||
+    if (dev_alloc(&c->d_ctr, kCtrSlots * kCtrSpread) || dev_alloc(&c->d_count, kDensityCounts) || dev_alloc(&c->d_count_heavy, 1) ||
         dev_alloc(&c->d_hmax, 1)) {
         gzm_ctx_destroy(c);
         return GZM_ERR_NOMEM;
@@ -773,7 +773,7 @@ gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const 
             s = s ? s : dev_alloc(&c->d_brow, (size_t)n * kPairRowCap);
             s = s ? s : dev_alloc(&c->d_bcount, n);
             s = s ? s : dev_alloc(&c->d_bwave, n);
-            s = s ? s : dev_alloc(&c->d_bwave_n, 1);
+            s = s ? s : dev_alloc(&c->d_bwave_n, 2);
         }
         if (s) { free_particles(c); return s; }
         if (c->p.precision != 2) {
@@ -1002,6 +1002,9 @@ DensityStageArgs density_stage_args(gzm_ctx *c)
     a.n_tail = c->d_count + 1;
     a.far_list = c->d_heavy_list;
     a.n_far = c->d_count + 2;
+    const bool tree = c->tree.nodes != nullptr;
+    a.walk_list = tree ? c->d_bwave : a.tail_list;
+    a.n_walk = tree ? c->d_count + 3 : a.n_tail;
     a.budget = c->p.density_budget == 0 ? kDensityBudget : (c->p.density_budget < 0 ? 0 : c->p.density_budget);
     a.lanes = c->n_active <= kFewParticles ? 8 : 1;
     a.ctr = c->d_ctr + kCtrDensity * kCtrSpread;
@@ -1013,7 +1016,7 @@ gzm_status density_fp64(gzm_ctx *c, bool captured)
     const DensityStageArgs a = density_stage_args(c);
     {
         Timed tm(c, kOther);
-        launch_density_begin(c->stream, captured ? nullptr : a.ctr, c->d_count + 1);
+        launch_density_begin(c->stream, captured ? nullptr : a.ctr, c->d_count);
     }
     if (a.n_active > 0) {
         {
@@ -1144,12 +1147,12 @@ gzm_status density_fp32(gzm_ctx *c, const Plan *gp, int *status, int *sweeps_out
         DensityStageArgs r = density_stage_args(c);
         r.row_idx = nullptr;
         r.row_n = nullptr;
-        r.tail_list = c->d_edge_list;
-        r.n_tail = c->d_n_edge;
+        r.tail_list = r.walk_list = c->d_edge_list;
+        r.n_tail = r.n_walk = c->d_n_edge;
         r.ctr = c->d_ctr + kCtrMisc * kCtrSpread;
         {
             Timed tm(c, kOther);
-            launch_density_begin(c->stream, nullptr, c->d_count + 1);
+            launch_density_begin(c->stream, nullptr, c->d_count);
             launch_edge_reset(c->stream, na, c->d_n_edge, c->d_edge_list, c->d_hsml_entry, c->d_hsml, c->d_left,
                               c->d_right, c->d_iter);
         }
@@ -1291,6 +1294,8 @@ gzm_status gradients_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
         a.dcache_r2 = c->d_dcache_r2;
         a.brow = c->d_brow;
         a.bcount = c->d_bcount;
+        a.far_list = c->d_bwave;  // its j have offered themselves
+        a.n_far = c->d_bwave_n + 1;
     } else if (!c->tree.nodes && c->d_dcache_idx) {
         a.dcache_idx = c->d_dcache_idx;
         a.dcache_n = c->d_dcache_n;

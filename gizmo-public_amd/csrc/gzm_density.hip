@@ -9,11 +9,14 @@
 //                         kDensityCacheFactor * hsml, in walk order (a pure
 //                         distance filter over the grid or tree)
 //   density_stage_kernel  the first two sweeps over the rows, a launch each
-//                         (nearly every particle needs exactly two)
+//                         (nearly every particle of an even set needs exactly two)
 //   density_tail_kernel   particles not converged by then, or without a usable
 //                         row: 16 lanes each, iterating to convergence
 //   density_far_kernel    particles whose walk passes the candidate budget: a
 //                         wavefront each, iterating to convergence
+//
+// The tree has density_more_kernel between the last two, and kernels of its own
+// for the particles that have to walk.
 //
 // The lists between them live on the device.
 //
@@ -30,6 +33,7 @@ namespace gzm {
 namespace {
 
 constexpr int kTailLanes = 16;
+constexpr int kFarWaves = 4;
 constexpr int kNoRow = kDensityCacheCap + 1;
 
 // sums of one candidate already known to lie within h (density.c:252-347).
@@ -37,8 +41,8 @@ constexpr int kNoRow = kDensityCacheCap + 1;
 // v_i - (v_i - v_j) otherwise), the sum behind ParticleVel.
 template <bool MFV>
 __device__ __forceinline__ void density_add(const double dp[3], double r2, double m_j, const double4 &vi,
-                                            const double4 *__restrict__ velu, int j, double hinv, double hinv3,
-                                            double hinv4, DensitySums &S, double *pv)
+                                            const double4 &vj, double hinv, double hinv3, double hinv4,
+                                            DensitySums &S, double *pv)
 {
     const double r = sqrt(r2);
     const double u = r * hinv;
@@ -57,7 +61,6 @@ __device__ __forceinline__ void density_add(const double dp[3], double r2, doubl
         S.f0 += wk * dp[0];
         S.f1 += wk * dp[1];
         S.f2 += wk * dp[2];
-        const double4 vj = velu[j];
         const double dv0 = vi.x - vj.x, dv1 = vi.y - vj.y, dv2 = vi.z - vj.z;
         if (MFV) {
             const double mj_wk = m_j * wk;
@@ -67,7 +70,6 @@ __device__ __forceinline__ void density_add(const double dp[3], double r2, doubl
         }
         S.divvel -= dwk * (dp[0] * dv0 + dp[1] * dv1 + dp[2] * dv2) / r;
     } else if (MFV) {
-        const double4 vj = velu[j];
         const double mj_wk = m_j * wk;
         pv[0] += mj_wk * vj.x;
         pv[1] += mj_wk * vj.y;
@@ -87,6 +89,33 @@ __device__ __forceinline__ void group_sums(DensitySums &S, double *pv)
         pv[0] = group_sum<G>(pv[0]);
         pv[1] = group_sum<G>(pv[1]);
         pv[2] = group_sum<G>(pv[2]);
+    }
+}
+
+// sums of a workgroup's wavefronts (each with its own in every lane), in their
+// order, to all of them
+template <int WAVES, bool MFV>
+__device__ __forceinline__ void block_sums(DensitySums &S, double *pv)
+{
+    constexpr int kSums = MFV ? 16 : 13;
+    __shared__ double lds[WAVES][16];
+    double v[16] = {S.ngb, S.rho, S.dhsml, S.divvel, S.t00, S.t01, S.t02, S.t11, S.t12, S.t22, S.f0, S.f1, S.f2,
+                    pv[0], pv[1], pv[2]};
+    if (threadIdx.x % 64 == 0)
+        for (int k = 0; k < kSums; k++) lds[threadIdx.x / 64][k] = v[k];
+    __syncthreads();
+    for (int k = 0; k < kSums; k++) {
+        v[k] = lds[0][k];
+        for (int w = 1; w < WAVES; w++) v[k] += lds[w][k];
+    }
+    __syncthreads();
+    S.ngb = v[0]; S.rho = v[1]; S.dhsml = v[2]; S.divvel = v[3];
+    S.t00 = v[4]; S.t01 = v[5]; S.t02 = v[6]; S.t11 = v[7]; S.t12 = v[8]; S.t22 = v[9];
+    S.f0 = v[10]; S.f1 = v[11]; S.f2 = v[12];
+    if (MFV) {
+        pv[0] = v[13];
+        pv[1] = v[14];
+        pv[2] = v[15];
     }
 }
 
@@ -175,7 +204,7 @@ __device__ __forceinline__ void count_sweeps(const DensityStageArgs &a, unsigned
 // per particle, entries staged in LDS and stored as whole 64-byte chunks.
 // G > 1 (few particles): G lanes share a cell, entries packed by ballot, same
 // order.
-template <bool TREE, int G>
+template <int G>
 __global__ __launch_bounds__(kBlock) void density_rows_kernel(DensityStageArgs a)
 {
     __shared__ __align__(16) int lds[G == 1 ? kListChunk * kBlock : 1];
@@ -195,7 +224,7 @@ __global__ __launch_bounds__(kBlock) void density_rows_kernel(DensityStageArgs a
             h = 0.99 * a.hp.max_hsml;
             if (sub == 0) a.hsml[i] = h;
         }
-        const double Rc = (TREE ? kDensityCacheFactor : kDensityCacheFactorGrid) * h, Rc2 = Rc * Rc;
+        const double Rc = kDensityCacheFactorGrid * h, Rc2 = Rc * Rc;
         const double xs[3] = {pi.x, pi.y, pi.z};
         constexpr int cap = kDensityCacheCap;
         int *row = a.row_idx + (size_t)i * cap;
@@ -220,57 +249,43 @@ __global__ __launch_bounds__(kBlock) void density_rows_kernel(DensityStageArgs a
                 m += __popc(bits);
             }
         };
-        if constexpr (TREE) {
-            auto visit = [&](int j) -> bool {
-                if (++visited > limit) return false;
-                const double4 pj = a.posm[j];
-                double dp[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
-                wrap_dp(B.box, dp);
-                const double r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
-                append(j, r2 < Rc2 && pj.w > 0);
-                return m <= cap;
-            };
-            static_assert(G == 1, "the tree rows take one lane per particle");
-            tree_walk_grouped(a.tree, B, xs, Rc, visit);
-        } else {
-            // FP32 distances with a margin for their rounding (2^-24 of a side per
-            // coordinate): the row may hold a few more than the exact radius
-            // asks for, never fewer, and a candidate is one 16-byte load.
-            const float Lmax = (float)fmax(B.box.L[0], fmax(B.box.L[1], B.box.L[2]));
-            const float Rf = (float)Rc * (1 + 1e-6f) + 5e-7f * Lmax, Rf2 = Rf * Rf * (1 + 1e-6f);
-            const float4 fi = a.posf[i];
-            for_each_run(B.grid, xs, Rc, [&](const bool full[3], int cx, int cy, int cz, int beg, int end) -> bool {
-                visited += end - beg;
-                if (visited > limit) return false;
-                // the image of this cell that the walk reached is the nearest
-                // one wherever the axis is not walked whole
-                const bool whole = full[0] || full[1] || full[2];
-                const float Lx = (float)B.box.L[0], Ly = (float)B.box.L[1], Lz = (float)B.box.L[2];
-                const float ox = fi.x - (cx < 0 ? -Lx : (cx >= B.grid.nc[0] ? Lx : 0.0f));
-                const float oy = fi.y - (cy < 0 ? -Ly : (cy >= B.grid.nc[1] ? Ly : 0.0f));
-                const float oz = fi.z - (cz < 0 ? -Lz : (cz >= B.grid.nc[2] ? Lz : 0.0f));
-                auto test = [&](const float4 &pj) {
-                    float dx = ox - pj.x, dy = oy - pj.y, dz = oz - pj.z;
-                    if (whole) {
-                        dx -= Lx * rintf(dx / Lx);
-                        dy -= Ly * rintf(dy / Ly);
-                        dz -= Lz * rintf(dz / Lz);
-                    }
-                    return dx * dx + dy * dy + dz * dz < Rf2 && pj.w > 0;
-                };
-                // two candidates in flight: the walk waits on these loads
-                constexpr int U = 2;
-                for (int k = beg + sub; k - sub < end; k += U * G) {
-                    float4 p[U];
-#pragma unroll
-                    for (int c = 0; c < U; c++) p[c] = a.posf[min(k + c * G, end - 1)];
-#pragma unroll
-                    for (int c = 0; c < U; c++)
-                        if (G > 1 || c == 0 || k + c < end) append(k + c * G, k + c * G < end && test(p[c]));
+        // FP32 distances with a margin for their rounding (2^-24 of a side per
+        // coordinate): the row may hold a few more than the exact radius
+        // asks for, never fewer, and a candidate is one 16-byte load.
+        const float Lmax = (float)fmax(B.box.L[0], fmax(B.box.L[1], B.box.L[2]));
+        const float Rf = (float)Rc * (1 + 1e-6f) + 5e-7f * Lmax, Rf2 = Rf * Rf * (1 + 1e-6f);
+        const float4 fi = a.posf[i];
+        for_each_run(B.grid, xs, Rc, [&](const bool full[3], int cx, int cy, int cz, int beg, int end) -> bool {
+            visited += end - beg;
+            if (visited > limit) return false;
+            // the image of this cell that the walk reached is the nearest
+            // one wherever the axis is not walked whole
+            const bool whole = full[0] || full[1] || full[2];
+            const float Lx = (float)B.box.L[0], Ly = (float)B.box.L[1], Lz = (float)B.box.L[2];
+            const float ox = fi.x - (cx < 0 ? -Lx : (cx >= B.grid.nc[0] ? Lx : 0.0f));
+            const float oy = fi.y - (cy < 0 ? -Ly : (cy >= B.grid.nc[1] ? Ly : 0.0f));
+            const float oz = fi.z - (cz < 0 ? -Lz : (cz >= B.grid.nc[2] ? Lz : 0.0f));
+            auto test = [&](const float4 &pj) {
+                float dx = ox - pj.x, dy = oy - pj.y, dz = oz - pj.z;
+                if (whole) {
+                    dx -= Lx * rintf(dx / Lx);
+                    dy -= Ly * rintf(dy / Ly);
+                    dz -= Lz * rintf(dz / Lz);
                 }
-                return m <= cap;
-            });
-        }
+                return dx * dx + dy * dy + dz * dz < Rf2 && pj.w > 0;
+            };
+            // two candidates in flight: the walk waits on these loads
+            constexpr int U = 2;
+            for (int k = beg + sub; k - sub < end; k += U * G) {
+                float4 p[U];
+#pragma unroll
+                for (int c = 0; c < U; c++) p[c] = a.posf[min(k + c * G, end - 1)];
+#pragma unroll
+                for (int c = 0; c < U; c++)
+                    if (G > 1 || c == 0 || k + c < end) append(k + c * G, k + c * G < end && test(p[c]));
+            }
+            return m <= cap;
+        });
         if (visited > limit) m = kNoRow;
         if (G == 1 && m < cap && (m & (kListChunk - 1)))
             flush_list_chunk(stage, row + (m & ~(kListChunk - 1)));
@@ -279,6 +294,93 @@ __global__ __launch_bounds__(kBlock) void density_rows_kernel(DensityStageArgs a
             a.row_r2[i] = Rc2;
         }
     });
+}
+
+// Candidate rows of the tree, kRowLanes lanes per particle (group_tree_walk).  With
+// one lane each the longest walks of a wavefront's lanes set its time, node after
+// node at the latency of each load: 1.15 ms for 250 k particles in Plummer spheres,
+// now 0.63
+// (16 lanes 0.69, 4 lanes 1.01).
+constexpr int kRowLanes = 8;
+__global__ __launch_bounds__(kBlock) void density_tree_rows_kernel(DensityStageArgs a)
+{
+    __shared__ GroupWalkLds<kRowLanes> walk[kBlock / kRowLanes];
+    const int gt = xcd_block() * kBlock + (int)threadIdx.x;
+    const int t = gt / kRowLanes, sub = gt % kRowLanes;
+    const bool valid = t < a.n_active;
+    for_box(a.boxes, a.box_of, valid ? a.active[t] : 0, valid, [&](const BoxDesc &B) {
+        const int i = a.active[t];
+        const double4 pi = a.posm[i];
+        if (!(pi.w > 0)) {  // density_isactive: gas with mass > 0 (density.c:85)
+            if (sub == 0) a.row_n[i] = kNoRow;
+            return;
+        }
+        double h = a.hsml[i];
+        if ((h < 0) || !isfinite(h) || (h > 0.99 * a.hp.max_hsml)) {  // density.c:484
+            h = 0.99 * a.hp.max_hsml;
+            if (sub == 0) a.hsml[i] = h;
+        }
+        const double Rc = kDensityCacheFactor * h, Rc2 = Rc * Rc;
+        const double xs[3] = {pi.x, pi.y, pi.z};
+        int *row = a.row_idx + (size_t)i * kDensityCacheCap;
+        int m = 0;
+        const bool whole = group_tree_walk<kRowLanes, true>(a.tree, B, xs, Rc, -1.0, sub, walk[threadIdx.x / kRowLanes],
+                                                            [&](int j, bool in) {
+            if (in) {
+                const double4 pj = a.posm[j];
+                double dp[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
+                wrap_dp(B.box, dp);
+                const double r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
+                in = r2 < Rc2 && pj.w > 0;
+            }
+            const uint64_t bits = group_ballot<kRowLanes>(in);
+            const int k = m + __popcll(bits & ((1ull << sub) - 1));
+            if (in && k < kDensityCacheCap) row[k] = j;
+            m += __popcll(bits);
+        }, a.budget ? 2 * a.budget : 0);
+        if (sub == 0) {
+            a.row_n[i] = whole && m <= kDensityCacheCap ? m : kNoRow;
+            a.row_r2[i] = Rc2;
+        }
+    });
+}
+
+// One sweep of a particle over its row, G lanes; true: sweep again.
+template <bool MFV, int G>
+__device__ __forceinline__ bool row_sweep(const DensityStageArgs &a, const BoxDesc &B, int i, const double4 &pi, int n,
+                                          int sub, int *chunk, Iterate &s, unsigned long long &cnt)
+{
+    const double4 vi = a.velu[i];
+    const int *row = a.row_idx + (size_t)i * kDensityCacheCap;
+    const double h2 = s.h * s.h;
+    double hinv, hinv3, hinv4;
+    kernel_hinv(s.h, hinv, hinv3, hinv4);
+    DensitySums S = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    double pv[3] = {0, 0, 0};
+    auto pair = [&](auto near, int j, const double4 &pj) {
+        double dp[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
+        if constexpr (near.value) wrap_near(B.box, dp);
+        else wrap_dp(B.box, dp);
+        const double r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
+        if (!(r2 < h2)) return;
+        cnt++;
+        density_add<MFV>(dp, r2, pj.w, vi, a.velu[j], hinv, hinv3, hinv4, S, pv);
+    };
+    auto scan = [&](auto near) {
+        if constexpr (G == 1) {
+            for_row_pairs(chunk, row, n, [&](int j0, int j1, bool second) {
+                const double4 p0 = a.posm[j0], p1 = a.posm[j1];
+                pair(near, j0, p0);
+                if (second) pair(near, j1, p1);
+            });
+        } else {
+            for (int k = sub; k < n; k += G) pair(near, row[k], a.posm[row[k]]);
+        }
+    };
+    if (__all(a.row_r2[i] < B.box.narrow2)) scan(std::true_type{});
+    else scan(std::false_type{});
+    if constexpr (G > 1) group_sums<G, MFV>(S, pv);
+    return density_step(a, i, sub == 0, S, pv, s);
 }
 
 // Sweep IT (0 or 1) over the rows, one launch each: nearly every particle of a
@@ -302,66 +404,111 @@ __global__ __launch_bounds__(kBlock, 3) void density_stage_kernel(DensityStageAr
         const double4 pi = a.posm[i];
         if (!(pi.w > 0)) return;
         if (IT == 1 && a.iter[i] != 1) return;  // done, or in the tail list
-        const double4 vi = a.velu[i];
         Iterate s = {a.hsml[i], IT ? a.left[i] : 0.0, IT ? a.right[i] : 0.0, a.cn[i], IT};
         const int n = a.row_n[i];
-        const int *row = a.row_idx + (size_t)i * kDensityCacheCap;
+        const double Rc2 = n <= kDensityCacheCap ? a.row_r2[i] : -1.0;
         bool again = true;
-        const double h2 = s.h * s.h;
-        if (n <= kDensityCacheCap && h2 <= a.row_r2[i]) {
-            double hinv, hinv3, hinv4;
-            kernel_hinv(s.h, hinv, hinv3, hinv4);
-            DensitySums S = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-            double pv[3] = {0, 0, 0};
-            auto pair = [&](auto near, int j, const double4 &pj) {
-                double dp[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
-                if constexpr (near.value) wrap_near(B.box, dp);
-                else wrap_dp(B.box, dp);
-                const double r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
-                if (!(r2 < h2)) return;
-                cnt++;
-                density_add<MFV>(dp, r2, pj.w, vi, a.velu, j, hinv, hinv3, hinv4, S, pv);
-            };
-            auto scan = [&](auto near) {
-                if constexpr (G == 1) {
-                    for_row_pairs(chunk, row, n, [&](int j0, int j1, bool second) {
-                        const double4 p0 = a.posm[j0], p1 = a.posm[j1];
-                        pair(near, j0, p0);
-                        if (second) pair(near, j1, p1);
-                    });
-                } else {
-                    for (int k = sub; k < n; k += G) pair(near, row[k], a.posm[row[k]]);
-                }
-            };
-            if (__all(a.row_r2[i] < B.box.narrow2)) scan(std::true_type{});
-            else scan(std::false_type{});
-            if constexpr (G > 1) group_sums<G, MFV>(S, pv);
+        if (s.h * s.h <= Rc2) {
+            again = row_sweep<MFV, G>(a, B, i, pi, n, sub, chunk, s, cnt);
             if (sub == 0) sweeps++;
-            again = density_step(a, i, sub == 0, S, pv, s);
         }
         if (sub == 0) {
             max_iter = s.iter;
             if (!again) a.iter[i] = 0;
             else if (IT == 0 && s.iter == 1) hand_on(a, i, s, nullptr, nullptr);
-            else hand_on(a, i, s, a.tail_list, a.n_tail);
+            else if (s.h * s.h <= Rc2) hand_on(a, i, s, a.tree.nodes ? nullptr : a.tail_list, a.n_tail);
+            else hand_on(a, i, s, a.walk_list, a.n_walk);
         }
     });
     count_sweeps(a, cnt, sweeps, max_iter);
 }
 
+// Tree: further sweeps over the rows.  Sets of strongly varying density leave
+// many particles after two (of 250 k in Plummer spheres 196 k need 2.6 more on
+// average, up to 10).  A workgroup takes a stretch of the active particles and
+// packs those not converged anew for every sweep, so that its wavefronts stay
+// full and keep neighbouring particles together; the last few go to the tail
+// list.  The 250 k: 0.50 ms (stretches of 256 or 1024: 0.67), against 2.0 ms with 16 lanes each to convergence
+// and 3.3 ms in four launches over lists whose order the atomics left.
+template <bool MFV, int G>
+__global__ __launch_bounds__(kBlock, 2) void density_more_kernel(DensityStageArgs a)
+{
+    constexpr int kStretch = 2 * kBlock / G, kFew = kStretch / 16;
+    __shared__ __align__(16) int lds[G == 1 ? kListChunk * kBlock : 1];
+    __shared__ int live[2][kStretch];
+    __shared__ int n_live[2];
+    int *chunk = wave_chunk(lds);
+    const int tid = (int)threadIdx.x, lane = tid & 63, sub = tid % G;
+    const int first = xcd_block() * kStretch;
+    unsigned long long cnt = 0, sweeps = 0;
+    int max_iter = 0;
+    // keeps i (one lane per entry calls) in list `to`
+    auto keep = [&](int to, int i, bool in) {
+        const uint64_t bits = __ballot(in);
+        int base = 0;
+        if (lane == 0 && bits) base = atomicAdd(&n_live[to], __popcll(bits));
+        base = __shfl(base, 0, 64);
+        if (in) live[to][base + __popcll(bits & ((1ull << lane) - 1))] = i;
+    };
+    if (tid == 0) n_live[0] = 0;
+    __syncthreads();
+    for (int k = tid; k < kStretch; k += kBlock) {
+        const int t = first + k;
+        const int i = t < a.n_active ? a.active[t] : 0;
+        bool in = t < a.n_active && a.posm[i].w > 0 && a.iter[i] != 0 && a.row_n[i] <= kDensityCacheCap;
+        if (in) {
+            const double h = a.hsml[i];
+            in = h * h <= a.row_r2[i];
+        }
+        keep(0, i, in);
+    }
+    for (int cur = 0;; cur ^= 1) {
+        __syncthreads();
+        const int n = n_live[cur];
+        if (tid == 0) n_live[cur ^ 1] = 0;
+        __syncthreads();
+        if (n <= kFew) {
+            for (int k = tid; k < n; k += kBlock) a.tail_list[atomicAdd(a.n_tail, 1)] = live[cur][k];
+            break;
+        }
+        for (int k0 = 0; k0 < n; k0 += kBlock / G) {
+            const int k = k0 + tid / G;
+            const bool valid = k < n;
+            const int i = valid ? live[cur][k] : 0;
+            bool stays = false;
+            if (valid) {
+                Iterate s = take_up(a, i);
+                const bool again = row_sweep<MFV, G>(a, a.boxes[a.box_of[i]], i, a.posm[i], a.row_n[i], sub, chunk, s, cnt);
+                if (sub == 0) {
+                    sweeps++;
+                    max_iter = s.iter > max_iter ? s.iter : max_iter;
+                    stays = again && s.h * s.h <= a.row_r2[i];
+                    if (stays) hand_on(a, i, s, nullptr, nullptr);
+                    else if (again) hand_on(a, i, s, a.walk_list, a.n_walk);
+                }
+            }
+            keep(cur ^ 1, i, stays);
+        }
+    }
+    count_sweeps(a, cnt, sweeps, max_iter);
+}
+
 // The listed particles, W lanes each, iterating to convergence: over the
 // particle's row while hsml stays inside it, else over a walk shared by the
-// lanes.  BUDGET: a walk past the candidate budget leaves the particle to
-// density_far_kernel.  A fixed grid strides over the device-side count.
-template <bool MFV, int W, bool BUDGET>
-__device__ __forceinline__ void density_iterate(const DensityStageArgs &a, const int *list, const int *count)
+// lanes.  A walk past the candidate budget (BUDGET) leaves the particle to the
+// far list, and any walk (kRowsOnly) to the walk list.  A fixed grid strides over
+// the device-side count.
+enum DensityWalk { kGridWalk, kTreeWalk, kRowsOnly };
+template <bool MFV, int W, bool BUDGET, DensityWalk WALK, int WAVES = 1>
+__device__ __forceinline__ void density_iterate(const DensityStageArgs &a, const int *list, const int *count,
+                                                WaveWalkLds *walk, BlockWalkLds<WAVES> *block_walk = nullptr)
 {
-    const int sub = (int)threadIdx.x % W;
-    const int n_groups = (int)(gridDim.x * (kBlock / W));
+    const int sub = (int)threadIdx.x % W, part = WAVES > 1 ? (int)threadIdx.x / 64 : 0;
+    const int n_groups = WAVES > 1 ? (int)gridDim.x : (int)(gridDim.x * (kBlock / W));
     const int n = *count;
     unsigned long long cnt = 0, sweeps = 0;
     int max_iter = 0;
-    for (int u = (int)(blockIdx.x * kBlock + threadIdx.x) / W; u < n; u += n_groups) {
+    for (int u = WAVES > 1 ? (int)blockIdx.x : (int)(blockIdx.x * kBlock + threadIdx.x) / W; u < n; u += n_groups) {
         const int i = list[u];
         const BoxDesc &B = a.boxes[a.box_of[i]];
         const double4 pi = a.posm[i];
@@ -378,32 +525,54 @@ __device__ __forceinline__ void density_iterate(const DensityStageArgs &a, const
             DensitySums S = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
             double pv[3] = {0, 0, 0};
             unsigned long long c = 0;
-            auto pair = [&](int j) {
-                const double4 pj = a.posm[j];
+            auto add = [&](const double4 &pj, const double4 &vj) {
                 double dp[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
                 wrap_dp(B.box, dp);
                 const double r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
                 if (!(r2 < h2 && pj.w > 0)) return;
                 c++;
-                density_add<MFV>(dp, r2, pj.w, vi, a.velu, j, hinv, hinv3, hinv4, S, pv);
+                density_add<MFV>(dp, r2, pj.w, vi, vj, hinv, hinv3, hinv4, S, pv);
             };
             if (h2 <= Rc2) {
                 const int *row = a.row_idx + (size_t)i * kDensityCacheCap;
-                for (int k = sub; k < n_row; k += W) pair(row[k]);
+                for (int k = sub + W * part; k < n_row; k += W * WAVES) add(a.posm[row[k]], a.velu[row[k]]);
+            } else if constexpr (WALK == kRowsOnly) {
+                far = true;
+                break;
+            } else if constexpr (WALK == kTreeWalk) {
+                // the loads of one step are used in the next
+                double4 pj = make_double4(0, 0, 0, 0), vj = pj;
+                auto step = [&](int j, bool valid) {
+                    add(pj, vj);
+                    pj.w = 0;
+                    if (valid) {
+                        pj = a.posm[j];
+                        vj = a.velu[j];
+                    }
+                };
+                if constexpr (WAVES > 1)
+                    block_tree_walk<WAVES>(a.tree, B, xs, s.h, *block_walk, step);
+                else
+                    far = !wave_tree_walk<false>(a.tree, B, xs, s.h, -1.0, sub, walk[threadIdx.x / 64], step,
+                                                 BUDGET ? a.budget : 0);
+                if (far) break;
+                add(pj, vj);
             } else {
                 const int budget = BUDGET ? a.budget : 0;
-                if (!group_candidates<W>(a.tree, B, xs, s.h, sub, budget, pair)) {
+                if (!group_candidates<W>(B, xs, s.h, sub, budget, [&](int j) { add(a.posm[j], a.velu[j]); })) {
                     far = true;
                     break;
                 }
             }
             group_sums<W, MFV>(S, pv);
+            if constexpr (WAVES > 1) block_sums<WAVES, MFV>(S, pv);
             cnt += c;
-            if (sub == 0) sweeps++;
-            again = density_step(a, i, sub == 0, S, pv, s);
+            if (sub == 0 && part == 0) sweeps++;
+            again = density_step(a, i, sub == 0 && part == 0, S, pv, s);
         }
-        if (sub == 0) {
-            if (far) hand_on(a, i, s, a.far_list, a.n_far);
+        if (sub == 0 && part == 0) {
+            if (far && WALK == kRowsOnly) hand_on(a, i, s, a.walk_list, a.n_walk);
+            else if (far) hand_on(a, i, s, a.far_list, a.n_far);
             max_iter = s.iter > max_iter ? s.iter : max_iter;
         }
     }
@@ -413,13 +582,38 @@ __device__ __forceinline__ void density_iterate(const DensityStageArgs &a, const
 template <bool MFV>
 __global__ __launch_bounds__(kBlock) void density_tail_kernel(DensityStageArgs a)
 {
-    density_iterate<MFV, kTailLanes, true>(a, a.tail_list, a.n_tail);
+    density_iterate<MFV, kTailLanes, true, kGridWalk>(a, a.tail_list, a.n_tail, nullptr);
 }
 
 template <bool MFV>
 __global__ __launch_bounds__(kBlock) void density_far_kernel(DensityStageArgs a)
 {
-    density_iterate<MFV, 64, false>(a, a.far_list, a.n_far);
+    density_iterate<MFV, 64, false, kGridWalk>(a, a.far_list, a.n_far, nullptr);
+}
+
+// Tree: what is left of the rows' sweeps, then the particles that have to walk, a
+// wavefront each, and a workgroup for those whose walk passes the candidate budget
+// (some hundred of 250 k particles in Plummer spheres, up to 50,000 slots in their
+// sweeps).  Those 250 k: walk 0.31 ms, far 0.59 ms (8 wavefronts 0.70), against 3.8
+// ms with a wavefront going from node to node.
+template <bool MFV>
+__global__ __launch_bounds__(kBlock) void density_tree_tail_kernel(DensityStageArgs a)
+{
+    density_iterate<MFV, kTailLanes, false, kRowsOnly>(a, a.tail_list, a.n_tail, nullptr);
+}
+
+template <bool MFV>
+__global__ __launch_bounds__(kBlock) void density_tree_walk_kernel(DensityStageArgs a)
+{
+    __shared__ WaveWalkLds walk[kBlock / 64];
+    density_iterate<MFV, 64, true, kTreeWalk>(a, a.walk_list, a.n_walk, walk);
+}
+
+template <bool MFV>
+__global__ __launch_bounds__(64 * kFarWaves) void density_tree_far_kernel(DensityStageArgs a)
+{
+    __shared__ BlockWalkLds<kFarWaves> walk;
+    density_iterate<MFV, 64, false, kTreeWalk, kFarWaves>(a, a.far_list, a.n_far, nullptr, &walk);
 }
 
 // no rows: every active particle starts in the tail list
@@ -432,7 +626,7 @@ __global__ void density_list_all_kernel(DensityStageArgs a)
     double h = a.hsml[i];
     if ((h < 0) || !isfinite(h) || (h > 0.99 * a.hp.max_hsml)) h = 0.99 * a.hp.max_hsml;  // density.c:484
     const Iterate s = {h, 0, 0, a.cn[i], 0};
-    hand_on(a, i, s, a.tail_list, a.n_tail);
+    hand_on(a, i, s, a.walk_list, a.n_walk);
 }
 
 inline unsigned nblocks(long long n) { return (unsigned)((n + kBlock - 1) / kBlock); }
@@ -444,11 +638,11 @@ void launch_density_rows(hipStream_t s, const DensityStageArgs &a)
     if (a.n_active <= 0) return;
     const dim3 block(kBlock);
     if (a.tree.nodes)
-        hipLaunchKernelGGL((density_rows_kernel<true, 1>), dim3(nblocks(a.n_active)), block, 0, s, a);
+        hipLaunchKernelGGL(density_tree_rows_kernel, dim3(nblocks((long long)kRowLanes * a.n_active)), block, 0, s, a);
     else if (a.lanes == 8)
-        hipLaunchKernelGGL((density_rows_kernel<false, 8>), dim3(nblocks(8LL * a.n_active)), block, 0, s, a);
+        hipLaunchKernelGGL(density_rows_kernel<8>, dim3(nblocks(8LL * a.n_active)), block, 0, s, a);
     else
-        hipLaunchKernelGGL((density_rows_kernel<false, 1>), dim3(nblocks(a.n_active)), block, 0, s, a);
+        hipLaunchKernelGGL(density_rows_kernel<1>, dim3(nblocks(a.n_active)), block, 0, s, a);
 }
 
 template <int G>
@@ -477,9 +671,31 @@ void launch_density_stage(hipStream_t s, const DensityStageArgs &a)
     }
 }
 
+// the counts are on the device: grids that fill the chip, at most one group per particle
+template <bool MFV>
+static void launch_tree_tail(hipStream_t s, const DensityStageArgs &a)
+{
+    const dim3 block(kBlock);
+    if (a.row_idx) {
+        const dim3 grid(nblocks((long long)a.lanes * a.n_active / 2 + a.lanes));
+        if (a.lanes == 8) hipLaunchKernelGGL((density_more_kernel<MFV, 8>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((density_more_kernel<MFV, 1>), grid, block, 0, s, a);
+        hipLaunchKernelGGL(density_tree_tail_kernel<MFV>, dim3(std::min(2048u, nblocks((long long)kTailLanes * a.n_active))),
+                           block, 0, s, a);
+    }
+    hipLaunchKernelGGL(density_tree_walk_kernel<MFV>, dim3(std::min(2048u, nblocks(64LL * a.n_active))), block, 0, s, a);
+    if (a.budget)
+        hipLaunchKernelGGL(density_tree_far_kernel<MFV>, dim3(std::min(512, a.n_active)), dim3(64 * kFarWaves), 0, s, a);
+}
+
 void launch_density_tail(hipStream_t s, const DensityStageArgs &a)
 {
     if (a.n_active <= 0) return;
+    if (a.tree.nodes) {
+        if (a.pvel) launch_tree_tail<true>(s, a);
+        else launch_tree_tail<false>(s, a);
+        return;
+    }
     // the count is on the device: enough workgroups to fill the chip, at most one group per particle
     const dim3 grid(std::min(2048u, nblocks((long long)kTailLanes * a.n_active))), block(kBlock);
     if (a.pvel) hipLaunchKernelGGL(density_tail_kernel<true>, grid, block, 0, s, a);

@@ -55,7 +55,7 @@ constexpr int kTreeBucket = 8;
 struct alignas(16) TreeNode {
     float4 lo;             // x, y, z rounded down; w = max hsml below the node, rounded up
     float4 hi;             // x, y, z rounded up; w = escape link (int bits)
-    int4 link;             // left child, first slot, last slot, unused
+    int4 link;             // left child, first slot, last slot, right child
 };
 
 struct TreeArgs {
@@ -180,7 +180,7 @@ struct SymRowArgs {
     int *brow;             // kPairRowCap per particle
     int *bcount;           // zeroed before the scatter
     int *wlist;            // particles j whose own row does not cover h_j (walked by a wavefront each)
-    int *wcount;
+    int *wcount;           // and the count of GradientArgs.far_list beside it; zeroed before the scatter
 };
 // a sweep over at most this many particles runs one wavefront per particle:
 // they all fit on the GPU at once, and a walk shared by 64 lanes is shorter
@@ -191,7 +191,9 @@ constexpr int kWaveSweepMax = 4096;
 // (measured 2.3e-7 on 31.5 M particles), and FP32 r^2 carries up to 2e-6 h^2.
 constexpr double kEdgeBand = 1e-5;
 
-// The density stage of precisions 0 and 1 (gzm_density.hip)
+// The density stage of precisions 0 and 1 (gzm_density.hip).  Its counts lie
+// together: select, tail, far, walk.
+constexpr int kDensityCounts = 4;
 struct DensityStageArgs {
     const BoxDesc *boxes;
     const int *box_of;
@@ -211,8 +213,9 @@ struct DensityStageArgs {
     int *row_idx, *row_n;
     double *row_r2;
     int *iter;             // sweeps done by a particle handed on to a list
-    int *tail_list, *n_tail;
-    int *far_list, *n_far;
+    int *tail_list, *n_tail;  // not converged after the stage's sweeps
+    int *far_list, *n_far;    // past the candidate budget
+    int *walk_list, *n_walk;  // tree: without a usable row (grid: the tail list)
     int budget;            // candidates of one walk in the tail kernel; 0: no limit
     int lanes;             // lanes per particle of the row and stage kernels: 1 or 8
     Counters *ctr;
@@ -298,6 +301,8 @@ struct GradientArgs {
     const double *dcache_r2;
     const int *brow;
     const int *bcount;
+    int *far_list;         // with brow: active entries whose rows do not hold their pair set, listed
+    int *n_far;            //   by the row kernel for gradients_walk_kernel (device count, zeroed)
 };
 
 // Pairs whose Riemann problem reaches the exact solver are taken out of the
@@ -390,7 +395,7 @@ void launch_clear_counters(hipStream_t s, Counters *ctr);
 void launch_map_active(hipStream_t s, int n_active, const int *active_caller, const int *inv, int *active_sorted);
 // density stage of precisions 0 and 1, in this order; counts[0] and [1] (tail
 // and far list) are cleared by the first, the counter block when ctr is given
-void launch_density_begin(hipStream_t s, Counters *ctr, int *counts);
+void launch_density_begin(hipStream_t s, Counters *ctr, int *counts);  // counts 1 .. kDensityCounts - 1
 void launch_density_rows(hipStream_t s, const DensityStageArgs &a);
 void launch_density_stage(hipStream_t s, const DensityStageArgs &a);
 void launch_density_tail(hipStream_t s, const DensityStageArgs &a);

@@ -132,10 +132,7 @@ __global__ void clear_counters_kernel(Counters *ctr)
 
 __global__ void density_begin_kernel(Counters *ctr, int *counts)
 {
-    if (threadIdx.x == 0) {
-        counts[0] = 0;
-        counts[1] = 0;
-    }
+    if (threadIdx.x >= 1 && threadIdx.x < kDensityCounts) counts[threadIdx.x] = 0;
     if (ctr) ctr[threadIdx.x] = Counters{};  // kCtrSpread threads
 }
 
@@ -255,6 +252,7 @@ __device__ __forceinline__ int density_store(const DensitySweepArgs &a, int t, i
 // the (device-side) count.
 __global__ __launch_bounds__(kBlock) void density_heavy_kernel(DensitySweepArgs a)
 {
+    __shared__ WaveWalkLds walk[kBlock / 64];
     const int lane = threadIdx.x & 63;
     const int n_waves = (int)(gridDim.x * (kBlock / 64));
     const int n = a.wave_all ? (a.n_live_dev ? *a.n_live_dev : a.n_live) : *a.n_heavy;
@@ -276,7 +274,7 @@ __global__ __launch_bounds__(kBlock) void density_heavy_kernel(DensitySweepArgs 
         const double xs[3] = {pi.x, pi.y, pi.z};
         unsigned long long c = 0;
         bool edge = false;
-        wave_candidates(a.tree, G, xs, h, lane, [&](int j) {
+        wave_candidates(a.tree, G, xs, h, lane, walk[threadIdx.x >> 6], [&](int j) {
             if (density_pair(G, pi, vi, a, j, h2, hinv, hinv3, hinv4, S, edge)) c++;
         });
         const bool any_edge = __any(edge);
@@ -407,6 +405,7 @@ __global__ __launch_bounds__(kBlock) void sym_rows_scatter_kernel(SymRowArgs a)
 // (wave_candidates).  A fixed grid strides over the device-side count.
 __global__ __launch_bounds__(kBlock) void sym_rows_wave_kernel(SymRowArgs a)
 {
+    __shared__ WaveWalkLds walk[kBlock / 64];
     const int lane = threadIdx.x & 63;
     const int n_waves = (int)(gridDim.x * (kBlock / 64));
     const int n = *a.wcount;
@@ -417,7 +416,7 @@ __global__ __launch_bounds__(kBlock) void sym_rows_wave_kernel(SymRowArgs a)
         const double h_j = a.hsml[j];
         const double hj2 = h_j * h_j;
         const double xs[3] = {pj.x, pj.y, pj.z};
-        wave_candidates(a.tree, G, xs, h_j, lane, [&](int i) { sym_offer(a, G, pj, hj2, j, i); });
+        wave_candidates(a.tree, G, xs, h_j, lane, walk[threadIdx.x >> 6], [&](int i) { sym_offer(a, G, pj, hj2, j, i); });
     }
 }
 
@@ -445,6 +444,40 @@ __global__ __launch_bounds__(kBlock) void sym_rows_sort_kernel(int n, int *brow,
 // back to the walk for a particle whose rows do not hold its pair set)
 enum GradSource { kFromWalk, kFromTreeRows, kFromGridRows };
 
+// One particle's sums of the gradient loop: g as stored (rho, P, v rows), the
+// extremes of the differences (rho, P, v), the largest distance.
+struct GradSums {
+    double g[15], mn[5], mx[5], maxd;
+};
+
+// NV_T, the limiter (SELFGRAVITY_OFF, no MAGNETIC/GALSF: h_lim = h, stol = 0.1;
+// gradients.c:1219-1232) and, with every particle active, the force record that
+// pack_force_kernel would write
+__device__ __forceinline__ void finish_gradients(const GradientArgs &a, int i, const double4 &xi, const GradRec &ri,
+                                                 GradSums &S, double g_out[15], ForceRec &f_out)
+{
+    const double h_i = xi.w, rho_i = ri.vr.w, p_i = ri.pm.x, m_i = ri.pm.y;
+    double nvt[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) nvt[k] = a.nvt[6 * (size_t)i + k];
+#pragma unroll
+    for (int q = 0; q < 5; q++) apply_nvt(nvt, S.g + 3 * q);
+    const double cn = a.cn[i];
+    const double d_max = (h_i > S.maxd) ? h_i : S.maxd;
+    double a_lim = 0.25;
+    if (cn > 100) a_lim = dmin(0.5, 0.25 + 0.25 * (cn - 100) / 100);
+    slope_limit(S.g + 0, S.mx[0], S.mn[0], a_lim, h_i, 0, 1, d_max, rho_i);
+    slope_limit(S.g + 3, S.mx[1], S.mn[1], a_lim, h_i, 0.1, 1, d_max, p_i);
+    slope_limit(S.g + 6, S.mx[2], S.mn[2], a_lim, h_i, 0.1, 0, 0, 0);
+    slope_limit(S.g + 9, S.mx[3], S.mn[3], a_lim, h_i, 0.1, 0, 0, 0);
+    slope_limit(S.g + 12, S.mx[4], S.mn[4], a_lim, h_i, 0.1, 0, 0, 0);
+#pragma unroll
+    for (int k = 0; k < 15; k++) g_out[k] = S.g[k];
+    if (a.frec_out)
+        f_out = make_force_rec(make_double4(xi.x, xi.y, xi.z, m_i), make_double4(ri.vr.x, ri.vr.y, ri.vr.z, 0.0),
+                               rho_i, p_i, h_i, a.dhsml[i], cn, a.fce[i], nvt, S.g, a.gamma);
+}
+
 // Bound by the L2 reads of the neighbours (5,500 lines per wavefront before the
 // split of GradRec and the chunked row reads): of 2.1 M particles 2.36 ms from
 // the walk, 1.72 from the rows entry by entry, 1.27 with rows read 64 bytes at
@@ -465,7 +498,7 @@ __global__ __launch_bounds__(BS, 3) void gradients_kernel(GradientArgs a)
     __shared__ __align__(16) int lds_row[G == 1 && SRC == kFromGridRows ? kListChunk * BS : 1];
     int *stage = wave_chunk(lds), *chunk = wave_chunk(lds_row);
     const int t = (xcd_block() * BS + (int)threadIdx.x) / G, sub = (int)threadIdx.x % G;
-    const bool valid = t < a.n_active;
+    bool valid = t < a.n_active;
     unsigned long long cnt = 0;
     int listed = 0, out_i = 0;
     double g_out[15];  // the particle's gradients and force record, stored by the whole wavefront
@@ -602,14 +635,19 @@ __global__ __launch_bounds__(BS, 3) void gradients_kernel(GradientArgs a)
                         jb = (kb < n_b) ? rb[kb] : kNoSlot;
                     }
                 }
-            } else if constexpr (G > 1) {  // grid
+            } else if constexpr (SRC == kFromTreeRows) {  // left to gradients_walk_kernel
+                a.far_list[atomicAdd(a.n_far, 1)] = t;
+                valid = false;
+                return;
+            } else if constexpr (G > 1) {
                 const double R = (B.hmax > h_i) ? B.hmax : h_i;
                 bool full[3];
                 for_each_cell(B.grid, xs, R, full, [&](int, int, int, int beg, int end) {
                     for (int k = beg; k < end; k += G) visit_step(std::false_type{}, k + sub, k + sub < end);
                 }, h_i);
             } else {
-                for_each_neighbour_candidate(a.tree, B, xs, h_i, true, visit);
+                const double R = (B.hmax > h_i) ? B.hmax : h_i;
+                for_each_candidate(B.grid, xs, R, visit, h_i);
             }
             // the partly filled last chunk (entries past `listed` are never read)
             if (G == 1 && list_row && listed < a.list.cap && (listed & (kListChunk - 1)))
@@ -630,33 +668,9 @@ __global__ __launch_bounds__(BS, 3) void gradients_kernel(GradientArgs a)
             mn_v1 = group_min<G>(mn_v1); mx_v1 = group_max<G>(mx_v1);
             mn_v2 = group_min<G>(mn_v2); mx_v2 = group_max<G>(mx_v2);
         }
-        double nvt[6];
-#pragma unroll
-        for (int k = 0; k < 6; k++) nvt[k] = a.nvt[6 * (size_t)i + k];
-        double gr[3] = {gr0, gr1, gr2}, gp[3] = {gp0, gp1, gp2};
-        double gv0[3] = {gv00, gv01, gv02}, gv1[3] = {gv10, gv11, gv12}, gv2[3] = {gv20, gv21, gv22};
-        apply_nvt(nvt, gr);
-        apply_nvt(nvt, gp);
-        apply_nvt(nvt, gv0);
-        apply_nvt(nvt, gv1);
-        apply_nvt(nvt, gv2);
-        // SELFGRAVITY_OFF, no MAGNETIC/GALSF: h_lim = h, stol = 0.1 (gradients.c:1219-1232)
-        const double cn = a.cn[i];
-        const double d_max = (h_i > maxd) ? h_i : maxd;
-        double a_lim = 0.25;
-        if (cn > 100) a_lim = dmin(0.5, 0.25 + 0.25 * (cn - 100) / 100);
-        slope_limit(gr, mx_r, mn_r, a_lim, h_i, 0, 1, d_max, rho_i);
-        slope_limit(gp, mx_p, mn_p, a_lim, h_i, 0.1, 1, d_max, p_i);
-        slope_limit(gv0, mx_v0, mn_v0, a_lim, h_i, 0.1, 0, 0, 0);
-        slope_limit(gv1, mx_v1, mn_v1, a_lim, h_i, 0.1, 0, 0, 0);
-        slope_limit(gv2, mx_v2, mn_v2, a_lim, h_i, 0.1, 0, 0, 0);
-        const double g[15] = {gr[0], gr[1], gr[2], gp[0], gp[1], gp[2], gv0[0], gv0[1], gv0[2],
-                              gv1[0], gv1[1], gv1[2], gv2[0], gv2[1], gv2[2]};
-#pragma unroll
-        for (int k = 0; k < 15; k++) g_out[k] = g[k];
-        if (a.frec_out)  // every particle active: its force record, as pack_force_kernel writes it
-            f_out = make_force_rec(make_double4(xi.x, xi.y, xi.z, m_i), make_double4(ri.vr.x, ri.vr.y, ri.vr.z, 0.0),
-                                   rho_i, p_i, h_i, a.dhsml[i], cn, a.fce[i], nvt, g, a.gamma);
+        GradSums S = {{gr0, gr1, gr2, gp0, gp1, gp2, gv00, gv01, gv02, gv10, gv11, gv12, gv20, gv21, gv22},
+                      {mn_r, mn_p, mn_v0, mn_v1, mn_v2}, {mx_r, mx_p, mx_v0, mx_v1, mx_v2}, maxd};
+        finish_gradients(a, i, xi, ri, S, g_out, f_out);
         if (a.list.idx && sub == 0) a.list.count[t] = listed;
     });
     if constexpr (G == 1) {
@@ -678,6 +692,111 @@ __global__ __launch_bounds__(BS, 3) void gradients_kernel(GradientArgs a)
         const bool over = __any(listed > a.list.cap);
         if ((threadIdx.x & 63) == 0 && over) atomicAdd(&ctr_slot(a.ctr)->overflow_slices, 1);
     }
+    wave_add_u64(&ctr_slot(a.ctr)->interactions, cnt);
+}
+
+// Tree: the particles whose rows do not hold their pair set (`list`, a device
+// count; W = 64), or, without rows, every active one (list NULL; W = 16, as there
+// are 15 sums: 40 k active of 400 k 0.48 ms, with W = 64 0.64, with one lane each
+// 2.6), W lanes each: the lanes share the walk and the pairs' terms.  Each sum is then added up by one
+// lane in ascending slot order, the order of the merged rows, so a particle's
+// bits do not depend on the rows.  250 k particles in Plummer spheres: row kernel
+// and this one 0.60 ms, against 4.2 ms for the row kernel with these particles
+// walking in a lane each.
+template <int W>
+__global__ __launch_bounds__(kBlock) void gradients_walk_kernel(GradientArgs a, const int *list, const int *count)
+{
+    static_assert(W >= 16, "15 sums");
+    __shared__ GroupWalkLds<W> walk[kBlock / W];
+    __shared__ double term_lds[kBlock / W][W][8];
+    const int lane = (int)threadIdx.x % W;
+    double (*term)[8] = term_lds[threadIdx.x / W];
+    const int n = list ? *count : a.n_active;
+    const int n_groups = (int)(gridDim.x * (kBlock / W));
+    const int q_a = lane % 3, q_b = 3 + min(lane / 3, 4);  // lane < 15: the sum of w[q_a] d[q_b - 3]
+    unsigned long long cnt = 0;
+    bool over = false;
+    for (int u = (int)(blockIdx.x * kBlock + threadIdx.x) / W; u < n; u += n_groups) {
+        const int t = list ? list[u] : u;
+        const int i = a.active[t];
+        const BoxDesc &B = a.boxes[a.box_of[i]];
+        const GradRec ri = a.rec[i];
+        const double4 xi = a.xh[i];
+        const double h_i = xi.w, rho_i = ri.vr.w, p_i = ri.pm.x, m_i = ri.pm.y;
+        int *list_row = a.list.idx ? a.list.idx + (size_t)t * a.list.cap : nullptr;
+        int listed = 0;
+        GradSums S = {};
+        if ((m_i > 0) && (rho_i > 0) && (h_i > 0)) {  // GasGrad_isactive (gradients.c:66-75)
+            double hinv, hinv3, hinv4, sum = 0;
+            kernel_hinv(h_i, hinv, hinv3, hinv4);
+            const double h2_i = h_i * h_i;
+            const double xs[3] = {xi.x, xi.y, xi.z};
+            group_tree_walk<W, true>(a.tree, B, xs, h_i, h_i, lane, walk[threadIdx.x / W], [&](int j, bool valid) {
+                double dp[3] = {0, 0, 0}, r2 = 0;
+                double4 xj = make_double4(0, 0, 0, 0), vr = xj;
+                double2 pm = make_double2(0, 0);
+                if (valid) {
+                    xj = a.xh[j];
+                    dp[0] = xs[0] - xj.x;
+                    dp[1] = xs[1] - xj.y;
+                    dp[2] = xs[2] - xj.z;
+                    wrap_dp(B.box, dp);
+                    r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
+                    valid = r2 > 0 && !((r2 >= h2_i) && (r2 >= xj.w * xj.w));
+                }
+                if (valid) {
+                    vr = a.rec[j].vr;
+                    pm = a.rec[j].pm;
+                    valid = (pm.y > 0) && (vr.w > 0);
+                }
+                const uint64_t below = (1ull << lane) - 1, pairs = group_ballot<W>(valid);
+                const int k = listed + __popcll(pairs & below);
+                if (valid && list_row && k < a.list.cap) list_row[k] = j;
+                listed += __popcll(pairs);
+                if (!(xj.w > 0)) valid = false;
+                const double r = sqrt(r2);
+                if (valid) {
+                    cnt++;
+                    if (r > S.maxd) S.maxd = r;
+                }
+                const double d[5] = {vr.w - rho_i, pm.x - p_i, vr.x - ri.vr.x, vr.y - ri.vr.y, vr.z - ri.vr.z};
+                if (valid)
+                    for (int q = 0; q < 5; q++) minmax_check(d[q], S.mn[q], S.mx[q]);
+                const bool inside = valid && r < h_i;
+                const uint64_t in = group_ballot<W>(inside);
+                if (inside) {
+                    const double wk_i = kernel_w(r * hinv, hinv3);
+                    double *o = term[__popcll(in & below)];
+                    for (int q = 0; q < 3; q++) o[q] = -wk_i * dp[q];
+                    for (int q = 0; q < 5; q++) o[3 + q] = d[q];
+                }
+                wave_lds_fence();
+                const int n_in = __popcll(in);
+#pragma unroll 4
+                for (int p = 0; p < n_in; p++) sum += term[p][q_a] * term[p][q_b];
+                wave_lds_fence();
+            });
+#pragma unroll
+            for (int q = 0; q < 15; q++) S.g[q] = __shfl(sum, q, W);
+            S.maxd = group_max<W>(S.maxd);
+            for (int q = 0; q < 5; q++) {
+                S.mn[q] = group_min<W>(S.mn[q]);
+                S.mx[q] = group_max<W>(S.mx[q]);
+            }
+        } else if ((m_i > 0) && (rho_i > 0)) {
+            listed = a.list.cap + 1;  // as in gradients_kernel
+        }
+        double g_out[15];
+        ForceRec f_out;
+        finish_gradients(a, i, xi, ri, S, g_out, f_out);
+        if (lane == 0) {
+            for (int k = 0; k < 15; k++) a.grad[15 * (size_t)i + k] = g_out[k];
+            if (a.frec_out) a.frec_out[i] = f_out;
+            if (a.list.idx) a.list.count[t] = listed;
+        }
+        over |= listed > a.list.cap;
+    }
+    if (a.list.idx && lane == 0 && over) atomicAdd(&ctr_slot(a.ctr)->overflow_slices, 1);
     wave_add_u64(&ctr_slot(a.ctr)->interactions, cnt);
 }
 
@@ -1083,7 +1202,7 @@ void launch_sym_rows(hipStream_t s, const SymRowArgs &a)
 {
     if (a.n <= 0) return;
     launch_fill_int(s, a.bcount, a.n, 0);
-    launch_fill_int(s, a.wcount, 1, 0);
+    launch_fill_int(s, a.wcount, 2, 0);
     hipLaunchKernelGGL(sym_rows_scatter_kernel, dim3(nblocks(a.n)), dim3(kBlock), 0, s, a);
     hipLaunchKernelGGL(sym_rows_wave_kernel, dim3(2048), dim3(kBlock), 0, s, a);
     hipLaunchKernelGGL(sym_rows_sort_kernel, dim3(nblocks(a.n)), dim3(kBlock), 0, s, a.n, a.brow, a.bcount);
@@ -1100,13 +1219,21 @@ void launch_gradients(hipStream_t s, const GradientArgs &a)
 {
     if (a.n_active <= 0) return;
     const dim3 grid(nblocks(a.n_active, a.block)), block(a.block);
-    if (a.lanes == 8 && !a.tree.nodes) {
+    if (a.lanes == 8) {
         const dim3 few(nblocks(8LL * a.n_active));
         if (a.dcache_idx) hipLaunchKernelGGL((gradients_kernel<kBlock, kFromGridRows, 8>), few, dim3(kBlock), 0, s, a);
         else hipLaunchKernelGGL((gradients_kernel<kBlock, kFromWalk, 8>), few, dim3(kBlock), 0, s, a);
-    } else if (a.brow) {
-        launch_gradients_from<kFromTreeRows>(s, a, grid, block);
-    } else if (a.dcache_idx && !a.tree.nodes) {
+    } else if (a.tree.nodes) {
+        // the list's length is on the device: at most what fills the chip
+        if (a.brow) {
+            const dim3 waves(std::min(2048u, nblocks(64LL * a.n_active)));
+            launch_gradients_from<kFromTreeRows>(s, a, grid, block);
+            hipLaunchKernelGGL(gradients_walk_kernel<64>, waves, dim3(kBlock), 0, s, a, a.far_list, a.n_far);
+        } else {
+            const dim3 groups(nblocks(16LL * a.n_active));
+            hipLaunchKernelGGL(gradients_walk_kernel<16>, groups, dim3(kBlock), 0, s, a, nullptr, nullptr);
+        }
+    } else if (a.dcache_idx) {
         launch_gradients_from<kFromGridRows>(s, a, grid, block);
     } else {
         launch_gradients_from<kFromWalk>(s, a, grid, block);

@@ -914,6 +914,7 @@ __global__ __launch_bounds__(kBlock, 4) void force_deferred_f32_kernel(ForceArgs
 // their partial sums, maxima and minima; lane 0 applies NV_T and the limiter.  Sums in another order than the FP64 pass: equal to ~1e-16.
 __global__ __launch_bounds__(kBlock) void gradients_redo_fp64_kernel(ForceArgs a)
 {
+    __shared__ WaveWalkLds walk[kBlock / 64];
     const int n_redo = a.redo_count[1];
     const int lane = threadIdx.x & 63;
     const int n_waves = gridDim.x * (kBlock / 64);
@@ -933,7 +934,7 @@ __global__ __launch_bounds__(kBlock) void gradients_redo_fp64_kernel(ForceArgs a
             const double h2_i = h_i * h_i;
             const double xs[3] = {pi.x, pi.y, pi.z};
             const double R = (h_i > G.hmax) ? h_i : G.hmax;
-            wave_pair_candidates(a.tree, G, xs, R, h_i, lane, [&](int j) {
+            wave_pair_candidates(a.tree, G, xs, R, h_i, lane, walk[threadIdx.x >> 6], [&](int j) {
                 const double4 xj = a.posm[j];
                 double dp[3] = {xs[0] - xj.x, xs[1] - xj.y, xs[2] - xj.z};
                 wrap_dp(G.box, dp);
@@ -1017,6 +1018,7 @@ __global__ __launch_bounds__(kBlock) void gradients_redo_fp64_kernel(ForceArgs a
 template <bool REDO>
 __global__ __launch_bounds__(kBlock) void force_wave_fp64_kernel(ForceArgs a, const int *list, const int *count)
 {
+    __shared__ WaveWalkLds walk[kBlock / 64];
     const int n_redo = *count;
     if (REDO && blockIdx.x == 0 && threadIdx.x == 0 && n_redo > 0) atomicAdd(&ctr_slot(a.ctr)->redo_n, n_redo);
     const int lane = threadIdx.x & 63;
@@ -1039,7 +1041,7 @@ __global__ __launch_bounds__(kBlock) void force_wave_fp64_kernel(ForceArgs a, co
             const double xs[3] = {pi.x, pi.y, pi.z};
             const double R = (h_i > G.hmax) ? h_i : G.hmax;
             ROut<double> ro = {0, 0, {0, 0, 0}, 0};
-            wave_pair_candidates(a.tree, G, xs, R, h_i, lane, [&](int j) {
+            wave_pair_candidates(a.tree, G, xs, R, h_i, lane, walk[threadIdx.x >> 6], [&](int j) {
                 if (j == i) return;
                 double dp[3];
                 const double r2 = exact_r2(G.box, pi, a.posm[j], dp);

@@ -273,7 +273,7 @@ __global__ void pack_nodes_kernel(TreeBuild t)
                         __double2float_ru(lo.w));
     nd.hi = make_float4(__double2float_ru(hi.x), __double2float_ru(hi.y), __double2float_ru(hi.z),
                         __int_as_float(t.esc[g]));
-    nd.link = make_int4(t.child[g].x, r.x, r.y, 0);
+    nd.link = make_int4(t.child[g].x, r.x, r.y, t.child[g].y);
     t.nodes[g] = nd;
 }
 
