@@ -153,6 +153,8 @@ struct gzm_ctx {
     TreeArgs tree;      // all null in grid mode
     TreeBuild tbuild;
 
+    Counters *h_ctr = nullptr;  // pinned: a stage's counters as the host reads them
+
     gzm_timing timing;
     std::vector<TimedLaunch> pending;
     std::vector<hipEvent_t> event_pool;
@@ -315,15 +317,56 @@ gzm_status upload_sorted(gzm_ctx *c, const double *host, double *dst, int width)
     return GZM_OK;
 }
 
-// sorted device array -> host array in caller order
-gzm_status download_sorted(gzm_ctx *c, const double *src, double *host, int width)
+// The device's address of host memory that it can write itself, all of
+// [host, host + bytes); NULL: it cannot.
+double *device_view(double *host, size_t bytes)
 {
-    size_t cnt = (size_t)c->n * width;
-    gzm_status s = ensure_stage(c, cnt);
-    if (s) return s;
-    launch_scatter_scalar(c->stream, c->n, c->d_perm, src, c->d_stage, width);
+    if (bytes == 0 || (uintptr_t)host % sizeof(double)) return nullptr;
+    hipPointerAttribute_t first, last;
+    if (hipPointerGetAttributes(&first, host) != hipSuccess ||
+        hipPointerGetAttributes(&last, (char *)host + bytes - 1) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (first.type != hipMemoryTypeHost || last.type != hipMemoryTypeHost || !first.devicePointer || !last.devicePointer)
+        return nullptr;
+    if ((char *)last.devicePointer - (char *)first.devicePointer != (ptrdiff_t)(bytes - 1)) return nullptr;
+    return (double *)first.devicePointer;
+}
+
+// Sorted device arrays -> host arrays in caller order.  Fields in memory that
+// the device can write (pinned) go there from one kernel; the others through a
+// staging array and a copy each.  Returns when all are there.
+gzm_status download_fields(gzm_ctx *c, const std::vector<ExportField> &fields)
+{
+    ExportArgs direct = {}, one = {};
+    direct.n = one.n = c->n;
+    direct.inv = one.inv = c->d_inv;
+    one.n_fields = 1;
+    int width = 0;
+    std::vector<const ExportField *> staged;
+    for (auto &f : fields) {
+        double *d = direct.n_fields < kMaxExport ? device_view(f.dst, (size_t)c->n * f.w * sizeof(double)) : nullptr;
+        if (d) {
+            direct.field[direct.n_fields] = f;
+            direct.field[direct.n_fields++].dst = d;
+        } else {
+            staged.push_back(&f);
+            width = std::max(width, f.w);
+        }
+    }
+    launch_export(c->stream, direct);
+    if (!staged.empty()) {
+        gzm_status s = ensure_stage(c, (size_t)c->n * width);
+        if (s) return s;
+    }
+    for (auto *f : staged) {
+        one.field[0] = *f;
+        one.field[0].dst = c->d_stage;
+        launch_export(c->stream, one);
+        GZM_HIP(hipMemcpyAsync(f->dst, c->d_stage, (size_t)c->n * f->w * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    }
     GZM_HIP(hipGetLastError());
-    GZM_HIP(hipMemcpyAsync(host, c->d_stage, cnt * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     GZM_HIP(hipStreamSynchronize(c->stream));
     return GZM_OK;
 }
@@ -348,15 +391,16 @@ void fold_counters(const Counters *part, Counters *h)
         h->overflow_slices += part[k].overflow_slices;
         h->sweeps = std::max(h->sweeps, part[k].sweeps);
         h->updates += part[k].updates;
+        h->deferred += part[k].deferred;
     }
 }
 
 gzm_status read_counters(gzm_ctx *c, int slot, Counters *h)
 {
-    Counters part[kCtrSpread];
-    GZM_HIP(hipMemcpyAsync(part, c->d_ctr + slot * kCtrSpread, sizeof(part), hipMemcpyDeviceToHost, c->stream));
+    launch_publish_counters(c->stream, c->d_ctr + slot * kCtrSpread, c->h_ctr);
+    GZM_HIP(hipGetLastError());
     GZM_HIP(hipStreamSynchronize(c->stream));
-    fold_counters(part, h);
+    *h = *c->h_ctr;
     return GZM_OK;
 }
 
@@ -444,12 +488,17 @@ gzm_status ensure_list(gzm_ctx *c)
 }
 
 // per-box max hsml into the device box descriptors (no host round trip)
-gzm_status compute_hmax(gzm_ctx *c)
+// and, with `ctr`, that stage's counters cleared
+gzm_status compute_hmax(gzm_ctx *c, Counters *ctr)
 {
-    if (c->hmax_valid) return GZM_OK;
+    if (c->hmax_valid) {
+        if (ctr) launch_clear_counters(c->stream, ctr);
+        return GZM_OK;
+    }
     c->hmax_valid = true;
     Timed tm(c, kOther);
-    launch_box_hmax(c->stream, c->n_boxes, c->d_boxes, c->d_hsml, c->n_hmax_tiles, c->d_hmax_tiles);
+    launch_box_hmax(c->stream, c->n_boxes, c->d_boxes, c->d_hsml, c->n_hmax_tiles, c->d_hmax_tiles,
+                    ctr);
     if (c->tree.nodes) launch_tree_hmax(c->stream, c->tbuild, c->d_hsml);
     else launch_cell_hmax(c->stream, c->ncell, c->d_range, c->d_hsml, c->d_cell_hmax);
     GZM_HIP(hipGetLastError());
@@ -563,7 +612,7 @@ gzm_status gzm_ctx_create(gzm_ctx **out, const gzm_params *params)
     c->G.G8 = (1.0 / g);
     c->G.G9 = (g - 1.0);
     if (dev_alloc(&c->d_ctr, kCtrSlots * kCtrSpread) || dev_alloc(&c->d_count, kDensityCounts) || dev_alloc(&c->d_count_heavy, 1) ||
-        dev_alloc(&c->d_hmax, 1)) {
+        dev_alloc(&c->d_hmax, 1) || hipHostMalloc((void **)&c->h_ctr, sizeof(Counters)) != hipSuccess) {
         gzm_ctx_destroy(c);
         return GZM_ERR_NOMEM;
     }
@@ -582,6 +631,7 @@ gzm_status gzm_ctx_destroy(gzm_ctx *c)
     dev_free(c->d_stage);
     dev_free(c->d_temp);
     dev_free(c->d_ctr);
+    if (c->h_ctr) (void)hipHostFree(c->h_ctr);
     dev_free(c->d_count);
     dev_free(c->d_count_heavy);
     dev_free(c->d_hmax);
@@ -954,11 +1004,9 @@ gzm_status restore_state(gzm_ctx *c)
 {
     c->hmax_valid = false;
     c->frec_fresh = false;
-    GZM_HIP(hipMemcpyAsync(c->d_hsml, c->d_hsml0, sizeof(double) * c->n, hipMemcpyDeviceToDevice, c->stream));
-    GZM_HIP(hipMemcpyAsync(c->d_cn, c->d_cn0, sizeof(double) * c->n, hipMemcpyDeviceToDevice, c->stream));
-    GZM_HIP(hipMemcpyAsync(c->d_vsig, c->d_vsig0, sizeof(double) * c->n, hipMemcpyDeviceToDevice, c->stream));
-    if (c->d_dmass0)
-        GZM_HIP(hipMemcpyAsync(c->d_dmass, c->d_dmass0, sizeof(double) * c->n, hipMemcpyDeviceToDevice, c->stream));
+    launch_restore(c->stream, c->n, c->d_hsml, c->d_hsml0, c->d_cn, c->d_cn0, c->d_vsig, c->d_vsig0, c->d_dmass,
+                   c->d_dmass0);
+    GZM_HIP(hipGetLastError());
     return GZM_OK;
 }
 
@@ -1210,11 +1258,7 @@ gzm_status density_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
 gzm_status gradients_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
 {
     gzm_status s;
-    if (!gp) {
-        s = reset_counters(c, kCtrGradients);
-        if (s) return s;
-    }
-    s = compute_hmax(c);
+    s = compute_hmax(c, gp ? nullptr : c->d_ctr + kCtrGradients * kCtrSpread);
     if (s) return s;
     {
         Timed tm(c, kOther);
@@ -1328,11 +1372,7 @@ gzm_status gradients_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
 gzm_status force_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
 {
     gzm_status s;
-    if (!gp) {
-        s = reset_counters(c, kCtrForce);
-        if (s) return s;
-    }
-    s = compute_hmax(c);
+    s = compute_hmax(c, gp ? nullptr : c->d_ctr + kCtrForce * kCtrSpread);
     if (s) return s;
     {
         Timed tm(c, kOther);
@@ -1437,6 +1477,41 @@ gzm_status force_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
         }
     }
     GZM_HIP(hipGetLastError());
+    auto reserve = [&](size_t want) -> gzm_status {
+        if (want <= c->defer_result_cap) return GZM_OK;
+        dev_free(c->d_defer_result);
+        dev_free(c->d_defer_pair);
+        c->defer_result_cap = 0;
+        gzm_status e = dev_alloc(&c->d_defer_result, want * (mfv ? 9 : 5));
+        e = e ? e : dev_alloc(&c->d_defer_pair, want);
+        if (e) return e;
+        c->defer_result_cap = want;
+        return GZM_OK;
+    };
+    // the deferred pairs [q0, q1), as far as there are so many, added to their particles
+    auto round = [&](int64_t q0, int64_t q1) {
+        a.defer.result = c->d_defer_result;
+        a.defer.pair = c->d_defer_pair;
+        a.defer.q_begin = (int)q0;
+        a.defer.q_end = (int)q1;
+        Timed tm(c, kForceDeferred);
+        launch_defer_owners(c->stream, a);
+        if (mfv) {
+            launch_force_mfv_deferred(c->stream, a, m, (int)(q1 - q0));
+            launch_force_mfv_finish(c->stream, a, m);
+        } else {
+            if (c->p.precision != 0) launch_force_deferred_f32(c->stream, a, (int)(q1 - q0));
+            else launch_force_deferred(c->stream, a, (int)(q1 - q0));
+            launch_force_finish(c->stream, a);
+        }
+    };
+    // FP64 redo of the FP32 particles listed for it, once every deferred pair is in
+    auto redo = [&]() {
+        if (c->p.precision == 0 || c->n_active == 0) return;
+        Timed tm(c, kForceDeferred);
+        launch_force_redo_fp64(c->stream, a);
+    };
+    int64_t first = 0;
     if (three_phase) {
         size_t bytes = 0;
         GZM_HIP(rocprim::exclusive_scan(nullptr, bytes, c->d_defer_count, c->d_defer_off, 0, (size_t)c->n_active,
@@ -1448,60 +1523,45 @@ gzm_status force_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
             Timed tm(c, kForceDeferred);
             GZM_HIP(rocprim::exclusive_scan(c->d_temp, bytes, c->d_defer_count, c->d_defer_off, 0, (size_t)c->n_active,
                                             rocprim::plus<int>(), c->stream));
-            launch_defer_total(c->stream, c->n_active, c->d_defer_off, c->d_defer_count, c->d_defer_total);
         }
-        int64_t D = 0;
         if (gp) {
-            D = gp->deferred;
+            const int64_t D = gp->deferred;
+            if (D > 0 && c->defer_result_cap == 0) { set_error("deferred-pair buffer missing while capturing"); return GZM_ERR_STATE; }
+            const int64_t chunk = D > 0 ? (int64_t)c->defer_result_cap : 1;
+            for (int64_t q0 = 0; q0 == 0 || q0 < D; q0 += chunk) round(q0, std::min<int64_t>(D, q0 + chunk));
         } else {
-            int h_total = 0;
-            GZM_HIP(hipMemcpyAsync(&h_total, c->d_defer_total, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-            GZM_HIP(hipStreamSynchronize(c->stream));
-            D = h_total;
-            // results of one round: all deferred pairs, or 2 per particle if more
-            const size_t want = (size_t)std::min<int64_t>(D, std::max<int64_t>(1 << 20, 2 * (int64_t)c->n));
-            if (want > c->defer_result_cap) {
-                dev_free(c->d_defer_result);
-                dev_free(c->d_defer_pair);
-                c->defer_result_cap = 0;
-                s = dev_alloc(&c->d_defer_result, want * (mfv ? 9 : 5));
-                s = s ? s : dev_alloc(&c->d_defer_pair, want);
+            // The first round takes as many as the buffer holds (at first a pair for
+            // every other particle, fewer where memory is short): only pairs past it
+            // have to wait for their number to reach the host.
+            size_t want = std::max<size_t>(1 << 16, (size_t)c->n_active / 2);
+            if (c->defer_result_cap == 0) {
+                while ((s = reserve(want)) && want > (1 << 16)) want = std::max<size_t>(1 << 16, want / 4);
                 if (s) return s;
-                c->defer_result_cap = want;
             }
-        }
-        c->last_deferred = D;
-        if (D > 0 && c->defer_result_cap == 0) { set_error("deferred-pair buffer missing while capturing"); return GZM_ERR_STATE; }
-        const int64_t chunk = D > 0 ? (int64_t)c->defer_result_cap : 1;
-        a.defer.result = c->d_defer_result;
-        a.defer.pair = c->d_defer_pair;
-        for (int64_t q0 = 0; q0 == 0 || q0 < D; q0 += chunk) {
-            const int64_t q1 = std::min<int64_t>(D, q0 + chunk);
-            a.defer.q_begin = (int)q0;
-            a.defer.q_end = (int)q1;
-            Timed tm(c, kForceDeferred);
-            if (q1 > q0) launch_defer_owners(c->stream, a);
-            if (mfv) {
-                launch_force_mfv_deferred(c->stream, a, m, (int)(q1 - q0));
-                launch_force_mfv_finish(c->stream, a, m);
-            } else {
-                if (c->p.precision != 0) launch_force_deferred_f32(c->stream, a, (int)(q1 - q0));
-                else launch_force_deferred(c->stream, a, (int)(q1 - q0));
-                launch_force_finish(c->stream, a);
-            }
-            if (D == 0) break;
+            first = (int64_t)c->defer_result_cap;
+            round(0, first);
         }
         GZM_HIP(hipGetLastError());
     }
-    if (c->p.precision != 0 && c->n_active > 0) {
-        Timed tm(c, kForceDeferred);
-        launch_force_redo_fp64(c->stream, a);
-        GZM_HIP(hipGetLastError());
-    }
+    redo();
+    GZM_HIP(hipGetLastError());
     if (gp) return GZM_OK;
     Counters h;
     s = read_counters(c, kCtrForce, &h);
     if (s) return s;
+    c->last_deferred = three_phase ? h.deferred : 0;
+    if (three_phase && h.deferred > first) {
+        // results of one round: all deferred pairs, or 2 per particle if more
+        const int64_t D = h.deferred;
+        s = reserve((size_t)std::min<int64_t>(D, std::max<int64_t>(1 << 20, 2 * (int64_t)c->n)));
+        if (s) return s;
+        const int64_t chunk = (int64_t)c->defer_result_cap;
+        for (int64_t q0 = first; q0 < D; q0 += chunk) round(q0, std::min<int64_t>(D, q0 + chunk));
+        redo();
+        GZM_HIP(hipGetLastError());
+        s = read_counters(c, kCtrForce, &h);
+        if (s) return s;
+    }
     collect_timings(c);
     if (stats) {
         stats->force_interactions = (int64_t)h.interactions;
@@ -1768,42 +1828,32 @@ gzm_status gzm_download(gzm_ctx *c, gzm_host_view *v)
     if (!c || !v) { set_error("NULL argument"); return GZM_ERR_ARG; }
     if (c->n == 0 || v->n != c->n) { set_error("view size %lld does not match uploaded %d", (long long)v->n, c->n); return GZM_ERR_ARG; }
     GZM_HIP(hipSetDevice(c->p.device));
-    GZM_HIP(hipStreamSynchronize(c->stream));
     const int n = c->n;
-    struct Out { double *h; const double *d; int w; } outs[] = {
-        {v->hsml, c->d_hsml, 1}, {v->cn, c->d_cn, 1}, {v->vsig, c->d_vsig, 1}, {v->num_ngb, c->d_num_ngb, 1},
-        {v->dhsml, c->d_dhsml, 1}, {v->divvel, c->d_divvel, 1}, {v->density, c->d_rho, 1},
-        {v->pressure, c->d_pres, 1}, {v->fce, c->d_fce, 1}, {v->acc, c->d_acc, 3}, {v->dtu, c->d_dtu, 1},
-        {v->particle_vel, c->d_pvel, 3}, {v->dt_mass, c->d_dtmass, 1}, {v->d_mass, c->d_dmass, 1},
-        {v->grav_work, c->d_gravwork, 3}};
-    for (auto &o : outs) {
-        if (!o.h || !o.d) continue;
-        gzm_status s = download_sorted(c, o.d, o.h, o.w);
-        if (s) return s;
-    }
-    if (v->nvt) {
-        std::vector<double> t6((size_t)n * 6);
-        gzm_status s = download_sorted(c, c->d_nvt, t6.data(), 6);
-        if (s) return s;
-        for (int i = 0; i < n; i++) {
-            const double *t = t6.data() + 6 * (size_t)i;
-            double *o = v->nvt + 9 * (size_t)i;
-            o[0] = t[0]; o[1] = t[1]; o[2] = t[2];
-            o[3] = t[1]; o[4] = t[3]; o[5] = t[4];
-            o[6] = t[2]; o[7] = t[4]; o[8] = t[5];
-        }
-    }
-    if (v->grad_rho || v->grad_p || v->grad_v) {
-        std::vector<double> g((size_t)n * 15);
-        gzm_status s = download_sorted(c, c->d_grad, g.data(), 15);
-        if (s) return s;
-        for (int i = 0; i < n; i++) {
-            const double *o = g.data() + 15 * (size_t)i;
-            if (v->grad_rho) for (int k = 0; k < 3; k++) v->grad_rho[3 * (size_t)i + k] = o[k];
-            if (v->grad_p) for (int k = 0; k < 3; k++) v->grad_p[3 * (size_t)i + k] = o[3 + k];
-            if (v->grad_v) for (int k = 0; k < 9; k++) v->grad_v[9 * (size_t)i + k] = o[6 + k];
-        }
-    }
+    std::vector<ExportField> fields;
+    auto add = [&](double *host, const double *dev, int w, int w_src, int off) {
+        if (host && dev) fields.push_back({host, dev, w, w_src, off});
+    };
+    add(v->hsml, c->d_hsml, 1, 1, 0);
+    add(v->cn, c->d_cn, 1, 1, 0);
+    add(v->vsig, c->d_vsig, 1, 1, 0);
+    add(v->num_ngb, c->d_num_ngb, 1, 1, 0);
+    add(v->dhsml, c->d_dhsml, 1, 1, 0);
+    add(v->divvel, c->d_divvel, 1, 1, 0);
+    add(v->density, c->d_rho, 1, 1, 0);
+    add(v->pressure, c->d_pres, 1, 1, 0);
+    add(v->fce, c->d_fce, 1, 1, 0);
+    add(v->acc, c->d_acc, 3, 3, 0);
+    add(v->dtu, c->d_dtu, 1, 1, 0);
+    add(v->particle_vel, c->d_pvel, 3, 3, 0);
+    add(v->dt_mass, c->d_dtmass, 1, 1, 0);
+    add(v->d_mass, c->d_dmass, 1, 1, 0);
+    add(v->grav_work, c->d_gravwork, 3, 3, 0);
+    add(v->nvt, c->d_nvt, 9, 6, 0);
+    add(v->grad_rho, c->d_grad, 3, 15, 0);
+    add(v->grad_p, c->d_grad, 3, 15, 3);
+    add(v->grad_v, c->d_grad, 9, 15, 6);
+    gzm_status s = download_fields(c, fields);
+    if (s) return s;
     if (v->wakeup) {
         std::vector<uint8_t> w(n);
         GZM_HIP(hipMemcpyAsync(w.data(), c->d_wakeup, n, hipMemcpyDeviceToHost, c->stream));
@@ -1836,7 +1886,7 @@ gzm_status gzm_neighbor_counts(gzm_ctx *c, int32_t mode, const int32_t *active, 
     }
     gzm_status s = reset_counters(c, kCtrMisc);
     if (s) return s;
-    s = compute_hmax(c);
+    s = compute_hmax(c, nullptr);
     if (s) return s;
     launch_neighbor_counts(c->stream, c->d_boxes, c->d_box_of, c->tree, mode, na, c->d_live, c->d_posm, c->d_hsml,
                            counts ? c->d_flags : nullptr, c->d_ctr + kCtrMisc * kCtrSpread);

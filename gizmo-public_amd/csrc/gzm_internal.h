@@ -134,6 +134,23 @@ struct alignas(128) Counters {
     int overflow_slices;
     int sweeps;  // density: sweeps of the particle that took most
     unsigned long long updates;  // density: sum over particles of their sweeps
+    int deferred;  // force: pairs deferred out of the list loop
+};
+
+// One field of an export from sorted slots to caller order: element c of
+// particle i is src[slot * w_src + off + c], or the full matrix of a packed
+// symmetric one (w = 9 from 6).
+struct ExportField {
+    double *dst;
+    const double *src;
+    int w, w_src, off;
+};
+constexpr int kMaxExport = 24;
+struct ExportArgs {
+    ExportField field[kMaxExport];
+    int n_fields, n;
+    const int *inv;        // caller index -> sorted slot
+    unsigned first_block[kMaxExport + 1];
 };
 
 // candidates a density-sweep lane walks before it defers its particle to the
@@ -315,7 +332,7 @@ struct DeferArgs {
     int *count;            // per active entry: number of deferred pairs
     uint8_t *raw;          // per active entry: 1 = acc, dtu, vsig hold the raw sums of the loop
     const int *offset;     // exclusive scan of count
-    const int *total;      // sum of count (device)
+    int *total;            // sum of count (device)
     double *result;        // per deferred pair of the round: dv/dt terms (3), du/dt term, v_sig
                            // (MFV: 9 per pair, see force_mfv_deferred_kernel)
     int2 *pair;            // per deferred pair of the round: particle i and neighbour j, written by
@@ -382,13 +399,17 @@ void launch_gather_sorted(hipStream_t s, int n, const int *perm, const double *p
                           const double *mass, const double *u, const int *box_caller, double4 *posm,
                           double4 *velu, float4 *posf, int *inv, int *box_of);
 void launch_gather_scalar(hipStream_t s, int n, const int *perm, const double *src, double *dst, int width);
-void launch_scatter_scalar(hipStream_t s, int n, const int *perm, const double *src, double *dst, int width);
 void launch_cell_ranges(hipStream_t s, int n, const double4 *posm, const BoxDesc *boxes, const int *box_of,
                         int2 *range, int ncell);
 // per-box max hsml into boxes[b].hmax; tiles = (box, first slot) of each
 // block, each tile at most kHmaxTile slots of one box
 constexpr int kHmaxTile = 4096;
-void launch_box_hmax(hipStream_t s, int n_boxes, BoxDesc *boxes, const double *hsml, int n_tiles, const int2 *tiles);
+void launch_box_hmax(hipStream_t s, int n_boxes, BoxDesc *boxes, const double *hsml, int n_tiles, const int2 *tiles,
+                     Counters *ctr);  // ctr (NULL: none): counters to clear on the way
+void launch_publish_counters(hipStream_t s, const Counters *ctr, Counters *host);
+void launch_export(hipStream_t s, ExportArgs &a);
+void launch_restore(hipStream_t s, int n, double *hsml, const double *hsml0, double *cn, const double *cn0, double *vsig,
+                    const double *vsig0, double *dmass, const double *dmass0);
 // status 1155 when live particles remain after the captured sweeps
 void launch_flag_unconverged(hipStream_t s, const int *n_live_dev, Counters *ctr);
 void launch_clear_counters(hipStream_t s, Counters *ctr);
@@ -422,7 +443,6 @@ void launch_force_deferred(hipStream_t s, const ForceArgs &a, int n_pairs);
 // owner entry and list position of each deferred pair of the round [q_begin, q_end)
 void launch_defer_owners(hipStream_t s, const ForceArgs &a);
 void launch_force_finish(hipStream_t s, const ForceArgs &a);
-void launch_defer_total(hipStream_t s, int n_active, const int *offset, const int *count, int *total);
 // FP32-bulk kernels (gzm_kernels_f32.hip)
 void launch_pack_geom_f32(hipStream_t s, int n, const double4 *posm, const double4 *velu, const BoxDesc *boxes,
                           const int *box_of, float4 *offm, float4 *velf, uint32_t *cellc);

@@ -67,12 +67,49 @@ __global__ void gather_scalar_kernel(int n, const int *perm, const double *src, 
     dst[t] = src[(long long)perm[k] * width + c];
 }
 
-__global__ void scatter_scalar_kernel(int n, const int *perm, const double *src, double *dst, int width)
+// Fields from sorted slots into caller order, all in one launch: consecutive
+// threads write consecutive elements, so that the destination may be host memory
+// (the writes then cross the bus as they are made, with no copy after them).
+__global__ __launch_bounds__(kBlock) void export_kernel(ExportArgs a)
 {
-    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long long)n * width) return;
-    int k = (int)(t / width), c = (int)(t % width);
-    dst[(long long)perm[k] * width + c] = src[t];
+    int q = 0;
+    while (q + 1 < a.n_fields && blockIdx.x >= a.first_block[q + 1]) q++;
+    const ExportField f = a.field[q];
+    const long long t = (long long)(blockIdx.x - a.first_block[q]) * kBlock + threadIdx.x;
+    if (t >= (long long)a.n * f.w) return;
+    const int i = (int)(t / f.w), c = (int)(t % f.w);
+    // (row, column) of the full matrix -> 00 01 02 11 12 22
+    const int e = f.w == 9 && f.w_src == 6 ? (c == 8 ? 5 : c / 3 + c % 3 + (c == 4 || c == 5 || c == 7 ? 1 : 0)) : c;
+    f.dst[t] = f.src[(long long)a.inv[i] * f.w_src + f.off + e];
+}
+
+__global__ void restore_kernel(int n, double *hsml, const double *hsml0, double *cn, const double *cn0, double *vsig,
+                               const double *vsig0, double *dmass, const double *dmass0)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    hsml[k] = hsml0[k];
+    cn[k] = cn0[k];
+    vsig[k] = vsig0[k];
+    if (dmass0) dmass[k] = dmass0[k];
+}
+
+// the sum of a stage's kCtrSpread counter copies, one lane each, into host memory
+__global__ void publish_counters_kernel(const Counters *ctr, Counters *host)
+{
+    Counters h = ctr[threadIdx.x];
+    for (int off = 32; off > 0; off >>= 1) {
+        h.interactions += __shfl_xor(h.interactions, off, 64);
+        h.retries += __shfl_xor(h.retries, off, 64);
+        h.exact_calls += __shfl_xor(h.exact_calls, off, 64);
+        h.updates += __shfl_xor(h.updates, off, 64);
+        h.redo_n += __shfl_xor(h.redo_n, off, 64);
+        h.overflow_slices += __shfl_xor(h.overflow_slices, off, 64);
+        h.deferred += __shfl_xor(h.deferred, off, 64);
+        h.status = max(h.status, __shfl_xor(h.status, off, 64));
+        h.sweeps = max(h.sweeps, __shfl_xor(h.sweeps, off, 64));
+    }
+    if (threadIdx.x == 0) *host = h;
 }
 
 __global__ void cell_ranges_kernel(int n, const double4 *posm, const BoxDesc *boxes, const int *box_of, int2 *range)
@@ -114,10 +151,11 @@ __global__ __launch_bounds__(kBlock) void box_hmax_kernel(BoxDesc *boxes, const 
     }
 }
 
-__global__ void clear_box_hmax_kernel(int n_boxes, BoxDesc *boxes)
+__global__ void clear_box_hmax_kernel(int n_boxes, BoxDesc *boxes, Counters *ctr)
 {
     int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b < n_boxes) boxes[b].hmax = 0.0;
+    if (ctr && b < kCtrSpread) ctr[b] = Counters{};
 }
 
 __global__ void flag_unconverged_kernel(const int *n_live_dev, Counters *ctr)
@@ -1075,11 +1113,6 @@ __global__ __launch_bounds__(kBlock) void force_finish_kernel(ForceArgs a)
     a.vsig[i] = out_vsig;
 }
 
-__global__ void defer_total_kernel(int n, const int *offset, const int *count, int *total)
-{
-    if (blockIdx.x == 0 && threadIdx.x == 0) *total = (n > 0) ? offset[n - 1] + count[n - 1] : 0;
-}
-
 // neighbour-set sizes for a fixed hsml (same predicates as the stage kernels)
 __global__ __launch_bounds__(kBlock) void neighbor_count_kernel(const BoxDesc *boxes, const int *box_of,
                                                                 TreeArgs tree, int mode, int n_active,
@@ -1140,10 +1173,25 @@ void launch_gather_scalar(hipStream_t s, int n, const int *perm, const double *s
     if (((long long)n * width) > 0) hipLaunchKernelGGL(gather_scalar_kernel, dim3(nblocks((long long)n * width)), dim3(kBlock), 0, s, n, perm, src,
                        dst, width);
 }
-void launch_scatter_scalar(hipStream_t s, int n, const int *perm, const double *src, double *dst, int width)
+void launch_export(hipStream_t s, ExportArgs &a)
 {
-    if (((long long)n * width) > 0) hipLaunchKernelGGL(scatter_scalar_kernel, dim3(nblocks((long long)n * width)), dim3(kBlock), 0, s, n, perm,
-                       src, dst, width);
+    unsigned blocks = 0;
+    for (int q = 0; q < a.n_fields; q++) {
+        a.first_block[q] = blocks;
+        blocks += nblocks((long long)a.n * a.field[q].w);
+    }
+    if (blocks > 0) hipLaunchKernelGGL(export_kernel, dim3(blocks), dim3(kBlock), 0, s, a);
+}
+void launch_restore(hipStream_t s, int n, double *hsml, const double *hsml0, double *cn, const double *cn0, double *vsig,
+                    const double *vsig0, double *dmass, const double *dmass0)
+{
+    if (n > 0)
+        hipLaunchKernelGGL(restore_kernel, dim3(nblocks(n)), dim3(kBlock), 0, s, n, hsml, hsml0, cn, cn0, vsig, vsig0,
+                           dmass, dmass0);
+}
+void launch_publish_counters(hipStream_t s, const Counters *ctr, Counters *host)
+{
+    hipLaunchKernelGGL(publish_counters_kernel, dim3(1), dim3(kCtrSpread), 0, s, ctr, host);
 }
 void launch_cell_ranges(hipStream_t s, int n, const double4 *posm, const BoxDesc *boxes, const int *box_of,
                         int2 *range, int ncell)
@@ -1151,9 +1199,11 @@ void launch_cell_ranges(hipStream_t s, int n, const double4 *posm, const BoxDesc
     if ((2LL * ncell) > 0) hipLaunchKernelGGL(fill_int_kernel, dim3(nblocks(2LL * ncell)), dim3(kBlock), 0, s, (int *)range, 2 * ncell, 0);
     if (n > 0) hipLaunchKernelGGL(cell_ranges_kernel, dim3(nblocks(n)), dim3(kBlock), 0, s, n, posm, boxes, box_of, range);
 }
-void launch_box_hmax(hipStream_t s, int n_boxes, BoxDesc *boxes, const double *hsml, int n_tiles, const int2 *tiles)
+void launch_box_hmax(hipStream_t s, int n_boxes, BoxDesc *boxes, const double *hsml, int n_tiles, const int2 *tiles,
+                     Counters *ctr)
 {
-    if (n_boxes > 0) hipLaunchKernelGGL(clear_box_hmax_kernel, dim3(nblocks(n_boxes)), dim3(kBlock), 0, s, n_boxes, boxes);
+    if (n_boxes > 0) hipLaunchKernelGGL(clear_box_hmax_kernel, dim3(nblocks(n_boxes)), dim3(kBlock), 0, s, n_boxes, boxes,
+                                       ctr);
     if (n_tiles > 0) hipLaunchKernelGGL(box_hmax_kernel, dim3(n_tiles), dim3(kBlock), 0, s, boxes, hsml, tiles);
 }
 void launch_flag_unconverged(hipStream_t s, const int *n_live_dev, Counters *ctr)
@@ -1266,6 +1316,11 @@ __global__ __launch_bounds__(kBlock) void defer_owners_kernel(ForceArgs a)
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= a.n_active) return;
     const int c = a.defer.count[t];
+    if (t == a.n_active - 1) {
+        const int total = a.defer.offset[t] + c;
+        *a.defer.total = total;
+        a.ctr->deferred = total;
+    }
     if (c == 0) return;
     const int q0 = a.defer.offset[t];
     if (q0 >= a.defer.q_end || q0 + c <= a.defer.q_begin) return;
@@ -1293,10 +1348,6 @@ void launch_force_deferred(hipStream_t s, const ForceArgs &a, int n_pairs)
 void launch_force_finish(hipStream_t s, const ForceArgs &a)
 {
     if (a.n_active > 0) hipLaunchKernelGGL(force_finish_kernel, dim3(nblocks(a.n_active)), dim3(kBlock), 0, s, a);
-}
-void launch_defer_total(hipStream_t s, int n_active, const int *offset, const int *count, int *total)
-{
-    hipLaunchKernelGGL(defer_total_kernel, dim3(1), dim3(64), 0, s, n_active, offset, count, total);
 }
 void launch_density_heavy(hipStream_t s, const DensitySweepArgs &a, int max_entries)
 {

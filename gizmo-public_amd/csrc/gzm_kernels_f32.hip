@@ -907,6 +907,12 @@ __global__ __launch_bounds__(kBlock, 4) void force_deferred_f32_kernel(ForceArgs
     wave_add_u64(&ctr_slot(a.ctr)->exact_calls, nexact);
 }
 
+// whether a later round holds more of the deferred pairs, the redo with it
+__device__ __forceinline__ bool deferred_left(const ForceArgs &a)
+{
+    return a.defer.mask && *a.defer.total > a.defer.q_end;
+}
+
 // The gradients of each particle listed by mark_redo, again, in FP64 from the
 // FP64 state with the arithmetic of gradients_kernel (gradients.c:66-75,
 // 1219-1232), written over the FP32 gradients.  One wavefront per listed
@@ -914,6 +920,7 @@ __global__ __launch_bounds__(kBlock, 4) void force_deferred_f32_kernel(ForceArgs
 // their partial sums, maxima and minima; lane 0 applies NV_T and the limiter.  Sums in another order than the FP64 pass: equal to ~1e-16.
 __global__ __launch_bounds__(kBlock) void gradients_redo_fp64_kernel(ForceArgs a)
 {
+    if (deferred_left(a)) return;
     __shared__ WaveWalkLds walk[kBlock / 64];
     const int n_redo = a.redo_count[1];
     const int lane = threadIdx.x & 63;
@@ -1018,6 +1025,7 @@ __global__ __launch_bounds__(kBlock) void gradients_redo_fp64_kernel(ForceArgs a
 template <bool REDO>
 __global__ __launch_bounds__(kBlock) void force_wave_fp64_kernel(ForceArgs a, const int *list, const int *count)
 {
+    if (REDO && deferred_left(a)) return;
     __shared__ WaveWalkLds walk[kBlock / 64];
     const int n_redo = *count;
     if (REDO && blockIdx.x == 0 && threadIdx.x == 0 && n_redo > 0) atomicAdd(&ctr_slot(a.ctr)->redo_n, n_redo);
