@@ -154,6 +154,8 @@ struct gzm_ctx {
     TreeBuild tbuild;
 
     Counters *h_ctr = nullptr;  // pinned: a stage's counters as the host reads them
+    double *h_bounce = nullptr; // pinned: fields on their way to pageable memory
+    size_t bounce_bytes = 0;
 
     gzm_timing timing;
     std::vector<TimedLaunch> pending;
@@ -317,6 +319,8 @@ gzm_status upload_sorted(gzm_ctx *c, const double *host, double *dst, int width)
     return GZM_OK;
 }
 
+constexpr size_t kBounceBytes = 32u << 20;
+
 // The device's address of host memory that it can write itself, all of
 // [host, host + bytes); NULL: it cannot.
 double *device_view(double *host, size_t bytes)
@@ -337,13 +341,14 @@ double *device_view(double *host, size_t bytes)
 // Sorted device arrays -> host arrays in caller order.  Fields in memory that
 // the device can write (pinned) go there from one kernel; the others through a
 // staging array and a copy each.  Returns when all are there.
-gzm_status download_fields(gzm_ctx *c, const std::vector<ExportField> &fields)
+gzm_status download_fields(gzm_ctx *c, const std::vector<ExportField> &fields, uint8_t *wakeup)
 {
     ExportArgs direct = {}, one = {};
     direct.n = one.n = c->n;
     direct.inv = one.inv = c->d_inv;
     one.n_fields = 1;
     int width = 0;
+    size_t bytes = wakeup ? (size_t)c->n : 0;
     std::vector<const ExportField *> staged;
     for (auto &f : fields) {
         double *d = direct.n_fields < kMaxExport ? device_view(f.dst, (size_t)c->n * f.w * sizeof(double)) : nullptr;
@@ -353,11 +358,44 @@ gzm_status download_fields(gzm_ctx *c, const std::vector<ExportField> &fields)
         } else {
             staged.push_back(&f);
             width = std::max(width, f.w);
+            bytes += (size_t)c->n * f.w * sizeof(double);
+        }
+    }
+    // A copy to pageable memory costs some 40 us whatever its size; below kBounceBytes
+    // in all, the fields go to a pinned array of the context and from there by
+    // memcpy (9,261 particles, 16 fields: 0.35 ms against 0.77; above it the
+    // runtime's copies, which overlap their own memcpy, are no slower).
+    if (bytes > 0 && bytes <= kBounceBytes && direct.n_fields + staged.size() <= (size_t)kMaxExport) {
+        if (bytes > c->bounce_bytes) {
+            if (c->h_bounce) (void)hipHostFree(c->h_bounce);
+            c->h_bounce = nullptr;
+            c->bounce_bytes = 0;
+            if (hipHostMalloc((void **)&c->h_bounce, bytes) == hipSuccess) c->bounce_bytes = bytes;
+            else (void)hipGetLastError();
+        }
+        if (c->h_bounce) {
+            double *p = c->h_bounce;
+            for (auto *f : staged) {
+                direct.field[direct.n_fields] = *f;
+                direct.field[direct.n_fields++].dst = p;
+                p += (size_t)c->n * f->w;
+            }
+            launch_export(c->stream, direct);
+            if (wakeup) launch_export_u8(c->stream, c->n, c->d_inv, c->d_wakeup, (uint8_t *)p);
+            GZM_HIP(hipGetLastError());
+            GZM_HIP(hipStreamSynchronize(c->stream));
+            p = c->h_bounce;
+            for (auto *f : staged) {
+                memcpy(f->dst, p, (size_t)c->n * f->w * sizeof(double));
+                p += (size_t)c->n * f->w;
+            }
+            if (wakeup) memcpy(wakeup, p, c->n);
+            return GZM_OK;
         }
     }
     launch_export(c->stream, direct);
-    if (!staged.empty()) {
-        gzm_status s = ensure_stage(c, (size_t)c->n * width);
+    if (!staged.empty() || wakeup) {
+        gzm_status s = ensure_stage(c, (size_t)c->n * std::max(width, 1));
         if (s) return s;
     }
     for (auto *f : staged) {
@@ -365,6 +403,10 @@ gzm_status download_fields(gzm_ctx *c, const std::vector<ExportField> &fields)
         one.field[0].dst = c->d_stage;
         launch_export(c->stream, one);
         GZM_HIP(hipMemcpyAsync(f->dst, c->d_stage, (size_t)c->n * f->w * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    }
+    if (wakeup) {
+        launch_export_u8(c->stream, c->n, c->d_inv, c->d_wakeup, (uint8_t *)c->d_stage);
+        GZM_HIP(hipMemcpyAsync(wakeup, c->d_stage, (size_t)c->n, hipMemcpyDeviceToHost, c->stream));
     }
     GZM_HIP(hipGetLastError());
     GZM_HIP(hipStreamSynchronize(c->stream));
@@ -632,6 +674,7 @@ gzm_status gzm_ctx_destroy(gzm_ctx *c)
     dev_free(c->d_temp);
     dev_free(c->d_ctr);
     if (c->h_ctr) (void)hipHostFree(c->h_ctr);
+    if (c->h_bounce) (void)hipHostFree(c->h_bounce);
     dev_free(c->d_count);
     dev_free(c->d_count_heavy);
     dev_free(c->d_hmax);
@@ -849,11 +892,15 @@ gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const 
     GZM_HIP(hipMemcpyAsync(st_vel, v->vel, sizeof(double) * 3 * n, hipMemcpyHostToDevice, c->stream));
     GZM_HIP(hipMemcpyAsync(st_mass, v->mass, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
     GZM_HIP(hipMemcpyAsync(st_u, v->u, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
-    std::vector<int> box_caller(n);
-    for (int b = 0; b < n_boxes; b++)
-        for (int64_t i = offsets[b]; i < offsets[b + 1]; i++) box_caller[i] = b;
-    int *d_box_caller = c->d_flags;  // free until the first stage call
-    GZM_HIP(hipMemcpyAsync(d_box_caller, box_caller.data(), sizeof(int) * n, hipMemcpyHostToDevice, c->stream));
+    std::vector<int> box_caller;
+    int *d_box_caller = nullptr;  // one box: no table
+    if (n_boxes > 1) {
+        box_caller.resize(n);
+        for (int b = 0; b < n_boxes; b++)
+            for (int64_t i = offsets[b]; i < offsets[b + 1]; i++) box_caller[i] = b;
+        d_box_caller = c->d_flags;  // free until the first stage call
+        GZM_HIP(hipMemcpyAsync(d_box_caller, box_caller.data(), sizeof(int) * n, hipMemcpyHostToDevice, c->stream));
+    }
     int box_bits = 0;
     while ((1 << box_bits) < n_boxes) box_bits++;
     const bool tree = c->p.search == 1;
@@ -882,21 +929,23 @@ gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const 
         GZM_HIP(hipGetLastError());
     }
     // d_iota was consumed as sort values; rebuild it as the identity for "all active"
-    std::vector<int> iota(n);
-    for (int i = 0; i < n; i++) iota[i] = i;
-    GZM_HIP(hipMemcpyAsync(c->d_iota, iota.data(), sizeof(int) * n, hipMemcpyHostToDevice, c->stream));
+    launch_iota(c->stream, n, c->d_iota);
+    // what the view does not give, filled in one launch
+    FillArgs fill = {};
+    fill.n = n;
+    auto fill_with = [&](double *p, int width, double value) {
+        fill.p[fill.n_fills] = p;
+        fill.width[fill.n_fills] = width;
+        fill.value[fill.n_fills++] = value;
+    };
 
     // carried state
     s = upload_sorted(c, v->hsml, c->d_hsml, 1);
     if (s) return s;
     if (v->cn) { s = upload_sorted(c, v->cn, c->d_cn, 1); if (s) return s; }
-    else launch_fill_double(c->stream, c->d_cn, n, 1.0);  // init.c:514
+    else fill_with(c->d_cn, 1, 1.0);  // init.c:514
     if (v->vsig) { s = upload_sorted(c, v->vsig, c->d_vsig, 1); if (s) return s; }
-    else launch_fill_double(c->stream, c->d_vsig, n, kMinReal);
-    GZM_HIP(hipStreamSynchronize(c->stream));
-    GZM_HIP(hipMemcpyAsync(c->d_hsml0, c->d_hsml, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
-    GZM_HIP(hipMemcpyAsync(c->d_cn0, c->d_cn, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
-    GZM_HIP(hipMemcpyAsync(c->d_vsig0, c->d_vsig, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
+    else fill_with(c->d_vsig, 1, kMinReal);
     if (tree) {
         TreeBuild &t = c->tbuild;
         t.n = n;
@@ -937,7 +986,7 @@ gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const 
         {v->density, c->d_rho, 1}, {v->pressure, c->d_pres, 1}, {v->fce, c->d_fce, 1}};
     for (auto &o : opts) {
         if (o.h) { s = upload_sorted(c, o.h, o.d, o.w); if (s) return s; }
-        else launch_fill_double(c->stream, o.d, (long long)n * o.w, 0.0);
+        else fill_with(o.d, o.w, 0.0);
     }
     if (v->nvt) {
         std::vector<double> t6((size_t)n * 6);
@@ -948,7 +997,7 @@ gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const 
         }
         s = upload_sorted(c, t6.data(), c->d_nvt, 6);
         if (s) return s;
-    } else launch_fill_double(c->stream, c->d_nvt, (long long)n * 6, 0.0);
+    } else fill_with(c->d_nvt, 6, 0.0);
     if (v->grad_rho && v->grad_p && v->grad_v) {
         std::vector<double> g((size_t)n * 15);
         for (int i = 0; i < n; i++) {
@@ -959,12 +1008,12 @@ gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const 
         }
         s = upload_sorted(c, g.data(), c->d_grad, 15);
         if (s) return s;
-    } else launch_fill_double(c->stream, c->d_grad, (long long)n * 15, 0.0);
+    } else fill_with(c->d_grad, 15, 0.0);
     // force outputs of particles that stay inactive round-trip unchanged
     if (v->acc) { s = upload_sorted(c, v->acc, c->d_acc, 3); if (s) return s; }
-    else launch_fill_double(c->stream, c->d_acc, (long long)n * 3, 0.0);
+    else fill_with(c->d_acc, 3, 0.0);
     if (v->dtu) { s = upload_sorted(c, v->dtu, c->d_dtu, 1); if (s) return s; }
-    else launch_fill_double(c->stream, c->d_dtu, n, 0.0);
+    else fill_with(c->d_dtu, 1, 0.0);
     launch_fill_u8(c->stream, c->d_wakeup, n, 0);
     if (c->p.method == 1) {
         // MFV state: the integer timesteps as doubles (exact below 2^53, as the
@@ -975,16 +1024,19 @@ gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const 
             for (int i = 0; i < n; i++) ti[i] = (double)v->ti_step[i];
             s = upload_sorted(c, ti.data(), c->d_ti, 1);
             if (s) return s;
-        } else launch_fill_double(c->stream, c->d_ti, n, 1.0);
+        } else fill_with(c->d_ti, 1, 1.0);
         struct MOpt { const double *h; double *d; int w; } mopts[] = {
             {v->particle_vel, c->d_pvel, 3}, {v->dt_mass, c->d_dtmass, 1}, {v->d_mass, c->d_dmass, 1},
             {v->grav_work, c->d_gravwork, 3}};
         for (auto &o : mopts) {
             if (o.h) { s = upload_sorted(c, o.h, o.d, o.w); if (s) return s; }
-            else launch_fill_double(c->stream, o.d, (long long)n * o.w, 0.0);
+            else fill_with(o.d, o.w, 0.0);
         }
-        GZM_HIP(hipMemcpyAsync(c->d_dmass0, c->d_dmass, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
     }
+    launch_fill_fields(c->stream, fill);
+    // the initial state of gzm_restore_initial_state
+    launch_restore(c->stream, n, c->d_hsml0, c->d_hsml, c->d_cn0, c->d_cn, c->d_vsig0, c->d_vsig, c->d_dmass0,
+                   c->d_dmass0 ? c->d_dmass : nullptr);
     GZM_HIP(hipGetLastError());
     GZM_HIP(hipStreamSynchronize(c->stream));
     collect_timings(c);
@@ -1828,7 +1880,6 @@ gzm_status gzm_download(gzm_ctx *c, gzm_host_view *v)
     if (!c || !v) { set_error("NULL argument"); return GZM_ERR_ARG; }
     if (c->n == 0 || v->n != c->n) { set_error("view size %lld does not match uploaded %d", (long long)v->n, c->n); return GZM_ERR_ARG; }
     GZM_HIP(hipSetDevice(c->p.device));
-    const int n = c->n;
     std::vector<ExportField> fields;
     auto add = [&](double *host, const double *dev, int w, int w_src, int off) {
         if (host && dev) fields.push_back({host, dev, w, w_src, off});
@@ -1852,17 +1903,7 @@ gzm_status gzm_download(gzm_ctx *c, gzm_host_view *v)
     add(v->grad_rho, c->d_grad, 3, 15, 0);
     add(v->grad_p, c->d_grad, 3, 15, 3);
     add(v->grad_v, c->d_grad, 9, 15, 6);
-    gzm_status s = download_fields(c, fields);
-    if (s) return s;
-    if (v->wakeup) {
-        std::vector<uint8_t> w(n);
-        GZM_HIP(hipMemcpyAsync(w.data(), c->d_wakeup, n, hipMemcpyDeviceToHost, c->stream));
-        std::vector<int> perm(n);
-        GZM_HIP(hipMemcpyAsync(perm.data(), c->d_perm, sizeof(int) * n, hipMemcpyDeviceToHost, c->stream));
-        GZM_HIP(hipStreamSynchronize(c->stream));
-        for (int k = 0; k < n; k++) v->wakeup[perm[k]] = w[k];
-    }
-    return GZM_OK;
+    return download_fields(c, fields, v->wakeup);
 }
 
 gzm_status gzm_neighbor_counts(gzm_ctx *c, int32_t mode, const int32_t *active, int64_t n_active, int32_t *counts,

@@ -408,6 +408,16 @@ void launch_box_hmax(hipStream_t s, int n_boxes, BoxDesc *boxes, const double *h
                      Counters *ctr);  // ctr (NULL: none): counters to clear on the way
 void launch_publish_counters(hipStream_t s, const Counters *ctr, Counters *host);
 void launch_export(hipStream_t s, ExportArgs &a);
+void launch_export_u8(hipStream_t s, int n, const int *inv, const uint8_t *src, uint8_t *dst);
+// several arrays to a value each, in one launch
+struct FillArgs {
+    static constexpr int kMax = 20;
+    double *p[kMax];
+    double value[kMax];
+    int width[kMax], n_fills, n;
+};
+void launch_fill_fields(hipStream_t s, const FillArgs &a);
+void launch_iota(hipStream_t s, int n, int *p);
 void launch_restore(hipStream_t s, int n, double *hsml, const double *hsml0, double *cn, const double *cn0, double *vsig,
                     const double *vsig0, double *dmass, const double *dmass0);
 // status 1155 when live particles remain after the captured sweeps
@@ -514,7 +524,6 @@ void launch_riemann_states_mfv(hipStream_t s, int mode, const GammaConsts &G, in
                                const double *R, const double *normal, const double *limiter, double *out, int *mask);
 void launch_fill_int(hipStream_t s, int *p, int n, int value);
 void launch_fill_u8(hipStream_t s, uint8_t *p, int n, uint8_t value);
-void launch_fill_double(hipStream_t s, double *p, long long n, double value);
 void launch_set_flags(hipStream_t s, int n_active, const int *active, uint8_t *flags);
 // the device Riemann solver on independent face states (gzm_elements.hip):
 // mode 0 riemann_solve, mode 1 the KT flux alone; precision 0 FP64, else FP32

@@ -83,6 +83,26 @@ __global__ __launch_bounds__(kBlock) void export_kernel(ExportArgs a)
     f.dst[t] = f.src[(long long)a.inv[i] * f.w_src + f.off + e];
 }
 
+__global__ void export_u8_kernel(int n, const int *inv, const uint8_t *src, uint8_t *dst)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) dst[i] = src[inv[i]];
+}
+
+__global__ void fill_fields_kernel(FillArgs a)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= a.n) return;
+    for (int q = 0; q < a.n_fills; q++)
+        for (int c = 0; c < a.width[q]; c++) a.p[q][(size_t)c * a.n + k] = a.value[q];
+}
+
+__global__ void iota_kernel(int n, int *p)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n) p[k] = k;
+}
+
 __global__ void restore_kernel(int n, double *hsml, const double *hsml0, double *cn, const double *cn0, double *vsig,
                                const double *vsig0, double *dmass, const double *dmass0)
 {
@@ -190,12 +210,6 @@ __global__ void fill_int_kernel(int *p, int n, int v)
 __global__ void fill_u8_kernel(uint8_t *p, int n, uint8_t v)
 {
     int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) p[t] = v;
-}
-
-__global__ void fill_double_kernel(double *p, long long n, double v)
-{
-    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t < n) p[t] = v;
 }
 
@@ -1182,6 +1196,18 @@ void launch_export(hipStream_t s, ExportArgs &a)
     }
     if (blocks > 0) hipLaunchKernelGGL(export_kernel, dim3(blocks), dim3(kBlock), 0, s, a);
 }
+void launch_export_u8(hipStream_t s, int n, const int *inv, const uint8_t *src, uint8_t *dst)
+{
+    if (n > 0) hipLaunchKernelGGL(export_u8_kernel, dim3(nblocks(n)), dim3(kBlock), 0, s, n, inv, src, dst);
+}
+void launch_fill_fields(hipStream_t s, const FillArgs &a)
+{
+    if (a.n > 0 && a.n_fills > 0) hipLaunchKernelGGL(fill_fields_kernel, dim3(nblocks(a.n)), dim3(kBlock), 0, s, a);
+}
+void launch_iota(hipStream_t s, int n, int *p)
+{
+    if (n > 0) hipLaunchKernelGGL(iota_kernel, dim3(nblocks(n)), dim3(kBlock), 0, s, n, p);
+}
 void launch_restore(hipStream_t s, int n, double *hsml, const double *hsml0, double *cn, const double *cn0, double *vsig,
                     const double *vsig0, double *dmass, const double *dmass0)
 {
@@ -1391,10 +1417,6 @@ void launch_fill_int(hipStream_t s, int *p, int n, int value)
 void launch_fill_u8(hipStream_t s, uint8_t *p, int n, uint8_t value)
 {
     if ((n) > 0) hipLaunchKernelGGL(fill_u8_kernel, dim3(nblocks(n)), dim3(kBlock), 0, s, p, n, value);
-}
-void launch_fill_double(hipStream_t s, double *p, long long n, double value)
-{
-    if ((n) > 0) hipLaunchKernelGGL(fill_double_kernel, dim3(nblocks(n)), dim3(kBlock), 0, s, p, n, value);
 }
 void launch_set_flags(hipStream_t s, int n_active, const int *active, uint8_t *flags)
 {
