@@ -913,15 +913,26 @@ __device__ __forceinline__ bool deferred_left(const ForceArgs &a)
     return a.defer.mask && *a.defer.total > a.defer.q_end;
 }
 
+// the pair list of a particle of the redo, where it holds the whole set: with
+// every particle active a particle's row is that of its slot
+__device__ __forceinline__ int redo_count(const ForceArgs &a, int i)
+{
+    return a.list.idx && !a.is_active && a.list.count[i] <= a.list.cap ? a.list.count[i] : -1;
+}
+__device__ __forceinline__ const int *redo_row(const ForceArgs &a, int i)
+{
+    return a.list.idx + (size_t)i * a.list.cap;
+}
+
 // The gradients of each particle listed by mark_redo, again, in FP64 from the
 // FP64 state with the arithmetic of gradients_kernel (gradients.c:66-75,
 // 1219-1232), written over the FP32 gradients.  One wavefront per listed
-// particle: the lanes share its candidates (wave_pair_candidates) and reduce
+// particle: the lanes share its candidates (wave_pairs) and reduce
 // their partial sums, maxima and minima; lane 0 applies NV_T and the limiter.  Sums in another order than the FP64 pass: equal to ~1e-16.
 __global__ __launch_bounds__(kBlock) void gradients_redo_fp64_kernel(ForceArgs a)
 {
     if (deferred_left(a)) return;
-    __shared__ WaveWalkLds walk[kBlock / 64];
+    __shared__ WavePairLds lds[kBlock / 64];
     const int n_redo = a.redo_count[1];
     const int lane = threadIdx.x & 63;
     const int n_waves = gridDim.x * (kBlock / 64);
@@ -941,17 +952,17 @@ __global__ __launch_bounds__(kBlock) void gradients_redo_fp64_kernel(ForceArgs a
             const double h2_i = h_i * h_i;
             const double xs[3] = {pi.x, pi.y, pi.z};
             const double R = (h_i > G.hmax) ? h_i : G.hmax;
-            wave_pair_candidates(a.tree, G, xs, R, h_i, lane, walk[threadIdx.x >> 6], [&](int j) {
-                const double4 xj = a.posm[j];
-                double dp[3] = {xs[0] - xj.x, xs[1] - xj.y, xs[2] - xj.z};
-                wrap_dp(G.box, dp);
-                const double r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
+            wave_pairs(a.tree, G, xs, R, h_i, lane, redo_row(a, i), redo_count(a, i), lds[threadIdx.x >> 6],
+                       [&](int j) {
+                double dp[3];
+                const double r2 = exact_r2(G.box, pi, a.posm[j], dp);
                 const double h_j = a.hsml[j];
-                if (r2 <= 0) return;
-                if ((r2 >= h2_i) && (r2 >= h_j * h_j)) return;
+                return (r2 > 0) && !((r2 >= h2_i) && (r2 >= h_j * h_j)) && (a.posm[j].w > 0) && (a.rho[j] > 0);
+            }, [&](int j) {
+                double dp[3];
+                const double r2 = exact_r2(G.box, pi, a.posm[j], dp);
                 const double rho_j = a.rho[j];
-                if (!((xj.w > 0) && (rho_j > 0))) return;
-                if (!(h_j > 0)) return;
+                if (!(a.hsml[j] > 0)) return;
                 const double4 vj = a.velu[j];
                 const double r = sqrt(r2);
                 const double wk_i = (r < h_i) ? kernel_w(r * hinv, hinv3) : 0.0;
@@ -1016,7 +1027,7 @@ __global__ __launch_bounds__(kBlock) void gradients_redo_fp64_kernel(ForceArgs a
 // The force loop of each listed particle in FP64 from the FP64 state: the
 // FP64 pass's neighbour predicate, pair arithmetic and inline exact solver
 // (hydro_evaluate.h:22-516).  One wavefront per listed particle: the lanes
-// share its candidates (wave_pair_candidates) and reduce their flux sums;
+// share its candidates (wave_pairs) and reduce their flux sums;
 // lane 0 applies the final operations.  REDO: the particles listed by
 // mark_redo (with the redone gradients), overwriting their FP32 result and
 // clearing their flags; their pairs were counted by the FP32 loop.  Otherwise:
@@ -1026,7 +1037,7 @@ template <bool REDO>
 __global__ __launch_bounds__(kBlock) void force_wave_fp64_kernel(ForceArgs a, const int *list, const int *count)
 {
     if (REDO && deferred_left(a)) return;
-    __shared__ WaveWalkLds walk[kBlock / 64];
+    __shared__ WavePairLds lds[kBlock / 64];
     const int n_redo = *count;
     if (REDO && blockIdx.x == 0 && threadIdx.x == 0 && n_redo > 0) atomicAdd(&ctr_slot(a.ctr)->redo_n, n_redo);
     const int lane = threadIdx.x & 63;
@@ -1049,13 +1060,15 @@ __global__ __launch_bounds__(kBlock) void force_wave_fp64_kernel(ForceArgs a, co
             const double xs[3] = {pi.x, pi.y, pi.z};
             const double R = (h_i > G.hmax) ? h_i : G.hmax;
             ROut<double> ro = {0, 0, {0, 0, 0}, 0};
-            wave_pair_candidates(a.tree, G, xs, R, h_i, lane, walk[threadIdx.x >> 6], [&](int j) {
-                if (j == i) return;
+            wave_pairs(a.tree, G, xs, R, h_i, lane, REDO ? redo_row(a, i) : nullptr, REDO ? redo_count(a, i) : -1,
+                       lds[threadIdx.x >> 6], [&](int j) {
                 double dp[3];
                 const double r2 = exact_r2(G.box, pi, a.posm[j], dp);
                 const double h_j = a.hsml[j];
-                if (!(r2 > 0) || (!(r2 < h2_i) && !(r2 < h_j * h_j))) return;
-                if (!(a.posm[j].w > 0) || !(a.rho[j] > 0)) return;  // hydro_evaluate.h:149-150
+                return (r2 > 0) && ((r2 < h2_i) || (r2 < h_j * h_j)) && (a.posm[j].w > 0) && (a.rho[j] > 0);  // hydro_evaluate.h:149-150
+            }, [&](int j) {
+                double dp[3];
+                const double r2 = exact_r2(G.box, pi, a.posm[j], dp);
                 PairSide<double> J;
                 side_fp64(a, j, J);
                 double Fv[3], Fp, vsig;
