@@ -180,6 +180,84 @@ __device__ __forceinline__ void for_each_run(const Grid &g, const double xs[3], 
     }
 }
 
+// the votes of a group of W lanes, from bit 0
+template <int W>
+__device__ __forceinline__ uint64_t group_ballot(bool v)
+{
+    const uint64_t bits = __ballot(v);
+    if constexpr (W == 64) return bits;
+    else return (bits >> ((threadIdx.x & 63) & ~(W - 1))) & ((1ull << W) - 1);
+}
+
+// The candidates of W lanes of one particle (`sub` = 0 .. W - 1), a z column of
+// cells for each lane: test(j, whole, cx, cy, cz) decides, hit(k, j) takes the hits
+// with their rank k in the order of for_each_cell.  Returns their number; -1: a
+// column held more hits than a lane keeps, or more than `limit` candidates.
+constexpr int kColumnHits = 32;
+template <int W, typename T, typename F>
+__device__ __forceinline__ int for_columns(const Grid &g, const double xs[3], double R, int sub, int limit,
+                                           int *kept /* kColumnHits of this lane, 256 apart */, T &&test, F &&hit)
+{
+    int lo[3], n[3];
+    bool full[3];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        full[a] = !(R * g.inv_s[a] < 0.5 * g.nc[a] - 2.0);
+        lo[a] = full[a] ? 0 : (int)floor((xs[a] - R) * g.inv_s[a] - 1e-6);
+        n[a] = (full[a] ? g.nc[a] - 1 : (int)floor((xs[a] + R) * g.inv_s[a] + 1e-6)) - lo[a] + 1;
+    }
+    const double R2 = R * R * (1.0 + 1e-9);
+    const bool whole = full[0] || full[1] || full[2];
+    const int columns = n[0] * n[1];
+    int total = 0, seen = 0;
+    for (int c0 = 0; c0 < columns; c0 += W) {
+        const int c = c0 + sub;
+        int hits = 0;
+        if (c < columns) {
+            const int cx = lo[0] + c / n[1], cy = lo[1] + c % n[1];
+            const double gx = full[0] ? 0.0 : axis_gap(xs[0], cx * g.s[0], g.s[0]);
+            const double gy = full[1] ? 0.0 : axis_gap(xs[1], cy * g.s[1], g.s[1]);
+            const double gxy2 = gx * gx + gy * gy;
+            const int wx = (cx < 0) ? cx + g.nc[0] : ((cx >= g.nc[0]) ? cx - g.nc[0] : cx);
+            const int wy = (cy < 0) ? cy + g.nc[1] : ((cy >= g.nc[1]) ? cy - g.nc[1] : cy);
+            const int2 *column = g.range + (wx * g.nc[1] + wy) * g.nc[2];
+            auto slots = [&](int cz) {
+                if (cz >= lo[2] + n[2]) return make_int2(0, 0);
+                const double gz = full[2] ? 0.0 : axis_gap(xs[2], cz * g.s[2], g.s[2]);
+                if (gxy2 > R2 || gxy2 + gz * gz > R2) return make_int2(0, 0);
+                return column[(cz < 0) ? cz + g.nc[2] : ((cz >= g.nc[2]) ? cz - g.nc[2] : cz)];
+            };
+            int2 r = slots(lo[2]);
+            for (int z = 0; z < n[2]; z++) {
+                const int2 next = slots(lo[2] + z + 1);  // under way while this cell is tested
+                seen += r.y - r.x;
+                for (int j = r.x; j < r.y; j += 4) {
+                    bool in[4];
+#pragma unroll
+                    for (int k = 0; k < 4; k++) in[k] = test(min(j + k, r.y - 1), whole, cx, cy, lo[2] + z) && j + k < r.y;
+#pragma unroll
+                    for (int k = 0; k < 4; k++)
+                        if (in[k]) {
+                            if (hits < kColumnHits) kept[256 * hits] = j + k;
+                            hits++;
+                        }
+                }
+                r = next;
+            }
+        }
+        if (group_ballot<W>(hits > kColumnHits || seen > limit)) return -1;
+        int sum = hits;
+#pragma unroll
+        for (int off = 1; off < W; off <<= 1) {
+            const int o = __shfl_up(sum, off, W);
+            if (sub >= off) sum += o;
+        }
+        for (int k = 0; k < hits; k++) hit(total + sum - hits + k, kept[256 * k]);
+        total += __shfl(sum, W - 1, W);
+    }
+    return total;
+}
+
 // Visit every sorted slot k whose cell may hold a particle within distance R
 // of (x, y, z), periodic.
 template <typename F>
@@ -339,15 +417,6 @@ __device__ __forceinline__ void walk_call(F &&f, int slot, bool valid, bool last
 {
     if constexpr (std::is_invocable<F, int, bool, bool>::value) f(slot, valid, last);
     else f(slot, valid);
-}
-
-// the votes of a group of W lanes, from bit 0
-template <int W>
-__device__ __forceinline__ uint64_t group_ballot(bool v)
-{
-    const uint64_t bits = __ballot(v);
-    if constexpr (W == 64) return bits;
-    else return (bits >> ((threadIdx.x & 63) & ~(W - 1))) & ((1ull << W) - 1);
 }
 
 // LDS of the tree walk of W lanes (group_tree_walk).  Past kWide entries fewer

@@ -529,20 +529,36 @@ gzm_status ensure_list(gzm_ctx *c)
     return GZM_OK;
 }
 
-// per-box max hsml into the device box descriptors (no host round trip)
-// and, with `ctr`, that stage's counters cleared
-gzm_status compute_hmax(gzm_ctx *c, Counters *ctr)
+// Per-box (and per-cell or per-node) max hsml into the device descriptors, with no
+// host round trip; with `ctr`, that stage's counters cleared; with `grad`, the
+// FP64 gradient records.
+gzm_status compute_hmax(gzm_ctx *c, Counters *ctr, bool grad = false)
 {
-    if (c->hmax_valid) {
-        if (ctr) launch_clear_counters(c->stream, ctr);
-        return GZM_OK;
+    PairPrepareArgs a = {};
+    a.boxes = c->d_boxes;
+    a.hsml = c->d_hsml;
+    if (!c->hmax_valid) {
+        a.tiles = c->d_hmax_tiles;
+        a.n_tiles = c->n_hmax_tiles;
+        if (!c->tree.nodes) {
+            a.range = c->d_range;
+            a.cell_hmax = c->d_cell_hmax;
+            a.n_cells = c->ncell;
+        }
     }
-    c->hmax_valid = true;
+    if (grad) {
+        a.n = c->n;
+        a.posm = c->d_posm;
+        a.velu = c->d_velu;
+        a.rho = c->d_rho;
+        a.pres = c->d_pres;
+        a.xh = c->d_gxh;
+        a.rec = c->d_grec;
+    }
     Timed tm(c, kOther);
-    launch_box_hmax(c->stream, c->n_boxes, c->d_boxes, c->d_hsml, c->n_hmax_tiles, c->d_hmax_tiles,
-                    ctr);
-    if (c->tree.nodes) launch_tree_hmax(c->stream, c->tbuild, c->d_hsml);
-    else launch_cell_hmax(c->stream, c->ncell, c->d_range, c->d_hsml, c->d_cell_hmax);
+    launch_pair_prepare(c->stream, a, c->hmax_valid ? 0 : c->n_boxes, ctr);
+    if (c->tree.nodes && !c->hmax_valid) launch_tree_hmax(c->stream, c->tbuild, c->d_hsml);
+    c->hmax_valid = true;
     GZM_HIP(hipGetLastError());
     return GZM_OK;
 }
@@ -1310,16 +1326,12 @@ gzm_status density_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
 gzm_status gradients_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
 {
     gzm_status s;
-    s = compute_hmax(c, gp ? nullptr : c->d_ctr + kCtrGradients * kCtrSpread);
+    s = compute_hmax(c, gp ? nullptr : c->d_ctr + kCtrGradients * kCtrSpread, c->p.precision == 0);
     if (s) return s;
-    {
+    if (c->p.precision != 0) {
         Timed tm(c, kOther);
-        if (c->p.precision != 0)
-            launch_pack_grad_f32(c->stream, c->n, c->d_offm, c->d_velf, c->d_hsml, c->d_rho, c->d_pres, c->d_gxhf,
-                                 c->d_grecf);
-        else
-            launch_pack_grad(c->stream, c->n, c->d_posm, c->d_velu, c->d_hsml, c->d_rho, c->d_pres, c->d_gxh,
-                             c->d_grec);
+        launch_pack_grad_f32(c->stream, c->n, c->d_offm, c->d_velf, c->d_hsml, c->d_rho, c->d_pres, c->d_gxhf,
+                             c->d_grecf);
     }
     GradientArgs a;
     memset(&a, 0, sizeof(a));
@@ -1565,13 +1577,16 @@ gzm_status force_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
     };
     int64_t first = 0;
     if (three_phase) {
-        size_t bytes = 0;
-        GZM_HIP(rocprim::exclusive_scan(nullptr, bytes, c->d_defer_count, c->d_defer_off, 0, (size_t)c->n_active,
-                                        rocprim::plus<int>(), c->stream));
-        if (c->capturing && bytes > c->temp_bytes) { set_error("temporary storage too small while capturing"); return GZM_ERR_STATE; }
-        s = ensure_temp(c, bytes);
-        if (s) return s;
-        {
+        if (c->n_active <= kOneBlockScan) {
+            Timed tm(c, kForceDeferred);
+            launch_defer_scan(c->stream, c->n_active, c->d_defer_count, c->d_defer_off);
+        } else {
+            size_t bytes = 0;
+            GZM_HIP(rocprim::exclusive_scan(nullptr, bytes, c->d_defer_count, c->d_defer_off, 0, (size_t)c->n_active,
+                                            rocprim::plus<int>(), c->stream));
+            if (c->capturing && bytes > c->temp_bytes) { set_error("temporary storage too small while capturing"); return GZM_ERR_STATE; }
+            s = ensure_temp(c, bytes);
+            if (s) return s;
             Timed tm(c, kForceDeferred);
             GZM_HIP(rocprim::exclusive_scan(c->d_temp, bytes, c->d_defer_count, c->d_defer_off, 0, (size_t)c->n_active,
                                             rocprim::plus<int>(), c->stream));

@@ -23,7 +23,7 @@
 // 128^3 blast (2.1 M particles, 33 pairs and 1.97 sweeps each): rows 0.86, sweeps
 // 0.66 + 0.66, tail and far 0.03 ms; the launch per sweep with its walk that this
 // replaces took 2 x 1.41 ms and a host round trip per sweep.  32^3 lattice: rows
-// 0.038, sweeps 2 x 0.024 ms (2 x 0.11 ms).  Bound by the latency of the
+// 0.033, sweeps 2 x 0.024 ms (2 x 0.11 ms).  Bound by the latency of the
 // candidate loads (45 % VALU busy, 500 cycles per load at 5 waves per SIMD).
 #include "grid_device.h"
 #include "gzm_internal.h"
@@ -202,13 +202,15 @@ __device__ __forceinline__ void count_sweeps(const DensityStageArgs &a, unsigned
 // together (in one loop nearly every candidate step of a wavefront runs the
 // pair body for the few lanes that have a neighbour there).  G = 1: one lane
 // per particle, entries staged in LDS and stored as whole 64-byte chunks.
-// G > 1 (few particles): G lanes share a cell, entries packed by ballot, same
-// order.
+// G > 1 (few particles): each of the G lanes walks a z column of cells, same order
+// (4,096 particles: 18 us, 32 k: 33 us; with the lanes sharing the candidates of one
+// cell after the other, waiting for each cell's slots, 28 and 38 us); a column with
+// more hits than a lane keeps sends its particle to that form.
 template <int G>
 __global__ __launch_bounds__(kBlock) void density_rows_kernel(DensityStageArgs a)
 {
-    __shared__ __align__(16) int lds[G == 1 ? kListChunk * kBlock : 1];
-    int *stage = wave_chunk(lds);
+    __shared__ __align__(16) int lds[G == 1 ? kListChunk * kBlock : kColumnHits * kBlock];
+    int *stage = wave_chunk(lds), *kept = lds;
     const int gt = xcd_block() * kBlock + (int)threadIdx.x;
     const int t = gt / G, sub = gt % G;
     const bool valid = t < a.n_active;
@@ -255,25 +257,25 @@ __global__ __launch_bounds__(kBlock) void density_rows_kernel(DensityStageArgs a
         const float Lmax = (float)fmax(B.box.L[0], fmax(B.box.L[1], B.box.L[2]));
         const float Rf = (float)Rc * (1 + 1e-6f) + 5e-7f * Lmax, Rf2 = Rf * Rf * (1 + 1e-6f);
         const float4 fi = a.posf[i];
-        for_each_run(B.grid, xs, Rc, [&](const bool full[3], int cx, int cy, int cz, int beg, int end) -> bool {
-            visited += end - beg;
-            if (visited > limit) return false;
-            // the image of this cell that the walk reached is the nearest
-            // one wherever the axis is not walked whole
-            const bool whole = full[0] || full[1] || full[2];
-            const float Lx = (float)B.box.L[0], Ly = (float)B.box.L[1], Lz = (float)B.box.L[2];
+        const float Lx = (float)B.box.L[0], Ly = (float)B.box.L[1], Lz = (float)B.box.L[2];
+        // the image of cell (cx, cy, cz) that the walk reached is the nearest one
+        // wherever the axis is not walked whole
+        auto near = [&](const float4 &pj, bool whole, int cx, int cy, int cz) {
             const float ox = fi.x - (cx < 0 ? -Lx : (cx >= B.grid.nc[0] ? Lx : 0.0f));
             const float oy = fi.y - (cy < 0 ? -Ly : (cy >= B.grid.nc[1] ? Ly : 0.0f));
             const float oz = fi.z - (cz < 0 ? -Lz : (cz >= B.grid.nc[2] ? Lz : 0.0f));
-            auto test = [&](const float4 &pj) {
-                float dx = ox - pj.x, dy = oy - pj.y, dz = oz - pj.z;
-                if (whole) {
-                    dx -= Lx * rintf(dx / Lx);
-                    dy -= Ly * rintf(dy / Ly);
-                    dz -= Lz * rintf(dz / Lz);
-                }
-                return dx * dx + dy * dy + dz * dz < Rf2 && pj.w > 0;
-            };
+            float dx = ox - pj.x, dy = oy - pj.y, dz = oz - pj.z;
+            if (whole) {
+                dx -= Lx * rintf(dx / Lx);
+                dy -= Ly * rintf(dy / Ly);
+                dz -= Lz * rintf(dz / Lz);
+            }
+            return dx * dx + dy * dy + dz * dz < Rf2 && pj.w > 0;
+        };
+        auto run = [&](const bool full[3], int cx, int cy, int cz, int beg, int end) -> bool {
+            visited += end - beg;
+            if (visited > limit) return false;
+            const bool whole = full[0] || full[1] || full[2];
             // two candidates in flight: the walk waits on these loads
             constexpr int U = 2;
             for (int k = beg + sub; k - sub < end; k += U * G) {
@@ -282,10 +284,22 @@ __global__ __launch_bounds__(kBlock) void density_rows_kernel(DensityStageArgs a
                 for (int c = 0; c < U; c++) p[c] = a.posf[min(k + c * G, end - 1)];
 #pragma unroll
                 for (int c = 0; c < U; c++)
-                    if (G > 1 || c == 0 || k + c < end) append(k + c * G, k + c * G < end && test(p[c]));
+                    if (G > 1 || c == 0 || k + c < end) append(k + c * G, k + c * G < end && near(p[c], whole, cx, cy, cz));
             }
             return m <= cap;
-        });
+        };
+        bool listed = false;
+        if constexpr (G > 1) {
+            m = for_columns<G>(B.grid, xs, Rc, sub, limit, kept + threadIdx.x,
+                               [&](int j, bool whole, int cx, int cy, int cz) {
+                return near(a.posf[j], whole, cx, cy, cz);
+            }, [&](int k, int j) {
+                if (k < cap) row[k] = j;
+            });
+            listed = m >= 0;
+            if (!listed) m = 0;
+        }
+        if (!listed) for_each_run(B.grid, xs, Rc, run);
         if (visited > limit) m = kNoRow;
         if (G == 1 && m < cap && (m & (kListChunk - 1)))
             flush_list_chunk(stage, row + (m & ~(kListChunk - 1)));
@@ -696,7 +710,18 @@ void launch_density_tail(hipStream_t s, const DensityStageArgs &a)
         else launch_tree_tail<false>(s, a);
         return;
     }
-    // the count is on the device: enough workgroups to fill the chip, at most one group per particle
+    // the counts are on the device: enough workgroups to fill the chip, at most one group per particle
+    if (a.lanes == 8) {
+        // few particles: the whole tail with a wavefront each, in one launch (a nearly
+        // empty tail of 32 k particles: 5.1 us against 4.1 + 3.5 and the gap between)
+        DensityStageArgs b = a;
+        b.far_list = a.tail_list;
+        b.n_far = a.n_tail;
+        const dim3 waves(std::min(2048u, nblocks(64LL * a.n_active)));
+        if (a.pvel) hipLaunchKernelGGL(density_far_kernel<true>, waves, dim3(kBlock), 0, s, b);
+        else hipLaunchKernelGGL(density_far_kernel<false>, waves, dim3(kBlock), 0, s, b);
+        return;
+    }
     const dim3 grid(std::min(2048u, nblocks((long long)kTailLanes * a.n_active))), block(kBlock);
     if (a.pvel) hipLaunchKernelGGL(density_tail_kernel<true>, grid, block, 0, s, a);
     else hipLaunchKernelGGL(density_tail_kernel<false>, grid, block, 0, s, a);

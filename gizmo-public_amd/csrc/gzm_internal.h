@@ -404,8 +404,20 @@ void launch_cell_ranges(hipStream_t s, int n, const double4 *posm, const BoxDesc
 // per-box max hsml into boxes[b].hmax; tiles = (box, first slot) of each
 // block, each tile at most kHmaxTile slots of one box
 constexpr int kHmaxTile = 4096;
-void launch_box_hmax(hipStream_t s, int n_boxes, BoxDesc *boxes, const double *hsml, int n_tiles, const int2 *tiles,
-                     Counters *ctr);  // ctr (NULL: none): counters to clear on the way
+// n_tiles, n_cells or rec may be none; ctr (NULL: none): counters to clear on the way
+struct PairPrepareArgs {
+    BoxDesc *boxes;
+    const double *hsml;
+    const int2 *tiles;
+    int n_tiles, n_cells, cell_blocks, n;
+    const int2 *range;
+    float *cell_hmax;
+    const double4 *posm, *velu;
+    const double *rho, *pres;
+    double4 *xh;
+    GradRec *rec;
+};
+void launch_pair_prepare(hipStream_t s, PairPrepareArgs &a, int n_boxes, Counters *ctr);
 void launch_publish_counters(hipStream_t s, const Counters *ctr, Counters *host);
 void launch_export(hipStream_t s, ExportArgs &a);
 void launch_export_u8(hipStream_t s, int n, const int *inv, const uint8_t *src, uint8_t *dst);
@@ -440,8 +452,6 @@ void launch_edge_reset(hipStream_t s, int cap, const int *n_edge, const int *edg
 void launch_density_finalize(hipStream_t s, int n_active, const int *active, const double4 *posm,
                              const double4 *velu, const double *hsml, double *num_ngb, double *rho,
                              double *pres, double gamma_minus_1);
-void launch_pack_grad(hipStream_t s, int n, const double4 *posm, const double4 *velu, const double *hsml,
-                      const double *rho, const double *pres, double4 *xh, GradRec *rec);
 void launch_sym_rows(hipStream_t s, const SymRowArgs &a);
 void launch_gradients(hipStream_t s, const GradientArgs &a);
 void launch_pack_force(hipStream_t s, int n, const double4 *posm, const double4 *velu, const double *hsml,
@@ -451,6 +461,10 @@ void launch_force(hipStream_t s, const ForceArgs &a);  // list-driven if a.list.
 // deferred exact-solver pairs [a.defer.q_begin, a.defer.q_end), then the per-particle finish
 void launch_force_deferred(hipStream_t s, const ForceArgs &a, int n_pairs);
 // owner entry and list position of each deferred pair of the round [q_begin, q_end)
+// Up to this many counts one workgroup scans them in one launch (4,096: 4 us; the
+// library's scan takes two, 6.6 us and the gap between); above it one is too few.
+constexpr int kOneBlockScan = 16384;
+void launch_defer_scan(hipStream_t s, int n, const int *count, int *offset);
 void launch_defer_owners(hipStream_t s, const ForceArgs &a);
 void launch_force_finish(hipStream_t s, const ForceArgs &a);
 // FP32-bulk kernels (gzm_kernels_f32.hip)
@@ -508,7 +522,6 @@ void launch_tree_build(hipStream_t s, const TreeBuild &b, const double *hsml);
 // node hmax from the current hsml (window-maximum table; node boxes unchanged)
 void launch_tree_hmax(hipStream_t s, const TreeBuild &b, const double *hsml);
 // per-cell max hsml (rounded up to FP32) of the cells' slot ranges
-void launch_cell_hmax(hipStream_t s, int ncell, const int2 *range, const double *hsml, float *hmax);
 // MFV force loop (gzm_mfv.hip): the preloop that zeroes the active
 // particles' DtMass, dMass and GravWorkTerm, then the loop
 void launch_mfv_preloop(hipStream_t s, const ForceArgs &a, const MfvArgs &m);

@@ -151,26 +151,6 @@ __global__ void cell_ranges_kernel(int n, const double4 *posm, const BoxDesc *bo
     if (c != cnext) range[c].y = k + 1;
 }
 
-// Per-box max hsml (the search radius of the pair loops, force_update_hmax):
-// block = one tile of up to kHmaxTile slots of one box; block maximum, then
-// one atomic max on the bit pattern (valid for hsml >= 0).
-__global__ __launch_bounds__(kBlock) void box_hmax_kernel(BoxDesc *boxes, const double *hsml, const int2 *tiles)
-{
-    __shared__ double red[kBlock / 64];
-    const int2 tile = tiles[blockIdx.x];  // (box, first slot)
-    const BoxDesc &B = boxes[tile.x];
-    const int end = min(tile.y + kHmaxTile, B.first + B.count);
-    double m = 0;
-    for (int k = tile.y + threadIdx.x; k < end; k += kBlock) m = fmax(m, hsml[k]);
-    for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < kBlock / 64; w++) m = fmax(m, red[w]);
-        atomicMax((unsigned long long *)&boxes[tile.x].hmax, (unsigned long long)__double_as_longlong(m));
-    }
-}
-
 __global__ void clear_box_hmax_kernel(int n_boxes, BoxDesc *boxes, Counters *ctr)
 {
     int b = blockIdx.x * blockDim.x + threadIdx.x;
@@ -376,11 +356,9 @@ __global__ void density_finalize_kernel(int n_active, const int *active, const d
 // ---------------------------------------------------------------------------
 // gradients (gradients.c:1477-2089 pair loop, 1052-1253 finalize)
 // ---------------------------------------------------------------------------
-__global__ void pack_grad_kernel(int n, const double4 *posm, const double4 *velu, const double *hsml,
-                                 const double *rho, const double *pres, double4 *xh, GradRec *rec)
+__device__ __forceinline__ void pack_grad(int k, const double4 *posm, const double4 *velu, const double *hsml,
+                                          const double *rho, const double *pres, double4 *xh, GradRec *rec)
 {
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
     double4 p = posm[k], v = velu[k];
     GradRec r;
     xh[k] = make_double4(p.x, p.y, p.z, hsml[k]);
@@ -406,6 +384,44 @@ __device__ __forceinline__ ForceRec make_force_rec(const double4 &p, const doubl
     for (int k = 0; k < 9; k++) r.gv[k] = g[6 + k];
     r.cn = cn; r.e = P / d;
     return r;
+}
+
+// What the pair stages read that hsml decides, in one launch of three parts by
+// workgroup: the largest hsml of each box (the search radius of the pair loops,
+// force_update_hmax), one tile of up to kHmaxTile slots of a box each (block
+// maximum, then one atomic max on the bit pattern, valid for hsml >= 0); that of
+// each cell, rounded up; and the FP64 gradient records (a.rec NULL: none).
+__global__ __launch_bounds__(kBlock) void pair_prepare_kernel(PairPrepareArgs a)
+{
+    __shared__ double red[kBlock / 64];
+    int block = blockIdx.x;
+    if (block < a.n_tiles) {
+        const int2 tile = a.tiles[block];  // (box, first slot)
+        const BoxDesc &B = a.boxes[tile.x];
+        const int end = min(tile.y + kHmaxTile, B.first + B.count);
+        double m = 0;
+        for (int k = tile.y + threadIdx.x; k < end; k += kBlock) m = fmax(m, a.hsml[k]);
+        for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int w = 1; w < kBlock / 64; w++) m = fmax(m, red[w]);
+            atomicMax((unsigned long long *)&a.boxes[tile.x].hmax, (unsigned long long)__double_as_longlong(m));
+        }
+        return;
+    }
+    block -= a.n_tiles;
+    if (block < a.cell_blocks) {
+        const int c = block * kBlock + (int)threadIdx.x;
+        if (c >= a.n_cells) return;
+        const int2 r = a.range[c];
+        double m = 0.0;
+        for (int k = r.x; k < r.y; ++k) m = (a.hsml[k] > m) ? a.hsml[k] : m;
+        a.cell_hmax[c] = __double2float_ru(m);
+        return;
+    }
+    const int k = (block - a.cell_blocks) * kBlock + (int)threadIdx.x;
+    if (k < a.n) pack_grad(k, a.posm, a.velu, a.hsml, a.rho, a.pres, a.xh, a.rec);
 }
 
 constexpr int kNoSlot = 0x7fffffff;  // above every sorted slot: the end of a merged row
@@ -1225,12 +1241,14 @@ void launch_cell_ranges(hipStream_t s, int n, const double4 *posm, const BoxDesc
     if ((2LL * ncell) > 0) hipLaunchKernelGGL(fill_int_kernel, dim3(nblocks(2LL * ncell)), dim3(kBlock), 0, s, (int *)range, 2 * ncell, 0);
     if (n > 0) hipLaunchKernelGGL(cell_ranges_kernel, dim3(nblocks(n)), dim3(kBlock), 0, s, n, posm, boxes, box_of, range);
 }
-void launch_box_hmax(hipStream_t s, int n_boxes, BoxDesc *boxes, const double *hsml, int n_tiles, const int2 *tiles,
-                     Counters *ctr)
+void launch_pair_prepare(hipStream_t s, PairPrepareArgs &a, int n_boxes, Counters *ctr)
 {
-    if (n_boxes > 0) hipLaunchKernelGGL(clear_box_hmax_kernel, dim3(nblocks(n_boxes)), dim3(kBlock), 0, s, n_boxes, boxes,
-                                       ctr);
-    if (n_tiles > 0) hipLaunchKernelGGL(box_hmax_kernel, dim3(n_tiles), dim3(kBlock), 0, s, boxes, hsml, tiles);
+    if (n_boxes > 0 || ctr)
+        hipLaunchKernelGGL(clear_box_hmax_kernel, dim3(nblocks(std::max(n_boxes, 1))), dim3(kBlock), 0, s, n_boxes, a.boxes,
+                           ctr);
+    a.cell_blocks = (int)nblocks(a.n_cells);
+    const unsigned blocks = a.n_tiles + a.cell_blocks + (a.rec ? nblocks(a.n) : 0);
+    if (blocks > 0) hipLaunchKernelGGL(pair_prepare_kernel, dim3(blocks), dim3(kBlock), 0, s, a);
 }
 void launch_flag_unconverged(hipStream_t s, const int *n_live_dev, Counters *ctr)
 {
@@ -1268,11 +1286,6 @@ void launch_density_finalize(hipStream_t s, int n_active, const int *active, con
 {
     if ((n_active) > 0) hipLaunchKernelGGL(density_finalize_kernel, dim3(nblocks(n_active)), dim3(kBlock), 0, s, n_active, active, posm,
                        velu, hsml, num_ngb, rho, pres, gm1);
-}
-void launch_pack_grad(hipStream_t s, int n, const double4 *posm, const double4 *velu, const double *hsml,
-                      const double *rho, const double *pres, double4 *xh, GradRec *rec)
-{
-    if ((n) > 0) hipLaunchKernelGGL(pack_grad_kernel, dim3(nblocks(n)), dim3(kBlock), 0, s, n, posm, velu, hsml, rho, pres, xh, rec);
 }
 void launch_sym_rows(hipStream_t s, const SymRowArgs &a)
 {
@@ -1334,6 +1347,31 @@ void launch_force(hipStream_t s, const ForceArgs &a)
 }
 namespace {
 
+// exclusive sums of up to kOneBlockScan counts, by one workgroup
+__global__ __launch_bounds__(1024) void defer_scan_kernel(int n, const int *count, int *offset)
+{
+    __shared__ int total[16];
+    const int per = (n + 1023) / 1024, lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+    const int beg = min(per * (int)threadIdx.x, n), end = min(beg + per, n);
+    int own = 0;
+    for (int k = beg; k < end; k++) own += count[k];
+    int sum = own;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int o = __shfl_up(sum, off, 64);
+        if (lane >= off) sum += o;
+    }
+    if (lane == 63) total[wave] = sum;
+    __syncthreads();
+    int at = sum - own;
+    for (int w = 0; w < wave; w++) at += total[w];
+    for (int k = beg; k < end; k++) {
+        const int c = count[k];
+        offset[k] = at;
+        at += c;
+    }
+}
+
 // one thread per active entry: its deferred pairs q = offset + r (r-th set
 // bit k of its mask) that fall in the round get their particle and neighbour
 // (i, list entry k), so that the pair kernel starts from both records' indices
@@ -1362,6 +1400,10 @@ __global__ __launch_bounds__(kBlock) void defer_owners_kernel(ForceArgs a)
 
 }  // namespace
 
+void launch_defer_scan(hipStream_t s, int n, const int *count, int *offset)
+{
+    hipLaunchKernelGGL(defer_scan_kernel, dim3(1), dim3(1024), 0, s, n, count, offset);
+}
 void launch_defer_owners(hipStream_t s, const ForceArgs &a)
 {
     if (a.n_active > 0) hipLaunchKernelGGL(defer_owners_kernel, dim3(nblocks(a.n_active)), dim3(kBlock), 0, s, a);
@@ -1382,24 +1424,6 @@ void launch_density_heavy(hipStream_t s, const DensitySweepArgs &a, int max_entr
     const long long blocks = ((long long)max_entries + 3) / 4;
     const dim3 grid((unsigned)(blocks < 2048 ? blocks : 2048));
     hipLaunchKernelGGL(density_heavy_kernel, grid, dim3(kBlock), 0, s, a);
-}
-
-namespace {
-__global__ void cell_hmax_kernel(int ncell, const int2 *range, const double *hsml, float *hmax)
-{
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ncell) return;
-    const int2 r = range[c];
-    double m = 0.0;
-    for (int k = r.x; k < r.y; ++k) m = (hsml[k] > m) ? hsml[k] : m;
-    hmax[c] = __double2float_ru(m);
-}
-}  // namespace
-
-void launch_cell_hmax(hipStream_t s, int ncell, const int2 *range, const double *hsml, float *hmax)
-{
-    if (ncell > 0)
-        hipLaunchKernelGGL(cell_hmax_kernel, dim3(nblocks(ncell)), dim3(kBlock), 0, s, ncell, range, hsml, hmax);
 }
 
 void launch_neighbor_counts(hipStream_t s, const BoxDesc *boxes, const int *box_of, const TreeArgs &tree, int mode,
