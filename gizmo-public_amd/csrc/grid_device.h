@@ -144,7 +144,7 @@ __device__ __forceinline__ void for_each_run(const Grid &g, const double xs[3], 
         lo[a] = full[a] ? 0 : (int)floor((xs[a] - R) * g.inv_s[a] - 1e-6);
         hi[a] = full[a] ? g.nc[a] - 1 : (int)floor((xs[a] + R) * g.inv_s[a] + 1e-6);
     }
-    const double R2 = R * R * (1.0 + 1e-9);
+    const double R2 = R * R * (1.0 + 1e-9), inv_R2 = 1.0 / R2;
     for (int cx = lo[0]; cx <= hi[0]; ++cx) {
         const int wx = (cx < 0) ? cx + g.nc[0] : ((cx >= g.nc[0]) ? cx - g.nc[0] : cx);
         const double gx = full[0] ? 0.0 : axis_gap(xs[0], cx * g.s[0], g.s[0]);
@@ -156,24 +156,34 @@ __device__ __forceinline__ void for_each_run(const Grid &g, const double xs[3], 
             const double gxy2 = gx2 + gy * gy;
             if (gxy2 > R2) continue;
             const int2 *column = g.range + (wx * g.nc[1] + wy) * g.nc[2];
+            // the cells in reach of this column, from the width of the sphere there
+            int z0 = lo[2], z1 = hi[2];
+            if (!full[2]) {
+                const double w = R * ((double)__builtin_amdgcn_sqrtf((float)((R2 - gxy2) * inv_R2)) * (1 + 1e-6));
+                z0 = max(z0, (int)floor((xs[2] - w) * g.inv_s[2] - 1e-6));
+                z1 = min(z1, (int)floor((xs[2] + w) * g.inv_s[2] + 1e-6));
+            }
+            auto slots = [&](int cz) {
+                if (cz > z1) return make_int2(0, 0);
+                return column[(cz < 0) ? cz + g.nc[2] : ((cz >= g.nc[2]) ? cz - g.nc[2] : cz)];
+            };
             int beg = 0, end = 0, first = 0;
+            int2 r = slots(z0);
             // one step past the last cell hands over the last run
-            for (int cz = lo[2]; cz <= hi[2] + 1; ++cz) {
-                int2 r = make_int2(0, 0);
-                if (cz <= hi[2]) {
-                    const double gz = full[2] ? 0.0 : axis_gap(xs[2], cz * g.s[2], g.s[2]);
-                    if (gxy2 + gz * gz > R2) continue;
-                    const int wz = (cz < 0) ? cz + g.nc[2] : ((cz >= g.nc[2]) ? cz - g.nc[2] : cz);
-                    r = column[wz];
-                    if (r.x == r.y) continue;
-                    if (r.x == end && end > beg && wz > 0) {
-                        end = r.y;
+            for (int cz = z0; cz <= z1 + 1; ++cz) {
+                const int2 next = slots(cz + 1);
+                const int2 c = r;
+                r = next;
+                if (cz <= z1) {
+                    if (c.x == c.y) continue;
+                    if (c.x == end && end > beg && cz != 0 && cz != g.nc[2]) {
+                        end = c.y;
                         continue;
                     }
                 }
                 if (end > beg && !f(full, cx, cy, first, beg, end)) return;
-                beg = r.x;
-                end = r.y;
+                beg = c.x;
+                end = c.y;
                 first = cz;
             }
         }

@@ -94,7 +94,7 @@ __device__ __forceinline__ void mfv_store(const ForceArgs &a, const MfvArgs &m, 
 // <= 64): pairs that reach the exact Riemann solver are left to
 // force_mfv_deferred_kernel (bit k of the particle's defer mask) and particles
 // whose pair set overflowed the list to force_mfv_kernel; raw sums go to
-// force_mfv_finish_kernel.  384 k particles: 1.37 ms against 1.79 ms with one lane
+// force_mfv_finish_kernel.  670 k particles: 1.37 ms against 1.79 ms with one lane
 // per particle, whose two records and nine sums spilled 82 registers.
 __global__ __launch_bounds__(64, 2) void force_mfv_list_kernel(ForceArgs a, MfvArgs m)
 {
