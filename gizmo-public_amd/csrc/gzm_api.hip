@@ -322,20 +322,25 @@ gzm_status upload_sorted(gzm_ctx *c, const double *host, double *dst, int width)
 constexpr size_t kBounceBytes = 32u << 20;
 
 // The device's address of host memory that it can write itself, all of
-// [host, host + bytes); NULL: it cannot.
-double *device_view(double *host, size_t bytes)
+// [host, host + bytes) in one allocation; NULL: it cannot.  `plain`: the host
+// can write there itself too (not the case of device memory).
+double *device_view(double *host, size_t bytes, bool *plain)
 {
-    if (bytes == 0 || (uintptr_t)host % sizeof(double)) return nullptr;
-    hipPointerAttribute_t first, last;
-    if (hipPointerGetAttributes(&first, host) != hipSuccess ||
-        hipPointerGetAttributes(&last, (char *)host + bytes - 1) != hipSuccess) {
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, host) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
     }
-    if (first.type != hipMemoryTypeHost || last.type != hipMemoryTypeHost || !first.devicePointer || !last.devicePointer)
+    if (at.type == hipMemoryTypeDevice) *plain = false;
+    if (at.type != hipMemoryTypeHost || !at.devicePointer || (uintptr_t)at.devicePointer % sizeof(double)) return nullptr;
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)at.devicePointer) != hipSuccess) {
+        (void)hipGetLastError();
         return nullptr;
-    if ((char *)last.devicePointer - (char *)first.devicePointer != (ptrdiff_t)(bytes - 1)) return nullptr;
-    return (double *)first.devicePointer;
+    }
+    const char *p = (const char *)at.devicePointer, *b = (const char *)base;
+    return (p >= b && (size_t)(p - b) <= size && bytes <= size - (size_t)(p - b)) ? (double *)at.devicePointer : nullptr;
 }
 
 // Sorted device arrays -> host arrays in caller order.  Fields in memory that
@@ -350,8 +355,9 @@ gzm_status download_fields(gzm_ctx *c, const std::vector<ExportField> &fields, u
     int width = 0;
     size_t bytes = wakeup ? (size_t)c->n : 0;
     std::vector<const ExportField *> staged;
+    bool plain = true;
     for (auto &f : fields) {
-        double *d = direct.n_fields < kMaxExport ? device_view(f.dst, (size_t)c->n * f.w * sizeof(double)) : nullptr;
+        double *d = direct.n_fields < kMaxExport ? device_view(f.dst, (size_t)c->n * f.w * sizeof(double), &plain) : nullptr;
         if (d) {
             direct.field[direct.n_fields] = f;
             direct.field[direct.n_fields++].dst = d;
@@ -365,7 +371,7 @@ gzm_status download_fields(gzm_ctx *c, const std::vector<ExportField> &fields, u
     // in all, the fields go to a pinned array of the context and from there by
     // memcpy (9,261 particles, 16 fields: 0.35 ms against 0.77; above it the
     // runtime's copies, which overlap their own memcpy, are no slower).
-    if (bytes > 0 && bytes <= kBounceBytes && direct.n_fields + staged.size() <= (size_t)kMaxExport) {
+    if (plain && bytes > 0 && bytes <= kBounceBytes && direct.n_fields + staged.size() <= (size_t)kMaxExport) {
         if (bytes > c->bounce_bytes) {
             if (c->h_bounce) (void)hipHostFree(c->h_bounce);
             c->h_bounce = nullptr;

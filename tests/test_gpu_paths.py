@@ -134,3 +134,22 @@ def test_downloads_into_pinned_and_ordinary_memory_agree(side):
         np.testing.assert_array_equal(pinned[k], out[k].reshape(-1), err_msg=k)
         if k in ic:
             np.testing.assert_array_equal(out[k].reshape(-1), np.asarray(ic[k]).reshape(-1), err_msg=k)
+
+
+def test_download_into_device_memory_and_into_part_of_a_pinned_array():
+    ic = ics.lattice_gaussian(9)
+    n = 9 ** 3
+    with gzm.MFMContext(params_for(ic)) as ctx:
+        ctx.upload(ic)
+        out = ctx.download()
+        on_card = torch.zeros(n, dtype=torch.float64, device="cuda")
+        pinned = torch.zeros(n + 12, dtype=torch.float64, pin_memory=True)
+        torch.cuda.synchronize()
+        view = gzm.HostView()
+        view.n = n
+        view.hsml = C.cast(C.c_void_p(on_card.data_ptr()), C.POINTER(C.c_double))
+        view.cn = C.cast(C.c_void_p(pinned[5:].data_ptr()), C.POINTER(C.c_double))
+        assert ctx.L.gzm_download(ctx.ctx, C.byref(view)) == 0
+    np.testing.assert_array_equal(on_card.cpu().numpy(), out["hsml"])
+    np.testing.assert_array_equal(pinned[5:5 + n].numpy(), out["cn"])
+    assert not pinned[:5].any() and not pinned[5 + n:].any()
