@@ -171,6 +171,7 @@ gzm_status dev_alloc(T **p, size_t count)
     hipError_t e = hipMalloc((void **)p, count * sizeof(T));
     if (e != hipSuccess) {
         set_error("hipMalloc of %zu bytes failed: %s", count * sizeof(T), hipGetErrorString(e));
+        (void)hipGetLastError();  // reported here: a caller that does without goes on
         *p = nullptr;
         return GZM_ERR_NOMEM;
     }
@@ -182,6 +183,25 @@ void dev_free(T *&p)
 {
     if (p) (void)hipFree((void *)p);
     p = nullptr;
+}
+
+// The candidate rows (up to 412 B per particle) are an optimisation: a set that
+// fills the memory without them runs without them.
+void free_rows(gzm_ctx *c)
+{
+    dev_free(c->d_dcache_idx); dev_free(c->d_dcache_n); dev_free(c->d_dcache_r2); dev_free(c->d_posf);
+    c->dcache_all = false;
+}
+
+// an array that the context needs, whose memory the candidate rows give up if they have to
+template <class T>
+gzm_status need(gzm_ctx *c, T **p, size_t count)
+{
+    gzm_status s = dev_alloc(p, count);
+    if (s == GZM_OK || c->capturing || !c->d_dcache_idx) return s;
+    (void)hipStreamSynchronize(c->stream);
+    free_rows(c);
+    return dev_alloc(p, count);
 }
 
 hipEvent_t take_event(gzm_ctx *c)
@@ -243,7 +263,7 @@ gzm_status ensure_temp(gzm_ctx *c, size_t bytes)
     if (bytes <= c->temp_bytes) return GZM_OK;
     dev_free(c->d_temp);
     c->temp_bytes = 0;
-    gzm_status s = dev_alloc((char **)&c->d_temp, bytes);
+    gzm_status s = need(c, (char **)&c->d_temp, bytes);
     if (s == GZM_OK) c->temp_bytes = bytes;
     return s;
 }
@@ -253,7 +273,7 @@ gzm_status ensure_stage(gzm_ctx *c, size_t doubles)
     if (doubles <= c->stage_doubles) return GZM_OK;
     dev_free(c->d_stage);
     c->stage_doubles = 0;
-    gzm_status s = dev_alloc(&c->d_stage, doubles);
+    gzm_status s = need(c, &c->d_stage, doubles);
     if (s == GZM_OK) c->stage_doubles = doubles;
     return s;
 }
@@ -284,9 +304,8 @@ void free_particles(gzm_ctx *c)
     dev_free(c->d_t_large_count);
     dev_free(c->d_t_split); dev_free(c->d_t_esc); dev_free(c->d_t_leaf_esc); dev_free(c->d_t_flag);
     dev_free(c->d_t_lo); dev_free(c->d_t_hi); dev_free(c->d_t_wmax); dev_free(c->d_t_nodes);
-    dev_free(c->d_dcache_idx); dev_free(c->d_dcache_n); dev_free(c->d_dcache_r2);
-    dev_free(c->d_posf); dev_free(c->d_brow); dev_free(c->d_bcount); dev_free(c->d_bwave); dev_free(c->d_bwave_n);
-    c->dcache_all = false;
+    dev_free(c->d_brow); dev_free(c->d_bcount); dev_free(c->d_bwave); dev_free(c->d_bwave_n);
+    free_rows(c);
     c->tree = TreeArgs{};
     c->defer_result_cap = 0;
     c->list_entries = 0;
@@ -512,11 +531,11 @@ F32Geom f32_geom(const gzm_ctx *c)
 gzm_status ensure_defer(gzm_ctx *c)
 {
     if (c->d_defer_mask) return GZM_OK;
-    gzm_status s = dev_alloc(&c->d_defer_mask, (size_t)c->n);
-    s = s ? s : dev_alloc(&c->d_defer_count, (size_t)c->n);
-    s = s ? s : dev_alloc(&c->d_defer_off, (size_t)c->n);
-    s = s ? s : dev_alloc(&c->d_defer_total, 1);
-    s = s ? s : dev_alloc(&c->d_defer_raw, (size_t)c->n);
+    gzm_status s = need(c, &c->d_defer_mask, (size_t)c->n);
+    s = s ? s : need(c, &c->d_defer_count, (size_t)c->n);
+    s = s ? s : need(c, &c->d_defer_off, (size_t)c->n);
+    s = s ? s : need(c, &c->d_defer_total, 1);
+    s = s ? s : need(c, &c->d_defer_raw, (size_t)c->n);
     return s;
 }
 
@@ -528,8 +547,8 @@ gzm_status ensure_list(gzm_ctx *c)
     if (entries <= c->list_entries && c->d_list_count) return GZM_OK;
     dev_free(c->d_list); dev_free(c->d_list_count);
     c->list_entries = 0;
-    gzm_status s = dev_alloc(&c->d_list, entries);
-    s = s ? s : dev_alloc(&c->d_list_count, (size_t)c->n + 64);
+    gzm_status s = need(c, &c->d_list, entries);
+    s = s ? s : need(c, &c->d_list_count, (size_t)c->n + 64);
     if (s) return s;
     c->list_entries = entries;
     return GZM_OK;
@@ -763,10 +782,10 @@ gzm_status setup_boxes(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const do
         for (int64_t k = i0; k < i1; k += kHmaxTile) tiles.push_back(make_int2(b, (int)k));
     }
     free_boxes(c);
-    gzm_status s = dev_alloc(&c->d_range, (size_t)ncell);
-    s = s ? s : dev_alloc(&c->d_cell_hmax, (size_t)ncell);
-    s = s ? s : dev_alloc(&c->d_boxes, (size_t)n_boxes);
-    s = s ? s : dev_alloc(&c->d_hmax_tiles, tiles.size());
+    gzm_status s = need(c, &c->d_range, (size_t)ncell);
+    s = s ? s : need(c, &c->d_cell_hmax, (size_t)ncell);
+    s = s ? s : need(c, &c->d_boxes, (size_t)n_boxes);
+    s = s ? s : need(c, &c->d_hmax_tiles, tiles.size());
     if (s) { free_boxes(c); return s; }
     for (auto &B : bx) {
         B.grid.range = c->d_range + B.cell_base;
@@ -892,13 +911,9 @@ gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const 
         }
         if (s) { free_particles(c); return s; }
         if (c->p.precision != 2) {
-            // the candidate rows are an optimisation (up to 412 B per particle): a set
-            // that fills the memory without them runs without them
             if (dev_alloc(&c->d_dcache_idx, (size_t)n * kDensityCacheCap) || dev_alloc(&c->d_dcache_n, n) ||
-                dev_alloc(&c->d_dcache_r2, n) || (c->p.search == 0 && dev_alloc(&c->d_posf, n))) {
-                (void)hipGetLastError();
-                dev_free(c->d_dcache_idx); dev_free(c->d_dcache_n); dev_free(c->d_dcache_r2); dev_free(c->d_posf);
-            }
+                dev_alloc(&c->d_dcache_r2, n) || (c->p.search == 0 && dev_alloc(&c->d_posf, n)))
+                free_rows(c);
         }
     }
     if (c->d_redo_flag) launch_fill_int(c->stream, c->d_redo_flag, n, 0);
@@ -985,7 +1000,7 @@ gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const 
         while ((2 << (levels - 1)) <= largest) levels++;  // 1 + floor(log2(largest))
         if (levels != t.levels || !c->d_t_wmax) {
             dev_free(c->d_t_wmax);
-            s = dev_alloc(&c->d_t_wmax, (size_t)levels * n);
+            s = need(c, &c->d_t_wmax, (size_t)levels * n);
             if (s) return s;
         }
         t.levels = levels;
@@ -1537,8 +1552,8 @@ gzm_status force_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
         if ((!mfv || three_phase) && use_list && c->list_overflow_slices > 0) {
             // particles whose pair set overflowed the list: one wavefront each, FP64
             if (!c->d_long_list) {
-                s = dev_alloc(&c->d_long_list, (size_t)c->n);
-                s = s ? s : dev_alloc(&c->d_long_count, 1);
+                s = need(c, &c->d_long_list, (size_t)c->n);
+                s = s ? s : need(c, &c->d_long_count, 1);
                 if (s) return s;
             }
             launch_fill_int(c->stream, c->d_long_count, 1, 0);
@@ -1552,8 +1567,8 @@ gzm_status force_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
         dev_free(c->d_defer_result);
         dev_free(c->d_defer_pair);
         c->defer_result_cap = 0;
-        gzm_status e = dev_alloc(&c->d_defer_result, want * (mfv ? 9 : 5));
-        e = e ? e : dev_alloc(&c->d_defer_pair, want);
+        gzm_status e = need(c, &c->d_defer_result, want * (mfv ? 9 : 5));
+        e = e ? e : need(c, &c->d_defer_pair, want);
         if (e) return e;
         c->defer_result_cap = want;
         return GZM_OK;
