@@ -771,6 +771,7 @@ gzm_status setup_boxes(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const do
         }
         const double side = 0.45 * std::min(L[0], std::min(L[1], L[2]));
         B.box.narrow2 = side * side;
+        B.unit = ldexp(1.0, -std::max(-1000, std::min(1000, ilogb(std::max(L[0], std::max(L[1], L[2]))))));
         B.cell_base = (int)ncell;
         ncell += nb;
         if (ncell > ((int64_t)1 << 30)) { set_error("grids of %lld cells too large", (long long)ncell); return GZM_ERR_ARG; }
@@ -957,8 +958,8 @@ gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const 
         if (s) return s;
         GZM_HIP(rocprim::radix_sort_pairs(c->d_temp, bytes, c->d_keys, c->d_keys_sorted, c->d_iota, c->d_perm, n, 0,
                                           key_bits, c->stream));
-        launch_gather_sorted(c->stream, n, c->d_perm, st_pos, st_vel, st_mass, st_u, d_box_caller, c->d_posm,
-                             c->d_velu, c->d_posf, c->d_inv, c->d_box_of);
+        launch_gather_sorted(c->stream, n, c->d_perm, st_pos, st_vel, st_mass, st_u, c->d_boxes, d_box_caller,
+                             c->d_posm, c->d_velu, c->d_posf, c->d_inv, c->d_box_of);
         if (!tree) launch_cell_ranges(c->stream, n, c->d_posm, c->d_boxes, c->d_box_of, c->d_range, c->ncell);
         if (c->p.precision != 0)
             launch_pack_geom_f32(c->stream, n, c->d_posm, c->d_velu, c->d_boxes, c->d_box_of, c->d_offm, c->d_velf,

@@ -256,11 +256,12 @@ __global__ __launch_bounds__(kBlock) void density_rows_kernel(DensityStageArgs a
         };
         // FP32 distances with a margin for their rounding (2^-24 of a side per
         // coordinate): the row may hold a few more than the exact radius
-        // asks for, never fewer, and a candidate is one 16-byte load.
-        const float Lmax = (float)fmax(B.box.L[0], fmax(B.box.L[1], B.box.L[2]));
-        const float Rf = (float)Rc * (1 + 1e-6f) + 5e-7f * Lmax, Rf2 = Rf * Rf * (1 + 1e-6f);
+        // asks for, never fewer, and a candidate is one 16-byte load.  In units
+        // of the box: the squares of a galaxy's centimetres overflow FP32.
+        const float Lx = (float)(B.box.L[0] * B.unit), Ly = (float)(B.box.L[1] * B.unit), Lz = (float)(B.box.L[2] * B.unit);
+        const float Rf = (float)(Rc * B.unit) * (1 + 1e-6f) + 5e-7f * fmaxf(Lx, fmaxf(Ly, Lz));
+        const float Rf2 = Rf * Rf * (1 + 1e-6f);
         const float4 fi = a.posf[i];
-        const float Lx = (float)B.box.L[0], Ly = (float)B.box.L[1], Lz = (float)B.box.L[2];
         // the image of cell (cx, cy, cz) that the walk reached is the nearest one
         // wherever the axis is not walked whole
         auto near = [&](const float4 &pj, bool whole, int cx, int cy, int cz) {

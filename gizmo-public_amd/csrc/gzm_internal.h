@@ -29,6 +29,8 @@ struct BoxDesc {
     BoxInfo box;           // side lengths and half side lengths
     double hmax;           // max hsml of the box (the pair loops' search radius)
     float s_f[3];          // cell side in FP32
+    double unit;           // power of two that brings the longest side to [1, 2): FP32 positions (posf)
+                           // are in these units, whose squares fit FP32 whatever the caller's units
     int cell_base;         // first cell of the box in the global range array
     int first, count;      // sorted slot range of the box
     int root;              // tree search: root node of the box (kTreeEnd if empty); with two or
@@ -221,7 +223,7 @@ struct DensityStageArgs {
     const int *active;
     int n_active;
     const double4 *posm, *velu;
-    const float4 *posf;    // positions in FP32, w = 1 for mass > 0, else 0 (grid rows)
+    const float4 *posf;    // positions * BoxDesc::unit in FP32, w = 1 for mass > 0, else 0 (grid rows)
     double *hsml, *left, *right, *cn;
     double *num_ngb, *dhsml, *divvel, *rho, *pres, *fce, *nvt;  // nvt: 6 per particle
     double *pvel;          // MFV: ParticleVel (NULL: MFM)
@@ -396,8 +398,8 @@ struct MfvArgs {
 void launch_cell_keys(hipStream_t s, int n, const double *pos, const BoxDesc *boxes, const int *box_caller,
                       uint64_t *keys, int *iota);
 void launch_gather_sorted(hipStream_t s, int n, const int *perm, const double *pos, const double *vel,
-                          const double *mass, const double *u, const int *box_caller, double4 *posm,
-                          double4 *velu, float4 *posf, int *inv, int *box_of);
+                          const double *mass, const double *u, const BoxDesc *boxes, const int *box_caller,
+                          double4 *posm, double4 *velu, float4 *posf, int *inv, int *box_of);
 void launch_gather_scalar(hipStream_t s, int n, const int *perm, const double *src, double *dst, int width);
 void launch_cell_ranges(hipStream_t s, int n, const double4 *posm, const BoxDesc *boxes, const int *box_of,
                         int2 *range, int ncell);

@@ -45,18 +45,22 @@ __global__ void cell_keys_kernel(int n, const double *pos, const BoxDesc *boxes,
 }
 
 __global__ void gather_sorted_kernel(int n, const int *perm, const double *pos, const double *vel,
-                                     const double *mass, const double *u, const int *box_caller, double4 *posm,
-                                     double4 *velu, float4 *posf, int *inv, int *box_of)
+                                     const double *mass, const double *u, const BoxDesc *boxes, const int *box_caller,
+                                     double4 *posm, double4 *velu, float4 *posf, int *inv, int *box_of)
 {
     int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
     int i = perm[k];
     posm[k] = make_double4(pos[3 * i + 0], pos[3 * i + 1], pos[3 * i + 2], mass[i]);
     velu[k] = make_double4(vel[3 * i + 0], vel[3 * i + 1], vel[3 * i + 2], u[i]);
-    if (posf)
-        posf[k] = make_float4((float)pos[3 * i + 0], (float)pos[3 * i + 1], (float)pos[3 * i + 2], mass[i] > 0 ? 1.0f : 0.0f);
+    const int b = box_caller ? box_caller[i] : 0;
+    if (posf) {
+        const double s = boxes[b].unit;
+        posf[k] = make_float4((float)(pos[3 * i + 0] * s), (float)(pos[3 * i + 1] * s), (float)(pos[3 * i + 2] * s),
+                              mass[i] > 0 ? 1.0f : 0.0f);
+    }
     inv[i] = k;
-    box_of[k] = box_caller ? box_caller[i] : 0;
+    box_of[k] = b;
 }
 
 __global__ void gather_scalar_kernel(int n, const int *perm, const double *src, double *dst, int width)
@@ -1191,12 +1195,12 @@ void launch_cell_keys(hipStream_t s, int n, const double *pos, const BoxDesc *bo
     if (n > 0) hipLaunchKernelGGL(cell_keys_kernel, dim3(nblocks(n)), dim3(kBlock), 0, s, n, pos, boxes, box_caller, keys, iota);
 }
 void launch_gather_sorted(hipStream_t s, int n, const int *perm, const double *pos, const double *vel,
-                          const double *mass, const double *u, const int *box_caller, double4 *posm,
-                          double4 *velu, float4 *posf, int *inv, int *box_of)
+                          const double *mass, const double *u, const BoxDesc *boxes, const int *box_caller,
+                          double4 *posm, double4 *velu, float4 *posf, int *inv, int *box_of)
 {
     if (n > 0)
-        hipLaunchKernelGGL(gather_sorted_kernel, dim3(nblocks(n)), dim3(kBlock), 0, s, n, perm, pos, vel, mass, u, box_caller,
-                           posm, velu, posf, inv, box_of);
+        hipLaunchKernelGGL(gather_sorted_kernel, dim3(nblocks(n)), dim3(kBlock), 0, s, n, perm, pos, vel, mass, u, boxes,
+                           box_caller, posm, velu, posf, inv, box_of);
 }
 void launch_gather_scalar(hipStream_t s, int n, const int *perm, const double *src, double *dst, int width)
 {
