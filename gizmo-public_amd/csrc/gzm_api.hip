@@ -1784,6 +1784,7 @@ gzm_status gzm_upload_batch(gzm_ctx *c, const gzm_host_view *v, int32_t n_boxes,
 gzm_status gzm_restore_initial_state(gzm_ctx *c)
 {
     if (!c || c->n == 0) { set_error("no particles uploaded"); return GZM_ERR_STATE; }
+    GZM_HIP(hipSetDevice(c->p.device));
     return restore_state(c);
 }
 

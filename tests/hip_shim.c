@@ -1,0 +1,49 @@
+/* Stands before the HIP runtime in a test process: counts hipSetDevice and
+ * bounds what hipMalloc hands out, as a card of `shim_budget` bytes would. */
+#include <pthread.h>
+#include <stddef.h>
+
+int (*shim_malloc)(void **, size_t), (*shim_free)(void *), (*shim_set_device)(int); /* the runtime's own */
+size_t shim_budget = (size_t)-1, shim_used, shim_peak;
+int shim_refused, shim_set_device_calls;
+
+#define SLOTS 65536
+static struct { void *p; size_t n; } held[SLOTS];
+static pthread_mutex_t mu = PTHREAD_MUTEX_INITIALIZER;
+
+int hipMalloc(void **p, size_t n)
+{
+    int e = 2; /* hipErrorOutOfMemory */
+    pthread_mutex_lock(&mu);
+    if (n > shim_budget || shim_used > shim_budget - n) {
+        shim_refused++;
+    } else if ((e = shim_malloc(p, n)) == 0) {
+        int k = 0;
+        while (k < SLOTS - 1 && held[k].p) k++;
+        held[k].p = *p;
+        held[k].n = n;
+        shim_used += n;
+        if (shim_used > shim_peak) shim_peak = shim_used;
+    }
+    pthread_mutex_unlock(&mu);
+    return e;
+}
+
+int hipFree(void *p)
+{
+    pthread_mutex_lock(&mu);
+    for (int k = 0; p && k < SLOTS; k++)
+        if (held[k].p == p) {
+            shim_used -= held[k].n;
+            held[k].p = NULL;
+            break;
+        }
+    pthread_mutex_unlock(&mu);
+    return shim_free(p);
+}
+
+int hipSetDevice(int device)
+{
+    shim_set_device_calls++;
+    return shim_set_device(device);
+}

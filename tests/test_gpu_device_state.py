@@ -1,0 +1,10 @@
+"""What the library asks of the HIP runtime, with a shim before it (hip_shim)."""
+import pytest
+
+import hip_shim
+
+pytestmark = pytest.mark.gpu
+
+
+def test_entry_points_make_their_device_current():
+    hip_shim.run("entry_points_make_their_device_current")
