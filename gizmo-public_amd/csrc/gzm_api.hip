@@ -1141,10 +1141,11 @@ DensityStageArgs density_stage_args(gzm_ctx *c)
     a.far_list = c->d_heavy_list;
     a.n_far = c->d_count + 2;
     const bool tree = c->tree.nodes != nullptr;
-    a.walk_list = tree ? c->d_bwave : a.tail_list;
+    const bool few = c->n_active <= kFewParticles;
+    a.walk_list = tree ? c->d_bwave : (few ? a.tail_list : nullptr);
     a.n_walk = tree ? c->d_count + 3 : a.n_tail;
     a.budget = c->p.density_budget == 0 ? kDensityBudget : (c->p.density_budget < 0 ? 0 : c->p.density_budget);
-    a.lanes = c->n_active <= kFewParticles ? 8 : 1;
+    a.lanes = few ? 8 : 1;
     a.ctr = c->d_ctr + kCtrDensity * kCtrSpread;
     return a;
 }

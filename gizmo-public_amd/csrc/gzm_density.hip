@@ -3,20 +3,21 @@
 //
 // A particle's iteration reads only its own sums, so no sweep has to be a
 // launch of its own and nothing is compacted or counted on the host between
-// sweeps.  Four kernels per stage:
+// sweeps.  The kernels of a stage:
 //
 //   density_rows_kernel   candidates of every active particle within
 //                         kDensityCacheFactor * hsml, in walk order (a pure
 //                         distance filter over the grid or tree)
 //   density_stage_kernel  the first two sweeps over the rows, a launch each
 //                         (nearly every particle of an even set needs exactly two)
-//   density_tail_kernel   particles not converged by then, or without a usable
-//                         row: 16 lanes each, iterating to convergence
-//   density_far_kernel    particles whose walk passes the candidate budget: a
-//                         wavefront each, iterating to convergence
+//   density_more_kernel   what is left by then, packed anew for every sweep (not
+//                         for few particles in the grid)
+//   density_tail_kernel   the last of those: 16 lanes each, iterating to convergence
+//   density_far_kernel    of those, the particles whose walk passes the candidate
+//                         budget; for few particles all that is left: a wavefront
+//                         each, iterating to convergence
 //
-// The tree has density_more_kernel between the last two, and kernels of its own
-// for the particles that have to walk.
+// The tree has kernels of its own for the particles that have to walk.
 //
 // The lists between them live on the device.
 //
@@ -35,6 +36,8 @@ namespace {
 constexpr int kTailLanes = 16;
 constexpr int kFarWaves = 4;
 constexpr int kNoRow = kDensityCacheCap + 1;
+constexpr int kWideRow = kNoRow + 1;  // row_n where the walk for the row passed twice the candidate budget
+constexpr int kDone = -1;  // iter of a particle whose iteration has ended
 
 // sums of one candidate already known to lie within h (density.c:252-347).
 // MFV: also m_j W_ij v_j into pv (density.c:291-293 for r = 0, 331-334 as
@@ -209,11 +212,108 @@ __device__ __forceinline__ void count_sweeps(const DensityStageArgs &a, unsigned
 // (4,096 particles: 18 us, 32 k: 33 us; with the lanes sharing the candidates of one
 // cell after the other, waiting for each cell's slots, 28 and 38 us); a column with
 // more hits than a lane keeps sends its particle to that form.
+// Returns the number of entries as stored in row_n, kNoRow or kWideRow where there is no row.
+__device__ __forceinline__ double grid_row_r2(double h)
+{
+    const double Rc = kDensityCacheFactorGrid * h;
+    return Rc * Rc;
+}
+template <int G>
+constexpr int kRowLds = G == 1 ? kListChunk * kBlock : kColumnHits * kBlock;
+template <int G>
+__device__ __forceinline__ int grid_row(const DensityStageArgs &a, const BoxDesc &B, int i, const double4 &pi, double h,
+                                        int sub, int *lds)
+{
+    int *stage = wave_chunk(lds), *kept = lds;
+    const double Rc = kDensityCacheFactorGrid * h;
+    const double xs[3] = {pi.x, pi.y, pi.z};
+    constexpr int cap = kDensityCacheCap;
+    int *row = a.row_idx + (size_t)i * cap;
+    // a row past its cap is of no use, so its walk ends there; the budget
+    // bounds the walk where cells hold many more particles than neighbours
+    const int limit = a.budget ? 2 * a.budget : 0x7fffffff;
+    int m = 0, visited = 0;
+    auto append = [&](int j, bool in) {
+        if constexpr (G == 1) {
+            if (!in) return;
+            if (m < cap) {
+                const int c = m & (kListChunk - 1);
+                stage[c * 64 + (threadIdx.x & 63)] = j;
+                if (c == kListChunk - 1) flush_list_chunk(stage, row + (m - c));
+            }
+            m++;
+        } else {
+            const uint64_t bits = group_ballot<G>(in);
+            const int k = m + __popcll(bits & ((1ull << sub) - 1));
+            if (in && k < cap) row[k] = j;
+            m += __popcll(bits);
+        }
+    };
+    // FP32 distances with a margin for their rounding (2^-24 of a side per
+    // coordinate): the row may hold a few more than the exact radius
+    // asks for, never fewer, and a candidate is one 16-byte load.  In units
+    // of the box: the squares of a galaxy's centimetres overflow FP32.
+    const float Lx = (float)(B.box.L[0] * B.unit), Ly = (float)(B.box.L[1] * B.unit), Lz = (float)(B.box.L[2] * B.unit);
+    const float Rf = (float)(Rc * B.unit) * (1 + 1e-6f) + 5e-7f * fmaxf(Lx, fmaxf(Ly, Lz));
+    const float Rf2 = Rf * Rf * (1 + 1e-6f);
+    const float4 fi = a.posf[i];
+    // the image of cell (cx, cy, cz) that the walk reached is the nearest one
+    // wherever the axis is not walked whole
+    auto near = [&](const float4 &pj, bool whole, int cx, int cy, int cz) {
+        const float ox = fi.x - (cx < 0 ? -Lx : (cx >= B.grid.nc[0] ? Lx : 0.0f));
+        const float oy = fi.y - (cy < 0 ? -Ly : (cy >= B.grid.nc[1] ? Ly : 0.0f));
+        const float oz = fi.z - (cz < 0 ? -Lz : (cz >= B.grid.nc[2] ? Lz : 0.0f));
+        float dx = ox - pj.x, dy = oy - pj.y, dz = oz - pj.z;
+        if (whole) {
+            dx -= Lx * rintf(dx / Lx);
+            dy -= Ly * rintf(dy / Ly);
+            dz -= Lz * rintf(dz / Lz);
+        }
+        return dx * dx + dy * dy + dz * dz < Rf2 && pj.w > 0;
+    };
+    auto run = [&](const bool full[3], int cx, int cy, int cz, int beg, int end) -> bool {
+        visited += end - beg;
+        if (visited > limit) return false;
+        const bool whole = full[0] || full[1] || full[2];
+        // two candidates in flight: the walk waits on these loads
+        constexpr int U = 2;
+        for (int k = beg + sub; k - sub < end; k += U * G) {
+            float4 p[U];
+#pragma unroll
+            for (int c = 0; c < U; c++) p[c] = a.posf[min(k + c * G, end - 1)];
+#pragma unroll
+            for (int c = 0; c < U; c++)
+                if (G > 1 || c == 0 || k + c < end) append(k + c * G, k + c * G < end && near(p[c], whole, cx, cy, cz));
+        }
+        return m <= cap;
+    };
+    bool listed = false;
+    if constexpr (G > 1) {
+        m = for_columns<G>(B.grid, xs, Rc, sub, limit, kept + threadIdx.x,
+                           [&](int j, bool whole, int cx, int cy, int cz) {
+            return near(a.posf[j], whole, cx, cy, cz);
+        }, [&](int k, int j) {
+            if (k < cap) row[k] = j;
+        });
+        listed = m >= 0;
+        if (!listed) m = 0;
+    }
+    if (!listed) for_each_run(B.grid, xs, Rc, run);
+    if (visited > limit) m = kWideRow;
+    if (G == 1 && m < cap && (m & (kListChunk - 1)))
+        flush_list_chunk(stage, row + (m & ~(kListChunk - 1)));
+    if (m > cap && m != kWideRow) m = kNoRow;
+    if (sub == 0) {
+        a.row_n[i] = m;
+        a.row_r2[i] = grid_row_r2(h);
+    }
+    return m;
+}
+
 template <int G>
 __global__ __launch_bounds__(kBlock) void density_rows_kernel(DensityStageArgs a)
 {
-    __shared__ __align__(16) int lds[G == 1 ? kListChunk * kBlock : kColumnHits * kBlock];
-    int *stage = wave_chunk(lds), *kept = lds;
+    __shared__ __align__(16) int lds[kRowLds<G>];
     const int gt = xcd_block() * kBlock + (int)threadIdx.x;
     const int t = gt / G, sub = gt % G;
     const bool valid = t < a.n_active;
@@ -229,88 +329,7 @@ __global__ __launch_bounds__(kBlock) void density_rows_kernel(DensityStageArgs a
             h = 0.99 * a.hp.max_hsml;
             if (sub == 0) a.hsml[i] = h;
         }
-        const double Rc = kDensityCacheFactorGrid * h, Rc2 = Rc * Rc;
-        const double xs[3] = {pi.x, pi.y, pi.z};
-        constexpr int cap = kDensityCacheCap;
-        int *row = a.row_idx + (size_t)i * cap;
-        // a row past its cap is of no use, so its walk ends there; the budget
-        // bounds the walk where cells hold many more particles than neighbours
-        const int limit = a.budget ? 2 * a.budget : 0x7fffffff;
-        int m = 0, visited = 0;
-        auto append = [&](int j, bool in) {
-            if constexpr (G == 1) {
-                if (!in) return;
-                if (m < cap) {
-                    const int c = m & (kListChunk - 1);
-                    stage[c * 64 + (threadIdx.x & 63)] = j;
-                    if (c == kListChunk - 1) flush_list_chunk(stage, row + (m - c));
-                }
-                m++;
-            } else {
-                const int first = (int)(threadIdx.x & 63) & ~(G - 1);
-                const unsigned bits = (unsigned)(__ballot(in) >> first) & ((1u << G) - 1);
-                const int k = m + __popc(bits & ((1u << sub) - 1));
-                if (in && k < cap) row[k] = j;
-                m += __popc(bits);
-            }
-        };
-        // FP32 distances with a margin for their rounding (2^-24 of a side per
-        // coordinate): the row may hold a few more than the exact radius
-        // asks for, never fewer, and a candidate is one 16-byte load.  In units
-        // of the box: the squares of a galaxy's centimetres overflow FP32.
-        const float Lx = (float)(B.box.L[0] * B.unit), Ly = (float)(B.box.L[1] * B.unit), Lz = (float)(B.box.L[2] * B.unit);
-        const float Rf = (float)(Rc * B.unit) * (1 + 1e-6f) + 5e-7f * fmaxf(Lx, fmaxf(Ly, Lz));
-        const float Rf2 = Rf * Rf * (1 + 1e-6f);
-        const float4 fi = a.posf[i];
-        // the image of cell (cx, cy, cz) that the walk reached is the nearest one
-        // wherever the axis is not walked whole
-        auto near = [&](const float4 &pj, bool whole, int cx, int cy, int cz) {
-            const float ox = fi.x - (cx < 0 ? -Lx : (cx >= B.grid.nc[0] ? Lx : 0.0f));
-            const float oy = fi.y - (cy < 0 ? -Ly : (cy >= B.grid.nc[1] ? Ly : 0.0f));
-            const float oz = fi.z - (cz < 0 ? -Lz : (cz >= B.grid.nc[2] ? Lz : 0.0f));
-            float dx = ox - pj.x, dy = oy - pj.y, dz = oz - pj.z;
-            if (whole) {
-                dx -= Lx * rintf(dx / Lx);
-                dy -= Ly * rintf(dy / Ly);
-                dz -= Lz * rintf(dz / Lz);
-            }
-            return dx * dx + dy * dy + dz * dz < Rf2 && pj.w > 0;
-        };
-        auto run = [&](const bool full[3], int cx, int cy, int cz, int beg, int end) -> bool {
-            visited += end - beg;
-            if (visited > limit) return false;
-            const bool whole = full[0] || full[1] || full[2];
-            // two candidates in flight: the walk waits on these loads
-            constexpr int U = 2;
-            for (int k = beg + sub; k - sub < end; k += U * G) {
-                float4 p[U];
-#pragma unroll
-                for (int c = 0; c < U; c++) p[c] = a.posf[min(k + c * G, end - 1)];
-#pragma unroll
-                for (int c = 0; c < U; c++)
-                    if (G > 1 || c == 0 || k + c < end) append(k + c * G, k + c * G < end && near(p[c], whole, cx, cy, cz));
-            }
-            return m <= cap;
-        };
-        bool listed = false;
-        if constexpr (G > 1) {
-            m = for_columns<G>(B.grid, xs, Rc, sub, limit, kept + threadIdx.x,
-                               [&](int j, bool whole, int cx, int cy, int cz) {
-                return near(a.posf[j], whole, cx, cy, cz);
-            }, [&](int k, int j) {
-                if (k < cap) row[k] = j;
-            });
-            listed = m >= 0;
-            if (!listed) m = 0;
-        }
-        if (!listed) for_each_run(B.grid, xs, Rc, run);
-        if (visited > limit) m = kNoRow;
-        if (G == 1 && m < cap && (m & (kListChunk - 1)))
-            flush_list_chunk(stage, row + (m & ~(kListChunk - 1)));
-        if (sub == 0) {
-            a.row_n[i] = m <= cap ? m : kNoRow;
-            a.row_r2[i] = Rc2;
-        }
+        grid_row<G>(a, B, i, pi, h, sub, lds);
     });
 }
 
@@ -421,7 +440,7 @@ __global__ __launch_bounds__(kBlock, 3) void density_stage_kernel(DensityStageAr
         const int i = a.active[t];
         const double4 pi = a.posm[i];
         if (!(pi.w > 0)) return;
-        if (IT == 1 && a.iter[i] != 1) return;  // done, or in the tail list
+        if (IT == 1 && a.iter[i] != 1) return;  // done, or without a usable row
         Iterate s = {a.hsml[i], IT ? a.left[i] : 0.0, IT ? a.right[i] : 0.0, a.cn[i], IT};
         const int n = a.row_n[i];
         const double Rc2 = n <= kDensityCacheCap ? a.row_r2[i] : -1.0;
@@ -432,29 +451,68 @@ __global__ __launch_bounds__(kBlock, 3) void density_stage_kernel(DensityStageAr
         }
         if (sub == 0) {
             max_iter = s.iter;
-            if (!again) a.iter[i] = 0;
+            if (!again) a.iter[i] = kDone;
             else if (IT == 0 && s.iter == 1) hand_on(a, i, s, nullptr, nullptr);
-            else if (s.h * s.h <= Rc2) hand_on(a, i, s, a.tree.nodes ? nullptr : a.tail_list, a.n_tail);
+            else if (s.h * s.h <= Rc2 && a.tree.nodes) hand_on(a, i, s, nullptr, nullptr);
             else hand_on(a, i, s, a.walk_list, a.n_walk);
         }
     });
     count_sweeps(a, cnt, sweeps, max_iter);
 }
 
-// Tree: further sweeps over the rows.  Sets of strongly varying density leave
-// many particles after two (of 250 k in Plummer spheres 196 k need 2.6 more on
-// average, up to 10).  A workgroup takes a stretch of the active particles and
-// packs those not converged anew for every sweep, so that its wavefronts stay
-// full and keep neighbouring particles together; the last few go to the tail
-// list.  The 250 k: 0.50 ms (stretches of 256 or 1024: 0.67), against 2.0 ms with 16 lanes each to convergence
-// and 3.3 ms in four launches over lists whose order the atomics left.
+// Grid: one sweep of a particle over a walk of its own, G lanes; 1: sweep again, 0:
+// done, -1: past the candidate budget (no limit to 64 lanes), the particle as it was.
 template <bool MFV, int G>
+__device__ __forceinline__ int walk_sweep(const DensityStageArgs &a, const BoxDesc &B, int i, const double4 &pi, int sub,
+                                          Iterate &s, unsigned long long &cnt)
+{
+    const double4 vi = a.velu[i];
+    const double h2 = s.h * s.h;
+    double hinv, hinv3, hinv4;
+    kernel_hinv(s.h, hinv, hinv3, hinv4);
+    DensitySums S = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    double pv[3] = {0, 0, 0};
+    const double xs[3] = {pi.x, pi.y, pi.z};
+    unsigned c = 0;
+    const bool ok = group_candidates<G>(B, xs, s.h, sub, G < 64 ? a.budget : 0, [&](int j) {
+        const double4 pj = a.posm[j];
+        double dp[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
+        wrap_dp(B.box, dp);
+        const double r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
+        if (!(r2 < h2 && pj.w > 0)) return;
+        c++;
+        density_add<MFV>(dp, r2, pj.w, vi, a.velu[j], hinv, hinv3, hinv4, S, pv);
+    });
+    if (!ok) return -1;
+    cnt += c;
+    if constexpr (G > 1) group_sums<G, MFV>(S, pv);
+    return density_step(a, i, sub == 0, S, pv, s) ? 1 : 0;
+}
+
+// Further sweeps over the rows.  Sets of strongly varying density, and all sets in
+// the first stage of a run, where hsml is a guess, leave many particles after two
+// (of 250 k in Plummer spheres 196 k need 2.6 more on average, up to 10).  A
+// workgroup takes a stretch of the active particles and packs those not converged
+// anew for every sweep, so that its wavefronts stay full and keep neighbouring
+// particles together; the last few go to the tail list.  The 250 k: 0.50 ms
+// (stretches of 256 or 1024: 0.67), against 2.0 ms with 16 lanes each to convergence
+// and 3.3 ms in four launches over lists whose order the atomics left.
+// Tree: a particle whose hsml leaves its row goes to the walk list.  Grid (GRID):
+// its row is built anew around the hsml reached, and where that is past the cap (a
+// guess far above) or the memory holds no rows, the sweep walks; a walk past the
+// candidate budget is done by a wavefront.  With the 16 lanes of the tail walking for
+// them, sweep by sweep, the density stage of a 128^3 lattice whose hsml starts 20 %
+// low took 35.3 ms, 50 % high 89.6; now 6.6 and 34.7 (a launch per sweep with a lane
+// each and no rows: 7.8 and 39.1).  A well guessed 128^3 blast pays 31 us of 10.7 ms
+// (stretches of 1024 22 us, but 61^3 20 % low 1.1 against 0.6 ms).
+template <bool MFV, int G, bool GRID>
 __global__ __launch_bounds__(kBlock, 2) void density_more_kernel(DensityStageArgs a)
 {
     constexpr int kStretch = 2 * kBlock / G, kFew = kStretch / 16;
-    __shared__ __align__(16) int lds[G == 1 ? kListChunk * kBlock : 1];
-    __shared__ int live[2][kStretch];
-    __shared__ int n_live[2];
+    constexpr int kLists = GRID ? 3 : 2;  // live ones of this sweep and the next, walks past the budget
+    __shared__ __align__(16) int lds[GRID ? kRowLds<G> : (G == 1 ? kListChunk * kBlock : 1)];
+    __shared__ int live[kLists][kStretch];
+    __shared__ int n_live[kLists];
     int *chunk = wave_chunk(lds);
     const int tid = (int)threadIdx.x, lane = tid & 63, sub = tid % G;
     const int first = xcd_block() * kStretch;
@@ -473,17 +531,21 @@ __global__ __launch_bounds__(kBlock, 2) void density_more_kernel(DensityStageArg
     for (int k = tid; k < kStretch; k += kBlock) {
         const int t = first + k;
         const int i = t < a.n_active ? a.active[t] : 0;
-        bool in = t < a.n_active && a.posm[i].w > 0 && a.iter[i] != 0 && a.row_n[i] <= kDensityCacheCap;
-        if (in) {
+        // (a particle without mass has no iter)
+        bool in = t < a.n_active && (GRID ? a.iter[i] != kDone : a.iter[i] > 0) && a.posm[i].w > 0;
+        if (!GRID && in) {
             const double h = a.hsml[i];
-            in = h * h <= a.row_r2[i];
+            in = a.row_n[i] <= kDensityCacheCap && h * h <= a.row_r2[i];
         }
         keep(0, i, in);
     }
     for (int cur = 0;; cur ^= 1) {
         __syncthreads();
         const int n = n_live[cur];
-        if (tid == 0) n_live[cur ^ 1] = 0;
+        if (tid == 0) {
+            n_live[cur ^ 1] = 0;
+            if (GRID) n_live[kLists - 1] = 0;
+        }
         __syncthreads();
         if (n <= kFew) {
             for (int k = tid; k < n; k += kBlock) a.tail_list[atomicAdd(a.n_tail, 1)] = live[cur][k];
@@ -493,33 +555,62 @@ __global__ __launch_bounds__(kBlock, 2) void density_more_kernel(DensityStageArg
             const int k = k0 + tid / G;
             const bool valid = k < n;
             const int i = valid ? live[cur][k] : 0;
-            bool stays = false;
-            if (valid) {
+            bool stays = false, wide = false;
+            for_box(a.boxes, a.box_of, i, valid, [&](const BoxDesc &B) {
                 Iterate s = take_up(a, i);
-                const bool again = row_sweep<MFV, G>(a, a.boxes[a.box_of[i]], i, a.posm[i], a.row_n[i], sub, chunk, s, cnt);
-                if (sub == 0) {
+                const double4 pi = a.posm[i];
+                int n_row = a.row_idx ? a.row_n[i] : kNoRow, again = -1;
+                // (before the first sweep the row is the one tried for this hsml)
+                if (GRID && a.row_idx && s.iter > 0 && !(n_row <= kDensityCacheCap && s.h * s.h <= a.row_r2[i])) {
+                    n_row = grid_row<G>(a, B, i, pi, s.h, sub, lds);
+                }
+                if (!GRID || n_row <= kDensityCacheCap)
+                    again = row_sweep<MFV, G>(a, B, i, pi, n_row, sub, chunk, s, cnt);
+                else if (n_row != kWideRow)
+                    again = walk_sweep<MFV, G>(a, B, i, pi, sub, s, cnt);
+                if (sub != 0) return;
+                wide = again < 0;
+                if (wide) return;
+                sweeps++;
+                max_iter = s.iter > max_iter ? s.iter : max_iter;
+                stays = again == 1 && (GRID || s.h * s.h <= a.row_r2[i]);
+                if (stays) hand_on(a, i, s, nullptr, nullptr);
+                else if (again == 1) hand_on(a, i, s, a.walk_list, a.n_walk);
+            });
+            keep(cur ^ 1, i, stays);
+            if (GRID) keep(kLists - 1, i, wide);
+        }
+        if constexpr (GRID) {
+            __syncthreads();
+            const int n_wide = n_live[kLists - 1];
+            for (int k = tid / 64; k < n_wide; k += kBlock / 64) {
+                const int i = live[kLists - 1][k];
+                Iterate s = take_up(a, i);
+                const bool stays = walk_sweep<MFV, 64>(a, a.boxes[a.box_of[i]], i, a.posm[i], lane, s, cnt) == 1;
+                if (lane == 0) {
                     sweeps++;
                     max_iter = s.iter > max_iter ? s.iter : max_iter;
-                    stays = again && s.h * s.h <= a.row_r2[i];
-                    if (stays) hand_on(a, i, s, nullptr, nullptr);
-                    else if (again) hand_on(a, i, s, a.walk_list, a.n_walk);
+                    if (stays) {
+                        hand_on(a, i, s, nullptr, nullptr);
+                        live[cur ^ 1][atomicAdd(&n_live[cur ^ 1], 1)] = i;
+                    }
                 }
             }
-            keep(cur ^ 1, i, stays);
         }
     }
     count_sweeps(a, cnt, sweeps, max_iter);
 }
 
 // The listed particles, W lanes each, iterating to convergence: over the
-// particle's row while hsml stays inside it, else over a walk shared by the
-// lanes.  A walk past the candidate budget (BUDGET) leaves the particle to the
+// particle's row while hsml stays inside it (grid: a row built anew once it leaves
+// it), else over a walk shared by the lanes.  A walk past the candidate budget (BUDGET) leaves the particle to the
 // far list, and any walk (kRowsOnly) to the walk list.  A fixed grid strides over
 // the device-side count.
 enum DensityWalk { kGridWalk, kTreeWalk, kRowsOnly };
 template <bool MFV, int W, bool BUDGET, DensityWalk WALK, int WAVES = 1>
 __device__ __forceinline__ void density_iterate(const DensityStageArgs &a, const int *list, const int *count,
-                                                WaveWalkLds *walk, BlockWalkLds<WAVES> *block_walk = nullptr)
+                                                WaveWalkLds *walk, int *row_lds = nullptr,
+                                                BlockWalkLds<WAVES> *block_walk = nullptr)
 {
     const int sub = (int)threadIdx.x % W, part = WAVES > 1 ? (int)threadIdx.x / 64 : 0;
     const int n_groups = WAVES > 1 ? (int)gridDim.x : (int)(gridDim.x * (kBlock / W));
@@ -532,12 +623,18 @@ __device__ __forceinline__ void density_iterate(const DensityStageArgs &a, const
         const double4 pi = a.posm[i];
         const double4 vi = a.velu[i];
         Iterate s = take_up(a, i);
-        const int n_row = a.row_n ? a.row_n[i] : kNoRow;
-        const double Rc2 = n_row <= kDensityCacheCap ? a.row_r2[i] : -1.0;
+        int n_row = a.row_n ? a.row_n[i] : kNoRow;
+        double Rc2 = n_row <= kDensityCacheCap ? a.row_r2[i] : -1.0;
         const double xs[3] = {pi.x, pi.y, pi.z};
         bool again = true, far = false;
         while (again) {
             const double h2 = s.h * s.h;
+            // (before the first sweep the row is the one tried for this hsml)
+            if (WALK == kGridWalk && a.row_n && s.iter > 0 && !(h2 <= Rc2)) {
+                n_row = grid_row<W>(a, B, i, pi, s.h, sub, row_lds);
+                wave_lds_fence();  // the other lanes' entries
+                Rc2 = n_row <= kDensityCacheCap ? grid_row_r2(s.h) : -1.0;
+            }
             double hinv, hinv3, hinv4;
             kernel_hinv(s.h, hinv, hinv3, hinv4);
             DensitySums S = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -598,15 +695,17 @@ __device__ __forceinline__ void density_iterate(const DensityStageArgs &a, const
 }
 
 template <bool MFV>
-__global__ __launch_bounds__(kBlock) void density_tail_kernel(DensityStageArgs a)
+__global__ __launch_bounds__(kBlock, 2) void density_tail_kernel(DensityStageArgs a)
 {
-    density_iterate<MFV, kTailLanes, true, kGridWalk>(a, a.tail_list, a.n_tail, nullptr);
+    __shared__ int row_lds[kRowLds<kTailLanes>];
+    density_iterate<MFV, kTailLanes, true, kGridWalk>(a, a.tail_list, a.n_tail, nullptr, row_lds);
 }
 
 template <bool MFV>
-__global__ __launch_bounds__(kBlock) void density_far_kernel(DensityStageArgs a)
+__global__ __launch_bounds__(kBlock, 2) void density_far_kernel(DensityStageArgs a)
 {
-    density_iterate<MFV, 64, false, kGridWalk>(a, a.far_list, a.n_far, nullptr);
+    __shared__ int row_lds[kRowLds<64>];
+    density_iterate<MFV, 64, false, kGridWalk>(a, a.far_list, a.n_far, nullptr, row_lds);
 }
 
 // Tree: what is left of the rows' sweeps, then the particles that have to walk, a
@@ -631,16 +730,16 @@ template <bool MFV>
 __global__ __launch_bounds__(64 * kFarWaves) void density_tree_far_kernel(DensityStageArgs a)
 {
     __shared__ BlockWalkLds<kFarWaves> walk;
-    density_iterate<MFV, 64, false, kTreeWalk, kFarWaves>(a, a.far_list, a.n_far, nullptr, &walk);
+    density_iterate<MFV, 64, false, kTreeWalk, kFarWaves>(a, a.far_list, a.n_far, nullptr, nullptr, &walk);
 }
 
-// no rows: every active particle starts in the tail list
+// no rows: where every active particle starts; the tree's in the walk list
 __global__ void density_list_all_kernel(DensityStageArgs a)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= a.n_active) return;
     const int i = a.active[t];
-    if (!(a.posm[i].w > 0)) return;
+    if (!(a.posm[i].w > 0)) return;  // density_isactive: gas with mass > 0 (density.c:85)
     double h = a.hsml[i];
     if ((h < 0) || !isfinite(h) || (h > 0.99 * a.hp.max_hsml)) h = 0.99 * a.hp.max_hsml;  // density.c:484
     const Iterate s = {h, 0, 0, a.cn[i], 0};
@@ -663,29 +762,25 @@ void launch_density_rows(hipStream_t s, const DensityStageArgs &a)
         hipLaunchKernelGGL(density_rows_kernel<1>, dim3(nblocks(a.n_active)), block, 0, s, a);
 }
 
-template <int G>
-static void launch_stage_lanes(hipStream_t s, const DensityStageArgs &a)
+template <int G, int IT>
+static void launch_stage_sweep(hipStream_t s, const DensityStageArgs &a)
 {
     const dim3 grid(nblocks((long long)G * a.n_active)), block(kBlock);
-    if (a.pvel) {
-        hipLaunchKernelGGL((density_stage_kernel<true, G, 0>), grid, block, 0, s, a);
-        hipLaunchKernelGGL((density_stage_kernel<true, G, 1>), grid, block, 0, s, a);
-    } else {
-        hipLaunchKernelGGL((density_stage_kernel<false, G, 0>), grid, block, 0, s, a);
-        hipLaunchKernelGGL((density_stage_kernel<false, G, 1>), grid, block, 0, s, a);
-    }
+    if (a.pvel) hipLaunchKernelGGL((density_stage_kernel<true, G, IT>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((density_stage_kernel<false, G, IT>), grid, block, 0, s, a);
 }
 
 void launch_density_stage(hipStream_t s, const DensityStageArgs &a)
 {
     if (a.n_active <= 0) return;
-    const dim3 block(kBlock);
     if (!a.row_idx) {
-        hipLaunchKernelGGL(density_list_all_kernel, dim3(nblocks(a.n_active)), block, 0, s, a);
+        hipLaunchKernelGGL(density_list_all_kernel, dim3(nblocks(a.n_active)), dim3(kBlock), 0, s, a);
     } else if (a.lanes == 8) {
-        launch_stage_lanes<8>(s, a);
+        launch_stage_sweep<8, 0>(s, a);
+        launch_stage_sweep<8, 1>(s, a);
     } else {
-        launch_stage_lanes<1>(s, a);
+        launch_stage_sweep<1, 0>(s, a);
+        launch_stage_sweep<1, 1>(s, a);
     }
 }
 
@@ -696,14 +791,35 @@ static void launch_tree_tail(hipStream_t s, const DensityStageArgs &a)
     const dim3 block(kBlock);
     if (a.row_idx) {
         const dim3 grid(nblocks((long long)a.lanes * a.n_active / 2 + a.lanes));
-        if (a.lanes == 8) hipLaunchKernelGGL((density_more_kernel<MFV, 8>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((density_more_kernel<MFV, 1>), grid, block, 0, s, a);
+        if (a.lanes == 8) hipLaunchKernelGGL((density_more_kernel<MFV, 8, false>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((density_more_kernel<MFV, 1, false>), grid, block, 0, s, a);
         hipLaunchKernelGGL(density_tree_tail_kernel<MFV>, dim3(std::min(2048u, nblocks((long long)kTailLanes * a.n_active))),
                            block, 0, s, a);
     }
     hipLaunchKernelGGL(density_tree_walk_kernel<MFV>, dim3(std::min(2048u, nblocks(64LL * a.n_active))), block, 0, s, a);
     if (a.budget)
         hipLaunchKernelGGL(density_tree_far_kernel<MFV>, dim3(std::min(512, a.n_active)), dim3(64 * kFarWaves), 0, s, a);
+}
+
+template <bool MFV>
+static void launch_grid_tail(hipStream_t s, const DensityStageArgs &a)
+{
+    // the counts are on the device: enough workgroups to fill the chip, at most one group per particle
+    const dim3 block(kBlock), waves(std::min(2048u, nblocks(64LL * a.n_active)));
+    if (a.lanes == 8) {
+        // few particles: the whole tail with a wavefront each, in one launch (a nearly
+        // empty tail of 32 k particles: 5.1 us against 4.1 + 3.5 and the gap between)
+        DensityStageArgs b = a;
+        b.far_list = a.tail_list;
+        b.n_far = a.n_tail;
+        hipLaunchKernelGGL(density_far_kernel<MFV>, waves, block, 0, s, b);
+        return;
+    }
+    if (!a.walk_list)
+        hipLaunchKernelGGL((density_more_kernel<MFV, 1, true>), dim3(nblocks((long long)a.n_active / 2 + 1)), block, 0, s, a);
+    hipLaunchKernelGGL(density_tail_kernel<MFV>, dim3(std::min(2048u, nblocks((long long)kTailLanes * a.n_active))), block, 0,
+                       s, a);
+    if (a.budget) hipLaunchKernelGGL(density_far_kernel<MFV>, waves, block, 0, s, a);
 }
 
 void launch_density_tail(hipStream_t s, const DensityStageArgs &a)
@@ -714,25 +830,8 @@ void launch_density_tail(hipStream_t s, const DensityStageArgs &a)
         else launch_tree_tail<false>(s, a);
         return;
     }
-    // the counts are on the device: enough workgroups to fill the chip, at most one group per particle
-    if (a.lanes == 8) {
-        // few particles: the whole tail with a wavefront each, in one launch (a nearly
-        // empty tail of 32 k particles: 5.1 us against 4.1 + 3.5 and the gap between)
-        DensityStageArgs b = a;
-        b.far_list = a.tail_list;
-        b.n_far = a.n_tail;
-        const dim3 waves(std::min(2048u, nblocks(64LL * a.n_active)));
-        if (a.pvel) hipLaunchKernelGGL(density_far_kernel<true>, waves, dim3(kBlock), 0, s, b);
-        else hipLaunchKernelGGL(density_far_kernel<false>, waves, dim3(kBlock), 0, s, b);
-        return;
-    }
-    const dim3 grid(std::min(2048u, nblocks((long long)kTailLanes * a.n_active))), block(kBlock);
-    if (a.pvel) hipLaunchKernelGGL(density_tail_kernel<true>, grid, block, 0, s, a);
-    else hipLaunchKernelGGL(density_tail_kernel<false>, grid, block, 0, s, a);
-    if (!a.budget) return;
-    const dim3 far(std::min(2048u, nblocks(64LL * a.n_active)));
-    if (a.pvel) hipLaunchKernelGGL(density_far_kernel<true>, far, block, 0, s, a);
-    else hipLaunchKernelGGL(density_far_kernel<false>, far, block, 0, s, a);
+    if (a.pvel) launch_grid_tail<true>(s, a);
+    else launch_grid_tail<false>(s, a);
 }
 
 }  // namespace gzm
