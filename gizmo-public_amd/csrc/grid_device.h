@@ -241,6 +241,7 @@ __device__ __forceinline__ int for_columns(const Grid &g, const double xs[3], do
             for (int z = 0; z < n[2]; z++) {
                 const int2 next = slots(lo[2] + z + 1);  // under way while this cell is tested
                 seen += r.y - r.x;
+                if (seen > limit) break;
                 for (int j = r.x; j < r.y; j += 4) {
                     bool in[4];
 #pragma unroll

@@ -729,6 +729,17 @@ gzm_status gzm_ctx_destroy(gzm_ctx *c)
 
 namespace {
 
+// Grid: whether the expected entries of a candidate row stay within its cap.  Above that
+// nearly every particle walks, over more candidates than a lane is given, so neither rows
+// nor the packed sweeps of a lane each are of use (68,921 particles of 128 neighbours,
+// density: 8.4 ms with both, 3.2 with rows tried, 2.85 with 16 lanes and more from the start;
+// of 80: 1.75 and 1.25).
+bool grid_rows_fit(const gzm_ctx *c)
+{
+    const double f = kDensityCacheFactorGrid;
+    return f * f * f * c->p.des_num_ngb <= kDensityCacheCap;
+}
+
 // Per-box grids, the global cell-range array and the hmax tiles of an upload.
 gzm_status setup_boxes(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const double *box_sizes,
                        const int64_t *offsets)
@@ -911,7 +922,7 @@ gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const 
             s = s ? s : dev_alloc(&c->d_bwave_n, 2);
         }
         if (s) { free_particles(c); return s; }
-        if (c->p.precision != 2) {
+        if (c->p.precision != 2 && (c->p.search == 1 || grid_rows_fit(c))) {
             if (dev_alloc(&c->d_dcache_idx, (size_t)n * kDensityCacheCap) || dev_alloc(&c->d_dcache_n, n) ||
                 dev_alloc(&c->d_dcache_r2, n) || (c->p.search == 0 && dev_alloc(&c->d_posf, n)))
                 free_rows(c);
@@ -1134,7 +1145,9 @@ DensityStageArgs density_stage_args(gzm_ctx *c)
     a.num_ngb = c->d_num_ngb; a.dhsml = c->d_dhsml; a.divvel = c->d_divvel; a.rho = c->d_rho; a.pres = c->d_pres;
     a.fce = c->d_fce; a.nvt = c->d_nvt;
     a.pvel = (c->p.method == 1) ? c->d_pvel : nullptr;
-    a.row_idx = c->d_dcache_idx; a.row_n = c->d_dcache_n; a.row_r2 = c->d_dcache_r2;
+    if (c->tree.nodes || grid_rows_fit(c)) {
+        a.row_idx = c->d_dcache_idx; a.row_n = c->d_dcache_n; a.row_r2 = c->d_dcache_r2;
+    }
     a.iter = c->d_iter;
     a.tail_list = c->d_live;
     a.n_tail = c->d_count + 1;
@@ -1142,7 +1155,7 @@ DensityStageArgs density_stage_args(gzm_ctx *c)
     a.n_far = c->d_count + 2;
     const bool tree = c->tree.nodes != nullptr;
     const bool few = c->n_active <= kFewParticles;
-    a.walk_list = tree ? c->d_bwave : (few ? a.tail_list : nullptr);
+    a.walk_list = tree ? c->d_bwave : (few || !grid_rows_fit(c) ? a.tail_list : nullptr);
     a.n_walk = tree ? c->d_count + 3 : a.n_tail;
     a.budget = c->p.density_budget == 0 ? kDensityBudget : (c->p.density_budget < 0 ? 0 : c->p.density_budget);
     a.lanes = few ? 8 : 1;

@@ -218,6 +218,21 @@ __device__ __forceinline__ double grid_row_r2(double h)
     const double Rc = kDensityCacheFactorGrid * h;
     return Rc * Rc;
 }
+// Whether to build a particle's row (of n_row entries in the radius^2 r2 tried last)
+// anew for hsml h: it left the row, or there was none and it is now so much smaller that
+// half the entries are left.
+__device__ __forceinline__ bool row_wanted(int n_row, double r2, double h)
+{
+    return n_row <= kDensityCacheCap ? h * h > r2 : grid_row_r2(h) < 0.64 * r2;
+}
+// whether a walk of radius h passes more cells than one lane should
+__device__ __forceinline__ bool many_cells(const Grid &g, double h)
+{
+    double cells = 1;
+#pragma unroll
+    for (int ax = 0; ax < 3; ax++) cells *= fmin((double)g.nc[ax], 2 * h * g.inv_s[ax] + 1);
+    return cells > 512;
+}
 template <int G>
 constexpr int kRowLds = G == 1 ? kListChunk * kBlock : kColumnHits * kBlock;
 template <int G>
@@ -289,7 +304,8 @@ __device__ __forceinline__ int grid_row(const DensityStageArgs &a, const BoxDesc
     };
     bool listed = false;
     if constexpr (G > 1) {
-        m = for_columns<G>(B.grid, xs, Rc, sub, limit, kept + threadIdx.x,
+        // (a column with that many candidates is better shared by many lanes)
+        m = for_columns<G>(B.grid, xs, Rc, sub, G > 8 ? min(limit, 4 * kColumnHits) : limit, kept + threadIdx.x,
                            [&](int j, bool whole, int cx, int cy, int cz) {
             return near(a.posf[j], whole, cx, cy, cz);
         }, [&](int k, int j) {
@@ -494,21 +510,25 @@ __device__ __forceinline__ int walk_sweep(const DensityStageArgs &a, const BoxDe
 // (of 250 k in Plummer spheres 196 k need 2.6 more on average, up to 10).  A
 // workgroup takes a stretch of the active particles and packs those not converged
 // anew for every sweep, so that its wavefronts stay full and keep neighbouring
-// particles together; the last few go to the tail list.  The 250 k: 0.50 ms
+// particles together; the last few (the last quarter in the grid: a random state of 61^3
+// has 14 % left, density 0.54 ms, with a sixteenth 0.60) go to the tail list.  The 250 k: 0.50 ms
 // (stretches of 256 or 1024: 0.67), against 2.0 ms with 16 lanes each to convergence
 // and 3.3 ms in four launches over lists whose order the atomics left.
 // Tree: a particle whose hsml leaves its row goes to the walk list.  Grid (GRID):
 // its row is built anew around the hsml reached, and where that is past the cap (a
 // guess far above) or the memory holds no rows, the sweep walks; a walk past the
-// candidate budget is done by a wavefront.  With the 16 lanes of the tail walking for
+// candidate budget is done by a wavefront.  Where already the walk for a row passed two
+// budgets (cells far wider than hsml, in clumps) or has many cells to pass (far smaller
+// ones, between clumps) the far list takes the particle: such walks come thousands to a
+// stretch and have to spread over the chip.  With the 16 lanes of the tail walking for
 // them, sweep by sweep, the density stage of a 128^3 lattice whose hsml starts 20 %
-// low took 35.3 ms, 50 % high 89.6; now 6.6 and 34.7 (a launch per sweep with a lane
+// low took 35.3 ms, 50 % high 89.6; now 6.7 and 38.0 (a launch per sweep with a lane
 // each and no rows: 7.8 and 39.1).  A well guessed 128^3 blast pays 31 us of 10.7 ms
 // (stretches of 1024 22 us, but 61^3 20 % low 1.1 against 0.6 ms).
 template <bool MFV, int G, bool GRID>
 __global__ __launch_bounds__(kBlock, 2) void density_more_kernel(DensityStageArgs a)
 {
-    constexpr int kStretch = 2 * kBlock / G, kFew = kStretch / 16;
+    constexpr int kStretch = 2 * kBlock / G, kFew = kStretch / (GRID ? 4 : 16);
     constexpr int kLists = GRID ? 3 : 2;  // live ones of this sweep and the next, walks past the budget
     __shared__ __align__(16) int lds[GRID ? kRowLds<G> : (G == 1 ? kListChunk * kBlock : 1)];
     __shared__ int live[kLists][kStretch];
@@ -560,17 +580,21 @@ __global__ __launch_bounds__(kBlock, 2) void density_more_kernel(DensityStageArg
                 Iterate s = take_up(a, i);
                 const double4 pi = a.posm[i];
                 int n_row = a.row_idx ? a.row_n[i] : kNoRow, again = -1;
-                // (before the first sweep the row is the one tried for this hsml)
-                if (GRID && a.row_idx && s.iter > 0 && !(n_row <= kDensityCacheCap && s.h * s.h <= a.row_r2[i])) {
-                    n_row = grid_row<G>(a, B, i, pi, s.h, sub, lds);
+                if (GRID) {
+                    const bool wanted = a.row_idx && row_wanted(n_row, a.row_r2[i], s.h);
+                    if ((wanted || n_row > kDensityCacheCap) && many_cells(B.grid, s.h)) n_row = kWideRow;
+                    else if (wanted) n_row = grid_row<G>(a, B, i, pi, s.h, sub, lds);
                 }
                 if (!GRID || n_row <= kDensityCacheCap)
                     again = row_sweep<MFV, G>(a, B, i, pi, n_row, sub, chunk, s, cnt);
                 else if (n_row != kWideRow)
                     again = walk_sweep<MFV, G>(a, B, i, pi, sub, s, cnt);
                 if (sub != 0) return;
-                wide = again < 0;
-                if (wide) return;
+                if (again < 0) {
+                    wide = n_row != kWideRow;
+                    if (!wide) a.far_list[atomicAdd(a.n_far, 1)] = i;
+                    return;
+                }
                 sweeps++;
                 max_iter = s.iter > max_iter ? s.iter : max_iter;
                 stays = again == 1 && (GRID || s.h * s.h <= a.row_r2[i]);
@@ -624,16 +648,16 @@ __device__ __forceinline__ void density_iterate(const DensityStageArgs &a, const
         const double4 vi = a.velu[i];
         Iterate s = take_up(a, i);
         int n_row = a.row_n ? a.row_n[i] : kNoRow;
-        double Rc2 = n_row <= kDensityCacheCap ? a.row_r2[i] : -1.0;
+        double tried = a.row_n ? a.row_r2[i] : 0.0, Rc2 = n_row <= kDensityCacheCap ? tried : -1.0;
         const double xs[3] = {pi.x, pi.y, pi.z};
         bool again = true, far = false;
         while (again) {
             const double h2 = s.h * s.h;
-            // (before the first sweep the row is the one tried for this hsml)
-            if (WALK == kGridWalk && a.row_n && s.iter > 0 && !(h2 <= Rc2)) {
+            if (WALK == kGridWalk && a.row_n && row_wanted(n_row, tried, s.h)) {
                 n_row = grid_row<W>(a, B, i, pi, s.h, sub, row_lds);
                 wave_lds_fence();  // the other lanes' entries
-                Rc2 = n_row <= kDensityCacheCap ? grid_row_r2(s.h) : -1.0;
+                tried = grid_row_r2(s.h);
+                Rc2 = n_row <= kDensityCacheCap ? tried : -1.0;
             }
             double hinv, hinv3, hinv4;
             kernel_hinv(s.h, hinv, hinv3, hinv4);

@@ -40,6 +40,22 @@ def test_poor_guess_of_hsml(side, guess, method):
         assert not bad, (cell, bad)
 
 
+@pytest.mark.parametrize("des", [60, 80, 130])
+@pytest.mark.parametrize("side", [14, 41])
+def test_more_neighbours_than_a_row_holds(side, des):
+    """60: some rows past their cap of 96; 80: none tried; 130: walks past the
+    candidate budget."""
+    ic = ics.random_state(side)
+    ic["hsml"] = ic["hsml"] * (des / 32.0) ** (1 / 3)
+    ref, st, _ = O.run_pass(ic, O.make_params(des_num_ngb=des), stages=STAGES)
+    out, gst = gzm.run_pass(ic, params=gzm.make_params(des_num_ngb=des), stages=STAGES)
+    assert gst["density_sweeps"] == st.iterations
+    assert gst["density_interactions"] == st.dens_interactions
+    assert gst["gradient_interactions"] == st.grad_interactions
+    errs, bad = check_pass(out, ref)
+    assert not bad, bad
+
+
 def density_ms(ic, passes=5):
     with gzm.MFMContext(gzm.make_params()) as ctx:
         ctx.upload(ic)
