@@ -1012,6 +1012,52 @@ __device__ __forceinline__ void force_final_ops(double acc[3], double &dte, cons
     if (h_i >= 0.99 * max_hsml) dte = 0;
 }
 
+// The sums of the list kernels' kForceLanes lanes kept by one lane for the forms
+// without them, added up in their order (group_sum's), so that all forms give the
+// same bits.  In LDS, part_bytes(threads) of it: an array indexed by the pair's
+// number lies in scratch memory, 256 bytes a lane.
+struct LaneSums {
+    double *at;  // [lane][component][thread]
+    int stride;
+    __device__ __forceinline__ LaneSums(double *lds) : at(lds + threadIdx.x), stride((int)blockDim.x)
+    {
+#pragma unroll
+        for (int k = 0; k < 4 * kForceLanes; k++) at[k * stride] = 0;
+    }
+    __device__ __forceinline__ void add(int lane, const double v[4])
+    {
+#pragma unroll
+        for (int c = 0; c < 4; c++) at[(4 * lane + c) * stride] += v[c];
+    }
+    __device__ __forceinline__ void fold()
+    {
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            double v[kForceLanes];
+#pragma unroll
+            for (int l = 0; l < kForceLanes; l++) v[l] = at[(4 * l + c) * stride];
+#pragma unroll
+            for (int off = kForceLanes / 2; off > 0; off >>= 1)
+#pragma unroll
+                for (int l = 0; l < off; l++) v[l] += v[l + off];
+            at[c * stride] = v[0];
+        }
+    }
+    __device__ __forceinline__ double total(int c) const { return at[c * stride]; }
+};
+// one sum, with the same face
+struct OwnSums {
+    double v[4] = {0, 0, 0, 0};
+    __device__ __forceinline__ OwnSums(double *) {}
+    __device__ __forceinline__ void add(int, const double x[4])
+    {
+#pragma unroll
+        for (int c = 0; c < 4; c++) v[c] += x[c];
+    }
+    __device__ __forceinline__ double total(int c) const { return v[c]; }
+};
+inline size_t part_bytes(unsigned threads) { return sizeof(double) * 4 * kForceLanes * threads; }
+
 // this workgroup's copy of a stage's counters
 __device__ __forceinline__ Counters *ctr_slot(Counters *c) { return c + (blockIdx.x & (kCtrSpread - 1)); }
 

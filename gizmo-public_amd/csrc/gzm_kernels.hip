@@ -985,6 +985,7 @@ __global__ __launch_bounds__(64, 2) void force_list_kernel(ForceArgs a)
 template <bool USE_LIST>
 __global__ __launch_bounds__(kBlock) void force_kernel(ForceArgs a)
 {
+    extern __shared__ double part_lds[];
     const int t = xcd_block() * (int)blockDim.x + threadIdx.x;
     bool valid = t < a.n_active;
     if (USE_LIST && valid && a.list.count[t] > a.list.cap) valid = false;
@@ -1002,14 +1003,13 @@ __global__ __launch_bounds__(kBlock) void force_kernel(ForceArgs a)
             ROut<double> ro = {0, 0, {0, 0, 0}, 0};
             const double h2_i = I.h * I.h;
             int n_deferred = 0, k_pair = 0;
-            // the sums of force_list_kernel's lanes, added up in its order
-            double part[kForceLanes][4] = {};
-            auto add = [&](double *sum, int j, const double Fv[3], double Fp, double vsig, int mask, int e) {
+            LaneSums part(part_lds);
+            auto add = [&](int lane, int j, const double Fv[3], double Fp, double vsig, int mask, int e) {
                 if (e > status) status = e;
                 nretry += (mask & 8) ? 1 : 0;
                 nexact += (mask & 4) ? 1 : 0;
-                for (int c = 0; c < 3; c++) sum[c] += Fv[c];
-                sum[3] += Fp;
+                const double v[4] = {Fv[0], Fv[1], Fv[2], Fp};
+                part.add(lane, v);
                 if (vsig > out_vsig) out_vsig = vsig;
                 if (a.is_active && !a.is_active[j]) {
                     if (vsig > kWakeup * a.vsig_old[j]) a.wakeup[j] = 1;  // WAKEUP (hydro_evaluate.h:485-495)
@@ -1037,17 +1037,15 @@ __global__ __launch_bounds__(kBlock) void force_kernel(ForceArgs a)
                         n_deferred++;
                         return;
                     }
-                    add(part[k % kForceLanes], j, Fv, Fp, vsig, mask, e);
+                    add(k % kForceLanes, j, Fv, Fp, vsig, mask, e);
                 } else if (e == kDeferred) {
                     const int e2 = force_pair<double, false>(I, J, dp, r2, a.G, ro, Fv, Fp, vsig, mask);
-                    add(part[0], j, Fv, Fp, vsig, mask, e2);
+                    add(0, j, Fv, Fp, vsig, mask, e2);
                 }
             };
             for (int pass = 0; pass < 2; pass++) {
                 if (pass == 1) {
-                    for (int off = kForceLanes / 2; off > 0; off >>= 1)
-                        for (int l = 0; l < off; l++)
-                            for (int c = 0; c < 4; c++) part[l][c] += part[l + off][c];
+                    part.fold();
                     if (n_deferred == 0) break;
                 }
                 if (USE_LIST) {
@@ -1060,8 +1058,8 @@ __global__ __launch_bounds__(kBlock) void force_kernel(ForceArgs a)
                     for_each_neighbour_candidate(a.tree, G, x_i, I.h, true, [&](int j) { visit(j, true, pass); });
                 }
             }
-            for (int c = 0; c < 3; c++) acc[c] = part[0][c];
-            dte = part[0][3];
+            for (int c = 0; c < 3; c++) acc[c] = part.total(c);
+            dte = part.total(3);
             if (vmax < out_vsig) vmax = out_vsig;
             force_final_ops(acc, dte, I.v, m_i, I.h, a.max_hsml);
         } else if (m_i > 0) {
@@ -1346,8 +1344,8 @@ void launch_force(hipStream_t s, const ForceArgs &a)
     const dim3 grid(nblocks(a.n_active, b)), block(b);
     if (a.list.idx && a.defer.mask)
         hipLaunchKernelGGL(force_list_kernel, dim3(nblocks((long long)kForceLanes * a.n_active, 64)), dim3(64), 0, s, a);
-    else if (a.list.idx) hipLaunchKernelGGL(force_kernel<true>, grid, block, 0, s, a);
-    else hipLaunchKernelGGL(force_kernel<false>, grid, block, 0, s, a);
+    else if (a.list.idx) hipLaunchKernelGGL(force_kernel<true>, grid, block, part_bytes(b), s, a);
+    else hipLaunchKernelGGL(force_kernel<false>, grid, block, part_bytes(b), s, a);
 }
 namespace {
 

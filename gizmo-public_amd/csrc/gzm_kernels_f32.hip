@@ -661,13 +661,19 @@ __device__ __forceinline__ void mark_redo(const ForceArgs &a, int i, int j)
 // overflowed it are left to force_wave_fp64_kernel); otherwise (no list) scan
 // the grid or tree with the same banded predicate as the gradient kernel.  Exact-solver pairs are summed
 // after the others, by force_deferred_f32_kernel + force_finish_kernel
-// (THREE_PHASE) or by a second walk over the pairs, as in the FP64 kernel.
+// (THREE_PHASE) or by a second walk over the pairs, a launch of its own (AGAIN) over
+// the particles that have any, which the first leaves marked by the sign of vsig:
+// in one kernel the second walk's registers cost the first its second wave on a SIMD
+// (226,981 particles, tree without lists: 27.3 ms with the sums in scratch, 27.4 with
+// them in LDS, 13.7 in two launches; lists of 128: 2.22, 2.15, 1.39).
 // Lists take kForceLanes lanes per particle, as in FP64 (pair_list_loop); the
 // FP32 records stay in registers, 158 of them.  3.55 M particles: 3.96 ms against
 // 4.03 ms with one lane each.
-template <bool USE_LIST, bool THREE_PHASE, bool TREE = false>
+template <bool USE_LIST, bool THREE_PHASE, bool TREE = false, bool AGAIN = false>
 __global__ __launch_bounds__((USE_LIST && THREE_PHASE) ? kMaxBlock : kBlock) void force_f32_kernel(ForceArgs a)
 {
+    constexpr bool IN_PARTS = !THREE_PHASE && !AGAIN;
+    extern __shared__ double part_lds[];  // with IN_PARTS
     constexpr int LANES = (USE_LIST && THREE_PHASE) ? kForceLanes : 1;
     const int gt = xcd_block() * (int)blockDim.x + (int)threadIdx.x;
     const int t = gt / LANES, sub = gt % LANES;
@@ -684,6 +690,7 @@ __global__ __launch_bounds__((USE_LIST && THREE_PHASE) ? kMaxBlock : kBlock) voi
     unsigned long long cnt = 0, nretry = 0, nexact = 0;
     for_box(a.boxes, a.box_of, valid ? a.active[t] : 0, valid, [&](const BoxDesc &G) {
         const int i = a.active[t];
+        if (AGAIN && !signbit(a.vsig[i])) return;
         const ForceRecF ri = a.recf[i];
         const double4 pi = a.posm[i];
         double acc[3] = {0, 0, 0}, dte = 0, vmax = kMinReal;
@@ -698,25 +705,34 @@ __global__ __launch_bounds__((USE_LIST && THREE_PHASE) ? kMaxBlock : kBlock) voi
             double out_vsig = I.cs;
             ROut<float> ro = {0, 0, {0, 0, 0}, 0};
             int n_deferred = 0, k_pair = 0;
-            // one lane per particle: the sums of the list form's lanes, added up in its order
-            double part[THREE_PHASE ? 1 : kForceLanes][4] = {};
-            auto add = [&](double *sum, int j, const float Fv[3], float Fp, float vsig, int mask, int e) {
+            std::conditional_t<IN_PARTS, LaneSums, OwnSums> part(part_lds);
+            if (AGAIN) {
+                const double v[4] = {a.acc[3 * (size_t)i + 0], a.acc[3 * (size_t)i + 1], a.acc[3 * (size_t)i + 2], a.dtu[i]};
+                part.add(0, v);
+                out_vsig = fabs(a.vsig[i]);
+            }
+            auto add = [&](int lane, int j, const float Fv[3], float Fp, float vsig, int mask, int e) {
                 if (e > status) status = e;
                 nretry += (mask & 8) ? 1 : 0;
                 nexact += (mask & 4) ? 1 : 0;
-                for (int c = 0; c < 3; c++) sum[c] += (double)Fv[c];
-                sum[3] += (double)Fp;
+                const double v[4] = {(double)Fv[0], (double)Fv[1], (double)Fv[2], (double)Fp};
+                part.add(lane, v);
                 if ((double)vsig > out_vsig) out_vsig = vsig;
                 if (a.is_active && !a.is_active[j]) {
                     if ((double)vsig > kWakeup * a.vsig_old[j]) a.wakeup[j] = 1;  // WAKEUP (hydro_evaluate.h:485-495)
                 }
             };
-            // pass 0: every pair but the deferred ones; pass 1: only those
-            auto eval = [&](int j, int k, const PairSide<float> &J, const float dp[3], float r2, int pass) {
+            // every pair but the deferred ones, or only those
+            auto eval = [&](int j, int k, const PairSide<float> &J, const float dp[3], float r2) {
                 float Fv[3], Fp, vsig;
                 int mask;
                 const int e = force_pair<float, true>(I, J, dp, r2, a.G, ro, Fv, Fp, vsig, mask);
-                if (pass == 0) {
+                if constexpr (AGAIN) {
+                    if (e != kDeferred) return;
+                    const int e2 = force_pair<float, false, true>(I, J, dp, r2, a.G, ro, Fv, Fp, vsig, mask);
+                    if (e2 == kNearThreshold) mark_redo(a, i, j);
+                    else add(0, j, Fv, Fp, vsig, mask, e2);
+                } else {
                     cnt++;
                     const int k_part = k_pair++;
                     if (e == kDeferred) {
@@ -724,11 +740,7 @@ __global__ __launch_bounds__((USE_LIST && THREE_PHASE) ? kMaxBlock : kBlock) voi
                         n_deferred++;
                         return;
                     }
-                    add(part[THREE_PHASE ? 0 : k_part % kForceLanes], j, Fv, Fp, vsig, mask, e);
-                } else if (!THREE_PHASE && e == kDeferred) {
-                    const int e2 = force_pair<float, false>(I, J, dp, r2, a.G, ro, Fv, Fp, vsig, mask);
-                    if (e2 == kNearThreshold) mark_redo(a, i, j);
-                    else add(part[0], j, Fv, Fp, vsig, mask, e2);
+                    add(k_part % kForceLanes, j, Fv, Fp, vsig, mask, e);
                 }
             };
             const double h_i = a.hsml[i];
@@ -739,85 +751,77 @@ __global__ __launch_bounds__((USE_LIST && THREE_PHASE) ? kMaxBlock : kBlock) voi
             const double R = (h_i > G.hmax) ? h_i : G.hmax;
             const bool exact_geom_list = a.tree.nodes != nullptr || list_needs_exact_geom(G);
             const float smax = smax_of(G);
-            for (int pass = 0; pass < 2; pass++) {
-                if (pass == 1) {
-                    if (!THREE_PHASE)
-                        for (int off = kForceLanes / 2; off > 0; off >>= 1)
-                            for (int l = 0; l < off; l++)
-                                for (int c = 0; c < 4; c++) part[l][c] += part[l + off][c];
-                    if (THREE_PHASE || n_deferred == 0) break;
+            if (USE_LIST) {
+                const int n = a.list.count[t];
+                const int *row = a.list.idx + (size_t)t * a.list.cap;
+                for (int k = sub; k < n; k += LANES) {
+                    const int j = row[k];
+                    const ForceRecF &Jr = a.recf[j];
+                    PairSide<float> J;
+                    unpack_side_f(Jr, J);
+                    float dp[3];
+                    list_dp(G, exact_geom_list, ri, ci, pi, Jr, a.posm, j, dp);
+                    const float r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
+                    eval(j, k, J, dp, r2);
                 }
-                if (USE_LIST) {
-                    const int n = a.list.count[t];
-                    const int *row = a.list.idx + (size_t)t * a.list.cap;
-                    for (int k = sub; k < n; k += LANES) {
-                        const int j = row[k];
-                        const ForceRecF &Jr = a.recf[j];
-                        PairSide<float> J;
-                        unpack_side_f(Jr, J);
-                        float dp[3];
-                        list_dp(G, exact_geom_list, ri, ci, pi, Jr, a.posm, j, dp);
-                        const float r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
-                        eval(j, k, J, dp, r2, pass);
-                    }
-                } else {
-                    auto visit = [&](int j, float sh0, float sh1, float sh2, bool exact_geom) {
-                        if (j == i) return;
-                        const float4 xj = a.recf[j].xh;
-                        const float hj2 = xj.w * xj.w;
-                        float dp[3];
-                        float r2;
-                        int in_i, in_j, pos;
-                        if (!exact_geom && !(fminf(ri.xh.w, xj.w) * kFineCells < smax)) {
-                            dp[0] = sh0 + (ri.xh.x - xj.x);
-                            dp[1] = sh1 + (ri.xh.y - xj.y);
-                            dp[2] = sh2 + (ri.xh.z - xj.z);
-                            r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
-                            if ((r2 >= bi.hi) && (r2 >= hj2 * (1 + kBandF))) return;
-                            in_i = decide(r2, bi);
-                            in_j = decide(r2, Band{hj2 * (1 - kBandF), hj2 * (1 + kBandF)});
-                            pos = (r2 >= pos_min) ? 1 : -1;
-                            if ((in_i < 0) || (in_j < 0) || (pos < 0)) {
-                                double d64[3];
-                                const double r2e = exact_r2(G.box, pi, a.posm[j], d64);
-                                const double h_j = a.hsml[j];
-                                in_i = r2e < h2_i;
-                                in_j = r2e < h_j * h_j;
-                                pos = r2e > 0;
-                            }
-                        } else {
+            } else {
+                auto visit = [&](int j, float sh0, float sh1, float sh2, bool exact_geom) {
+                    if (j == i) return;
+                    const float4 xj = a.recf[j].xh;
+                    const float hj2 = xj.w * xj.w;
+                    float dp[3];
+                    float r2;
+                    int in_i, in_j, pos;
+                    if (!exact_geom && !(fminf(ri.xh.w, xj.w) * kFineCells < smax)) {
+                        dp[0] = sh0 + (ri.xh.x - xj.x);
+                        dp[1] = sh1 + (ri.xh.y - xj.y);
+                        dp[2] = sh2 + (ri.xh.z - xj.z);
+                        r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
+                        if ((r2 >= bi.hi) && (r2 >= hj2 * (1 + kBandF))) return;
+                        in_i = decide(r2, bi);
+                        in_j = decide(r2, Band{hj2 * (1 - kBandF), hj2 * (1 + kBandF)});
+                        pos = (r2 >= pos_min) ? 1 : -1;
+                        if ((in_i < 0) || (in_j < 0) || (pos < 0)) {
                             double d64[3];
                             const double r2e = exact_r2(G.box, pi, a.posm[j], d64);
                             const double h_j = a.hsml[j];
                             in_i = r2e < h2_i;
                             in_j = r2e < h_j * h_j;
                             pos = r2e > 0;
-                            dp[0] = (float)d64[0]; dp[1] = (float)d64[1]; dp[2] = (float)d64[2];
-                            r2 = (float)r2e;
                         }
-                        if (!pos || (!in_i && !in_j)) return;
-                        const ForceRecF &Jr = a.recf[j];
-                        if (!(a.posm[j].w > 0) || !(Jr.th.x > 0)) return;  // hydro_evaluate.h:149-150
-                        PairSide<float> J;
-                        unpack_side_f(Jr, J);
-                        eval(j, 0, J, dp, r2, pass);
-                    };
-                    if (TREE) {
-                        tree_walk(a.tree, G, xs, h_i, true, [&](int j) { visit(j, 0.0f, 0.0f, 0.0f, true); });
                     } else {
-                        bool full[3];
-                        for_each_cell(G.grid, xs, R, full, [&](int cx, int cy, int cz, int beg, int end) {
-                            const bool exact_geom = full[0] || full[1] || full[2];
-                            const float sh0 = cell_shift(ci[0] - cx, G.s_f[0]);
-                            const float sh1 = cell_shift(ci[1] - cy, G.s_f[1]);
-                            const float sh2 = cell_shift(ci[2] - cz, G.s_f[2]);
-                            for (int j = beg; j < end; ++j) visit(j, sh0, sh1, sh2, exact_geom);
-                        }, h_i);
+                        double d64[3];
+                        const double r2e = exact_r2(G.box, pi, a.posm[j], d64);
+                        const double h_j = a.hsml[j];
+                        in_i = r2e < h2_i;
+                        in_j = r2e < h_j * h_j;
+                        pos = r2e > 0;
+                        dp[0] = (float)d64[0]; dp[1] = (float)d64[1]; dp[2] = (float)d64[2];
+                        r2 = (float)r2e;
                     }
+                    if (!pos || (!in_i && !in_j)) return;
+                    const ForceRecF &Jr = a.recf[j];
+                    if (!(a.posm[j].w > 0) || !(Jr.th.x > 0)) return;  // hydro_evaluate.h:149-150
+                    PairSide<float> J;
+                    unpack_side_f(Jr, J);
+                    eval(j, 0, J, dp, r2);
+                };
+                if (TREE) {
+                    tree_walk(a.tree, G, xs, h_i, true, [&](int j) { visit(j, 0.0f, 0.0f, 0.0f, true); });
+                } else {
+                    bool full[3];
+                    for_each_cell(G.grid, xs, R, full, [&](int cx, int cy, int cz, int beg, int end) {
+                        const bool exact_geom = full[0] || full[1] || full[2];
+                        const float sh0 = cell_shift(ci[0] - cx, G.s_f[0]);
+                        const float sh1 = cell_shift(ci[1] - cy, G.s_f[1]);
+                        const float sh2 = cell_shift(ci[2] - cz, G.s_f[2]);
+                        for (int j = beg; j < end; ++j) visit(j, sh0, sh1, sh2, exact_geom);
+                    }, h_i);
                 }
             }
-            for (int c = 0; c < 3; c++) acc[c] = part[0][c];
-            dte = part[0][3];
+            if constexpr (IN_PARTS) part.fold();
+            for (int c = 0; c < 3; c++) acc[c] = part.total(c);
+            dte = part.total(3);
             if (THREE_PHASE) {
                 // raw sums: finished by force_finish_kernel after the deferred pairs
                 if (status) atomicMax(&ctr_slot(a.ctr)->status, status);
@@ -837,10 +841,14 @@ __global__ __launch_bounds__((USE_LIST && THREE_PHASE) ? kMaxBlock : kBlock) voi
                 a.defer.raw[t] = 1;
                 return;
             }
-            if (vmax < out_vsig) vmax = out_vsig;
-            const double4 v = a.velu[i];
-            const double vi[3] = {v.x, v.y, v.z};
-            force_final_ops(acc, dte, vi, m_i, h_i, a.max_hsml);
+            if (n_deferred > 0) {  // raw sums for the second walk
+                vmax = -fabs(out_vsig);  // the sign also of NaN
+            } else {
+                if (vmax < out_vsig) vmax = out_vsig;
+                const double4 v = a.velu[i];
+                const double vi[3] = {v.x, v.y, v.z};
+                force_final_ops(acc, dte, vi, m_i, h_i, a.max_hsml);
+            }
         } else if (m_i > 0) {
             dte /= m_i;
         }
@@ -1186,6 +1194,12 @@ void launch_pack_force_f32(hipStream_t s, int n, const float4 *offm, const float
         hipLaunchKernelGGL(pack_force_f32_kernel, dim3(nblocks(n)), dim3(kBlock), 0, s, n, offm, velf, cellc, posm, hsml,
                            rho, pres, dhsml, cn, fce, nvt, grad, gamma, rec);
 }
+template <bool USE_LIST, bool TREE>
+static void launch_force_walks_f32(hipStream_t s, const ForceArgs &a, dim3 grid, dim3 block)
+{
+    hipLaunchKernelGGL((force_f32_kernel<USE_LIST, false, TREE, false>), grid, block, part_bytes(block.x), s, a);
+    hipLaunchKernelGGL((force_f32_kernel<USE_LIST, false, TREE, true>), grid, block, 0, s, a);
+}
 void launch_force_f32(hipStream_t s, const ForceArgs &a)
 {
     if (a.n_active <= 0) return;
@@ -1196,11 +1210,11 @@ void launch_force_f32(hipStream_t s, const ForceArgs &a)
         if (a.defer.mask)
             hipLaunchKernelGGL((force_f32_kernel<true, true>), dim3(nblocks((long long)kForceLanes * a.n_active, b)),
                                block, 0, s, a);
-        else hipLaunchKernelGGL((force_f32_kernel<true, false>), grid, block, 0, s, a);
+        else launch_force_walks_f32<true, false>(s, a, grid, block);
     } else if (a.tree.nodes) {
-        hipLaunchKernelGGL((force_f32_kernel<false, false, true>), grid, block, 0, s, a);
+        launch_force_walks_f32<false, true>(s, a, grid, block);
     } else {
-        hipLaunchKernelGGL((force_f32_kernel<false, false>), grid, block, 0, s, a);
+        launch_force_walks_f32<false, false>(s, a, grid, block);
     }
 }
 void launch_force_redo_fp64(hipStream_t s, const ForceArgs &a)
