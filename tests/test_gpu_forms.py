@@ -6,6 +6,8 @@ import pytest
 
 import gzm
 import ics
+import oracle as O
+from parity import check_pass
 
 pytestmark = pytest.mark.gpu
 
@@ -59,3 +61,25 @@ def test_fp32_force_without_lists_keeps_two_waves():
     ic = ics.random_state(61)
     kw = dict(precision=1, search=1)
     assert force_ms(gzm.make_params(pair_list_cap=-1, **kw), ic) < 45 * force_ms(gzm.make_params(**kw), ic)
+
+
+@pytest.mark.parametrize("cell_size", [0.02, 0.06, 0.3])
+def test_long_pair_sets_in_any_cells(cell_size):
+    """Lists of 16 leave nearly all particles to the wavefront loop: cells of less
+    than a particle, of one and of a hundred, more than 64 cells and fewer."""
+    ic = ics.random_state(13)
+    ref, st, _ = O.run_pass(ic)
+    out, gst = gzm.run_pass(ic, params=gzm.make_params(cell_size=cell_size, pair_list_cap=16))
+    assert gst["force_interactions"] == st.force_interactions
+    assert gst["exact_solver_calls"] == st.exact_solver_calls
+    errs, bad = check_pass(out, ref)
+    assert not bad, bad
+
+
+def test_long_pair_sets_in_dense_cells_cost_their_candidates():
+    """Plummer spheres, thousands of particles in a grid cell: the force stage takes
+    as long as with the tree; 100 times and more where a cell is tested anew for
+    each 64 pairs."""
+    ic = ics.plummer_clusters(32768, 50)
+    grid, tree = force_ms(gzm.make_params(), ic), force_ms(gzm.make_params(search=1), ic)
+    assert grid < 20 * tree
