@@ -1156,7 +1156,7 @@ DensityStageArgs density_stage_args(gzm_ctx *c)
     const bool tree = c->tree.nodes != nullptr;
     const bool few = c->n_active <= kFewParticles;
     a.walk_list = tree ? c->d_bwave : (few || !grid_rows_fit(c) ? a.tail_list : nullptr);
-    a.n_walk = tree ? c->d_count + 3 : a.n_tail;
+    a.n_walk = a.walk_list == a.tail_list ? a.n_tail : c->d_count + 3;
     a.budget = c->p.density_budget == 0 ? kDensityBudget : (c->p.density_budget < 0 ? 0 : c->p.density_budget);
     a.lanes = few ? 8 : 1;
     a.ctr = c->d_ctr + kCtrDensity * kCtrSpread;

@@ -37,7 +37,9 @@ constexpr int kTailLanes = 16;
 constexpr int kFarWaves = 4;
 constexpr int kNoRow = kDensityCacheCap + 1;
 constexpr int kWideRow = kNoRow + 1;  // row_n where the walk for the row passed twice the candidate budget
-constexpr int kDone = -1;  // iter of a particle whose iteration has ended
+// iter of a particle whose iteration has ended; beside the sweeps done, of one that is in
+// the tail list
+constexpr int kDone = -1, kListed = 1 << 30;
 
 // sums of one candidate already known to lie within h (density.c:252-347).
 // MFV: also m_j W_ij v_j into pv (density.c:291-293 for r = 0, 331-334 as
@@ -184,7 +186,7 @@ __device__ __forceinline__ void hand_on(const DensityStageArgs &a, int i, const 
 
 __device__ __forceinline__ Iterate take_up(const DensityStageArgs &a, int i)
 {
-    return {a.hsml[i], a.left[i], a.right[i], a.cn[i], a.iter[i]};
+    return {a.hsml[i], a.left[i], a.right[i], a.cn[i], a.iter[i] & ~kListed};
 }
 
 __device__ __forceinline__ void count_sweeps(const DensityStageArgs &a, unsigned long long pairs,
@@ -451,12 +453,16 @@ __global__ __launch_bounds__(kBlock, 3) void density_stage_kernel(DensityStageAr
     __shared__ __align__(16) int lds[G == 1 ? kListChunk * kBlock : 1];
     int *chunk = wave_chunk(lds);
     unsigned long long cnt = 0, sweeps = 0;
-    int max_iter = 0;
+    int max_iter = 0, left = -1;  // the particle, not done after IT = 1
+    const bool packed = G == 1 && IT == 1 && !a.walk_list;  // density_more_kernel follows in the grid
     for_box(a.boxes, a.box_of, valid ? a.active[t] : 0, valid, [&](const BoxDesc &B) {
         const int i = a.active[t];
         const double4 pi = a.posm[i];
         if (!(pi.w > 0)) return;
-        if (IT == 1 && a.iter[i] != 1) return;  // done, or without a usable row
+        if (IT == 1 && a.iter[i] != 1) {  // done, or without a usable row
+            if (a.iter[i] == 0) left = i;
+            return;
+        }
         Iterate s = {a.hsml[i], IT ? a.left[i] : 0.0, IT ? a.right[i] : 0.0, a.cn[i], IT};
         const int n = a.row_n[i];
         const double Rc2 = n <= kDensityCacheCap ? a.row_r2[i] : -1.0;
@@ -471,8 +477,25 @@ __global__ __launch_bounds__(kBlock, 3) void density_stage_kernel(DensityStageAr
             else if (IT == 0 && s.iter == 1) hand_on(a, i, s, nullptr, nullptr);
             else if (s.h * s.h <= Rc2 && a.tree.nodes) hand_on(a, i, s, nullptr, nullptr);
             else hand_on(a, i, s, a.walk_list, a.n_walk);
+            if (again) left = i;
         }
     });
+    if (packed) {
+        // up to a quarter of the wavefront goes to the tail list; more wait for density_more_kernel
+        const uint64_t bits = __ballot(left >= 0);
+        const int n = __popcll(bits), lane = (int)threadIdx.x & 63;
+        if (n > 16) {
+            if (lane == 0) *a.n_walk = 1;
+        } else if (n > 0) {
+            int base = 0;
+            if (lane == 0) base = atomicAdd(a.n_tail, n);
+            base = __shfl(base, 0, 64);
+            if (left >= 0) {
+                a.tail_list[base + __popcll(bits & ((1ull << lane) - 1))] = left;
+                a.iter[left] |= kListed;
+            }
+        }
+    }
     count_sweeps(a, cnt, sweeps, max_iter);
 }
 
@@ -510,8 +533,9 @@ __device__ __forceinline__ int walk_sweep(const DensityStageArgs &a, const BoxDe
 // (of 250 k in Plummer spheres 196 k need 2.6 more on average, up to 10).  A
 // workgroup takes a stretch of the active particles and packs those not converged
 // anew for every sweep, so that its wavefronts stay full and keep neighbouring
-// particles together; the last few (the last quarter in the grid: a random state of 61^3
-// has 14 % left, density 0.54 ms, with a sixteenth 0.60) go to the tail list.  The 250 k: 0.50 ms
+// particles together; the last few (in the grid the last quarter, and the second sweep's
+// wavefronts with as few left list them themselves: a random state of 61^3 has 14 % left,
+// density 0.54 ms, with a sixteenth 0.60) go to the tail list.  The 250 k: 0.50 ms
 // (stretches of 256 or 1024: 0.67), against 2.0 ms with 16 lanes each to convergence
 // and 3.3 ms in four launches over lists whose order the atomics left.
 // Tree: a particle whose hsml leaves its row goes to the walk list.  Grid (GRID):
@@ -523,13 +547,14 @@ __device__ __forceinline__ int walk_sweep(const DensityStageArgs &a, const BoxDe
 // stretch and have to spread over the chip.  With the 16 lanes of the tail walking for
 // them, sweep by sweep, the density stage of a 128^3 lattice whose hsml starts 20 %
 // low took 35.3 ms, 50 % high 89.6; now 6.7 and 38.0 (a launch per sweep with a lane
-// each and no rows: 7.8 and 39.1).  A well guessed 128^3 blast pays 31 us of 10.7 ms
-// (stretches of 1024 22 us, but 61^3 20 % low 1.1 against 0.6 ms).
+// each and no rows: 7.8 and 39.1).  A well guessed 128^3 blast pays under 8 us of 10.7 ms.
+// (Stretches of 1024: 61^3 20 % low 1.1 against 0.6 ms.)
 template <bool MFV, int G, bool GRID>
 __global__ __launch_bounds__(kBlock, 2) void density_more_kernel(DensityStageArgs a)
 {
     constexpr int kStretch = 2 * kBlock / G, kFew = kStretch / (GRID ? 4 : 16);
     constexpr int kLists = GRID ? 3 : 2;  // live ones of this sweep and the next, walks past the budget
+    if (GRID && *a.n_walk == 0) return;
     __shared__ __align__(16) int lds[GRID ? kRowLds<G> : (G == 1 ? kListChunk * kBlock : 1)];
     __shared__ int live[kLists][kStretch];
     __shared__ int n_live[kLists];
@@ -552,7 +577,7 @@ __global__ __launch_bounds__(kBlock, 2) void density_more_kernel(DensityStageArg
         const int t = first + k;
         const int i = t < a.n_active ? a.active[t] : 0;
         // (a particle without mass has no iter)
-        bool in = t < a.n_active && (GRID ? a.iter[i] != kDone : a.iter[i] > 0) && a.posm[i].w > 0;
+        bool in = t < a.n_active && (GRID ? (a.iter[i] & (1u << 31 | kListed)) == 0 : a.iter[i] > 0) && a.posm[i].w > 0;
         if (!GRID && in) {
             const double h = a.hsml[i];
             in = a.row_n[i] <= kDensityCacheCap && h * h <= a.row_r2[i];
@@ -768,6 +793,7 @@ __global__ void density_list_all_kernel(DensityStageArgs a)
     if ((h < 0) || !isfinite(h) || (h > 0.99 * a.hp.max_hsml)) h = 0.99 * a.hp.max_hsml;  // density.c:484
     const Iterate s = {h, 0, 0, a.cn[i], 0};
     hand_on(a, i, s, a.walk_list, a.n_walk);
+    if (!a.walk_list) *a.n_walk = 1;
 }
 
 inline unsigned nblocks(long long n) { return (unsigned)((n + kBlock - 1) / kBlock); }

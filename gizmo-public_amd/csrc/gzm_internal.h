@@ -235,7 +235,7 @@ struct DensityStageArgs {
     int *tail_list, *n_tail;  // not converged after the stage's packed sweeps
     int *far_list, *n_far;    // past the candidate budget
     int *walk_list, *n_walk;  // tree: without a usable row; grid: the tail list, or NULL where
-                              // density_more_kernel finds for itself what is left
+                              // density_more_kernel finds for itself what is left (*n_walk: whether any is)
     int budget;            // candidates of one walk in the tail kernel; 0: no limit
     int lanes;             // lanes per particle of the row and stage kernels: 1 or 8
     Counters *ctr;
