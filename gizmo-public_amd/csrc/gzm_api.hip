@@ -1909,6 +1909,13 @@ gzm_status gzm_run_passes(gzm_ctx *c, int32_t n_passes, gzm_pass_stats *stats)
     int status = 0;
     for (int k = 0; k < kCtrSlots; k++) status = std::max(status, h[k].status);
     if (status == 6) status = GZM_ERR_BRACKET;
+    // passes that left the probe's routes: pairs past its number were not evaluated, and
+    // neither were lists past their cap where it had none
+    const bool strayed = h[kCtrForce].deferred > gp.deferred || (!gp.overflow && h[kCtrGradients].overflow_slices > 0);
+    if (strayed) {
+        if (c->d_redo_flag) launch_fill_int(c->stream, c->d_redo_flag, c->n, 0);
+        GZM_HIP(hipGetLastError());
+    }
     if (stats) {
         stats->density_sweeps = gp.sweeps;
         stats->density_interactions = (int64_t)h[kCtrDensity].interactions;
@@ -1918,11 +1925,15 @@ gzm_status gzm_run_passes(gzm_ctx *c, int32_t n_passes, gzm_pass_stats *stats)
         stats->exact_solver_calls = (int64_t)h[kCtrForce].exact_calls;
         stats->fp64_force_particles = (int64_t)h[kCtrForce].redo_n;
         stats->density_updates = 0;
-        stats->status = status;
+        stats->status = status ? status : (strayed ? (int)GZM_ERR_STATE : 0);
     }
     if (status != 0) {
         set_error("%s", gzm_status_string(status));
         return (gzm_status)status;
+    }
+    if (strayed) {
+        set_error("the captured passes found more deferred pairs or longer lists than their probe: outputs incomplete");
+        return GZM_ERR_STATE;
     }
     return GZM_OK;
 }

@@ -136,7 +136,7 @@ struct alignas(128) Counters {
     int overflow_slices;
     int sweeps;  // density: sweeps of the particle that took most
     unsigned long long updates;  // density: sum over particles of their sweeps
-    int deferred;  // force: pairs deferred out of the list loop
+    int deferred;  // force: pairs deferred out of the list loop (of the pass that had most)
 };
 
 // One field of an export from sorted slots to caller order: element c of

@@ -1385,7 +1385,7 @@ __global__ __launch_bounds__(kBlock) void defer_owners_kernel(ForceArgs a)
     if (t == a.n_active - 1) {
         const int total = a.defer.offset[t] + c;
         *a.defer.total = total;
-        a.ctr->deferred = total;
+        atomicMax(&a.ctr->deferred, total);  // a graph's passes: the most of any
     }
     if (c == 0) return;
     const int q0 = a.defer.offset[t];

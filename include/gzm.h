@@ -236,7 +236,8 @@ gzm_status gzm_restore_initial_state(gzm_ctx *ctx);
  * graph and launched once.  One eager probe pass first fixes what the graph
  * cannot decide on the host (number of density sweeps, pair-list overflow);
  * the graph replays the same input, so every pass repeats the probe's
- * decisions.  stats hold the sums over the n_passes passes (density_sweeps:
+ * decisions; should one meet more than the probe did, the call ends with
+ * GZM_ERR_STATE, its outputs incomplete.  stats hold the sums over the n_passes passes (density_sweeps:
  * per pass); gzm_timing's graph fields hold the graph's device time.  The
  * outputs left on the device are those of the last pass.  No counterpart in
  * the reference: for callers that repeat passes without host round trips. */

@@ -1,11 +1,17 @@
-/* Stands before the HIP runtime in a test process: counts hipSetDevice and
- * bounds what hipMalloc hands out, as a card of `shim_budget` bytes would. */
+/* Stands before the HIP runtime in a test process: counts hipSetDevice, bounds
+ * what hipMalloc hands out, as a card of `shim_budget` bytes would (and refuses
+ * more than `shim_largest` at once), keeps the last allocations' addresses and
+ * calls `shim_before_graph` before a graph is launched. */
 #include <pthread.h>
 #include <stddef.h>
 
 int (*shim_malloc)(void **, size_t), (*shim_free)(void *), (*shim_set_device)(int); /* the runtime's own */
-size_t shim_budget = (size_t)-1, shim_used, shim_peak;
+int (*shim_graph_launch)(void *, void *);
+void (*shim_before_graph)(void);
+size_t shim_budget = (size_t)-1, shim_largest = (size_t)-1, shim_used, shim_peak;
 int shim_refused, shim_set_device_calls;
+int shim_n_recent;
+struct { void *p; size_t n; } shim_recent[256]; /* ring, in order of allocation */
 
 #define SLOTS 65536
 static struct { void *p; size_t n; } held[SLOTS];
@@ -15,13 +21,15 @@ int hipMalloc(void **p, size_t n)
 {
     int e = 2; /* hipErrorOutOfMemory */
     pthread_mutex_lock(&mu);
-    if (n > shim_budget || shim_used > shim_budget - n) {
+    if (n > shim_largest || n > shim_budget || shim_used > shim_budget - n) {
         shim_refused++;
     } else if ((e = shim_malloc(p, n)) == 0) {
         int k = 0;
         while (k < SLOTS - 1 && held[k].p) k++;
         held[k].p = *p;
         held[k].n = n;
+        shim_recent[shim_n_recent % 256].p = *p;
+        shim_recent[shim_n_recent++ % 256].n = n;
         shim_used += n;
         if (shim_used > shim_peak) shim_peak = shim_used;
     }
@@ -40,6 +48,12 @@ int hipFree(void *p)
         }
     pthread_mutex_unlock(&mu);
     return shim_free(p);
+}
+
+int hipGraphLaunch(void *exec, void *stream)
+{
+    if (shim_before_graph) shim_before_graph();
+    return shim_graph_launch(exec, stream);
 }
 
 int hipSetDevice(int device)

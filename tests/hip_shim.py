@@ -23,20 +23,33 @@ class Shim:
         self.lib = C.CDLL(path, mode=C.RTLD_GLOBAL)  # before libgzm.so, whose calls it then takes
 
     def __getattr__(self, name):
-        return C.c_size_t.in_dll(self.lib, "shim_" + name).value if name in ("budget", "used", "peak") else \
-            C.c_int.in_dll(self.lib, "shim_" + name).value
+        return self._var(name).value
 
     def set(self, name, value):
-        t = C.c_size_t if name in ("budget", "used", "peak") else C.c_int
-        t.in_dll(self.lib, "shim_" + name).value = value
+        self._var(name).value = value
+
+    def _var(self, name):
+        t = C.c_size_t if name in ("budget", "largest", "used", "peak") else C.c_int
+        return t.in_dll(self.lib, "shim_" + name)
+
+    def recent(self):
+        """(address, bytes) of the last allocations, in order"""
+        ring = (C.c_size_t * 512).in_dll(self.lib, "shim_recent")
+        return [(ring[2 * (k % 256)], ring[2 * (k % 256) + 1]) for k in
+                range(max(0, self.n_recent - 256), self.n_recent)]
+
+    def before_graph(self, function):
+        self.hook = C.CFUNCTYPE(None)(function)
+        C.c_void_p.in_dll(self.lib, "shim_before_graph").value = C.cast(self.hook, C.c_void_p).value
 
     def connect(self):
         """the runtime that libgzm.so brought with it"""
         with open("/proc/self/maps") as f:
             path = next(line.split()[-1] for line in f if "libamdhip64" in line)
-        hip = C.CDLL(path)
-        for name, symbol in (("malloc", "hipMalloc"), ("free", "hipFree"), ("set_device", "hipSetDevice")):
-            C.c_void_p.in_dll(self.lib, "shim_" + name).value = C.cast(getattr(hip, symbol), C.c_void_p).value
+        self.hip = C.CDLL(path)
+        for name, symbol in (("malloc", "hipMalloc"), ("free", "hipFree"), ("set_device", "hipSetDevice"),
+                             ("graph_launch", "hipGraphLaunch")):
+            C.c_void_p.in_dll(self.lib, "shim_" + name).value = C.cast(getattr(self.hip, symbol), C.c_void_p).value
 
 
 def main():

@@ -1,6 +1,19 @@
 """Checks that run in hip_shim's process, each called with the shim."""
+import ctypes as C
+
+import numpy as np
+
 import gzm
 import ics
+
+OUT_KEYS = ("hsml", "density", "grad_v", "acc", "dtu", "vsig")
+
+
+def one_pass(ctx):
+    ctx.restore_initial_state()
+    ctx.density()
+    ctx.gradients()
+    return ctx.hydro_force()
 
 
 def entry_points_make_their_device_current(shim):
@@ -12,3 +25,35 @@ def entry_points_make_their_device_current(shim):
             before = shim.set_device_calls
             call()
             assert shim.set_device_calls > before, k
+
+
+def run_passes_reports_what_its_probe_did_not_meet(shim, precision):
+    """Velocities that rise between the probe and the graph's launch send pairs to the
+    exact solver for which the graph has no room."""
+    ic = ics.random_state(12)
+    n = ic["mass"].size
+    with gzm.MFMContext(gzm.make_params(precision=int(precision))) as ctx:
+        ctx.upload(ic)
+        # the velocities that the force loop reads, FP64 or FP32, after the positions
+        v = np.zeros((n, 4), dtype=np.float32 if int(precision) else np.float64)
+        velu = [p for p, size in shim.recent() if size == v.nbytes][1]
+        copy = shim.hip.hipMemcpy
+        copy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
+
+        def faster():
+            assert copy(v.ctypes.data, velu, v.nbytes, 2) == 0
+            v[:, :3] *= 60
+            assert copy(velu, v.ctypes.data, v.nbytes, 1) == 0
+
+        before = one_pass(ctx)
+        shim.before_graph(faster)
+        try:
+            ctx.run_passes(1)
+            raise AssertionError("the incomplete passes were reported as complete")
+        except gzm.GzmError as e:
+            assert e.status == 4 and "probe" in str(e), e
+        # the context goes on with what it holds now
+        after = one_pass(ctx)
+        again = one_pass(ctx)
+        assert after.exact_solver_calls == again.exact_solver_calls > before.exact_solver_calls
+        assert after.fp64_force_particles == again.fp64_force_particles

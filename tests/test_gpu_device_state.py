@@ -8,3 +8,8 @@ pytestmark = pytest.mark.gpu
 
 def test_entry_points_make_their_device_current():
     hip_shim.run("entry_points_make_their_device_current")
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_run_passes_reports_what_its_probe_did_not_meet(precision):
+    hip_shim.run("run_passes_reports_what_its_probe_did_not_meet", precision)
