@@ -1836,15 +1836,22 @@ gzm_status gzm_run_passes(gzm_ctx *c, int32_t n_passes, gzm_pass_stats *stats)
     if (!c || c->n == 0) { set_error("no particles uploaded"); return GZM_ERR_STATE; }
     if (n_passes < 1 || n_passes > 100000) { set_error("n_passes=%d out of range [1, 100000]", n_passes); return GZM_ERR_ARG; }
     GZM_HIP(hipSetDevice(c->p.device));
-    // probe pass (eager): sizes every buffer, gives the sweep count and the list overflow
+    // probe pass (eager): sizes every buffer, gives the sweep count and the list overflow.
+    // Where it gave up the candidate rows (need), another: the captured passes go without
+    // them, and with the last bits of hsml the pairs that reach the exact solver may change.
     gzm_pass_stats probe;
-    memset(&probe, 0, sizeof(probe));
-    gzm_status s = restore_state(c);
-    s = s ? s : set_active(c, nullptr, 0);
-    s = s ? s : density_impl(c, nullptr, &probe);
-    s = s ? s : gradients_impl(c, nullptr, &probe);
-    s = s ? s : force_impl(c, nullptr, &probe);
-    if (s) return s;
+    gzm_status s = GZM_OK;
+    for (bool again = true; again;) {
+        const bool rows = c->d_dcache_idx != nullptr;
+        memset(&probe, 0, sizeof(probe));
+        s = restore_state(c);
+        s = s ? s : set_active(c, nullptr, 0);
+        s = s ? s : density_impl(c, nullptr, &probe);
+        s = s ? s : gradients_impl(c, nullptr, &probe);
+        s = s ? s : force_impl(c, nullptr, &probe);
+        if (s) return s;
+        again = rows && !c->d_dcache_idx;
+    }
     const Plan gp = {probe.density_sweeps, c->list_overflow_slices > 0, c->last_deferred, c->last_sweep_live};
     {
         // the captured compactions run over the whole active list

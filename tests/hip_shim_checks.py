@@ -27,6 +27,27 @@ def entry_points_make_their_device_current(shim):
             assert shim.set_device_calls > before, k
 
 
+def run_passes_probes_again_without_rows(shim):
+    """The probe has no memory for its pair list until it gives up the candidate
+    rows: the captured passes, without rows, are probed without them too."""
+    ic = ics.random_state(32)
+    n = ic["mass"].size
+    with gzm.MFMContext(gzm.make_params()) as ctx:
+        ctx.upload(ic)
+        with_rows = shim.used
+        shim.set("budget", with_rows + n)
+        ctx.timing_reset()
+        st = ctx.run_passes(2)
+        assert shim.refused > 0 and shim.used < with_rows + n
+        assert ctx.timing()["density_launches"] == 2, "one probe with rows, one without"
+        out = ctx.download()
+        eager = one_pass(ctx)
+        ref = ctx.download()
+        assert st.force_interactions == 2 * eager.force_interactions
+        for k in OUT_KEYS:
+            np.testing.assert_array_equal(out[k], ref[k], err_msg=k)
+
+
 def run_passes_reports_what_its_probe_did_not_meet(shim, precision):
     """Velocities that rise between the probe and the graph's launch send pairs to the
     exact solver for which the graph has no room."""

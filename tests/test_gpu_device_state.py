@@ -10,6 +10,10 @@ def test_entry_points_make_their_device_current():
     hip_shim.run("entry_points_make_their_device_current")
 
 
+def test_run_passes_probes_again_without_rows():
+    hip_shim.run("run_passes_probes_again_without_rows")
+
+
 @pytest.mark.parametrize("precision", [0, 1])
 def test_run_passes_reports_what_its_probe_did_not_meet(precision):
     hip_shim.run("run_passes_reports_what_its_probe_did_not_meet", precision)
