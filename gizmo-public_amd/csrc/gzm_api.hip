@@ -1577,14 +1577,19 @@ gzm_status force_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
         }
     }
     GZM_HIP(hipGetLastError());
-    auto reserve = [&](size_t want) -> gzm_status {
+    // room for the results of `want` pairs; `must`: the candidate rows give up their memory for it
+    auto reserve = [&](size_t want, bool must) -> gzm_status {
         if (want <= c->defer_result_cap) return GZM_OK;
         dev_free(c->d_defer_result);
         dev_free(c->d_defer_pair);
         c->defer_result_cap = 0;
-        gzm_status e = need(c, &c->d_defer_result, want * (mfv ? 9 : 5));
-        e = e ? e : need(c, &c->d_defer_pair, want);
-        if (e) return e;
+        const size_t words = want * (mfv ? 9 : 5);
+        gzm_status e = must ? need(c, &c->d_defer_result, words) : dev_alloc(&c->d_defer_result, words);
+        e = e ? e : (must ? need(c, &c->d_defer_pair, want) : dev_alloc(&c->d_defer_pair, want));
+        if (e) {
+            dev_free(c->d_defer_result);
+            return e;
+        }
         c->defer_result_cap = want;
         return GZM_OK;
     };
@@ -1638,7 +1643,7 @@ gzm_status force_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
             // have to wait for their number to reach the host.
             size_t want = std::max<size_t>(1 << 16, (size_t)c->n_active / 2);
             if (c->defer_result_cap == 0) {
-                while ((s = reserve(want)) && want > (1 << 16)) want = std::max<size_t>(1 << 16, want / 4);
+                while ((s = reserve(want, want == (1 << 16))) && want > (1 << 16)) want = std::max<size_t>(1 << 16, want / 4);
                 if (s) return s;
             }
             first = (int64_t)c->defer_result_cap;
@@ -1656,7 +1661,9 @@ gzm_status force_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
     if (three_phase && h.deferred > first) {
         // results of one round: all deferred pairs, or 2 per particle if more
         const int64_t D = h.deferred;
-        s = reserve((size_t)std::min<int64_t>(D, std::max<int64_t>(1 << 20, 2 * (int64_t)c->n)));
+        size_t want = (size_t)std::min<int64_t>(D, std::max<int64_t>(1 << 20, 2 * (int64_t)c->n));
+        const size_t had = c->defer_result_cap;
+        while ((s = reserve(want, want <= had)) && want > had) want = std::max<size_t>(had, want / 4);
         if (s) return s;
         const int64_t chunk = (int64_t)c->defer_result_cap;
         for (int64_t q0 = first; q0 < D; q0 += chunk) round(q0, std::min<int64_t>(D, q0 + chunk));

@@ -78,3 +78,45 @@ def run_passes_reports_what_its_probe_did_not_meet(shim, precision):
         again = one_pass(ctx)
         assert after.exact_solver_calls == again.exact_solver_calls > before.exact_solver_calls
         assert after.fp64_force_particles == again.fp64_force_particles
+
+
+def deferred_buffer_shrinks_before_rows_go(shim):
+    """The deferred pairs' buffer, half a pair per particle, has a smaller form: no
+    reason to give up the candidate rows, at first or when it has to grow."""
+    ic = ics.random_state(64)
+    n = ic["mass"].size
+    with gzm.MFMContext(gzm.make_params()) as ctx:
+        ctx.upload(ic)
+        ctx.density()
+        ctx.gradients()
+        before = shim.used
+        shim.set("budget", before + 17 * n + (48 << 16) + 4096)  # per-particle arrays and the smallest buffer
+        few = ctx.hydro_force()
+        assert shim.refused > 0 and shim.used >= before
+        out = ctx.download()
+    shim.set("budget", 1 << 62)
+    ref, st = gzm.run_pass(ic)
+    assert st["exact_solver_calls"] == few.exact_solver_calls > 0
+    for k in OUT_KEYS:
+        np.testing.assert_array_equal(out[k], ref[k], err_msg=k)
+
+
+def deferred_buffer_grows_within_what_is_free(shim):
+    """More pairs than the buffer holds, and no memory for all of them: rounds."""
+    ic = ics.random_state(42)
+    ic["vel"] = 60 * ic["vel"]
+    n = ic["mass"].size
+    with gzm.MFMContext(gzm.make_params()) as ctx:
+        ctx.upload(ic)
+        ctx.density()
+        ctx.gradients()
+        before = shim.used
+        shim.set("budget", before + 17 * n + (48 << 16) + 4096)
+        many = ctx.hydro_force()
+        assert shim.refused > 0 and shim.used >= before
+        out = ctx.download()
+    shim.set("budget", 1 << 62)
+    ref, st = gzm.run_pass(ic)
+    assert st["exact_solver_calls"] == many.exact_solver_calls > 1 << 16
+    for k in OUT_KEYS:
+        np.testing.assert_array_equal(out[k], ref[k], err_msg=k)

@@ -17,3 +17,8 @@ def test_run_passes_probes_again_without_rows():
 @pytest.mark.parametrize("precision", [0, 1])
 def test_run_passes_reports_what_its_probe_did_not_meet(precision):
     hip_shim.run("run_passes_reports_what_its_probe_did_not_meet", precision)
+
+
+@pytest.mark.parametrize("check", ["deferred_buffer_shrinks_before_rows_go", "deferred_buffer_grows_within_what_is_free"])
+def test_deferred_pairs_leave_the_rows_their_memory(check):
+    hip_shim.run(check)
