@@ -185,12 +185,37 @@ void dev_free(T *&p)
     p = nullptr;
 }
 
+// Grid: whether the expected entries of a candidate row stay within its cap.  Above that
+// nearly every particle walks, over more candidates than a lane is given, so neither rows
+// nor the packed sweeps of a lane each are of use (68,921 particles of 128 neighbours,
+// density: 8.4 ms with both, 3.2 with rows tried, 2.85 with 16 lanes and more from the start;
+// of 80: 1.75 and 1.25).
+bool grid_rows_fit(const gzm_ctx *c)
+{
+    const double f = kDensityCacheFactorGrid;
+    return f * f * f * c->p.des_num_ngb <= kDensityCacheCap;
+}
+
 // The candidate rows (up to 412 B per particle) are an optimisation: a set that
 // fills the memory without them runs without them.
 void free_rows(gzm_ctx *c)
 {
     dev_free(c->d_dcache_idx); dev_free(c->d_dcache_n); dev_free(c->d_dcache_r2); dev_free(c->d_posf);
     c->dcache_all = false;
+}
+
+constexpr size_t kRowBytes = kDensityCacheCap * sizeof(int) + sizeof(int) + sizeof(double) + sizeof(float4);
+
+// whether the density stage can use rows
+bool rows_useful(const gzm_ctx *c) { return c->p.precision != 2 && (c->p.search == 1 || grid_rows_fit(c)); }
+
+// memory for them where the card has it
+void alloc_rows(gzm_ctx *c)
+{
+    const size_t n = (size_t)c->n;
+    if (dev_alloc(&c->d_dcache_idx, n * kDensityCacheCap) || dev_alloc(&c->d_dcache_n, n) ||
+        dev_alloc(&c->d_dcache_r2, n) || (c->p.search == 0 && dev_alloc(&c->d_posf, n)))
+        free_rows(c);
 }
 
 // an array that the context needs, whose memory the candidate rows give up if they have to
@@ -729,17 +754,6 @@ gzm_status gzm_ctx_destroy(gzm_ctx *c)
 
 namespace {
 
-// Grid: whether the expected entries of a candidate row stay within its cap.  Above that
-// nearly every particle walks, over more candidates than a lane is given, so neither rows
-// nor the packed sweeps of a lane each are of use (68,921 particles of 128 neighbours,
-// density: 8.4 ms with both, 3.2 with rows tried, 2.85 with 16 lanes and more from the start;
-// of 80: 1.75 and 1.25).
-bool grid_rows_fit(const gzm_ctx *c)
-{
-    const double f = kDensityCacheFactorGrid;
-    return f * f * f * c->p.des_num_ngb <= kDensityCacheCap;
-}
-
 // Per-box grids, the global cell-range array and the hmax tiles of an upload.
 gzm_status setup_boxes(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const double *box_sizes,
                        const int64_t *offsets)
@@ -922,11 +936,12 @@ gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const 
             s = s ? s : dev_alloc(&c->d_bwave_n, 2);
         }
         if (s) { free_particles(c); return s; }
-        if (c->p.precision != 2 && (c->p.search == 1 || grid_rows_fit(c))) {
-            if (dev_alloc(&c->d_dcache_idx, (size_t)n * kDensityCacheCap) || dev_alloc(&c->d_dcache_n, n) ||
-                dev_alloc(&c->d_dcache_r2, n) || (c->p.search == 0 && dev_alloc(&c->d_posf, n)))
-                free_rows(c);
-        }
+        if (rows_useful(c)) alloc_rows(c);
+    } else if (rows_useful(c) && !c->d_dcache_idx) {
+        // given up since the first upload of this many particles: again once memory is not short any more
+        size_t free_bytes = 0, total_bytes = 0;
+        if (hipMemGetInfo(&free_bytes, &total_bytes) == hipSuccess && free_bytes / 2 >= (size_t)n * kRowBytes) alloc_rows(c);
+        else (void)hipGetLastError();
     }
     if (c->d_redo_flag) launch_fill_int(c->stream, c->d_redo_flag, n, 0);
     gzm_status s = setup_boxes(c, v, n_boxes, box_sizes, offsets);

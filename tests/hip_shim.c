@@ -6,7 +6,7 @@
 #include <stddef.h>
 
 int (*shim_malloc)(void **, size_t), (*shim_free)(void *), (*shim_set_device)(int); /* the runtime's own */
-int (*shim_graph_launch)(void *, void *);
+int (*shim_graph_launch)(void *, void *), (*shim_mem_info)(size_t *, size_t *);
 void (*shim_before_graph)(void);
 size_t shim_budget = (size_t)-1, shim_largest = (size_t)-1, shim_used, shim_peak;
 int shim_refused, shim_set_device_calls;
@@ -48,6 +48,14 @@ int hipFree(void *p)
         }
     pthread_mutex_unlock(&mu);
     return shim_free(p);
+}
+
+int hipMemGetInfo(size_t *free_bytes, size_t *total)
+{
+    const int e = shim_mem_info(free_bytes, total);
+    const size_t left = shim_budget > shim_used ? shim_budget - shim_used : 0;
+    if (e == 0 && *free_bytes > left) *free_bytes = left;
+    return e;
 }
 
 int hipGraphLaunch(void *exec, void *stream)

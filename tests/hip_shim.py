@@ -48,7 +48,7 @@ class Shim:
             path = next(line.split()[-1] for line in f if "libamdhip64" in line)
         self.hip = C.CDLL(path)
         for name, symbol in (("malloc", "hipMalloc"), ("free", "hipFree"), ("set_device", "hipSetDevice"),
-                             ("graph_launch", "hipGraphLaunch")):
+                             ("graph_launch", "hipGraphLaunch"), ("mem_info", "hipMemGetInfo")):
             C.c_void_p.in_dll(self.lib, "shim_" + name).value = C.cast(getattr(self.hip, symbol), C.c_void_p).value
 
 

@@ -120,3 +120,30 @@ def deferred_buffer_grows_within_what_is_free(shim):
     assert st["exact_solver_calls"] == many.exact_solver_calls > 1 << 16
     for k in OUT_KEYS:
         np.testing.assert_array_equal(out[k], ref[k], err_msg=k)
+
+
+def rows_come_back_with_the_memory(shim):
+    """Rows given up for want of memory are there again after an upload that finds it,
+    and are not asked for while it is short."""
+    ic = ics.random_state(32)
+    n = ic["mass"].size
+    ref, _ = gzm.run_pass(ic)
+    with gzm.MFMContext(gzm.make_params()) as ctx:
+        ctx.upload(ic)
+        with_rows = shim.used
+        shim.set("budget", with_rows + n)
+        one_pass(ctx)
+        given_up = shim.used
+        assert shim.refused > 0 and given_up < with_rows + n
+        ctx.upload(ic)
+        assert shim.used == given_up
+        refused = shim.refused
+        ctx.upload(ic)
+        assert shim.used == given_up and shim.refused == refused
+        shim.set("budget", 1 << 62)
+        ctx.upload(ic)
+        assert shim.used == given_up + 412 * n
+        one_pass(ctx)
+        out = ctx.download()
+    for k in OUT_KEYS:
+        np.testing.assert_array_equal(out[k], ref[k], err_msg=k)

@@ -22,3 +22,7 @@ def test_run_passes_reports_what_its_probe_did_not_meet(precision):
 @pytest.mark.parametrize("check", ["deferred_buffer_shrinks_before_rows_go", "deferred_buffer_grows_within_what_is_free"])
 def test_deferred_pairs_leave_the_rows_their_memory(check):
     hip_shim.run(check)
+
+
+def test_rows_come_back_with_the_memory():
+    hip_shim.run("rows_come_back_with_the_memory")
