@@ -1,14 +1,14 @@
 /* Stands before the HIP runtime in a test process: counts hipSetDevice, bounds
  * what hipMalloc hands out, as a card of `shim_budget` bytes would (and refuses
- * more than `shim_largest` at once), keeps the last allocations' addresses and
- * calls `shim_before_graph` before a graph is launched. */
+ * requests of just `shim_unwanted` bytes), keeps the last allocations' addresses
+ * and calls `shim_before_graph` before a graph is launched. */
 #include <pthread.h>
 #include <stddef.h>
 
 int (*shim_malloc)(void **, size_t), (*shim_free)(void *), (*shim_set_device)(int); /* the runtime's own */
 int (*shim_graph_launch)(void *, void *), (*shim_mem_info)(size_t *, size_t *);
 void (*shim_before_graph)(void);
-size_t shim_budget = (size_t)-1, shim_largest = (size_t)-1, shim_used, shim_peak;
+size_t shim_budget = (size_t)-1, shim_unwanted, shim_used, shim_peak;
 int shim_refused, shim_set_device_calls;
 int shim_n_recent;
 struct { void *p; size_t n; } shim_recent[256]; /* ring, in order of allocation */
@@ -21,7 +21,7 @@ int hipMalloc(void **p, size_t n)
 {
     int e = 2; /* hipErrorOutOfMemory */
     pthread_mutex_lock(&mu);
-    if (n > shim_largest || n > shim_budget || shim_used > shim_budget - n) {
+    if (n == shim_unwanted || n > shim_budget || shim_used > shim_budget - n) {
         shim_refused++;
     } else if ((e = shim_malloc(p, n)) == 0) {
         int k = 0;

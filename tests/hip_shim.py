@@ -29,7 +29,7 @@ class Shim:
         self._var(name).value = value
 
     def _var(self, name):
-        t = C.c_size_t if name in ("budget", "largest", "used", "peak") else C.c_int
+        t = C.c_size_t if name in ("budget", "unwanted", "used", "peak") else C.c_int
         return t.in_dll(self.lib, "shim_" + name)
 
     def recent(self):

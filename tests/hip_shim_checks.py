@@ -5,6 +5,8 @@ import numpy as np
 
 import gzm
 import ics
+import oracle as O
+from parity import TOL32_DENSITY, TOL32_FLUX, check_mfv, check_pass, error_stats
 
 OUT_KEYS = ("hsml", "density", "grad_v", "acc", "dtu", "vsig")
 
@@ -147,3 +149,82 @@ def rows_come_back_with_the_memory(shim):
         out = ctx.download()
     for k in OUT_KEYS:
         np.testing.assert_array_equal(out[k], ref[k], err_msg=k)
+
+
+def params_of(ic, method=0, **kw):
+    return dict(gpu=gzm.make_params(method=method, **kw), oracle=O.make_params(method=method))
+
+
+def without_rows(shim, side, search, method):
+    """A context that never gets candidate rows: density from the tail's and the walk's
+    kernels, gradients from walks, hsml well guessed, poorly guessed and of a part,
+    against the oracle; the passes of a graph against the eager one."""
+    side, search, method = int(side), int(search), int(method)
+    check = check_mfv if method else check_pass
+    ic = ics.random_state(side)
+    n = ic["mass"].size
+    shim.set("unwanted", 96 * 4 * n)
+    poor = dict(ic, hsml=ic["hsml"] * (0.6 + 1.2 * ics.uniform(5, 1, n)))
+    for which, s in (("good", ic), ("poor", poor)):
+        p = params_of(s, method=method, search=search)
+        refused = shim.refused
+        ref, st, _ = O.run_pass(s, p["oracle"])
+        with gzm.MFMContext(p["gpu"]) as ctx:
+            ctx.upload(s)
+            assert shim.refused > refused, "no rows asked for"
+            d, g, f = ctx.density(), ctx.gradients(), ctx.hydro_force()
+            out = ctx.download()
+            assert (d.density_sweeps, d.density_interactions, g.gradient_interactions, f.force_interactions,
+                    f.exact_solver_calls) == (st.iterations, st.dens_interactions, st.grad_interactions,
+                                              st.force_interactions, st.exact_solver_calls), which
+            errs, bad = check(out, ref)
+            assert not bad, (which, bad)
+            if method == 0:
+                ctx.restore_initial_state()
+                ctx.run_passes(2)
+                again = ctx.download()
+                for k in OUT_KEYS:
+                    np.testing.assert_array_equal(again[k], out[k], err_msg=f"{which} {k}")
+    if method:
+        return
+    state = dict(ic)
+    for k in ("hsml", "num_ngb", "dhsml", "divvel", "density", "pressure", "nvt", "cn", "fce", "grad_rho", "grad_p",
+              "grad_v"):
+        state[k] = out[k]
+    active = ics.random_subset(n, 0.4)
+    ref, st, _ = O.run_pass(state, active=active)
+    part, gst = gzm.run_pass(state, active=active, params=gzm.make_params(search=search))
+    assert gst["density_interactions"] == st.dens_interactions
+    assert gst["force_interactions"] == st.force_interactions
+    errs, bad = check_pass(part, ref, active)
+    assert not bad, bad
+    ref, st, _ = O.run_pass(ic)
+    half, gst = gzm.run_pass(ic, params=gzm.make_params(search=search, precision=1))
+    assert gst["density_interactions"] == st.dens_interactions
+    assert gst["force_interactions"] == st.force_interactions
+    es = error_stats(half, ref)
+    for k in ("density", "hsml", "pressure"):
+        assert es[k]["max"] <= TOL32_DENSITY, (k, es[k])
+    for k in ("acc", "dtu"):
+        assert es[k]["max"] <= TOL32_FLUX, (k, es[k])
+
+
+def rows_given_up_between_stages(shim, search):
+    """Rows that served the density stage and are gone at the gradients."""
+    ic = ics.random_state(32)
+    n = ic["mass"].size
+    ref, st, _ = O.run_pass(ic)
+    with gzm.MFMContext(gzm.make_params(search=int(search))) as ctx:
+        ctx.upload(ic)
+        d = ctx.density()
+        with_rows = shim.used
+        shim.set("budget", with_rows + n)
+        g = ctx.gradients()
+        assert shim.refused > 0 and shim.used < with_rows
+        f = ctx.hydro_force()
+        out = ctx.download()
+    assert d.density_interactions == st.dens_interactions
+    assert g.gradient_interactions == st.grad_interactions
+    assert f.force_interactions == st.force_interactions
+    errs, bad = check_pass(out, ref)
+    assert not bad, bad

@@ -26,3 +26,15 @@ def test_deferred_pairs_leave_the_rows_their_memory(check):
 
 def test_rows_come_back_with_the_memory():
     hip_shim.run("rows_come_back_with_the_memory")
+
+
+@pytest.mark.parametrize("method", [0, 1])
+@pytest.mark.parametrize("search", [0, 1])
+@pytest.mark.parametrize("side", [12, 41])  # eight lanes and one lane per particle
+def test_pass_without_candidate_rows(side, search, method):
+    hip_shim.run("without_rows", side, search, method)
+
+
+@pytest.mark.parametrize("search", [0, 1])
+def test_rows_given_up_between_stages(search):
+    hip_shim.run("rows_given_up_between_stages", search)
