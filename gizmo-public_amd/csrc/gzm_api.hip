@@ -14,7 +14,9 @@
 #include <rocprim/device/device_select.hpp>
 
 #include <algorithm>
+#include <atomic>
 #include <mutex>
+#include <thread>
 #include <vector>
 
 #include "../../include/gzm.h"
@@ -160,15 +162,39 @@ struct gzm_ctx {
     gzm_timing timing;
     std::vector<TimedLaunch> pending;
     std::vector<hipEvent_t> event_pool;
+
+    std::atomic<bool> busy{false};  // in a call, or giving its rows to another context (reclaim_rows)
+    gzm_ctx *next = nullptr;        // of g_contexts
 };
 
 namespace {
 
+// the contexts of this process
+std::mutex g_contexts_mu;
+gzm_ctx *g_contexts = nullptr;
+
+// held by every call that works on a context
+struct InUse {
+    gzm_ctx *c;
+    explicit InUse(gzm_ctx *ctx) : c(ctx)
+    {
+        while (c && c->busy.exchange(true, std::memory_order_acquire)) std::this_thread::yield();
+    }
+    ~InUse()
+    {
+        if (c) c->busy.store(false, std::memory_order_release);
+    }
+};
+
+bool reclaim_rows();
+
+// `ask`: where the card is full, idle contexts give up their candidate rows
 template <class T>
-gzm_status dev_alloc(T **p, size_t count)
+gzm_status dev_alloc(T **p, size_t count, bool ask = true)
 {
     if (count == 0) count = 1;
     hipError_t e = hipMalloc((void **)p, count * sizeof(T));
+    if (e != hipSuccess && ask && reclaim_rows()) e = hipMalloc((void **)p, count * sizeof(T));
     if (e != hipSuccess) {
         set_error("hipMalloc of %zu bytes failed: %s", count * sizeof(T), hipGetErrorString(e));
         (void)hipGetLastError();  // reported here: a caller that does without goes on
@@ -213,9 +239,29 @@ bool rows_useful(const gzm_ctx *c) { return c->p.precision != 2 && (c->p.search 
 void alloc_rows(gzm_ctx *c)
 {
     const size_t n = (size_t)c->n;
-    if (dev_alloc(&c->d_dcache_idx, n * kDensityCacheCap) || dev_alloc(&c->d_dcache_n, n) ||
-        dev_alloc(&c->d_dcache_r2, n) || (c->p.search == 0 && dev_alloc(&c->d_posf, n)))
+    if (dev_alloc(&c->d_dcache_idx, n * kDensityCacheCap, false) || dev_alloc(&c->d_dcache_n, n, false) ||
+        dev_alloc(&c->d_dcache_r2, n, false) || (c->p.search == 0 && dev_alloc(&c->d_posf, n, false)))
         free_rows(c);
+}
+
+// The rows of the contexts on the current device that are in no call, given back to
+// the card for another's arrays; whether there were any.
+bool reclaim_rows()
+{
+    int device = -1;
+    if (hipGetDevice(&device) != hipSuccess) return false;
+    bool any = false;
+    std::lock_guard<std::mutex> lock(g_contexts_mu);
+    for (gzm_ctx *c = g_contexts; c; c = c->next) {
+        if (c->p.device != device || c->busy.exchange(true, std::memory_order_acquire)) continue;
+        if (c->d_dcache_idx) {
+            (void)hipStreamSynchronize(c->stream);
+            free_rows(c);
+            any = true;
+        }
+        c->busy.store(false, std::memory_order_release);
+    }
+    return any;
 }
 
 // an array that the context needs, whose memory the candidate rows give up if they have to
@@ -724,6 +770,11 @@ gzm_status gzm_ctx_create(gzm_ctx **out, const gzm_params *params)
         gzm_ctx_destroy(c);
         return GZM_ERR_NOMEM;
     }
+    {
+        std::lock_guard<std::mutex> lock(g_contexts_mu);
+        c->next = g_contexts;
+        g_contexts = c;
+    }
     *out = c;
     return GZM_OK;
 }
@@ -731,6 +782,14 @@ gzm_status gzm_ctx_create(gzm_ctx **out, const gzm_params *params)
 gzm_status gzm_ctx_destroy(gzm_ctx *c)
 {
     if (!c) return GZM_OK;
+    {
+        std::lock_guard<std::mutex> lock(g_contexts_mu);
+        for (gzm_ctx **p = &g_contexts; *p; p = &(*p)->next)
+            if (*p == c) {
+                *p = c->next;
+                break;
+            }
+    }
     (void)hipSetDevice(c->p.device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     collect_timings(c);
@@ -1599,8 +1658,8 @@ gzm_status force_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
         dev_free(c->d_defer_pair);
         c->defer_result_cap = 0;
         const size_t words = want * (mfv ? 9 : 5);
-        gzm_status e = must ? need(c, &c->d_defer_result, words) : dev_alloc(&c->d_defer_result, words);
-        e = e ? e : (must ? need(c, &c->d_defer_pair, want) : dev_alloc(&c->d_defer_pair, want));
+        gzm_status e = must ? need(c, &c->d_defer_result, words) : dev_alloc(&c->d_defer_result, words, false);
+        e = e ? e : (must ? need(c, &c->d_defer_pair, want) : dev_alloc(&c->d_defer_pair, want, false));
         if (e) {
             dev_free(c->d_defer_result);
             return e;
@@ -1806,6 +1865,7 @@ extern "C" {
 gzm_status gzm_upload(gzm_ctx *c, const gzm_host_view *v)
 {
     if (!c || !v) { set_error("NULL argument"); return GZM_ERR_ARG; }
+    const InUse in_use(c);
     const int64_t offsets[2] = {0, v->n};
     return upload_common(c, v, 1, c->p.box, offsets);
 }
@@ -1814,11 +1874,13 @@ gzm_status gzm_upload_batch(gzm_ctx *c, const gzm_host_view *v, int32_t n_boxes,
                             const int64_t *box_offsets)
 {
     if (!c || !v || !box_sizes || !box_offsets) { set_error("NULL argument"); return GZM_ERR_ARG; }
+    const InUse in_use(c);
     return upload_common(c, v, n_boxes, box_sizes, box_offsets);
 }
 
 gzm_status gzm_restore_initial_state(gzm_ctx *c)
 {
+    const InUse in_use(c);
     if (!c || c->n == 0) { set_error("no particles uploaded"); return GZM_ERR_STATE; }
     GZM_HIP(hipSetDevice(c->p.device));
     return restore_state(c);
@@ -1826,6 +1888,7 @@ gzm_status gzm_restore_initial_state(gzm_ctx *c)
 
 gzm_status gzm_density(gzm_ctx *c, const int32_t *active, int64_t n_active, gzm_pass_stats *stats)
 {
+    const InUse in_use(c);
     if (!c || c->n == 0) { set_error("no particles uploaded"); return GZM_ERR_STATE; }
     GZM_HIP(hipSetDevice(c->p.device));
     gzm_status s = set_active(c, active, n_active);
@@ -1835,6 +1898,7 @@ gzm_status gzm_density(gzm_ctx *c, const int32_t *active, int64_t n_active, gzm_
 
 gzm_status gzm_gradients(gzm_ctx *c, const int32_t *active, int64_t n_active, gzm_pass_stats *stats)
 {
+    const InUse in_use(c);
     if (!c || c->n == 0) { set_error("no particles uploaded"); return GZM_ERR_STATE; }
     if (!c->have_density) { set_error("gradients need density results (run gzm_density or upload them)"); return GZM_ERR_STATE; }
     GZM_HIP(hipSetDevice(c->p.device));
@@ -1845,6 +1909,7 @@ gzm_status gzm_gradients(gzm_ctx *c, const int32_t *active, int64_t n_active, gz
 
 gzm_status gzm_hydro_force(gzm_ctx *c, const int32_t *active, int64_t n_active, gzm_pass_stats *stats)
 {
+    const InUse in_use(c);
     if (!c || c->n == 0) { set_error("no particles uploaded"); return GZM_ERR_STATE; }
     if (!c->have_density) { set_error("force needs density results"); return GZM_ERR_STATE; }
     GZM_HIP(hipSetDevice(c->p.device));
@@ -1855,6 +1920,7 @@ gzm_status gzm_hydro_force(gzm_ctx *c, const int32_t *active, int64_t n_active, 
 
 gzm_status gzm_run_passes(gzm_ctx *c, int32_t n_passes, gzm_pass_stats *stats)
 {
+    const InUse in_use(c);
     if (!c || c->n == 0) { set_error("no particles uploaded"); return GZM_ERR_STATE; }
     if (n_passes < 1 || n_passes > 100000) { set_error("n_passes=%d out of range [1, 100000]", n_passes); return GZM_ERR_ARG; }
     GZM_HIP(hipSetDevice(c->p.device));
@@ -1970,6 +2036,7 @@ gzm_status gzm_run_passes(gzm_ctx *c, int32_t n_passes, gzm_pass_stats *stats)
 gzm_status gzm_download(gzm_ctx *c, gzm_host_view *v)
 {
     if (!c || !v) { set_error("NULL argument"); return GZM_ERR_ARG; }
+    const InUse in_use(c);
     if (c->n == 0 || v->n != c->n) { set_error("view size %lld does not match uploaded %d", (long long)v->n, c->n); return GZM_ERR_ARG; }
     GZM_HIP(hipSetDevice(c->p.device));
     std::vector<ExportField> fields;
@@ -2001,6 +2068,7 @@ gzm_status gzm_download(gzm_ctx *c, gzm_host_view *v)
 gzm_status gzm_neighbor_counts(gzm_ctx *c, int32_t mode, const int32_t *active, int64_t n_active, int32_t *counts,
                                int64_t *total)
 {
+    const InUse in_use(c);
     if (!c || c->n == 0) { set_error("no particles uploaded"); return GZM_ERR_STATE; }
     if (mode != 0 && mode != 1) { set_error("mode must be 0 or 1"); return GZM_ERR_ARG; }
     GZM_HIP(hipSetDevice(c->p.device));

@@ -228,3 +228,67 @@ def rows_given_up_between_stages(shim, search):
     assert f.force_interactions == st.force_interactions
     errs, bad = check_pass(out, ref)
     assert not bad, bad
+
+
+def idle_contexts_give_their_rows(shim, search):
+    """A second context fits beside one with candidate rows where it fits beside one
+    without: the idle one gives them up, between its density and gradients."""
+    search = int(search)
+    one, two = ics.random_state(32), ics.random_state(32, seed=8)
+    n = one["mass"].size
+    refs = [O.run_pass(ic)[0] for ic in (one, two)]
+    with gzm.MFMContext(gzm.make_params(search=search)) as a:
+        empty = shim.used
+        a.upload(one)
+        one_pass(a)  # every array that a pass needs
+        a.upload(one)
+        a.density()
+        full = shim.used
+        rows = n * (96 * 4 + 12 + (0 if search else 16))
+        budget = full + (full - empty - rows) - 100 * n  # a second set of that size, without rows, lacks 100 n
+        shim.set("budget", budget)
+        with gzm.MFMContext(gzm.make_params(search=search)) as b:
+            b.upload(two)
+            one_pass(b)
+            assert shim.refused > 0 and shim.used <= budget
+            a.gradients()
+            a.hydro_force()
+            for ctx, ref in ((a, refs[0]), (b, refs[1])):
+                errs, bad = check_pass(ctx.download(), ref)
+                assert not bad, bad
+
+
+def contexts_of_threads_share_a_full_card(shim):
+    """Threads with a context each on a card that holds the rows of one or two."""
+    import threading
+    sets = [ics.random_state(side) for side in (30, 28, 26)]
+    refs = [O.run_pass(ic)[0] for ic in sets]
+    with gzm.MFMContext(gzm.make_params()) as ctx:
+        empty = shim.used
+        ctx.upload(sets[0])
+        one_pass(ctx)
+        each = shim.used - empty
+    shim.set("budget", shim.used + int(2.2 * each))
+    failures = []
+
+    def work(ic, ref):
+        try:
+            for _ in range(4):
+                with gzm.MFMContext(gzm.make_params()) as ctx:
+                    for _ in range(3):
+                        ctx.upload(ic)
+                        one_pass(ctx)
+                        errs, bad = check_pass(ctx.download(), ref)
+                        assert not bad, bad
+        except gzm.GzmError as e:
+            if e.status != 3:  # no memory left even without rows
+                failures.append(repr(e))
+        except BaseException as e:  # noqa: B902
+            failures.append(repr(e))
+
+    threads = [threading.Thread(target=work, args=a) for a in zip(sets, refs)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not failures and not any(t.is_alive() for t in threads), failures

@@ -38,3 +38,12 @@ def test_pass_without_candidate_rows(side, search, method):
 @pytest.mark.parametrize("search", [0, 1])
 def test_rows_given_up_between_stages(search):
     hip_shim.run("rows_given_up_between_stages", search)
+
+
+@pytest.mark.parametrize("search", [0, 1])
+def test_idle_contexts_give_their_rows(search):
+    hip_shim.run("idle_contexts_give_their_rows", search)
+
+
+def test_contexts_of_threads_share_a_full_card():
+    hip_shim.run("contexts_of_threads_share_a_full_card")
