@@ -29,6 +29,7 @@ constexpr int kBlock = 256;
 constexpr int kMaxBlock = 512;
 constexpr int kXcds = 8;         // MI355X: 8 XCDs, each with its own L2
 constexpr int kListChunk = 16;   // pair-list entries a lane stages before one 64-byte store
+static_assert(kDensityCacheCap % kListChunk == 0, "a row's last chunk would reach into the next row");
 
 // Workgroups are dealt to the XCDs round-robin (block b runs on XCD b % 8).
 // Renumber them so that each XCD receives one contiguous run of the

@@ -168,7 +168,7 @@ constexpr int kDensityBudget = 512;
 // beyond the few percent by which hsml changes within a stage.
 constexpr double kDensityCacheFactor = 1.2;      // tree
 constexpr double kDensityCacheFactorGrid = 1.1;  // grid
-constexpr int kDensityCacheCap = 96;  // a multiple of 4: rows are read as int4
+constexpr int kDensityCacheCap = 96;  // whole chunks (kListChunk, 16 entries): rows are stored and read by them
 
 // At most this many active particles: 8 lanes per particle in the density stage
 // instead of one, which would leave most SIMDs without a wavefront (rows + two
