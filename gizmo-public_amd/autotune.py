@@ -9,15 +9,18 @@ library's defaults) and returns the fastest setting it met:
                   against cells walked
   pair_list_cap   neighbours per particle kept in the gradient-to-force pair
                   list (longer pair sets take the wavefront fallback)
-  block_size      workgroup size of the density-sweep, gradient and force
-                  loops (64, 128, 256, 512), one axis each (threads per
-                  particle are fixed at one, so this trades scheduling
-                  granularity against tail effects)
-  density_budget  candidates a density-sweep thread tests before its particle
-                  moves to a wavefront of its own
-  wave_sweep_max  density sweeps over at most this many particles give every
-                  particle a wavefront (neighbours per wavefront rather than
-                  per thread)
+  block_size      workgroup size of the density-sweep (precision 2), gradient
+                  and force (precisions 1 and 2) loops (64, 128, 256, 512), one
+                  axis each (lanes per particle are the library's choice, so this
+                  trades scheduling granularity against tail effects)
+  density_budget  candidates a density walk tests before its particle moves to
+                  a wavefront of its own
+  wave_sweep_max  density sweeps of precision 2 over at most this many particles
+                  give every particle a wavefront (neighbours per wavefront rather
+                  than per thread)
+
+An axis that the library does not read at the precision and size in question is not
+timed: its candidates are one setting, and noise would choose among them.
 
 A batch is tuned on a sample of its boxes spread over the size range, so that
 tuning costs a small fraction of a full pass.  None of these settings changes
@@ -48,6 +51,21 @@ AXES = (("cell_factor", CELL_FACTORS), ("pair_list_cap", LIST_CAPS), ("block_den
 # run to run, and a choice made on noise would differ between otherwise
 # identical runs.
 MIN_GAIN = 0.02
+
+
+# at most this many particles: the FP64 gradient kernel's workgroups are fixed
+FEW_PARTICLES = 65536
+
+
+def axis_is_read(name: str, precision: int, n: int) -> bool:
+    """Whether a pass over n particles depends on the axis."""
+    if name in ("block_density", "wave_sweep_max"):
+        return precision == 2
+    if name == "block_force":
+        return precision != 0  # the FP64 list loop's workgroup is a wavefront
+    if name == "block_gradients":
+        return precision != 0 or n > FEW_PARTICLES
+    return True
 
 
 def make_params_kwargs(setting: dict) -> dict:
@@ -108,7 +126,8 @@ def tune(ic: dict, precision: int, axes=AXES, n_sample: int = 32, min_gain: floa
     kwargs, "cell_factor", "pair_list_cap", "table": {label: ms},
     "axes": {axis: {candidate: ms}}}.  Along an axis the candidates are tried
     in the order given, the others held at the best setting so far; one
-    replaces the best only when it is faster by more than `min_gain`."""
+    replaces the best only when it is faster by more than `min_gain`.  An axis
+    that the pass does not read shows the best time so far for each candidate."""
     sample = sample_boxes(ic, n_sample) if "box_offsets" in ic else ic
     best = dict(DEFAULTS)
     timed = {}
@@ -123,6 +142,9 @@ def tune(ic: dict, precision: int, axes=AXES, n_sample: int = 32, min_gain: floa
     per_axis = {}
     for name, candidates in axes:
         per_axis[name] = {}
+        if not axis_is_read(name, precision, int(sample["pos"].shape[0])):
+            per_axis[name] = {str(v): round(best_t * 1e3, 3) for v in candidates}
+            continue
         for v in candidates:
             trial = dict(best, **{name: v})
             t = measure(trial)
