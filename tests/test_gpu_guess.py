@@ -56,6 +56,31 @@ def test_more_neighbours_than_a_row_holds(side, des):
     assert not bad, bad
 
 
+@pytest.mark.parametrize("budget", [0, -1])
+@pytest.mark.parametrize("search", [0, 1])
+def test_sums_of_the_widest_walks(search, budget):
+    """Search spheres over a clump of 6,000 massive particles: the walks past every
+    budget, with their sums.  Any number of neighbours will do, so one sweep is all
+    and no step of hsml turns on a sum's rounding."""
+    rng = np.random.default_rng(6)
+    n_bg, n_clump = 2000, 6000
+    pos = np.concatenate([rng.uniform(0, 1, (n_bg, 3)), 0.37 + 0.01 * rng.normal(size=(n_clump, 3))])
+    n = pos.shape[0]
+    ic = dict(pos=pos, vel=0.1 * rng.normal(size=(n, 3)), mass=np.full(n, 1.0 / n), u=1 + 0.1 * rng.uniform(size=n),
+              hsml=ics.local_hsml(pos), cn=np.ones(n), box=np.ones(3))
+    active = np.concatenate([np.arange(40), n_bg + np.arange(30)]).astype(np.int32)
+    ic["hsml"][active] = 0.3 + 0.15 * rng.uniform(size=active.size)
+    kw = dict(des_num_ngb=1000.0, max_num_ngb_dev=1e6, first_step=0)
+    ref, st, _ = O.run_pass(ic, O.make_params(**kw), active=active, stages=("density",))
+    assert st.iterations == 1 and st.dens_interactions > 6000 * 30
+    out, gst = gzm.run_pass(ic, active=active, params=gzm.make_params(search=search, density_budget=budget, **kw),
+                            stages=("density",))
+    assert gst["density_sweeps"] == 1
+    assert gst["density_interactions"] == st.dens_interactions
+    errs, bad = check_pass(out, ref, active)
+    assert not bad, bad
+
+
 def density_ms(ic, passes=5):
     with gzm.MFMContext(gzm.make_params()) as ctx:
         ctx.upload(ic)
