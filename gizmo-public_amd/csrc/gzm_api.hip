@@ -601,12 +601,12 @@ F32Geom f32_geom(const gzm_ctx *c)
 // per-particle arrays of the deferred exact-solver pairs (sized for all particles)
 gzm_status ensure_defer(gzm_ctx *c)
 {
-    if (c->d_defer_mask) return GZM_OK;
-    gzm_status s = need(c, &c->d_defer_mask, (size_t)c->n);
-    s = s ? s : need(c, &c->d_defer_count, (size_t)c->n);
-    s = s ? s : need(c, &c->d_defer_off, (size_t)c->n);
-    s = s ? s : need(c, &c->d_defer_total, 1);
-    s = s ? s : need(c, &c->d_defer_raw, (size_t)c->n);
+    gzm_status s = GZM_OK;  // (a call that ran out of memory may have left some of them)
+    if (!c->d_defer_mask) s = need(c, &c->d_defer_mask, (size_t)c->n);
+    if (!s && !c->d_defer_count) s = need(c, &c->d_defer_count, (size_t)c->n);
+    if (!s && !c->d_defer_off) s = need(c, &c->d_defer_off, (size_t)c->n);
+    if (!s && !c->d_defer_total) s = need(c, &c->d_defer_total, 1);
+    if (!s && !c->d_defer_raw) s = need(c, &c->d_defer_raw, (size_t)c->n);
     return s;
 }
 
@@ -888,38 +888,10 @@ gzm_status setup_boxes(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const do
     return GZM_OK;
 }
 
-gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const double *box_sizes,
-                         const int64_t *offsets)
+// the checked view onto the device
+gzm_status upload_checked(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const double *box_sizes,
+                          const int64_t *offsets)
 {
-    if (!c || !v) { set_error("NULL argument"); return GZM_ERR_ARG; }
-    if (v->n <= 0 || v->n > (int64_t)0x7fffffff / 16) { set_error("n=%lld out of range", (long long)v->n); return GZM_ERR_ARG; }
-    if (!v->pos || !v->vel || !v->mass || !v->u || !v->hsml) {
-        set_error("pos, vel, mass, u and hsml are required");
-        return GZM_ERR_ARG;
-    }
-    if (n_boxes < 1 || n_boxes > (1 << 20)) { set_error("n_boxes=%d out of range", n_boxes); return GZM_ERR_ARG; }
-    if (offsets[0] != 0 || offsets[n_boxes] != v->n) {
-        set_error("box offsets must start at 0 and end at n=%lld", (long long)v->n);
-        return GZM_ERR_ARG;
-    }
-    for (int b = 0; b < n_boxes; b++) {
-        if (offsets[b + 1] < offsets[b]) { set_error("box offsets must not decrease (box %d)", b); return GZM_ERR_ARG; }
-        for (int ax = 0; ax < 3; ax++) {
-            const double L = box_sizes[3 * (size_t)b + ax];
-            if (!(L > 0) || !isfinite(L)) { set_error("box %d side %d must be > 0", b, ax); return GZM_ERR_ARG; }
-        }
-        // positions must lie inside their box: the grid maps [0, L) to cells
-        for (int64_t i = offsets[b]; i < offsets[b + 1]; i++) {
-            for (int ax = 0; ax < 3; ax++) {
-                const double x = v->pos[3 * i + ax], L = box_sizes[3 * (size_t)b + ax];
-                if (!(x >= 0.0 && x < L)) {
-                    set_error("pos[%lld][%d]=%g outside [0, %g) of box %d", (long long)i, ax, x, L, b);
-                    return GZM_ERR_ARG;
-                }
-            }
-        }
-    }
-    GZM_HIP(hipSetDevice(c->p.device));
     const int n = (int)v->n;
     if (n != c->n) {
         free_particles(c);
@@ -1172,6 +1144,47 @@ gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const 
     c->frec_fresh = false;
     c->hmax_valid = false;
     return GZM_OK;
+}
+
+gzm_status upload_common(gzm_ctx *c, const gzm_host_view *v, int n_boxes, const double *box_sizes,
+                         const int64_t *offsets)
+{
+    if (!c || !v) { set_error("NULL argument"); return GZM_ERR_ARG; }
+    if (v->n <= 0 || v->n > (int64_t)0x7fffffff / 16) { set_error("n=%lld out of range", (long long)v->n); return GZM_ERR_ARG; }
+    if (!v->pos || !v->vel || !v->mass || !v->u || !v->hsml) {
+        set_error("pos, vel, mass, u and hsml are required");
+        return GZM_ERR_ARG;
+    }
+    if (n_boxes < 1 || n_boxes > (1 << 20)) { set_error("n_boxes=%d out of range", n_boxes); return GZM_ERR_ARG; }
+    if (offsets[0] != 0 || offsets[n_boxes] != v->n) {
+        set_error("box offsets must start at 0 and end at n=%lld", (long long)v->n);
+        return GZM_ERR_ARG;
+    }
+    for (int b = 0; b < n_boxes; b++) {
+        if (offsets[b + 1] < offsets[b]) { set_error("box offsets must not decrease (box %d)", b); return GZM_ERR_ARG; }
+        for (int ax = 0; ax < 3; ax++) {
+            const double L = box_sizes[3 * (size_t)b + ax];
+            if (!(L > 0) || !isfinite(L)) { set_error("box %d side %d must be > 0", b, ax); return GZM_ERR_ARG; }
+        }
+        // positions must lie inside their box: the grid maps [0, L) to cells
+        for (int64_t i = offsets[b]; i < offsets[b + 1]; i++) {
+            for (int ax = 0; ax < 3; ax++) {
+                const double x = v->pos[3 * i + ax], L = box_sizes[3 * (size_t)b + ax];
+                if (!(x >= 0.0 && x < L)) {
+                    set_error("pos[%lld][%d]=%g outside [0, %g) of box %d", (long long)i, ax, x, L, b);
+                    return GZM_ERR_ARG;
+                }
+            }
+        }
+    }
+    GZM_HIP(hipSetDevice(c->p.device));
+    const bool same = (int)v->n == c->n;
+    const gzm_status s = upload_checked(c, v, n_boxes, box_sizes, offsets);
+    if (s && !(same && s == GZM_ERR_ARG)) {  // half a particle set is none (grids too large: the old one still whole)
+        (void)hipStreamSynchronize(c->stream);
+        free_particles(c);
+    }
+    return s;
 }
 
 
@@ -1640,11 +1653,9 @@ gzm_status force_impl(gzm_ctx *c, const Plan *gp, gzm_pass_stats *stats)
         }
         if ((!mfv || three_phase) && use_list && c->list_overflow_slices > 0) {
             // particles whose pair set overflowed the list: one wavefront each, FP64
-            if (!c->d_long_list) {
-                s = need(c, &c->d_long_list, (size_t)c->n);
-                s = s ? s : need(c, &c->d_long_count, 1);
-                if (s) return s;
-            }
+            if (!c->d_long_list) s = need(c, &c->d_long_list, (size_t)c->n);
+            if (!s && !c->d_long_count) s = need(c, &c->d_long_count, 1);
+            if (s) return s;
             launch_fill_int(c->stream, c->d_long_count, 1, 0);
             if (mfv) launch_force_mfv_overflow(c->stream, a, m, c->d_long_list, c->d_long_count);
             else launch_force_long_lists(c->stream, a, c->d_long_list, c->d_long_count);

@@ -292,3 +292,39 @@ def contexts_of_threads_share_a_full_card(shim):
     for t in threads:
         t.join(60)
     assert not failures and not any(t.is_alive() for t in threads), failures
+
+
+def failed_allocations_leave_nothing_half_made(shim):
+    """An upload without memory leaves no particles, and a force stage that ran out
+    of it half-way can be called again."""
+    ic = ics.random_state(12)
+    n = ic["mass"].size
+    ref, st = gzm.run_pass(ic, params=gzm.make_params(pair_list_cap=16))
+    with gzm.MFMContext(gzm.make_params(pair_list_cap=16)) as ctx:
+        ctx.upload(ic)
+        shim.set("budget", shim.used)
+        other = ics.random_state(14)
+        for call in (lambda: ctx.upload(other), ctx.density, ctx.hydro_force):
+            try:
+                call()
+                raise AssertionError("a context without particles worked")
+            except gzm.GzmError as e:
+                assert e.status == (3 if call.__name__ == "<lambda>" else 4), e
+        shim.set("budget", 1 << 62)
+        ctx.upload(ic)
+        ctx.density()
+        ctx.gradients()
+        # the counts of the deferred pairs, then their total
+        for unwanted in (4 * n, 4):
+            shim.set("unwanted", unwanted)
+            try:
+                ctx.hydro_force()
+                raise AssertionError("the force stage had what it was refused")
+            except gzm.GzmError as e:
+                assert e.status == 3, e
+        shim.set("unwanted", 0)
+        f = ctx.hydro_force()
+        out = ctx.download()
+    assert f.force_interactions == st["force_interactions"]
+    for k in OUT_KEYS:
+        np.testing.assert_array_equal(out[k], ref[k], err_msg=k)

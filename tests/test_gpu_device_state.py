@@ -47,3 +47,7 @@ def test_idle_contexts_give_their_rows(search):
 
 def test_contexts_of_threads_share_a_full_card():
     hip_shim.run("contexts_of_threads_share_a_full_card")
+
+
+def test_failed_allocations_leave_nothing_half_made():
+    hip_shim.run("failed_allocations_leave_nothing_half_made")
