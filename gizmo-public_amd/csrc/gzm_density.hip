@@ -36,7 +36,7 @@ namespace {
 constexpr int kTailLanes = 16;
 constexpr int kFarWaves = 4;
 constexpr int kNoRow = kDensityCacheCap + 1;
-constexpr int kWideRow = kNoRow + 1;  // row_n where the walk for the row passed twice the candidate budget
+constexpr int kWideRow = kNoRow + 1;  // row_n where the walk for the row passed its candidate budgets
 // iter of a particle whose iteration has ended; beside the sweeps done, of one that is in
 // the tail list
 constexpr int kDone = -1, kListed = 1 << 30;
@@ -239,16 +239,16 @@ template <int G>
 constexpr int kRowLds = G == 1 ? kListChunk * kBlock : kColumnHits * kBlock;
 template <int G>
 __device__ __forceinline__ int grid_row(const DensityStageArgs &a, const BoxDesc &B, int i, const double4 &pi, double h,
-                                        int sub, int *lds)
+                                        int sub, int *lds, int budgets = 2)
 {
     int *stage = wave_chunk(lds), *kept = lds;
     const double Rc = kDensityCacheFactorGrid * h;
     const double xs[3] = {pi.x, pi.y, pi.z};
     constexpr int cap = kDensityCacheCap;
     int *row = a.row_idx + (size_t)i * cap;
-    // a row past its cap is of no use, so its walk ends there; the budget
-    // bounds the walk where cells hold many more particles than neighbours
-    const int limit = a.budget ? 2 * a.budget : 0x7fffffff;
+    // a row past its cap is of no use, so its walk ends there; a number of candidate
+    // budgets bounds the walk where cells hold many more particles than neighbours
+    const int limit = a.budget ? budgets * a.budget : 0x7fffffff;
     int m = 0, visited = 0;
     auto append = [&](int j, bool in) {
         if constexpr (G == 1) {
@@ -541,9 +541,9 @@ __device__ __forceinline__ int walk_sweep(const DensityStageArgs &a, const BoxDe
 // Tree: a particle whose hsml leaves its row goes to the walk list.  Grid (GRID):
 // its row is built anew around the hsml reached, and where that is past the cap (a
 // guess far above) or the memory holds no rows, the sweep walks; a walk past the
-// candidate budget is done by a wavefront.  Where already the walk for a row passed two
-// budgets (cells far wider than hsml, in clumps) or has many cells to pass (far smaller
-// ones, between clumps) the far list takes the particle: such walks come thousands to a
+// candidate budget is done by a wavefront.  Where already the walk for a row passed the
+// budget (cells far wider than hsml, in clumps) or has many cells to pass (far smaller
+// ones, between clumps) the tail list takes the particle: such walks come thousands to a
 // stretch and have to spread over the chip.  With the 16 lanes of the tail walking for
 // them, sweep by sweep, the density stage of a 128^3 lattice whose hsml starts 20 %
 // low took 35.3 ms, 50 % high 89.6; now 6.7 and 38.0 (a launch per sweep with a lane
@@ -608,7 +608,7 @@ __global__ __launch_bounds__(kBlock, 2) void density_more_kernel(DensityStageArg
                 if (GRID) {
                     const bool wanted = a.row_idx && row_wanted(n_row, a.row_r2[i], s.h);
                     if ((wanted || n_row > kDensityCacheCap) && many_cells(B.grid, s.h)) n_row = kWideRow;
-                    else if (wanted) n_row = grid_row<G>(a, B, i, pi, s.h, sub, lds);
+                    else if (wanted) n_row = grid_row<G>(a, B, i, pi, s.h, sub, lds, 1);
                 }
                 if (!GRID || n_row <= kDensityCacheCap)
                     again = row_sweep<MFV, G>(a, B, i, pi, n_row, sub, chunk, s, cnt);
@@ -617,7 +617,7 @@ __global__ __launch_bounds__(kBlock, 2) void density_more_kernel(DensityStageArg
                 if (sub != 0) return;
                 if (again < 0) {
                     wide = n_row != kWideRow;
-                    if (!wide) a.far_list[atomicAdd(a.n_far, 1)] = i;
+                    if (!wide) a.tail_list[atomicAdd(a.n_tail, 1)] = i;
                     return;
                 }
                 sweeps++;
