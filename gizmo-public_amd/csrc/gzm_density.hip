@@ -652,9 +652,9 @@ __global__ __launch_bounds__(kBlock, 2) void density_more_kernel(DensityStageArg
 
 // The listed particles, W lanes each, iterating to convergence: over the
 // particle's row while hsml stays inside it (grid: a row built anew once it leaves
-// it), else over a walk shared by the lanes.  A walk past the candidate budget (BUDGET) leaves the particle to the
-// far list, and any walk (kRowsOnly) to the walk list.  A fixed grid strides over
-// the device-side count.
+// it), else over a walk shared by the lanes.  A walk past the candidate budget (BUDGET)
+// leaves the particle to the far list, and any walk (kRowsOnly) to the walk list.  A
+// fixed grid strides over the device-side count.
 enum DensityWalk { kGridWalk, kTreeWalk, kRowsOnly };
 template <bool MFV, int W, bool BUDGET, DensityWalk WALK, int WAVES = 1>
 __device__ __forceinline__ void density_iterate(const DensityStageArgs &a, const int *list, const int *count,

@@ -155,8 +155,8 @@ struct ExportArgs {
     unsigned first_block[kMaxExport + 1];
 };
 
-// candidates a density-sweep lane walks before it defers its particle to the
-// second, load-balanced launch (gzm_params.density_budget = 0)
+// candidates that a walk of the density stage tests before it leaves its particle to
+// more lanes (gzm_params.density_budget = 0); precision 2: to the wavefront launch
 constexpr int kDensityBudget = 512;
 
 // Candidate rows of the FP64 density sums: the particles (of mass > 0) within

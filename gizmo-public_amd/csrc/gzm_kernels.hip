@@ -1,12 +1,13 @@
 // gzm_kernels.hip -- HIP kernels of the MFM hydro pass for gfx950 (FP64).
 //
-// One thread per active particle i ("gather form"): the thread walks the
-// cells of the grid that can hold neighbours, evaluates every pair (i, j) for
-// its own particle only, and finishes the per-particle work (hsml update,
-// gradient construction + limiter, flux sums -> dv/dt, du/dt) in registers.
-// Consecutive threads hold consecutive particles of the Morton-sorted order,
-// so the lanes of a wavefront walk almost the same cells and their neighbour
-// loads hit the same cache lines.
+// "Gather form": one lane or a small group of lanes per active particle i
+// evaluates every pair (i, j) for its own particle only -- from the candidate
+// rows of the density stage (gzm_density.hip) or the pair list where they hold
+// the set, else over a walk of the grid or tree -- and finishes the particle's
+// work (gradient construction + limiter, flux sums -> dv/dt, du/dt).
+// Consecutive lanes hold consecutive particles of the Morton-sorted order, so
+// those of a wavefront meet almost the same neighbours and their loads hit the
+// same cache lines.
 //
 // No pair writes to j (the reference disables its pair-symmetric writes too,
 // hydro_evaluate.h:159-168, gradients.c:1554-1565), so every kernel is free of

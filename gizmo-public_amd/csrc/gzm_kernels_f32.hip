@@ -1,7 +1,7 @@
 // gzm_kernels_f32.hip -- FP32-bulk kernels of the MFM hydro pass (gfx950).
 //
-// Same loops as gzm_kernels.hip (one thread per active particle, gather
-// form), with the per-pair arithmetic in FP32:
+// Same loops as gzm_kernels.hip (gather form; the list force loop gives a
+// particle eight lanes, the others one), with the per-pair arithmetic in FP32:
 //   * geometry: FP32 offsets from FP64 cell origins plus exact integer cell
 //     differences (the F32Geom layout in gzm_internal.h);
 //   * neighbour predicates: decided on the FP32 r^2 unless it lies within a

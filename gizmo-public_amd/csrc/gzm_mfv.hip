@@ -3,8 +3,8 @@
 //
 // The density iteration (which also sums the smoothed mesh velocity,
 // density_pair<.., MFV>), the gradients and the pair list are those of the
-// MFM pass.  The force loop keeps its gather form (one thread per active
-// particle, its flux sums in registers) with one scatter: the reference gives
+// MFM pass.  The force loop keeps its gather form (eight lanes per particle
+// over the pair list, one over a walk) with one scatter: the reference gives
 // each neighbour its share of the exchanged mass (SphP[j].dMass -= ...,
 // hydro_evaluate.h:384-392, under `omp atomic` there), an FP64 atomic add here.
 // dMass is therefore summed in a run-dependent order; every other output is

@@ -82,14 +82,15 @@ typedef struct gzm_params {
                                Morton-sorted particles with per-node hsml maxima, for
                                strongly clustered sets */
     int32_t density_budget; /* candidates a density walk tests before its particle
-                               is deferred to a launch that gives it a wavefront
+                               is deferred to a launch that gives it more lanes
                                (load balance where a few hsml jump far in one iteration):
-                               0 = default (512), < 0 = no limit; results do not depend
-                               on it */
+                               0 = default (512), < 0 = no limit.  It decides how many
+                               lanes share a particle's sums, which then run in another
+                               order, within the parity bar */
     int32_t block_size[3];  /* threads per workgroup of the per-particle loop kernels of
                                [0] the density sweeps of precision 2, [1] the gradient loop, [2] the force
                                loop: 64, 128, 256 or 512 (the force loop's grid-scanning
-                               fallbacks stay at 256, its FP64 list loop at 64); 0 = 256.
+                               fallbacks and FP64 list loop have sizes of their own); 0 = 256.
                                Results do not depend on it */
     int32_t wave_sweep_max; /* precision 2: a density sweep over at most this many particles gives each
                                one a wavefront whose lanes share its walk: 0 = default
@@ -204,7 +205,9 @@ gzm_status gzm_upload(gzm_ctx *ctx, const gzm_host_view *view);
  * holds the caller rows [box_offsets[b], box_offsets[b+1]) of `view` and has
  * side lengths box_sizes[3b..3b+2]; gzm_params.box is not used.  Every stage
  * call then runs over all boxes at once, each particle seeing only its own
- * box, with the results of running each box alone. */
+ * box: the neighbour sets and results of running each box alone (a particle's
+ * sums may run in another order, since a small set gives it more lanes; within
+ * the parity bar). */
 gzm_status gzm_upload_batch(gzm_ctx *ctx, const gzm_host_view *view, int32_t n_boxes, const double *box_sizes,
                             const int64_t *box_offsets);
 
@@ -237,9 +240,9 @@ gzm_status gzm_restore_initial_state(gzm_ctx *ctx);
  * cannot decide on the host (number of density sweeps, pair-list overflow);
  * the graph replays the same input, so every pass repeats the probe's
  * decisions; should one meet more than the probe did, the call ends with
- * GZM_ERR_STATE, its outputs incomplete.  stats hold the sums over the n_passes passes (density_sweeps:
- * per pass); gzm_timing's graph fields hold the graph's device time.  The
- * outputs left on the device are those of the last pass.  No counterpart in
+ * GZM_ERR_STATE, its outputs incomplete.  stats hold the sums over the
+ * n_passes passes (density_sweeps: per pass); gzm_timing's graph fields hold
+ * the graph's device time.  The outputs left on the device are those of the last pass.  No counterpart in
  * the reference: for callers that repeat passes without host round trips. */
 gzm_status gzm_run_passes(gzm_ctx *ctx, int32_t n_passes, gzm_pass_stats *stats);
 
